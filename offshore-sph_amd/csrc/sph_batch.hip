@@ -641,7 +641,7 @@ int b_pair_pec(sph_batch *b, hipStream_t s) {
     State st = b->buf[b->cur];
     PairIn in{b->recA, b->recB, st.h, b->cxy_s, b->cellStart};
     PairOut out{st.ax, st.ay, st.drho, nullptr, 0};
-    const PecArgs pec{st, b->buf[1 - b->cur], b->perm, b->part_d, HmConst{}, 0, &b->view->pec_parts};
+    const PecArgs pec{st, b->buf[1 - b->cur], b->perm, b->part_d, nullptr, HmConst{}, 0, &b->view->pec_parts};
     hipError_t e = b->precision == SPH_PREC_FP32C
                        ? launch_pair_batch_fp32u_pec(b->inst, b->ts, b->tileInst, b->NT, in, out, b->uniK, b->kernel,
                                                      b->n, pec, s)

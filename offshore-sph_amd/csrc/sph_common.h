@@ -109,6 +109,15 @@ __device__ inline void block_partials(double (&v)[NQ], const int (&kind)[NQ], do
     }
 }
 
+// Doubles as unsigned integers of the same order (no NaN), and back.
+__device__ inline unsigned long long order_key(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x + 0.0);  // -0.0 as 0.0
+    return b ^ ((b >> 63) ? ~0ull : 0x8000000000000000ull);
+}
+__device__ inline double order_value(unsigned long long k) {
+    return __longlong_as_double((long long)(k ^ ((k >> 63) ? 0x8000000000000000ull : ~0ull)));
+}
+
 // src/Integrators/PEC.py:32-59 (useXSPH = False branch), one particle. The
 // fused step evaluates the same expressions inside the neighbour update.
 __device__ inline double pec_half_pos(double x, double v, double dt) { return x + 0.5 * dt * v; }
@@ -184,6 +193,18 @@ struct DtVars {
         block_partials<kDtQ>(v, kind, lds, part, R, k);
     }
     __device__ void publish(double *part, double *lds) { store(part, gridDim.x, blockIdx.x, lds); }
+    // into the dt slots (one h for every particle: min h is not folded).
+    // |a|^2 >= 0 orders as its bits. lds holds 3 * 16 doubles.
+    __device__ void publish_slots(unsigned long long *d, double *lds) {
+        const int kind[3] = {1, 2, 2};
+        double v[3] = {mx, cnt, bad};
+        block_fold<3>(v, kind, lds);
+        if (threadIdx.x == 0 && v[1] > 0.0) {
+            unsigned long long *p = d + (size_t)(blockIdx.x % kDtSlotCount) * kDtStride;
+            if (v[0] >= 0.0) atomicMax(p, (unsigned long long)__double_as_longlong(v[0]));
+            atomicOr(p + 1, kDtAny | (v[2] > 0.0 ? kDtBad : 0ull));
+        }
+    }
 };
 __device__ inline double pec_half_rho(double rho, double drho, double dt, int strict) {
     double r = rho + 0.5 * dt * drho;
@@ -276,6 +297,105 @@ __global__ void k_scan_apply(const Ctrl *ctrl, int *counts, const int *tileSums,
         }
         if (tile == ntiles - 1 && threadIdx.x == blockDim.x - 1) cellStart[nbins] = ex;
     }
+}
+
+// The scan in one kernel of kScanBlocks workgroups, for a state small enough
+// that a launch costs more than reading counts again: workgroup i sums every
+// count before its share itself (nbins / 2 counts on average, from L2; 25k
+// bins of a 50k-particle tank: 3 loads of 16 bytes per thread), then scans its
+// share. counts is cleared by the next kernel (k_place): other workgroups
+// still read it here.
+constexpr int kScanBlocks = 64, kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, const int *counts, int *cellStart) {
+    if (!ctrl->active) return;
+    const long long nbins = ctrl->grid.ncells + 1;
+    __shared__ int lds[16];
+    const long long share = ((nbins + gridDim.x - 1) / gridDim.x + 3) / 4 * 4;
+    const long long b0 = blockIdx.x * share;
+    if (b0 >= nbins) return;
+    const long long b1 = b0 + share < nbins ? b0 + share : nbins;
+    int pre = 0;
+    constexpr int U = 8;  // loads in flight per thread
+    const long long step = 4 * (long long)blockDim.x;
+    for (long long j = 4 * (long long)threadIdx.x; j < b0; j += U * step) {  // b0 is a multiple of 4
+        int4 c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            c[u] = j + u * step < b0 ? *reinterpret_cast<const int4 *>(counts + j + u * step) : make_int4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) pre += c[u].x + c[u].y + c[u].z + c[u].w;
+    }
+    int run, tot;
+    block_scan_excl(pre, lds, &run);  // run: the sum before the share
+    for (long long b = b0; b < b1; b += blockDim.x) {
+        const long long k = b + threadIdx.x;
+        const int v = k < b1 ? counts[k] : 0;
+        const int ex = block_scan_excl(v, lds, &tot) + run;
+        if (k < b1) cellStart[k] = ex;
+        run += tot;
+    }
+    if (b1 == nbins && threadIdx.x == 0) cellStart[nbins] = run;
+}
+
+// Each particle's place from its bin's offset and its rank there: perm0 maps
+// places to slots. Inside a bin the order is that of the ranks' atomics;
+// bin_place orders it. clear (after k_scan_one): also zeroes the counts for
+// the next update. The bounds slots, folded by now, are cleared for the next
+// update too, active or not (a halted step's k_bounds may have filled them).
+__global__ void k_place(const Ctrl *ctrl, const int *cellStart, const int *bin, const int *rank, int *perm0, int n,
+                        int *clear, unsigned long long *bslots) {
+    if (blockIdx.x == 0 && threadIdx.x < kBoundsSlots * kBoundsStride) bslots[threadIdx.x] = 0;
+    if (!ctrl->active) return;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (clear) {
+        const long long nbins = ctrl->grid.ncells + 1;
+        for (long long b = t; b < nbins; b += (long long)gridDim.x * blockDim.x) clear[b] = 0;
+    }
+    if (t < n) perm0[cellStart[bin[t]] + rank[t]] = t;
+}
+
+// The place of the particle that k_place put at t, with its bin in order of
+// the reference index (what the reference's head-inserted lists are ordered
+// by, descending there; the pair pass walks the bin backwards): the bin's
+// start plus the number of smaller indices in it. Only a bin filled by more
+// than one run of k_keys (binflag[b] holds this update's epoch) can be out
+// of order. The places of a bin are consecutive, so its indices are mostly in
+// other lanes of the wavefront and are compared there; a bin that crosses
+// into the next wavefront reads them through perm0. (A kernel of its own for
+// the flagged bins took 8.9 us on the 1M dam break and its permuted indices
+// 1.4 us in the scatter; here the reorder takes 39.9 us instead of 34.0.)
+// Called by every thread with t < n of a wavefront of consecutive t together (my: its particle's
+// index).
+__device__ inline int bin_place(int t, int my, long long b, const int *cellStart, const int *binflag, int epoch,
+                                const int *perm0, const int *id) {
+    const int lane = threadIdx.x & 63, t0 = t - lane;
+    const bool flagged = binflag[b] == epoch;
+    int s = t, e = t;
+    if (flagged) {
+        s = cellStart[b];
+        e = cellStart[b + 1];
+    }
+    const bool inside = s >= t0 && e <= t0 + 64;
+    const int len = flagged && inside ? e - s : 0;
+    int r = 0;
+    for (int j = 0; __ballot(j < len) != 0; ++j) {  // every lane takes part in every exchange
+        const int other = __shfl(my, (s - t0 + j) & 63, 64);
+        r += j < len && other < my;
+    }
+    if (!flagged) return t;
+    if (inside) return s + r;
+    int j = s;
+    for (; j + 4 <= e; j += 4) {
+        int q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = perm0[j + u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = id[q[u]];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) r += q[u] < my;
+    }
+    for (; j < e; ++j) r += id[perm0[j]] < my;
+    return s + r;
 }
 
 __global__ void k_scatter(const Ctrl *ctrl, const int *cellStart, const int *bin, const int *rank, const int *id,

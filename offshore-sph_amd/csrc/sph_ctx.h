@@ -16,7 +16,9 @@ struct sph_ctx {
     int cur = 0;
     hipsph::Ctrl *ctrl = nullptr;
     double *dt_hist = nullptr;
-    int *bin = nullptr, *rank = nullptr, *perm = nullptr, *permKey = nullptr;
+    // perm0: the source slot of each place before the bins are ordered; perm: after
+    int *bin = nullptr, *rank = nullptr, *perm0 = nullptr, *perm = nullptr;
+    unsigned long long *slots = nullptr;  // reduction slots (Slots)
     int2 *cxy_s = nullptr;  // raw cell (cx, cy) of each slot in cell order
     int *counts = nullptr, *cellStart = nullptr, *tileSums = nullptr, *binflag = nullptr;
     double *part_b = nullptr, *part_d = nullptr;  // per-workgroup partials: bounds, dt

@@ -76,13 +76,13 @@ __global__ void k_dt_partial(Ctrl *ctrl, const int8_t *label, const double *h, c
 }
 
 // Solver._minTimeStep (src/Solver.py:210-230): courant (TimeStep.py:47-49),
-// force (:51-56), min(c, f) (:45), from the partials of the fluid reduction
-// (ctrl->dt_parts of them, as the kernel that wrote them recorded). Also opens the step: the reference's loop condition
-// `while self.t < self.duration` (src/Solver.py:366) and `self.t += self.dt`
-// (:409) move here, so a captured step needs no host. It also bounds how far
+// force (:51-56), min(c, f) (:45), from the folded fluid reduction v. Also
+// opens the step: the reference's loop condition `while self.t <
+// self.duration` (src/Solver.py:366) and `self.t += self.dt` (:409) move
+// here, so a step needs no host. It also bounds how far
 // this step's predictor puts any particle from where the last update binned
-// it (ctrl->disp, for k_bounds): after the fused PEC pass of the last step
-// (ctrl->pec_parts; dt0 its dt, V = ctrl->vbound its velocity bound at the
+// it (disp, for the border-cell bounds): after the fused PEC pass of the last
+// step (ctrl->pec_parts; dt0 its dt, V = ctrl->vbound its velocity bound at the
 // start, A0 = ctrl->abound its predictor's rates, A1 this fold's), a fluid
 // particle binned at x + dt0 v / 2 was corrected to x + dt0 vh, with |vh| <=
 // V + dt0 A0 / 2 (damping only shrinks it), and its new velocity v' has
@@ -90,22 +90,116 @@ __global__ void k_dt_partial(Ctrl *ctrl, const int8_t *label, const double *h, c
 // dt0 V / 2 of where it was binned and this step's predictor moves it dt |v'|
 // / 2 further; V + dt0 A1 bounds the next step's start. Anything else (other
 // partials, non-finite rates, a halted step, a second call on the same
-// partials) leaves +inf: the next update scans every particle. One workgroup.
-__global__ void k_dt_final(Ctrl *ctrl, double gamma_c, double gamma_f, double *hist, const double *part) {
-    __shared__ double lds[kDtQ * 16];
-    const int R = ctrl->dt_parts;
-    // control fields are loaded with the partials (used after the fold)
-    unsigned flags = ctrl->flags;
-    const double t0 = ctrl->t, duration = ctrl->duration, fixed_dt = ctrl->fixed_dt, co = ctrl->co;
-    const long long step = ctrl->step;
-    const int advance_t = ctrl->advance_t;
+// partials) leaves +inf: the next update scans every particle. Reads the
+// control block and changes nothing (dt_commit does).
+struct DtIn {  // the control fields of the decision, loaded before the fold
+    double t, dt, dt_c, dt_f, duration, fixed_dt, co, V, A0;
+    long long step;
+    unsigned flags;
+    int advance_t, pec;
+    __device__ explicit DtIn(const Ctrl *c)
+        : t(c->t), dt(c->dt), dt_c(c->dt_c), dt_f(c->dt_f), duration(c->duration), fixed_dt(c->fixed_dt), co(c->co),
+          V(c->vbound), A0(c->abound), step(c->step), flags(c->flags), advance_t(c->advance_t), pec(c->pec_parts) {}
+};
+__device__ inline DtNext dt_decide(const DtIn &in, const double *v, double gamma_c, double gamma_f) {
+    DtNext x;
+    x.t = in.t;
+    x.dt = in.dt;
+    x.dt_c = in.dt_c;
+    x.dt_f = in.dt_f;
+    x.step = in.step;
+    x.disp = x.vbound = x.abound = INFINITY;
+    x.flags = 0;
+    x.active = 0;
+    const double mn = v[0], mx = v[1], cnt = v[2], bad = v[3];
+    const unsigned halt = SPH_FLAG_CAPACITY | SPH_FLAG_NONFINITE | SPH_FLAG_NO_FLUID | SPH_FLAG_ZERO_DENSITY;
+    if ((in.flags & halt) || !(x.t < in.duration)) return x;
+    if (cnt == 0) {
+        x.flags = SPH_FLAG_NO_FLUID;
+        return x;
+    }
+    if (bad != 0) x.flags |= SPH_FLAG_NONFINITE;
+    double dt, c, f;
+    if (in.fixed_dt > 0.0) {
+        dt = in.fixed_dt;  // src/Solver.py:370-372
+        c = 0.0;
+        f = 0.0;
+    } else {
+        const double max_c = in.co;  // c = co for every fluid particle (WCSPH.py:110-129)
+        c = gamma_c * mn / max_c;
+        f = (mx < 1e-12) ? 1e10 : gamma_f * sqrt(mn / mx);
+        dt = (f < c) ? f : c;
+        if (dt < 1e-6) x.flags |= SPH_FLAG_DT_SMALL;  // src/Solver.py:220-224
+    }
+    const double dt0 = x.dt;
+    x.dt = dt;
+    x.dt_c = c;
+    x.dt_f = f;
+    if (in.advance_t) x.t = x.t + dt;
+    x.step = x.step + 1;
+    x.active = 1;
+    if (bad == 0) {
+        const double A1 = sqrt(mx);
+        x.abound = A1;
+        if (in.pec) {
+            const double V1 = in.V + dt0 * A1;
+            const double d = dt0 * (in.V + 0.5 * dt0 * in.A0) + 0.5 * dt0 * in.V + 0.5 * dt * V1;
+            if (d == d) x.disp = d;  // NaN: +inf
+            x.vbound = V1;
+        }
+    }
+    return x;
+}
+
+// The decision takes effect: clock, dt, bounds, flags and the dt series.
+__device__ inline void dt_commit(Ctrl *ctrl, const DtNext &x, double *hist) {
+    ctrl->pec_parts = 0;  // these partials are used once
+    ctrl->disp = x.disp;
+    ctrl->vbound = x.vbound;
+    ctrl->abound = x.abound;
+    if (x.flags) atomicOr(&ctrl->flags, x.flags);
+    ctrl->active = x.active;
+    if (!x.active) return;
+    const long long k = (x.step - 1) % SPH_DT_HISTORY;
+    hist[3 * k + 0] = x.dt;
+    hist[3 * k + 1] = x.dt_c;
+    hist[3 * k + 2] = x.dt_f;
+    ctrl->dt = x.dt;
+    ctrl->dt_c = x.dt_c;
+    ctrl->dt_f = x.dt_f;
+    ctrl->t = x.t;
+    ctrl->step = x.step;
+}
+
+// One workgroup's fold of the dt partials: R of them (k_dt_partial,
+// k_correct), or the dt slots of the fused pair pass (R = kDtSlots), whose
+// state has one h. The result is valid in thread 0; lds holds kDtQ * 16
+// doubles.
+__device__ inline void dt_fold(int R, const double *part, const unsigned long long *dslots, double h1, double (&v)[kDtQ],
+                               double *lds) {
     const int kind[kDtQ] = {0, 1, 2, 2};
-    double v[kDtQ] = {INFINITY, -INFINITY, 0.0, 0.0};
-    // eight partials per thread per round, their loads issued together (the
-    // fused pair pass leaves one per workgroup: ~5,000 at 1M particles, one
-    // round; four per round: 6.64 against 6.38 us; 512 threads in two
-    // rounds 6.85, 256 threads with sixteen per round 12.0)
-    constexpr int U = 8;
+    v[0] = INFINITY;
+    v[1] = -INFINITY;
+    v[2] = v[3] = 0.0;
+    const unsigned long long *p = dslots + (size_t)(threadIdx.x % kDtSlotCount) * kDtStride;
+    unsigned long long a = p[0], f = p[1];  // in flight together with R
+    if (R == kDtSlots) {
+        if (threadIdx.x < kDtSlotCount) {  // one wavefront
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long a2 = __shfl_xor(a, o, 64);
+                a = a2 > a ? a2 : a;
+                f |= __shfl_xor(f, o, 64);
+            }
+            v[0] = h1;
+            v[1] = __longlong_as_double((long long)a);
+            v[2] = f & kDtAny ? 1.0 : 0.0;
+            v[3] = f & kDtBad ? 1.0 : 0.0;
+        }
+        return;
+    }
+    // four partials per thread per round, their loads issued together
+    constexpr int U = 4;
     for (int k0 = threadIdx.x; k0 < R; k0 += U * blockDim.x) {
         double u[U][kDtQ];
 #pragma unroll
@@ -123,58 +217,17 @@ __global__ void k_dt_final(Ctrl *ctrl, double gamma_c, double gamma_f, double *h
         }
     }
     block_fold<kDtQ>(v, kind, lds);
-    if (threadIdx.x != 0) return;
-    const int pec = ctrl->pec_parts;
-    const double dt0 = ctrl->dt, V = ctrl->vbound, A0 = ctrl->abound;
-    ctrl->pec_parts = 0;  // these partials are used once
-    ctrl->disp = INFINITY;
-    ctrl->vbound = INFINITY;
-    ctrl->abound = INFINITY;
-    const double mn = v[0], mx = v[1], cnt = v[2], bad = v[3];
-    const unsigned halt = SPH_FLAG_CAPACITY | SPH_FLAG_NONFINITE | SPH_FLAG_NO_FLUID | SPH_FLAG_ZERO_DENSITY;
-    if ((flags & halt) || !(t0 < duration)) {
-        ctrl->active = 0;
-        return;
-    }
-    if (cnt == 0) {
-        ctrl->flags = flags | SPH_FLAG_NO_FLUID;
-        ctrl->active = 0;
-        return;
-    }
-    if (bad != 0) flags |= SPH_FLAG_NONFINITE;
-    double dt, c, f;
-    if (fixed_dt > 0.0) {
-        dt = fixed_dt;  // src/Solver.py:370-372
-        c = 0.0;
-        f = 0.0;
-    } else {
-        const double max_c = co;  // c = co for every fluid particle (WCSPH.py:110-129)
-        c = gamma_c * mn / max_c;
-        f = (mx < 1e-12) ? 1e10 : gamma_f * sqrt(mn / mx);
-        dt = (f < c) ? f : c;
-        if (dt < 1e-6) flags |= SPH_FLAG_DT_SMALL;  // src/Solver.py:220-224
-    }
-    const long long k = step % SPH_DT_HISTORY;
-    hist[3 * k + 0] = dt;
-    hist[3 * k + 1] = c;
-    hist[3 * k + 2] = f;
-    ctrl->flags = flags;
-    ctrl->dt = dt;
-    ctrl->dt_c = c;
-    ctrl->dt_f = f;
-    if (advance_t) ctrl->t = t0 + dt;
-    ctrl->step = step + 1;
-    ctrl->active = 1;
-    if (bad == 0) {
-        const double A1 = sqrt(mx);
-        ctrl->abound = A1;
-        if (pec) {
-            const double V1 = V + dt0 * A1;
-            const double d = dt0 * (V + 0.5 * dt0 * A0) + 0.5 * dt0 * V + 0.5 * dt * V1;
-            if (d == d) ctrl->disp = d;  // NaN: +inf
-            ctrl->vbound = V1;
-        }
-    }
+}
+
+// sph_dt: the fold and its decision by themselves (a step folds them in
+// k_bounds). One workgroup.
+__global__ void k_dt_final(Ctrl *ctrl, double gamma_c, double gamma_f, double *hist, const double *part,
+                           const unsigned long long *dslots, double h1) {
+    __shared__ double lds[kDtQ * 16];
+    double v[kDtQ];
+    const DtIn in(ctrl);
+    dt_fold(ctrl->dt_parts, part, dslots, h1, v, lds);
+    if (threadIdx.x == 0) dt_commit(ctrl, dt_decide(in, v, gamma_c, gamma_f), hist);
 }
 
 // KineticEnergy (src/Equations/KineticEnergy.py:5-12) over the fluid:
@@ -322,7 +375,7 @@ __device__ inline void upd_pos(const Ctrl *ctrl, const State &a, int i, int pred
 // Whether this update's bounds can come from the border cells alone (the
 // fused PEC step's update, with one h): the state is in the cell order of
 // the grid it was last binned on (ctrl->grid, the offsets in cellStart) and
-// no particle's predicted position lies more than ctrl->disp from where it
+// no particle's predicted position lies more than disp from where it
 // was binned, per axis, with 2 disp under the cell size by a margin far
 // above the rounding of the positions and of the cell arithmetic. Then the
 // particle binned at the old minimum x (column 0) is now at most disp to its
@@ -331,13 +384,29 @@ __device__ inline void upd_pos(const Ctrl *ctrl, const State &a, int i, int pred
 // binned at the old maximum x lies beyond ncx - 1 cells and one of a column
 // <= ncx - 3 within ncx - 2, so the maximum lies in columns ncx - 2 or
 // ncx - 1; y likewise with rows 0, ncy - 2 and ncy - 1.
-__device__ inline bool border_bounds_ok(const Ctrl *ctrl, const int *cellStart, int pred, const HmConst &hc) {
+__device__ inline bool border_bounds_ok(const Ctrl *ctrl, const int *cellStart, int pred, const HmConst &hc,
+                                        double disp) {
     if (!cellStart || pred != 1 || !hc.on || ctrl->nm || !ctrl->nn_valid) return false;
-    return border_margin_ok(ctrl->grid, ctrl->disp);
+    return border_margin_ok(ctrl->grid, disp);
 }
 
+// What k_bounds takes to fold the dt partials itself (a step's update);
+// on = 0: the control block's dt stands (sph_nn_update).
+struct DtFold {
+    int on;
+    double gamma_c, gamma_f, h1;  // h1: the one h of a state whose partials are in the dt slots
+    double *hist;
+    const double *part;
+    const unsigned long long *dslots;
+};
+
 // _init :86-101 bounds and _get_cell_size :103-110 min h, over all active
-// particles: per-workgroup partials, folded by k_grid. Grid-stride over at
+// particles, into the bounds slots (folded by k_keys). In a step every
+// workgroup first folds the dt partials (64 slots, or up to 2,048 partials
+// after k_correct) and decides dt for itself, since the predicted positions
+// need it; the first leaves the decision in ctrl->nx. That fold costs the
+// kernel 1.6 us (5k particles) to 2 us (1M) and saves a single-workgroup
+// kernel of 4.6 to 6.6 us and its launch. Grid-stride over at
 // most kBoundsBlocks workgroups, four particles per thread per round with
 // their loads issued together (one workgroup per 256 particles measured 40 %
 // slower, the per-workgroup fold paid in more rounds; 2048 workgroups with
@@ -345,18 +414,41 @@ __device__ inline bool border_bounds_ok(const Ctrl *ctrl, const int *cellStart, 
 // and border_bounds_ok, only the particles of the border cells
 // (border_walk), over the first kBorderBlocks workgroups. The extremes are
 // the same values the full scan finds. With PEC's
-// predictor the full scan also finds the largest |vx|, |vy| (k_grid keeps it
+// predictor the full scan also finds the largest |vx|, |vy| (k_keys keeps it
 // as ctrl->vbound; +inf if one is not finite).
 constexpr int kBoundsBlocks = 1024;
 // workgroups that walk the border cells (one per CU: 8.4 us on the 1M dam
 // break, against 9.6 with all 1,024 and 10.1 with 64)
 constexpr int kBorderBlocks = 256;
-__global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, double *part, HmConst hc, const int *cellStart) {
-    if (!ctrl->active) return;
+__global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const int *cellStart, DtFold D,
+                         unsigned long long *bslots) {
     __shared__ double lds[kBoundsVQ * 16];
+    __shared__ double s_dt, s_disp;
+    __shared__ int s_active;
+    double dt, disp;
+    if (D.on) {
+        double v[kDtQ];
+        const DtIn in(ctrl);
+        dt_fold(ctrl->dt_parts, D.part, D.dslots, D.h1, v, lds);
+        if (threadIdx.x == 0) {
+            const DtNext x = dt_decide(in, v, D.gamma_c, D.gamma_f);
+            s_dt = x.dt;
+            s_disp = x.disp;
+            s_active = x.active;
+            if (blockIdx.x == 0) ctrl->nx = x;
+        }
+        __syncthreads();
+        if (!s_active) return;
+        dt = s_dt;
+        disp = s_disp;
+    } else {
+        if (!ctrl->active) return;
+        dt = ctrl->dt;
+        disp = ctrl->disp;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->epoch += 1;
     double xmn = INFINITY, xmx = -INFINITY, ymn = INFINITY, ymx = -INFINITY, hmn = INFINITY, hmx = -INFINITY;
     double bad = 0.0, vmx = -INFINITY;
-    const double dt = ctrl->dt;
     auto take = [&](int i) {
         double xi, yi;
         upd_pos(ctrl, a, i, pred, dt, xi, yi);
@@ -371,15 +463,8 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, double *part, HmC
     };
     const int stride = gridDim.x * blockDim.x;
     const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-    if (border_bounds_ok(ctrl, cellStart, pred, hc)) {
-        if (blockIdx.x >= kBorderBlocks) {  // the rest store empty partials
-            if (threadIdx.x == 0) {
-                const double e[kBoundsVQ] = {INFINITY, -INFINITY, INFINITY, -INFINITY, hc.h, hc.h, 0.0, -INFINITY};
-#pragma unroll
-                for (int q = 0; q < kBoundsVQ; ++q) part[q * gridDim.x + blockIdx.x] = e[q];
-            }
-            return;
-        }
+    if (border_bounds_ok(ctrl, cellStart, pred, hc, disp)) {
+        if (blockIdx.x >= kBorderBlocks) return;
         const int fstride = (kBorderBlocks < (int)gridDim.x ? kBorderBlocks : (int)gridDim.x) * blockDim.x;
         if (gt == 0) ctrl->border_updates += 1;
         hmn = hmx = hc.h;  // every particle's h
@@ -402,15 +487,22 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, double *part, HmC
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
     double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
-    block_partials<kBoundsVQ>(v, kind, lds, part, gridDim.x, blockIdx.x);
+    __syncthreads();  // lds held the dt fold
+    block_fold<kBoundsVQ>(v, kind, lds);
+    if (threadIdx.x == 0) {
+        unsigned long long *p = bslots + (size_t)(blockIdx.x % kBoundsSlots) * kBoundsStride;
+        v[0] = -v[0];  // minima as maxima
+        v[2] = -v[2];
+        v[4] = -v[4];
+#pragma unroll
+        for (int q = 0; q < kBoundsVQ; ++q) atomicMax(p + q, order_key(v[q]));
+    }
 }
 
 // _get_cell_size :103-110 and _get_number_of_cells :112-127 from the folded
-// bounds; writes the grid (or the halt flags) to the control block. Returns
-// false when the step must halt.
-__device__ bool derive_grid(Ctrl *ctrl, double scale, long long cap, const double *v) {
+// bounds. Returns the halt flag (0: the grid is valid).
+__device__ inline unsigned derive_grid(const double *v, double scale, long long cap, Grid &g) {
     const double xmn = v[0], xmx = v[1], ymn = v[2], ymx = v[3], hmn = v[4], hmx = v[5], bad = v[6];
-    Grid g;
     g.xmin = xmn;
     g.xmax = xmx;
     g.ymin = ymn;
@@ -422,68 +514,89 @@ __device__ bool derive_grid(Ctrl *ctrl, double scale, long long cap, const doubl
     double cell_size1 = 1. / cell_size;
     double fx = ceil(cell_size1 * (xmx - xmn));
     double fy = ceil(cell_size1 * (ymx - ymn));
-    if (bad != 0.0 || !(fx < 2.0e9) || !(fy < 2.0e9)) {
-        ctrl->flags |= SPH_FLAG_NONFINITE;
-        ctrl->active = 0;
-        ctrl->nn_valid = 0;
-        return false;
-    }
+    if (bad != 0.0 || !(fx < 2.0e9) || !(fy < 2.0e9)) return SPH_FLAG_NONFINITE;
     long long ncx = (long long)fx, ncy = (long long)fy;
     if (ncx < 1) ncx = 1;
     if (ncy < 1) ncy = 1;
     g.ncx = ncx;
     g.ncy = ncy;
     g.ncells = ncx * ncy;
-    ctrl->grid = g;
-    if (g.ncells > cap) {
-        ctrl->flags |= SPH_FLAG_CAPACITY;
-        ctrl->active = 0;
-        ctrl->nn_valid = 0;
-        return false;
-    }
-    return true;
-}
-
-// Fold the R bounds partials and derive the grid; a velocity bound that the
-// scan found (>= 0) becomes ctrl->vbound. One workgroup of kGridThreads
-// (256: 6.6 us on the 1M dam break against 7.9 with 1,024, four partials per
-// thread); every load, the active flag's included, is issued before the
-// fold.
-constexpr int kGridThreads = 256;
-__global__ void k_grid(Ctrl *ctrl, const double *part, int R, double scale, long long cap) {
-    const int active = ctrl->active;
-    __shared__ double lds[kBoundsVQ * 16];
-    const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
-    double v[kBoundsVQ] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY, 0.0, -INFINITY};
-    for (int k = threadIdx.x; k < R; k += blockDim.x) {
-        double u[kBoundsVQ];
-#pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q) u[q] = part[q * R + k];
-#pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q)
-            v[q] = kind[q] == 0 ? (u[q] < v[q] ? u[q] : v[q]) : kind[q] == 1 ? (u[q] > v[q] ? u[q] : v[q]) : v[q] + u[q];
-    }
-    block_fold<kBoundsVQ>(v, kind, lds);
-    if (threadIdx.x == 0 && active) {
-        if (v[7] >= 0.0) ctrl->vbound = v[7];
-        derive_grid(ctrl, scale, cap, v);
-    }
+    return g.ncells > cap ? SPH_FLAG_CAPACITY : 0u;
 }
 
 // _bin :129-141: cid = floor((x - xmin) / cs) per axis (:146-176), flat key
 // cx + ncx * cy (:200-208). Counts per bin; the rank inside a bin comes from
 // one atomic per run of equal bins within a wavefront (the state is already
 // in the previous step's cell order, so ~7 consecutive lanes share a bin).
-// k_cellsort fixes the order inside each bin afterwards.
-__global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int *counts, int *bin, int *rank, int *binflag) {
-    if (!ctrl->active) return;
+// bin_place fixes the order inside each bin afterwards.
+// Every workgroup derives the grid itself from the 16 bounds slots (two
+// wavefronts, one round of loads and four shuffles, under the loads of its
+// particles), 0.6 us (5k particles) to 2.3 us (1M), which saves a
+// single-workgroup kernel of 4.6 to 6.6 us and its launch; the first one also moves the grid and, in a step (fold),
+// the dt decision ctrl->nx into the control block, whose fields no other
+// workgroup reads here (they take nx and their own grid), and clears the dt
+// slots that k_bounds has folded.
+__global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double scale, long long cap,
+                       const unsigned long long *bslots, unsigned long long *dslots, double *hist, int *counts, int *bin,
+                       int *rank, int *binflag) {
+    if (!(fold ? ctrl->nx.active : ctrl->active)) {
+        if (fold && blockIdx.x == 0 && threadIdx.x == 0) dt_commit(ctrl, ctrl->nx, hist);
+        return;
+    }
+    __shared__ double s_v[kBoundsVQ];
+    __shared__ Grid s_g;
+    __shared__ unsigned s_halt;
+    const double dt = fold ? ctrl->nx.dt : ctrl->dt;
+    const int epoch = ctrl->epoch;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const Grid g = ctrl->grid;
+    double x = 0.0, y = 0.0;
+    int id = 0x7fffffff;
+    if (t < n) {
+        upd_pos(ctrl, a, t, pred, dt, x, y);
+        id = a.id[t];
+    }
+    if (threadIdx.x < kBoundsVQ * kBoundsSlots) {
+        const int q = threadIdx.x / kBoundsSlots, k = threadIdx.x % kBoundsSlots;
+        unsigned long long m = bslots[k * kBoundsStride + q];
+#pragma unroll
+        for (int o = kBoundsSlots / 2; o > 0; o >>= 1) {
+            const unsigned long long m2 = __shfl_xor(m, o, 64);
+            m = m2 > m ? m2 : m;
+        }
+        if (k == 0) {
+            const double u = order_value(m);
+            s_v[q] = q == 0 || q == 2 || q == 4 ? -u : u;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        Grid g;
+        const unsigned halt = derive_grid(s_v, scale, cap, g);
+        s_halt = halt;
+        s_g = g;
+        if (blockIdx.x == 0) {
+            if (fold) dt_commit(ctrl, ctrl->nx, hist);
+            if (s_v[7] >= 0.0) ctrl->vbound = s_v[7];  // a full scan's velocity bound
+            if (halt) {
+                atomicOr(&ctrl->flags, halt);
+                ctrl->active = 0;
+                ctrl->nn_valid = 0;
+                if (halt == SPH_FLAG_CAPACITY) ctrl->grid = g;
+            } else {
+                ctrl->grid = g;
+            }
+        }
+    }
+    if (fold && blockIdx.x == 0 && threadIdx.x < kDtSlotCount) {
+        dslots[(size_t)threadIdx.x * kDtStride] = 0;
+        dslots[(size_t)threadIdx.x * kDtStride + 1] = 0;
+    }
+    __syncthreads();
+    if (s_halt) return;
+    const Grid &g = s_g;
     int b = -1;
     if (t < n) {
-        double x, y;
-        upd_pos(ctrl, a, t, pred, ctrl->dt, x, y);
         const int2 c = cell_of(x, y, g);
         const long long key = (long long)c.x + g.ncx * (long long)c.y;
         if (key >= 0 && key < g.ncells) {
@@ -496,8 +609,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int *counts, int *b
     // Runs of equal bins in lane order, one atomic per run. A run also breaks
     // where the reference index drops (consecutive slots from two old cells),
     // so every run is in reference-index order; a bin that receives two runs
-    // is listed for k_cellsort below.
-    const int id = t < n ? a.id[t] : 0x7fffffff;
+    // is flagged for bin_place below.
     const int prev = __shfl_up(b, 1, 64);
     const int prev_id = __shfl_up(id, 1, 64);
     const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
@@ -509,10 +621,10 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int *counts, int *b
     if (lane == leader && b >= 0) {
         base = atomicAdd(&counts[b], next - leader);
         // A bin filled by more than one run may be out of reference-index
-        // order: flag it for k_cellsort, which clears the flag again. Every
+        // order: flag it with this update's epoch. Every
         // run but the first to arrive sees base != 0, so such a bin is always
         // flagged; the store is idempotent, so no atomic is needed.
-        if (base != 0) binflag[b] = 1;
+        if (base != 0) binflag[b] = epoch;
     }
     base = __shfl(base, leader, 64);
     if (t < n) {
@@ -539,44 +651,60 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int *counts, int *b
 // dynamic h for the fluid, formed here, after the keys were binned with the
 // previous h (Solver._compute: nn.update :238, then computeH :242-246) and
 // from the density the loop sees (the predicted one with PEC).
-__global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm, int2 *cxy_s, Phys ph, int n, int fmt,
-                          void *recA, void *recB, int pred, int strict, int lean, int xs, int dyn, HmConst hc) {
+// perm0 gives the source slot of each place, in any order inside a bin; the
+// slot t that a thread writes is the place of its particle in index order
+// (bin_place), and perm[t] records the source slot for the corrector.
+__global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *perm, const int *cellStart,
+                          const int *binflag, int2 *cxy_s, Phys ph, int n, int fmt, void *recA, void *recB, int pred,
+                          int strict, int lean, int xs, int dyn, HmConst hc) {
     // An inactive step (halted, or past the duration) still flips the
     // buffers on the host, so copy the state unpermuted.
     const int act = ctrl->active;
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     if (t == 0 && act) ctrl->nn_valid = 1;
-    int s = act ? perm[t] : t;
+    const int s = act ? perm0[t] : t;
+    const int id = a.id[s];
     double x = a.x[s], y = a.y[s], vx = a.vx[s], vy = a.vy[s], rho = a.rho[s];
     double m = hc.on ? hc.m : a.m[s], h = hc.on ? hc.h : a.h[s];
     const double ax = a.ax[s], ay = a.ay[s], drho = a.drho[s];
     int8_t lab = a.label[s];
     const bool skip = lean && act && pred && lab == kFluid;
-    if (act && pred && lab == kFluid) {
+    const bool moved = act && pred && lab == kFluid;
+    const double x0 = x, y0 = y, vx0 = vx, vy0 = vy, rho0 = rho;
+    if (moved) {
         // PEC.predict (src/Integrators/PEC.py:32-59) fused into the permutation
         const double dt = ctrl->dt, damping = ctrl->damping;
-        if (!skip) {
-            b.x0[t] = x;
-            b.y0[t] = y;
-            b.vx0[t] = vx;
-            b.vy0[t] = vy;
-            b.rho0[t] = rho;
-        }
         x = pec_half_pos(x, pred == 2 ? a.xsphx[s] : vx, dt);
         y = pec_half_pos(y, pred == 2 ? a.xsphy[s] : vy, dt);
         vx = pec_half_vel(vx, ax, dt, damping);
         vy = pec_half_vel(vy, ay, dt, damping);
         rho = pec_half_rho(rho, drho, dt, strict);
-    } else {
-        if (act && lab == kCoupled && ctrl->nm) {
-            // NewmarkBeta.predict (src/Integrators/NewmarkBeta.py:41-52), src/Solver.py:381-382
-            const double dt = ctrl->dt, nb = ctrl->nm_beta, ng = ctrl->nm_gamma;
-            x = nm_pred_pos(x, vx, ax, nb, dt);
-            y = nm_pred_pos(y, vy, ay, nb, dt);
-            vx = nm_pred_vel(vx, ax, ng, dt);
-            vy = nm_pred_vel(vy, ay, ng, dt);
+    } else if (act && lab == kCoupled && ctrl->nm) {
+        // NewmarkBeta.predict (src/Integrators/NewmarkBeta.py:41-52), src/Solver.py:381-382
+        const double dt = ctrl->dt, nb = ctrl->nm_beta, ng = ctrl->nm_gamma;
+        x = nm_pred_pos(x, vx, ax, nb, dt);
+        y = nm_pred_pos(y, vy, ay, nb, dt);
+        vx = nm_pred_vel(vx, ax, ng, dt);
+        vy = nm_pred_vel(vy, ay, ng, dt);
+    }
+    const Grid &g = ctrl->grid;
+    int2 cc = make_int2(0, 0);
+    if (act) {
+        cc = cell_of(x, y, g);
+        const long long key = (long long)cc.x + g.ncx * (long long)cc.y;  // k_keys' bin
+        t = bin_place(t, id, key >= 0 && key < g.ncells ? key : g.ncells, cellStart, binflag, ctrl->epoch, perm0, a.id);
+        perm[t] = s;
+    }
+    if (moved) {
+        if (!skip) {
+            b.x0[t] = x0;
+            b.y0[t] = y0;
+            b.vx0[t] = vx0;
+            b.vy0[t] = vy0;
+            b.rho0[t] = rho0;
         }
+    } else {
         b.x0[t] = a.x0[s];
         b.y0[t] = a.y0[s];
         b.vx0[t] = a.vx0[s];
@@ -586,8 +714,6 @@ __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm, int2 *c
     // SolverTools.computeH :106-118, sigma 1.3, d = 2 (the reference's fastmath
     // (m / rho) ** 0.5 is the square root)
     if (dyn && act && lab == kFluid) h = rho > 1e-12 ? 1.3 * sqrt(m / rho) : 0.0;
-    const Grid &g = ctrl->grid;
-    const int2 cc = act ? cell_of(x, y, g) : make_int2(0, 0);
     if (!skip) {
         b.x[t] = x;
         b.y[t] = y;
@@ -600,7 +726,7 @@ __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm, int2 *c
         b.h[t] = h;
     }
     b.label[t] = lab;
-    b.id[t] = a.id[s];
+    b.id[t] = id;
     if (xs || lab != kFluid) {  // without XSPH the fluid's is 0 after every loop (WCSPH.py:187-189)
         b.xsphx[t] = a.xsphx[s];
         b.xsphy[t] = a.xsphy[s];
@@ -990,7 +1116,7 @@ static void free_ctx(sph_ctx *c) {
         if (c->arena[k]) hipFree(c->arena[k]);
         if (c->gexec[k]) hipGraphExecDestroy(c->gexec[k]);
     }
-    void *ptrs[] = {c->ctrl, c->dt_hist, c->bin, c->rank, c->perm, c->permKey, c->cxy_s,
+    void *ptrs[] = {c->ctrl, c->dt_hist, c->bin, c->rank, c->perm, c->perm0, c->slots, c->cxy_s,
                     c->counts, c->cellStart, c->tileSums, c->binflag, c->part_b, c->part_d, c->part_k, c->recA, c->recB,
                     c->slot_of};
     for (void *p : ptrs)
@@ -1175,14 +1301,12 @@ int sph_ctx_create(const sph_params_t *params, sph_ctx_t **out) {
               hipMalloc(&c->dt_hist, sizeof(double) * 3 * SPH_DT_HISTORY) == hipSuccess &&
               hipMalloc(&c->bin, sizeof(int) * n) == hipSuccess && hipMalloc(&c->rank, sizeof(int) * n) == hipSuccess &&
               hipMalloc(&c->perm, sizeof(int) * n) == hipSuccess &&
-              hipMalloc(&c->permKey, sizeof(int) * n) == hipSuccess &&
+              hipMalloc(&c->perm0, sizeof(int) * n) == hipSuccess &&
+              hipMalloc(&c->slots, sizeof(unsigned long long) * kSlotWords) == hipSuccess &&
               hipMalloc(&c->cxy_s, sizeof(int2) * n) == hipSuccess &&
 
               hipMalloc(&c->part_b, sizeof(double) * kBoundsVQ * kRedBlocks) == hipSuccess &&
-              // dt partials: a reduction's workgroups or the fused pair pass's
-              hipMalloc(&c->part_d, sizeof(double) * kDtQ * (kRedBlocks > xcd_blocks(n, 256) ? kRedBlocks
-                                                                                             : xcd_blocks(n, 256))) ==
-                  hipSuccess &&
+              hipMalloc(&c->part_d, sizeof(double) * kDtQ * kRedBlocks) == hipSuccess &&
               hipMalloc(&c->part_k, sizeof(double) * (kRedBlocks + 1)) == hipSuccess &&
               hipMalloc(&c->slot_of, sizeof(int) * n) == hipSuccess;
     if (ok) {
@@ -1211,7 +1335,8 @@ int sph_ctx_create(const sph_params_t *params, sph_ctx_t **out) {
     h.active = 1;
     h.disp = h.vbound = h.abound = INFINITY;
     if (hipMemcpy(c->ctrl, &h, sizeof h, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(c->dt_hist, 0, sizeof(double) * 3 * SPH_DT_HISTORY) != hipSuccess) {
+        hipMemset(c->dt_hist, 0, sizeof(double) * 3 * SPH_DT_HISTORY) != hipSuccess ||
+        hipMemset(c->slots, 0, sizeof(unsigned long long) * kSlotWords) != hipSuccess) {
         free_ctx(c);
         return fail(SPH_EHIP, "control block init failed");
     }
@@ -1372,8 +1497,9 @@ static int refresh_uniform(sph_ctx *c, hipStream_t s) {
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s));
     }
+    // captured steps bake the one h and m into their kernels' arguments
     if (rec_format(c) != before || c->static_hm != static_before ||
-        (c->static_hm && (c->uni_h != h_before || v[4] != m_before)))
+        ((c->uni_hm || c->static_hm) && (c->uni_h != h_before || c->uni_m != m_before)))
         drop_graphs(c);
     return 0;
 }
@@ -1386,9 +1512,44 @@ static HmConst hm_const(const sph_ctx *c) {
     return hc;
 }
 
+static Slots slots_of(unsigned long long *w) { return Slots{w, w + (size_t)kBoundsSlots * kBoundsStride}; }
+
+// The scan's form: one kernel up to kScanOneMax particles, else two. Measured
+// per step: 4.7 us against 3.1 + 3.6 us and a launch gap at 5k particles
+// (4.6k bins), 8.0 against 2.9 + 3.9 us and the gap at 90k (72k bins).
+constexpr int kScanOneMax = 1 << 16;
+
+// The neighbour update's kernels on the state a of n particles: bounds, keys,
+// scan, places (perm0, cellStart, binflag). D.on: the dt fold in the bounds.
+struct NnWork {
+    Ctrl *ctrl;
+    Slots slots;
+    int *counts, *cellStart, *tileSums, *binflag, *bin, *rank, *perm0;
+    long long cap;
+};
+static void nn_launch(const NnWork &w, const State &a, int n, int pred, const HmConst &hc, const int *border,
+                      double scale, const DtFold &D, hipStream_t s) {
+    const int R = redblk(n) < kBoundsBlocks ? redblk(n) : kBoundsBlocks;
+    k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b);
+    k_keys<<<nblk(n), kBlock, 0, s>>>(w.ctrl, a, n, pred, D.on, scale, w.cap, w.slots.b, w.slots.d, D.hist, w.counts,
+                                      w.bin, w.rank, w.binflag);
+    const bool one = n <= kScanOneMax;
+    if (one) {
+        k_scan_one<<<kScanBlocks, kScanThreads, 0, s>>>(w.ctrl, w.counts, w.cellStart);
+    } else {
+        const long long tiles_cap = (w.cap + 1 + kScanTile - 1) / kScanTile;
+        const int tiles = (int)(tiles_cap < 1024 ? tiles_cap : 1024);
+        k_scan_reduce<<<tiles, kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums);
+        k_scan_apply<<<tiles, kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums, w.cellStart);
+    }
+    k_place<<<nblk(n), kBlock, 0, s>>>(w.ctrl, w.cellStart, w.bin, w.rank, w.perm0, n, one ? w.counts : nullptr,
+                                       w.slots.b);
+}
+
 // pred != 0: the PEC predictor runs inside the update (bounds and keys see
-// the predicted positions, the reorder writes the predicted state).
-static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0) {
+// the predicted positions, the reorder writes the predicted state). fold: the
+// update opens a step (dt from the partials of the current state).
+static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int fold = 0) {
     if (pred && c->P.use_xsph) pred = 2;  // PEC with XSPH moves x by the XSPH velocity
     const int n = c->n;
     State a = c->buf[c->cur];
@@ -1397,24 +1558,17 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0) {
         int rc = ev_record(c, c->ev_nn, c->n_nn, s);
         if (rc) return rc;
     }
-    const int R = redblk(n) < kBoundsBlocks ? redblk(n) : kBoundsBlocks;
     // the border-cell bounds only in the step's update with PEC's predictor
     const int *border = c->border_bounds && pred == 1 ? c->cellStart : nullptr;
-    k_bounds<<<R, kBlock, 0, s>>>(c->ctrl, a, n, pred, c->part_b, hm_const(c), border);
-    k_grid<<<1, kGridThreads, 0, s>>>(c->ctrl, c->part_b, R, c->P.scale, c->cap_cells);
-    k_keys<<<nblk(n), kBlock, 0, s>>>(c->ctrl, a, n, pred, c->counts, c->bin, c->rank, c->binflag);
-    long long tiles_cap = (c->cap_cells + 1 + kScanTile - 1) / kScanTile;
-    int tiles = (int)(tiles_cap < 1024 ? tiles_cap : 1024);
-    k_scan_reduce<<<tiles, kBlock, 0, s>>>(c->ctrl, c->counts, c->tileSums);
-    k_scan_apply<<<tiles, kBlock, 0, s>>>(c->ctrl, c->counts, c->tileSums, c->cellStart);
-    k_scatter<<<nblk(n), kBlock, 0, s>>>(c->ctrl, c->cellStart, c->bin, c->rank, a.id, c->perm, c->permKey, n);
-    // bin/rank are free once scattered: they stage the rare bins of more than 64
-    k_cellsort<<<redblk(c->cap_cells + 1), kBlock, 0, s>>>(c->ctrl, c->cellStart, c->perm, c->permKey,
-                                                           c->binflag, c->bin, c->rank);
+    const HmConst hc = hm_const(c);
+    const Slots sl = slots_of(c->slots);
+    const NnWork w{c->ctrl, sl, c->counts, c->cellStart, c->tileSums, c->binflag, c->bin, c->rank, c->perm0, c->cap_cells};
+    nn_launch(w, a, n, pred, hc, border, c->P.scale,
+              DtFold{fold, c->P.gamma_c, c->P.gamma_f, c->uni_h, c->dt_hist, c->part_d, sl.d}, s);
     c->rec_fmt = rec_format(c);
-    k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, a, b, c->perm, c->cxy_s, make_phys(c->P), n, c->rec_fmt,
-                                         c->recA, c->recB, pred, c->P.strict, lean, c->P.use_xsph, c->P.dynamic_h,
-                                         hm_const(c));
+    k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, a, b, c->perm0, c->perm, c->cellStart, c->binflag, c->cxy_s,
+                                         make_phys(c->P), n, c->rec_fmt, c->recA, c->recB, pred, c->P.strict, lean,
+                                         c->P.use_xsph, c->P.dynamic_h, hc);
     HIPCHK(hipGetLastError());
     if (!c->P.use_xsph) c->xs_fluid_zero = true;
     if (c->timing) {
@@ -1486,12 +1640,20 @@ static int compute(sph_ctx *c, hipStream_t s, int *count = nullptr, int mode = 0
     return 0;
 }
 
-static int dt_step(sph_ctx *c, hipStream_t s) {
+// The dt partials of the current state, if no corrector left them.
+static int dt_partials(sph_ctx *c, hipStream_t s) {
+    if (c->dt_fresh) return 0;
     State st = c->buf[c->cur];
-    if (!c->dt_fresh) {
-        k_dt_partial<<<redblk(c->n), kBlock, 0, s>>>(c->ctrl, st.label, st.h, st.ax, st.ay, c->n, c->part_d);
-    }
-    k_dt_final<<<1, 1024, 0, s>>>(c->ctrl, c->P.gamma_c, c->P.gamma_f, c->dt_hist, c->part_d);
+    k_dt_partial<<<redblk(c->n), kBlock, 0, s>>>(c->ctrl, st.label, st.h, st.ax, st.ay, c->n, c->part_d);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+static int dt_step(sph_ctx *c, hipStream_t s) {
+    int rc = dt_partials(c, s);
+    if (rc) return rc;
+    k_dt_final<<<1, kBlock, 0, s>>>(c->ctrl, c->P.gamma_c, c->P.gamma_f, c->dt_hist, c->part_d, slots_of(c->slots).d,
+                                    c->uni_h);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1520,7 +1682,7 @@ static int compute_pec(sph_ctx *c, hipStream_t s) {
     State st = c->buf[c->cur];
     PairIn in{c->recA, c->recB, st.h, c->cxy_s, c->cellStart};
     PairOut out{st.ax, st.ay, st.drho, nullptr, 0};
-    const PecArgs pec{st, c->buf[1 - c->cur], c->perm, c->part_d, hm_const(c), c->P.strict};
+    const PecArgs pec{st, c->buf[1 - c->cur], c->perm, nullptr, slots_of(c->slots).d, hm_const(c), c->P.strict};
     if (c->timing) {
         int rc = ev_record(c, c->ev_pair, c->n_pair, s);
         if (rc) return rc;
@@ -1545,8 +1707,8 @@ static int one_step(sph_ctx *c, hipStream_t s) {
     // the lean reorder leaves the half-step velocity and density out of the
     // state; XSPH and the summation density read them there
     const bool lean = pec && !c->P.use_xsph && !c->P.use_summation_density;
-    if ((rc = dt_step(c, s))) return rc;
-    if ((rc = nn_update(c, s, pec, lean))) return rc;
+    if ((rc = dt_partials(c, s))) return rc;
+    if ((rc = nn_update(c, s, pec, lean, 1))) return rc;
     if (lean && c->P.coupled_integrator != SPH_COUPLED_NEWMARK && uniform_pass(c)) {
         if ((rc = compute_pec(c, s))) return rc;
     } else {
@@ -1579,8 +1741,8 @@ static int record_step(sph_ctx *ctx, sph_tape *tape, int slot, hipStream_t s) {
     int rc;
     const bool pec = ctx->P.integrator == SPH_INTEGRATOR_PEC;
     const bool fused = pec && uniform_pass(ctx);  // the tape covers no XSPH, summation density or coupling
-    if ((rc = dt_step(ctx, s))) return rc;
-    if ((rc = nn_update(ctx, s, pec, fused))) return rc;
+    if ((rc = dt_partials(ctx, s))) return rc;
+    if ((rc = nn_update(ctx, s, pec, fused, 1))) return rc;
     if (fused) {
         if ((rc = compute_pec(ctx, s))) return rc;
         if ((rc = tape_record_pair(ctx, tape, slot, s, true))) return rc;
@@ -1771,8 +1933,8 @@ int sph_step_begin(sph_ctx_t *ctx, void *stream) {
     if (closed(ctx)) return SPH_ESTATE;
     hipStream_t s = S(stream);
     int rc;
-    if ((rc = dt_step(ctx, s))) return rc;
-    if ((rc = nn_update(ctx, s, ctx->P.integrator == SPH_INTEGRATOR_PEC))) return rc;
+    if ((rc = dt_partials(ctx, s))) return rc;
+    if ((rc = nn_update(ctx, s, ctx->P.integrator == SPH_INTEGRATOR_PEC, 0, 1))) return rc;
     if ((rc = compute(ctx, s))) return rc;
     ctx->mid = true;
     return 0;
@@ -2162,13 +2324,13 @@ static_assert(sizeof(Rec<double>::A) == 32 && sizeof(Rec<double>::B) == 32 && si
                   sizeof(Rec<float>::B) <= 32,
               "pair records are sized at 32 bytes in the workspace");
 constexpr size_t kNaOffCtrl = 0;
-constexpr size_t kNaOffPart = kNaOffCtrl + al256(sizeof(Ctrl));
-constexpr size_t kNaOffId = kNaOffPart + al256(sizeof(double) * kBoundsVQ * kBoundsBlocks);
+constexpr size_t kNaOffSlots = kNaOffCtrl + al256(sizeof(Ctrl));
+constexpr size_t kNaOffId = kNaOffSlots + al256(sizeof(unsigned long long) * kSlotWords);
 constexpr size_t kNaOffBin = kNaOffId + al256(4 * kNaParticles);
 constexpr size_t kNaOffRank = kNaOffBin + al256(4 * kNaParticles);
 constexpr size_t kNaOffPerm = kNaOffRank + al256(4 * kNaParticles);
-constexpr size_t kNaOffPermKey = kNaOffPerm + al256(4 * kNaParticles);
-constexpr size_t kNaOffCxy = kNaOffPermKey + al256(4 * kNaParticles);
+constexpr size_t kNaOffPerm0 = kNaOffPerm + al256(4 * kNaParticles);
+constexpr size_t kNaOffCxy = kNaOffPerm0 + al256(4 * kNaParticles);
 constexpr size_t kNaOffRecA = kNaOffCxy + al256(8 * kNaParticles);
 constexpr size_t kNaOffRecB = kNaOffRecA + al256(32 * kNaParticles);
 constexpr size_t kNaOffH = kNaOffRecB + al256(32 * kNaParticles);
@@ -2210,13 +2372,15 @@ static int na_workspace(unsigned char **out) {
 // no coupled integrator; the cell counts and bin flags cleared over the whole
 // capacity (the workspace keeps the last call's contents); the identity as
 // each particle's reference index.
-__global__ void k_na_init(Ctrl *ctrl, int *counts, int *binflag, int *id, int n, long long ncap) {
+__global__ void k_na_init(Ctrl *ctrl, unsigned long long *slots, int *counts, int *binflag, int *id, int n,
+                          long long ncap) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         Ctrl c{};
         c.active = 1;
         *ctrl = c;
     }
+    if (i < (long long)kSlotWords) slots[i] = 0;
     if (i <= ncap) {
         counts[i] = 0;
         binflag[i] = 0;
@@ -2228,18 +2392,24 @@ __global__ void k_na_init(Ctrl *ctrl, int *counts, int *binflag, int *id, int n,
 // arrays through the permutation: records (as k_reorder writes them without
 // a predictor), the double h, each slot's raw cell, and the rates a target
 // keeps when it finds no neighbour (src/Tools/SolverTools.py:166-169).
-__global__ void k_na_reorder(const Ctrl *ctrl, sph_state_t in, const int *perm, int2 *cxy, double *H, double *ax,
-                             double *ay, double *drho, Phys ph, int n, int fp32, void *recA, void *recB) {
+__global__ void k_na_reorder(const Ctrl *ctrl, sph_state_t in, const int *perm0, int *perm, const int *cellStart,
+                             const int *binflag, const int *id, int2 *cxy, double *H, double *ax, double *ay,
+                             double *drho, Phys ph, int n, int fp32, void *recA, void *recB) {
     if (!ctrl->active) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    const int s = perm[t];
+    const int s = perm0[t];
     const double x = in.x[s], y = in.y[s], vx = in.vx[s], vy = in.vy[s], rho = in.rho[s], m = in.m[s], h = in.h[s];
     const int8_t lab = in.label[s];
+    const Grid &g = ctrl->grid;
+    const int2 cc = cell_of(x, y, g);
+    const long long key = (long long)cc.x + g.ncx * (long long)cc.y;
+    t = bin_place(t, s, key >= 0 && key < g.ncells ? key : g.ncells, cellStart, binflag, ctrl->epoch, perm0, id);
+    perm[t] = s;
     ax[t] = in.ax ? in.ax[s] : 0.0;
     ay[t] = in.ay ? in.ay[s] : 0.0;
     drho[t] = in.drho ? in.drho[s] : 0.0;
-    cxy[t] = cell_of(x, y, ctrl->grid);
+    cxy[t] = cc;
     H[t] = h;
     write_pair_records(t, x, y, vx, vy, rho, m, h, lab, ph, fp32, recA, recB);
 }
@@ -2273,9 +2443,9 @@ extern "C" int sph_loop_noalloc(const sph_params_t *params, const sph_state_t *s
     unsigned char *w = nullptr;
     if ((rc = na_workspace(&w))) return rc;
     Ctrl *ctrl = (Ctrl *)(w + kNaOffCtrl);
-    double *part = (double *)(w + kNaOffPart);
+    unsigned long long *slots = (unsigned long long *)(w + kNaOffSlots);
     int *id = (int *)(w + kNaOffId), *bin = (int *)(w + kNaOffBin), *rank = (int *)(w + kNaOffRank);
-    int *perm = (int *)(w + kNaOffPerm), *permKey = (int *)(w + kNaOffPermKey);
+    int *perm = (int *)(w + kNaOffPerm), *perm0 = (int *)(w + kNaOffPerm0);
     int2 *cxy = (int2 *)(w + kNaOffCxy);
     void *recA = w + kNaOffRecA, *recB = w + kNaOffRecB;
     double *H = (double *)(w + kNaOffH), *ax_s = (double *)(w + kNaOffAx), *ay_s = (double *)(w + kNaOffAy);
@@ -2291,19 +2461,13 @@ extern "C" int sph_loop_noalloc(const sph_params_t *params, const sph_state_t *s
     a.label = st->label;
     a.id = id;
     const long long ninit = (kNaCells + 1 > n ? kNaCells + 1 : n);
-    k_na_init<<<nblk(ninit), kBlock, 0, s>>>(ctrl, counts, binflag, id, nn, kNaCells);
-    const int R = redblk(n) < kBoundsBlocks ? redblk(n) : kBoundsBlocks;
-    k_bounds<<<R, kBlock, 0, s>>>(ctrl, a, nn, 0, part, HmConst{}, nullptr);
-    k_grid<<<1, kGridThreads, 0, s>>>(ctrl, part, R, params->scale, kNaCells);
-    k_keys<<<nblk(n), kBlock, 0, s>>>(ctrl, a, nn, 0, counts, bin, rank, binflag);
-    const int tiles = (int)((kNaCells + 1 + kScanTile - 1) / kScanTile);
-    k_scan_reduce<<<tiles, kBlock, 0, s>>>(ctrl, counts, tileSums);
-    k_scan_apply<<<tiles, kBlock, 0, s>>>(ctrl, counts, tileSums, cellStart);
-    k_scatter<<<nblk(n), kBlock, 0, s>>>(ctrl, cellStart, bin, rank, id, perm, permKey, nn);
-    k_cellsort<<<redblk(kNaCells + 1), kBlock, 0, s>>>(ctrl, cellStart, perm, permKey, binflag, bin, rank);
+    k_na_init<<<nblk(ninit), kBlock, 0, s>>>(ctrl, slots, counts, binflag, id, nn, kNaCells);
+    const NnWork nw{ctrl, slots_of(slots), counts, cellStart, tileSums, binflag, bin, rank, perm0, kNaCells};
+    nn_launch(nw, a, nn, 0, HmConst{}, nullptr, params->scale, DtFold{}, s);
     const bool f32 = params->precision == SPH_PREC_FP32C;
     const Phys ph = make_phys(*params);
-    k_na_reorder<<<nblk(n), kBlock, 0, s>>>(ctrl, *st, perm, cxy, H, ax_s, ay_s, drho_s, ph, nn, f32, recA, recB);
+    k_na_reorder<<<nblk(n), kBlock, 0, s>>>(ctrl, *st, perm0, perm, cellStart, binflag, id, cxy, H, ax_s, ay_s, drho_s, ph,
+                                            nn, f32, recA, recB);
     HIPCHK(hipGetLastError());
     PairIn in{recA, recB, H, cxy, cellStart};
     PairOut out{ax_s, ay_s, drho_s, nullptr, 0};

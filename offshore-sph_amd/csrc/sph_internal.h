@@ -38,6 +38,18 @@ struct Grid {
     int uniform_h;  // min h == max h over all particles
 };
 
+// What the dt fold of a step decided, before it takes effect: k_bounds folds
+// the partials in every workgroup (each needs dt), and its first workgroup
+// leaves the result here; the next kernel (k_keys) moves it into the control
+// block, whose old values the other workgroups of k_bounds may still read.
+struct DtNext {
+    double t, dt, dt_c, dt_f;
+    double disp, vbound, abound;
+    long long step;
+    unsigned flags;  // flags to add
+    int active;
+};
+
 struct Ctrl {
     double t, dt, dt_c, dt_f;
     long long step;
@@ -50,13 +62,16 @@ struct Ctrl {
     int nn_valid;        // cell order and offsets match the positions
     int nm;              // Newmark-beta on the coupled particles
     double nm_beta, nm_gamma;
-    int dt_parts;        // workgroups whose dt partials the partials buffer holds (set by their kernel)
+    int dt_parts;        // workgroups whose dt partials the partials buffer holds (set by their kernel;
+                         // kDtSlots: the dt slots hold them)
     int pec_parts;       // 1 when those partials come from the fused PEC pass (cleared by k_dt_final)
     double disp;         // bound on how far any particle's predicted position lies from where it was
                          // last binned, per axis (k_dt_final; +inf when unknown)
     double vbound;       // bound on every particle's |vx|, |vy| at the start of the step (+inf: unknown)
     double abound;       // bound on every fluid particle's |a| in the rates the step's predictor uses
     long long border_updates;  // neighbour updates whose bounds came from the border cells
+    DtNext nx;
+    int epoch;           // neighbour updates so far: a bin flag holds the update that set it
 };
 
 // Grid-wide reductions (bounds, dt) run over at most kRedBlocks workgroups in
@@ -65,9 +80,26 @@ struct Ctrl {
 // launch) and a single-workgroup kernel folds the R partials. Same-address
 // device-scope atomics from every workgroup serialise across the XCDs and
 // cost ~10 ns each, far more than the second launch.
-constexpr int kBoundsQ = 7;  // min/max x, min/max y, min/max h, non-finite count
 constexpr int kDtQ = 4;      // min h, max |a|^2, fluid count, non-finite count
-constexpr int kBoundsVQ = 8;  // the single engine's bounds: kBoundsQ, then the largest |vx|, |vy|
+constexpr int kBoundsVQ = 8;  // min/max x, min/max y, min/max h, non-finite count, largest |vx|, |vy|
+
+// Reductions whose result every workgroup of the next kernel needs (the
+// single engine's bounds; the dt partials of the fused pair pass, up to one
+// per 256 particles): each workgroup adds its partial to one of a few slots
+// with device-scope atomic maxima (order-preserving integer keys of the
+// doubles), so the next kernel's workgroups fold 16 or 64 entries instead of
+// one per workgroup. Slots lie on lines of their own: about 16 (bounds) to 80
+// (dt, 1M particles) workgroups meet on one, far from the serialisation of a
+// single address.
+constexpr int kBoundsSlots = 16, kBoundsStride = 16;  // u64 entries
+constexpr int kDtSlotCount = 64, kDtStride = 16;
+constexpr int kDtSlots = -1;  // Ctrl::dt_parts: the partials are in the dt slots
+struct Slots {
+    unsigned long long *b;  // kBoundsSlots x kBoundsStride: the kBoundsVQ quantities as maxima
+    unsigned long long *d;  // kDtSlotCount x kDtStride: bits of max |a|^2, kDt* flags
+};
+constexpr unsigned long long kDtAny = 1ull, kDtBad = 2ull;  // a fluid particle; a NaN rate
+constexpr size_t kSlotWords = (size_t)kBoundsSlots * kBoundsStride + (size_t)kDtSlotCount * kDtStride;
 
 // One cell-ordered buffer set.
 struct State {
@@ -107,11 +139,13 @@ struct HmConst {
 // PEC's corrector fused into the uniform pair passes (a step whose reorder
 // ran lean): slot j of s (this step's cell order) came from slot perm[j] of
 // o (the start-of-step buffer), which holds the start-of-step state and the
-// previous rates; part receives the next dt's partials (kDtQ per workgroup).
+// previous rates; the next dt's partials go to part (kDtQ per workgroup) or
+// the dt slots.
 struct PecArgs {
     State s, o;
     const int *perm;
-    double *part;
+    double *part;                      // the batch: one partial per tile
+    unsigned long long *dslots = nullptr;  // the single engine: the dt slots
     HmConst hc;
     int strict;
     int *mark = nullptr;  // when set, the pass stores 1 there (its partials come from a corrector that moved the fluid)

@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void k_pair_uniform64_pec(Ctrl *ctrl, Uniform6
     __shared__ double lds[kDtQ * 16];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctrl->dt_parts = gridDim.x;
+        ctrl->dt_parts = kDtSlots;
         ctrl->pec_parts = 1;
     }
     const int t = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) void k_pair_uniform64_pec(Ctrl *ctrl, Uniform6
             pec_finish(C, t, p0, ax, ay, drho, dt, damping);
         }
     }
-    v.publish(C.part, lds);
+    v.publish_slots(C.dslots, lds);
 }
 
 // The batched ensemble (one thread per slot, and the persistent work-queue
