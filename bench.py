@@ -9,9 +9,8 @@ A "step" is one pass of the Solver loop body on the device: dt reduction,
 predict, neighbour search (bounds, keys, counting sort, reorder), fused pair
 pass (Tait EOS, continuity, momentum + artificial viscosity + gravity,
 Lennard-Jones wall force), correct. The state is resident in HBM before the
-timed region; W untimed steps (which capture the step as a hipGraph) precede
-K timed ones replayed from the graphs with no per-launch timing, bracketed by
-device synchronisation.
+timed region; W untimed steps precede K timed ones launched back to back with
+no per-launch timing, bracketed by device synchronisation.
 
 `value` is particle-steps/s (fluid particles x steps / s) with the FP32
 compensated pair pass and the FP64 integrator; the FP64 pair pass is
@@ -56,10 +55,9 @@ def algorithmic_pair_bytes(precision, n, nf, cells, corrector=False):
 
 
 def run_gpu(sc, precision, steps, warmup, timing_steps=50, host_reps=0):
-    """The headline timing: W warm-up steps (the first captures the step as a
-    hipGraph per buffer parity), then K steps replayed from the graphs with
-    no per-launch timing, bracketed by device synchronisation. Then, apart
-    from that timed region, `timing_steps` eager steps with HIP events around
+    """The headline timing: W warm-up steps, then K steps launched back to back
+    with no per-launch timing, bracketed by device synchronisation. Then, apart
+    from that timed region, `timing_steps` steps with HIP events around
     every pair pass and neighbour update (on the stream they run on) for the
     per-stage times and the roofline."""
     import torch
@@ -117,7 +115,7 @@ def run_gpu(sc, precision, steps, warmup, timing_steps=50, host_reps=0):
 def evolved_timing(sc, before=4000, steps=200, timing_steps=50):
     """The FP32C step on a flow that has run `before` steps from the initial
     lattice (the flow disorders it: more candidates per target, uneven
-    contributor counts): K steps replayed from the graphs, then eager steps
+    contributor counts): K steps launched back to back, then steps
     with HIP events around the pair pass and the neighbour update."""
     import torch
     from hipsph.device import Engine, EngineParams, soa_from_particles
@@ -281,10 +279,9 @@ def ensemble(steps=500, count=256, seq_steps=10, seq_instances=64):
     """The batched ensemble: `count` dam breaks (width U(0.5, 1.5), height
     U(0.5, 2.5), dx from {0.005, 0.01, 0.02}, alpha U(0.005, 0.05), seeded per
     instance), FP32C pairs and FP64 integrator, `steps` steps each in one batch
-    (one launch per stage, hipGraph replay, pair workgroup size,
-    contributor-list length and schedule autotuned).
+    (one launch per stage, pair workgroup size, contributor-list length and schedule autotuned).
     Beside it: the same instances as separate engines one after another
-    (graph replay each), timed on the first `seq_instances` for `seq_steps`."""
+    (as above), timed on the first `seq_instances` for `seq_steps`."""
     import torch
     import numpy as np
     from hipsph import scenarios
@@ -645,7 +642,7 @@ def write_summaries(traffic, valu, phases, build, n=None, nf=None, cells=None):
 
     L = ['# Kernel statistics of the 1M dam break step', '',
          'The headline run, shortened: `bench.py --steps 200 --warmup 10` (FP32C run, then FP64 run; each 10 '
-         'warm-up steps, 200 steps replayed from hipGraphs, then 50 eager steps with HIP events around the pair '
+         'warm-up steps, 200 steps, then 50 steps with HIP events around the pair '
          'pass and the neighbour update, and the host round trip). Kernels of the engine only; the split between '
          'the runs is the first double pair dispatch.', '', head]
     for tag in ('fp32c', 'fp64'):
@@ -682,7 +679,7 @@ STATS_NOTES = {
     'kt_ens': 'Workload: 256 dam breaks (column width U(0.5, 1.5) m, height U(0.5, 2.5) m, dx from '
               '{0.005, 0.01, 0.02} m, alpha U(0.005, 0.05), 4.0 x 3.0 m tank), 961 to 136,948 fluid particles '
               'each, FP32C pairs, FP64 integrator, PEC, per-instance dt; every stage one launch over all '
-              'instances, the step replayed as a hipGraph. Every instance has one h and one fluid mass, so the '
+              'instances. Every instance has one h and one fluid mass, so the '
               'pair pass is the uniform one with the corrector fused in (`k_pair_batch_uniform_pec`, one '
               'workgroup per 256-slot tile of one instance); the autotuner times it against the persistent '
               'work-queue schedule (`k_pair_batch_uniform_queue` + `kb_correct`).',
@@ -879,7 +876,7 @@ def main():
         'config': {'workload': sc.name, 'n_particles': n, 'n_fluid': nf, 'dx': sc.dx, 'kernel': 'cubic',
                    'integrator': 'pec', 'pair_precision': 'fp32c (float pairs, compensated sums)',
                    'pair_form': r32['pair_form'], 'integrator_dtype': 'f64', 'h': sc.h, 'cells': cells,
-                   'timed_region': 'K steps replayed from hipGraphs, no per-launch timing',
+                   'timed_region': 'K steps launched back to back, no per-launch timing',
                    'parallelism': 'single GPU'},
         'roofline': {'bound': 'hbm', 'achieved': ach32, 'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
                      'frac': ach32 / HBM_PEAK_GBS, 'traffic': prof(traffic, 'fp32c', 'hbm_bytes_per_launch'),

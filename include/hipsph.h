@@ -185,7 +185,9 @@ int sph_predict(sph_ctx_t *ctx, void *stream);
 int sph_correct(sph_ctx_t *ctx, void *stream);
 /* nsteps iterations of the Solver.run loop body (src/Solver.py:366-410):
  * dt -> predict -> nn_update -> compute -> correct, all on the device.
- * use_graph != 0 captures the step in a hipGraph and replays it. */
+ * Nothing waits for the host between launches; use_graph is accepted and
+ * changes nothing (replaying captured steps measured slower than launching
+ * them). */
 int sph_step(sph_ctx_t *ctx, int64_t nsteps, int32_t use_graph, void *stream);
 
 /* One loop body split at the coupling hook (src/Solver.py:389-392):
@@ -275,10 +277,7 @@ int sph_step_record(sph_ctx_t *ctx, sph_tape_t *tape, int32_t slot, void *stream
 int sph_adjoint_step(sph_ctx_t *ctx, sph_tape_t *tape, int32_t slot, const sph_adjoint_t *adj, void *stream);
 /* One checkpoint segment in a single call: record `nsteps` steps from the
  * current state into slots 0..nsteps-1, then reverse them (as
- * sph_step_record and sph_adjoint_step, in that order). Steps after the first
- * are replayed from hipGraphs cached in the tape (per slot and buffer parity
- * for the recording; per slot for the reversal, for the adjoint buffers of
- * the last call). */
+ * sph_step_record and sph_adjoint_step, in that order). */
 int sph_adjoint_segment(sph_ctx_t *ctx, sph_tape_t *tape, int32_t nsteps, const sph_adjoint_t *adj, void *stream);
 /* A saved state back into the context without a host round trip (for
  * checkpoint restores): as sph_state_upload without resetting the step count,
@@ -288,7 +287,7 @@ int sph_state_restore(sph_ctx_t *ctx, const sph_state_t *st, double t, void *str
 /* ---- batched ensemble (no counterpart in the reference) ----
  * K independent simulations of uneven sizes advanced together: one launch per
  * stage covers every instance (segmented cell grid, per-instance clock, dt,
- * grid and constants), and a step replays as one hipGraph. Each instance
+ * grid and constants). Each instance
  * evolves exactly as sph_step would advance it alone. params[k] describes
  * instance k (n, constants, duration, cell_capacity); kernel, precision and
  * integrator must be the same for all. State arrays are the instances'

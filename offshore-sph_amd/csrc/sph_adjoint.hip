@@ -661,9 +661,6 @@ int sph_tape_create(sph_ctx_t *ctx, int32_t nslots, sph_tape_t **out) {
     for (double **d : scr) *d = (double *)take(n * sizeof(double));
     t->lk = (double4 *)take(n * sizeof(double4));
     t->slot.resize(nslots);
-    t->rec_exec.assign(2 * (size_t)nslots, nullptr);
-    t->adj_exec.assign(nslots, nullptr);
-    t->gen = ctx->gen;
     for (int k = 0; k < nslots; ++k) {
         TapeSlot &S = t->slot[k];
         double **f[] = {&S.vxh, &S.vyh, &S.ax, &S.ay, &S.drho, &S.vx0, &S.vy0, &S.axp, &S.ayp, &S.drhop};
@@ -702,7 +699,6 @@ int sph_tape_create(sph_ctx_t *ctx, int32_t nslots, sph_tape_t **out) {
 int sph_tape_destroy(sph_tape_t *tape) {
     if (!tape) return 0;
     hipDeviceSynchronize();
-    tape_drop_graphs(tape);
     hipFree(tape->arena);
     delete tape;
     return 0;
@@ -728,13 +724,6 @@ int sph_adjoint_step(sph_ctx_t *ctx, sph_tape_t *tape, int32_t slot, const sph_a
 }
 
 }  // extern "C"
-
-void hipsph::tape_drop_graphs(sph_tape *t) {
-    for (auto &g : t->rec_exec)
-        if (g) hipGraphExecDestroy(g), g = nullptr;
-    for (auto &g : t->adj_exec)
-        if (g) hipGraphExecDestroy(g), g = nullptr;
-}
 
 int hipsph::adjoint_launch(sph_ctx *ctx, sph_tape *tape, int slot, const sph_adjoint_t *adj, hipStream_t s) {
     const int n = ctx->n;

@@ -16,7 +16,7 @@
 //     the instances' bins);
 //   * every instance has its own control block (BInst): clock, dt, grid,
 //     halt flags and constants (alpha, c0, B, r0, D ...).
-// A step is captured in a hipGraph like the single simulation's. The
+// A step needs no host round trip, like the single simulation's. The
 // arithmetic per particle is the single engine's, in the same order, so an
 // instance evolves exactly as it would alone.
 //
@@ -515,8 +515,6 @@ struct sph_batch {
     long long capBins = 0;
     bool dt_fresh = false;
     bool loaded = false;  // a state was uploaded: every id indexes its instance
-    hipStream_t own = nullptr;
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int pair_threads = 256;
     int list_len = 0;  // 0: the single-simulation pass's length
     int persistent = 0;    // the pair pass as a persistent work-queue kernel
@@ -542,7 +540,6 @@ void free_batch(sph_batch *b) {
     if (!b) return;
     for (int k = 0; k < 2; ++k) {
         if (b->arena[k]) hipFree(b->arena[k]);
-        if (b->gexec[k]) hipGraphExecDestroy(b->gexec[k]);
     }
     void *ptrs[] = {b->inst, b->view, b->instOf, b->cs, b->chunkInst, b->chunk0, b->ts, b->tileInst, b->tile0,
                     b->bin, b->rank, b->perm,
@@ -551,13 +548,12 @@ void free_batch(sph_batch *b) {
     for (void *p : ptrs)
         if (p) hipFree(p);
     for (auto e : b->ev) hipEventDestroy(e);
-    if (b->own) hipStreamDestroy(b->own);
     delete b;
 }
 
 // The persistent pair pass's grid: one resident occupancy of the device
 // (hipOccupancy for the chosen kernel, list and workgroup size). Host only;
-// sized before a step is launched or captured.
+// sized before a step is launched.
 void size_queue(sph_batch *b) {
     if (!b->persistent || b->queue_grid > 0) return;
     const int per = b->uni ? (b->precision == SPH_PREC_FP32C ? pair_batch_uniform_occupancy_fp32(b->kernel)
@@ -838,8 +834,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMemset(b->counts, 0, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMemset(b->cellStart, 0, sizeof(int) * (capTot + 2)) == hipSuccess &&
          hipMemset(b->binflag, 0, sizeof(int) * (capTot + 1)) == hipSuccess &&
-         hipMemset(b->queue, 0, sizeof(int) * kQueueInts) == hipSuccess &&
-         hipStreamCreateWithFlags(&b->own, hipStreamNonBlocking) == hipSuccess;
+         hipMemset(b->queue, 0, sizeof(int) * kQueueInts) == hipSuccess;
     int dev = 0;
     if (ok && hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -911,12 +906,10 @@ int sph_batch_upload(sph_batch_t *b, const sph_state_t *st, void *stream) {
         hI[k].uh = uni ? hm[4 * (size_t)k] : 0.0;
     }
     HIPCHK(hipMemcpy(b->inst, hI.data(), sizeof(BInst) * b->K, hipMemcpyHostToDevice));
-    if (uni != b->uni) {  // another record format and pair kernel: recapture
+    if (uni != b->uni) {  // another record format and pair kernel
         b->uni = uni;
         b->queue_grid = 0;
-        for (auto &g : b->gexec)
-            if (g) hipGraphExecDestroy(g), g = nullptr;
-    }  // same form: the graphs read the constants from uniK, rewritten above
+    }
     return 0;
 }
 
@@ -937,60 +930,18 @@ int sph_batch_download(sph_batch_t *b, const sph_state_t *st, void *stream) {
     return 0;
 }
 
+// Launched one by one, whatever use_graph, as sph_step.
 int sph_batch_step(sph_batch_t *b, int64_t nsteps, int32_t use_graph, void *stream) {
+    (void)use_graph;
     if (!b) return fail(SPH_EINVAL, "batch is NULL");
     if (nsteps < 0) return fail(SPH_EINVAL, "nsteps < 0");
     if (!b->loaded) return fail(SPH_ESTATE, "no state: call sph_batch_upload first");
     size_queue(b);
-    hipStream_t s = (hipStream_t)stream;
-    if (!use_graph || b->timing) {
-        for (int64_t k = 0; k < nsteps; ++k) {
-            int rc = b_step(b, s);
-            if (rc) return rc;
-        }
-        return 0;
+    for (int64_t k = 0; k < nsteps; ++k) {
+        int rc = b_step(b, (hipStream_t)stream);
+        if (rc) return rc;
     }
-    hipStream_t g = b->own;
-    hipEvent_t e0, e1;
-    HIPCHK(hipEventCreateWithFlags(&e0, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&e1, hipEventDisableTiming));
-    HIPCHK(hipEventRecord(e0, s));
-    HIPCHK(hipStreamWaitEvent(g, e0, 0));
-    int rc = 0;
-    if (!b->dt_fresh && nsteps > 0) {
-        rc = b_step(b, g);
-        --nsteps;
-    }
-    for (int64_t k = 0; k < nsteps && !rc; ++k) {
-        const int start = b->cur;
-        if (!b->gexec[start]) {
-            // the capture ends, and the graph is released, whatever fails
-            hipGraph_t graph = nullptr;
-            hipError_t ce = hipStreamBeginCapture(g, hipStreamCaptureModeThreadLocal);
-            if (ce != hipSuccess) {
-                rc = fail(SPH_EHIP, "begin capture: %s", hipGetErrorString(ce));
-                break;
-            }
-            rc = b_step(b, g);
-            ce = hipStreamEndCapture(g, &graph);
-            b->cur = start;  // capture flipped it without running anything
-            if (!rc && ce != hipSuccess) rc = fail(SPH_EHIP, "end capture: %s", hipGetErrorString(ce));
-            if (!rc && (ce = hipGraphInstantiate(&b->gexec[start], graph, nullptr, nullptr, 0)) != hipSuccess) {
-                b->gexec[start] = nullptr;
-                rc = fail(SPH_EHIP, "graph instantiate: %s", hipGetErrorString(ce));
-            }
-            if (graph) hipGraphDestroy(graph);
-            if (rc) break;
-        }
-        hipError_t le = hipGraphLaunch(b->gexec[start], g);
-        if (le != hipSuccess) rc = fail(SPH_EHIP, "graph launch: %s", hipGetErrorString(le));
-        else b->cur = 1 - start;
-    }
-    hipEventRecord(e1, g);
-    hipStreamWaitEvent(s, e1, 0);
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    return rc;
+    return 0;
 }
 
 int sph_batch_status(sph_batch_t *b, double *out_d, int64_t *out_i, void *stream) {
@@ -1020,8 +971,6 @@ int sph_batch_set_tuning(sph_batch_t *b, int32_t pair_threads) {
     if (pair_threads != b->pair_threads) {
         b->pair_threads = pair_threads;
         b->queue_grid = 0;
-        for (auto &g : b->gexec)
-            if (g) hipGraphExecDestroy(g), g = nullptr;
     }
     return 0;
 }
@@ -1033,8 +982,6 @@ int sph_batch_set_list_len(sph_batch_t *b, int32_t list_len) {
     if (list_len != b->list_len) {
         b->list_len = list_len;
         b->queue_grid = 0;
-        for (auto &g : b->gexec)
-            if (g) hipGraphExecDestroy(g), g = nullptr;
     }
     return 0;
 }
@@ -1045,8 +992,6 @@ int sph_batch_set_persistent(sph_batch_t *b, int32_t on) {
     if (on != b->persistent) {
         b->persistent = on;
         b->queue_grid = 0;
-        for (auto &g : b->gexec)
-            if (g) hipGraphExecDestroy(g), g = nullptr;
     }
     return 0;
 }
@@ -1054,8 +999,6 @@ int sph_batch_set_persistent(sph_batch_t *b, int32_t on) {
 int sph_batch_set_border_bounds(sph_batch_t *b, int32_t on) {
     if (!b) return fail(SPH_EINVAL, "batch is NULL");
     b->border_bounds = on ? 1 : 0;
-    for (auto &g : b->gexec)
-        if (g) hipGraphExecDestroy(g), g = nullptr;
     return 0;
 }
 

@@ -30,12 +30,6 @@ struct sph_ctx {
     bool xs_fluid_zero = false;  // XSPH off and a reorder ran: the fluid's XSPH velocity reads as 0
     void *recA = nullptr, *recB = nullptr;  // packed pair-pass records (Rec<double> / Rec<float>)
     int *slot_of = nullptr;
-    hipStream_t own = nullptr;
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
-    // bumped whenever values that captured graphs bake into kernel arguments
-    // (constants, launch shape) change; graphs captured under another value
-    // are stale
-    unsigned long long gen = 0;
     int pair_threads = 256;
     int pair_staging = 1;  // the uniform float pair passes stage each workgroup's records in LDS
     int border_bounds = 1;  // the fused PEC step's bounds from the border cells when the displacement allows
@@ -104,11 +98,6 @@ struct sph_tape {
     double *amax_v = nullptr;  // argmax partials (value, id) per workgroup
     int *amax_i = nullptr;
     int *force_steps = nullptr;  // device counter: reversed steps whose dt came from the force criterion
-    // captured steps of sph_adjoint_segment: recording per (slot, buffer
-    // parity), reversal per slot for the adjoint buffers in adj_key
-    std::vector<hipGraphExec_t> rec_exec, adj_exec;
-    sph_adjoint_t adj_key{};
-    unsigned long long gen = 0;  // the context's gen when the cached graphs were captured
 };
 
 namespace hipsph {
@@ -121,7 +110,6 @@ Phys make_phys(const sph_params_t &P);
 int tape_record_pair(sph_ctx *c, sph_tape *t, int slot, hipStream_t s, bool lean);
 // The reverse of one recorded step (the kernels of sph_adjoint_step).
 int adjoint_launch(sph_ctx *c, sph_tape *t, int slot, const sph_adjoint_t *adj, hipStream_t s);
-void tape_drop_graphs(sph_tape *t);
 int tape_supported(const sph_ctx *c);
 int tape_refresh_labels(sph_ctx *c, sph_tape *t, hipStream_t s);
 

@@ -1114,7 +1114,6 @@ static void free_ctx(sph_ctx *c) {
     if (!c) return;
     for (int k = 0; k < 2; ++k) {
         if (c->arena[k]) hipFree(c->arena[k]);
-        if (c->gexec[k]) hipGraphExecDestroy(c->gexec[k]);
     }
     void *ptrs[] = {c->ctrl, c->dt_hist, c->bin, c->rank, c->perm, c->perm0, c->slots, c->cxy_s,
                     c->counts, c->cellStart, c->tileSums, c->binflag, c->part_b, c->part_d, c->part_k, c->recA, c->recB,
@@ -1123,7 +1122,6 @@ static void free_ctx(sph_ctx *c) {
         if (p) hipFree(p);
     for (auto e : c->ev_pair) hipEventDestroy(e);
     for (auto e : c->ev_nn) hipEventDestroy(e);
-    if (c->own) hipStreamDestroy(c->own);
     delete c;
 }
 
@@ -1340,10 +1338,6 @@ int sph_ctx_create(const sph_params_t *params, sph_ctx_t **out) {
         free_ctx(c);
         return fail(SPH_EHIP, "control block init failed");
     }
-    if (hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) != hipSuccess) {
-        free_ctx(c);
-        return fail(SPH_EHIP, "stream creation failed");
-    }
     *out = c;
     return 0;
 }
@@ -1372,12 +1366,6 @@ int sph_ctx_set_params(sph_ctx_t *ctx, const sph_params_t *params) {
     HIPCHK(hipMemcpy(&h, ctx->ctrl, sizeof h, hipMemcpyDeviceToHost));
     ctrl_from_params(h, ctx->P);
     HIPCHK(hipMemcpy(ctx->ctrl, &h, sizeof h, hipMemcpyHostToDevice));
-    for (int k = 0; k < 2; ++k)
-        if (ctx->gexec[k]) {
-            hipGraphExecDestroy(ctx->gexec[k]);
-            ctx->gexec[k] = nullptr;
-        }
-    ++ctx->gen;  // a tape's cached segment graphs hold the old constants
     return 0;
 }
 
@@ -1407,11 +1395,6 @@ int sph_state_upload(sph_ctx_t *ctx, const sph_state_t *st, int32_t reset_clock,
     h.disp = h.vbound = h.abound = INFINITY;
     ctrl_from_params(h, ctx->P);
     HIPCHK(hipMemcpy(ctx->ctrl, &h, sizeof h, hipMemcpyHostToDevice));
-    for (int k = 0; k < 2; ++k)
-        if (ctx->gexec[k]) {
-            hipGraphExecDestroy(ctx->gexec[k]);
-            ctx->gexec[k] = nullptr;
-        }
     return refresh_uniform(ctx, s);
 }
 
@@ -1464,22 +1447,9 @@ static UniformParams uniform_params(const sph_ctx *c) {
     return u;
 }
 
-static void drop_graphs(sph_ctx *c) {
-    for (int k = 0; k < 2; ++k)
-        if (c->gexec[k]) {
-            hipGraphExecDestroy(c->gexec[k]);
-            c->gexec[k] = nullptr;
-        }
-    ++c->gen;
-}
-
 // The h range of the state and the mass range of its fluid: one h and one
-// mass make the fused float pass uniform. Synchronises s; a change of form
-// drops the captured steps.
+// mass make the fused pass uniform. Synchronises s.
 static int refresh_uniform(sph_ctx *c, hipStream_t s) {
-    const int before = rec_format(c);
-    const bool static_before = c->static_hm;
-    const double h_before = c->uni_h, m_before = c->uni_m;
     // partials in the bounds buffer (free between updates), result in part_k
     const int R = redblk(c->n) < kBoundsBlocks ? redblk(c->n) : kBoundsBlocks;
     k_hm_range<<<R, kBlock, 0, s>>>(c->buf[c->cur], c->n, c->part_b);
@@ -1497,10 +1467,6 @@ static int refresh_uniform(sph_ctx *c, hipStream_t s) {
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s));
     }
-    // captured steps bake the one h and m into their kernels' arguments
-    if (rec_format(c) != before || c->static_hm != static_before ||
-        ((c->uni_hm || c->static_hm) && (c->uni_h != h_before || c->uni_m != m_before)))
-        drop_graphs(c);
     return 0;
 }
 
@@ -1755,37 +1721,6 @@ static int record_step(sph_ctx *ctx, sph_tape *tape, int slot, hipStream_t s) {
     return 0;
 }
 
-// Capture `body` on stream g into *exec. The capture always ends, and the
-// graph is released, whatever fails.
-extern "C++" template <typename F>
-static int capture_step(hipGraphExec_t *exec, hipStream_t g, F body) {
-    hipGraph_t graph = nullptr;
-    HIPCHK(hipStreamBeginCapture(g, hipStreamCaptureModeThreadLocal));
-    int rc = body();
-    hipError_t ce = hipStreamEndCapture(g, &graph);
-    if (!rc && ce != hipSuccess) rc = fail(SPH_EHIP, "end capture: %s", hipGetErrorString(ce));
-    if (!rc) {
-        ce = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
-        if (ce != hipSuccess) {
-            *exec = nullptr;
-            rc = fail(SPH_EHIP, "graph instantiate: %s", hipGetErrorString(ce));
-        }
-    }
-    if (graph) hipGraphDestroy(graph);
-    return rc;
-}
-
-// Capture `body` on stream g into *exec (once) and launch it.
-extern "C++" template <typename F>
-static int graph_launch(hipGraphExec_t *exec, hipStream_t g, F body) {
-    if (!*exec) {
-        int rc = capture_step(exec, g, body);
-        if (rc) return rc;
-    }
-    HIPCHK(hipGraphLaunch(*exec, g));
-    return 0;
-}
-
 int sph_adjoint_segment(sph_ctx_t *ctx, sph_tape_t *tape, int32_t nsteps, const sph_adjoint_t *adj, void *stream) {
     if (ctx && closed(ctx)) return SPH_ESTATE;
     if (!ctx || !tape || !adj) return fail(SPH_EINVAL, "NULL argument");
@@ -1796,39 +1731,10 @@ int sph_adjoint_segment(sph_ctx_t *ctx, sph_tape_t *tape, int32_t nsteps, const 
         return fail(SPH_EINVAL, "every sph_adjoint_t pointer is required");
     int rc = tape_supported(ctx);
     if (rc) return rc;
-    if (tape->gen != ctx->gen) {  // constants or launch shape changed since the capture: every graph is stale
-        tape_drop_graphs(tape);
-        tape->gen = ctx->gen;
-    }
-    if (std::memcmp(&tape->adj_key, adj, sizeof *adj) != 0) {  // other buffers: the reverse graphs are stale
-        for (auto &g : tape->adj_exec)
-            if (g) hipGraphExecDestroy(g), g = nullptr;
-        tape->adj_key = *adj;
-    }
-    hipStream_t s = S(stream), g = ctx->own;
-    hipEvent_t e0, e1;
-    HIPCHK(hipEventCreateWithFlags(&e0, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&e1, hipEventDisableTiming));
-    HIPCHK(hipEventRecord(e0, s));
-    HIPCHK(hipStreamWaitEvent(g, e0, 0));
-    rc = tape_refresh_labels(ctx, tape, g);
-    for (int k = 0; k < nsteps && !rc; ++k) {
-        if (!ctx->dt_fresh) {  // a captured step expects the corrector's dt partials
-            rc = record_step(ctx, tape, k, g);
-            continue;
-        }
-        const int start = ctx->cur;
-        rc = graph_launch(&tape->rec_exec[2 * (size_t)k + start], g, [&] { return record_step(ctx, tape, k, g); });
-        // a capture flips it without running; a launched step ends on the other buffer
-        ctx->cur = rc ? start : 1 - start;
-    }
-    for (int k = nsteps - 1; k >= 0 && !rc; --k)
-        rc = graph_launch(&tape->adj_exec[k], g, [&] { return adjoint_launch(ctx, tape, k, adj, g); });
-    // the caller's stream waits for whatever was queued, also after an error
-    hipEventRecord(e1, g);
-    hipStreamWaitEvent(s, e1, 0);
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
+    hipStream_t s = S(stream);
+    rc = tape_refresh_labels(ctx, tape, s);
+    for (int k = 0; k < nsteps && !rc; ++k) rc = record_step(ctx, tape, k, s);
+    for (int k = nsteps - 1; k >= 0 && !rc; --k) rc = adjoint_launch(ctx, tape, k, adj, s);
     return rc;
 }
 
@@ -1880,49 +1786,23 @@ int sph_correct(sph_ctx_t *ctx, void *stream) {
     return rc;
 }
 
+// The steps are launched one by one, whatever use_graph: on this runtime a
+// graph's node costs the GPU about 0.7 us more than a launch, and each graph
+// launch another 7 us (5k particles, per step: 54.8 us launched, 59.5 in
+// graphs of 8 steps, 62.3 in graphs of one; 1M: 179.6, 182.0 and 186). Six or
+// seven launches take the host 16 to 20 us, so the queue stays ahead of the
+// GPU.
 int sph_step(sph_ctx_t *ctx, int64_t nsteps, int32_t use_graph, void *stream) {
+    (void)use_graph;
     if (!ctx) return fail(SPH_EINVAL, "ctx is NULL");
     if (closed(ctx)) return SPH_ESTATE;
     if (nsteps < 0) return fail(SPH_EINVAL, "nsteps < 0");
     hipStream_t s = S(stream);
-    if (!use_graph || ctx->timing) {
-        for (int64_t k = 0; k < nsteps; ++k) {
-            int rc = one_step(ctx, s);
-            if (rc) return rc;
-        }
-        return 0;
+    for (int64_t k = 0; k < nsteps; ++k) {
+        int rc = one_step(ctx, s);
+        if (rc) return rc;
     }
-    // Graph path: one captured step per starting buffer (the step flips
-    // `cur`), replayed alternately on the context's own stream, ordered after
-    // and before the caller's stream with events.
-    hipStream_t g = ctx->own;
-    hipEvent_t e0, e1;
-    HIPCHK(hipEventCreateWithFlags(&e0, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&e1, hipEventDisableTiming));
-    HIPCHK(hipEventRecord(e0, s));
-    HIPCHK(hipStreamWaitEvent(g, e0, 0));
-    int rc = 0;
-    if (!ctx->dt_fresh && nsteps > 0) {  // the captured step expects the corrector's dt partials
-        rc = one_step(ctx, g);
-        --nsteps;
-    }
-    for (int64_t k = 0; k < nsteps && !rc; ++k) {
-        const int start = ctx->cur;
-        if (!ctx->gexec[start]) {
-            rc = capture_step(&ctx->gexec[start], g, [&] { return one_step(ctx, g); });
-            ctx->cur = start;  // capture flipped it without running anything
-            if (rc) break;
-        }
-        hipError_t le = hipGraphLaunch(ctx->gexec[start], g);
-        if (le != hipSuccess) rc = fail(SPH_EHIP, "graph launch: %s", hipGetErrorString(le));
-        else ctx->cur = 1 - start;
-    }
-    // the caller's stream waits for whatever was queued, also after an error
-    hipEventRecord(e1, g);
-    hipStreamWaitEvent(s, e1, 0);
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    return rc;
+    return 0;
 }
 
 // The loop body split at the coupling hook (src/Solver.py:389-392). The
@@ -2229,26 +2109,18 @@ int sph_ctx_set_tuning(sph_ctx_t *ctx, int32_t pair_threads) {
     if (pair_threads != 64 && pair_threads != 128 && pair_threads != 256)
         return fail(SPH_EINVAL, "pair_threads must be 64, 128 or 256");
     ctx->pair_threads = pair_threads;
-    for (int k = 0; k < 2; ++k)
-        if (ctx->gexec[k]) {
-            hipGraphExecDestroy(ctx->gexec[k]);
-            ctx->gexec[k] = nullptr;
-        }
-    ++ctx->gen;
     return 0;
 }
 
 int sph_ctx_set_pair_staging(sph_ctx_t *ctx, int32_t on) {
     if (!ctx) return fail(SPH_EINVAL, "ctx is NULL");
     ctx->pair_staging = on ? 1 : 0;
-    drop_graphs(ctx);
     return 0;
 }
 
 int sph_ctx_set_border_bounds(sph_ctx_t *ctx, int32_t on) {
     if (!ctx) return fail(SPH_EINVAL, "ctx is NULL");
     ctx->border_bounds = on ? 1 : 0;
-    drop_graphs(ctx);
     return 0;
 }
 

@@ -13,7 +13,7 @@
 //     ever visits it.
 //   * Control block (Ctrl): time, dt, step count, flags and the grid of the
 //     last update live on the device, so a whole step runs without a host
-//     round trip and can be captured in a hipGraph.
+//     round trip.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -7,7 +7,7 @@ fluid velocity field. The gradient comes from the adjoint kernels of
 libhipsph (``sph_step_record`` / ``sph_adjoint_step``), not from autograd:
 
 * forward: the state is saved every ``checkpoint_every`` steps (device
-  tensors), the steps themselves run as captured device steps;
+  tensors), the steps themselves run on the device without the host;
 * backward: for each segment, last first, the saved state is restored, the
   segment is recomputed while recording a tape (bit-identical to the forward:
   the engine is deterministic), and the recorded steps are reversed.
@@ -61,7 +61,7 @@ class Tape:
         call('sph_adjoint_step', self.engine._ctx, self._t, int(slot), C.byref(a), self.engine._stream())
 
     def segment(self, nsteps, adj, g_alpha, g_co):
-        """Record nsteps from the current state and reverse them (hipGraph replays)."""
+        """Record nsteps from the current state and reverse them, in one call."""
         a = self._adj(adj, g_alpha, g_co)
         call('sph_adjoint_segment', self.engine._ctx, self._t, int(nsteps), C.byref(a), self.engine._stream())
 
@@ -105,7 +105,7 @@ class SPHRun:
         self._tape = None
         self._ckpt = None
         self.force_steps = 0
-        # adjoint buffers kept for the run's lifetime (the reverse graphs bind them)
+        # adjoint buffers kept for the run's lifetime (no allocation per backward)
         self._adjbuf = {f: torch.zeros(self.n, dtype=torch.float64, device=self.device) for f in ADJ_FIELDS}
         self._gbuf = torch.zeros(2, dtype=torch.float64, device=self.device)
 

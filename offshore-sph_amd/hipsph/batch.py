@@ -3,7 +3,7 @@
 ``BatchEngine`` holds K instances of uneven particle counts (C ABI
 ``sph_batch_*``). Every stage of a step is one launch over all instances
 (segmented cell grid, per-instance clock, dt, grid and constants) and a step
-replays as one hipGraph; each instance evolves exactly as an ``Engine`` with
+needs no host round trip; each instance evolves exactly as an ``Engine`` with
 the same parameters would advance it alone.
 
 ``autotune(batch)`` picks the pair pass's launch shape for the batch's own
