@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/hipsph.h"
 
 namespace hipsph {
@@ -216,6 +218,37 @@ struct Phys {
 };
 
 struct BInst;
+
+// Lanes per target of the single-simulation pair passes (sph_pair_group.h) for
+// n particles; 0: one thread per target. A group shortens a target's serial
+// chain at about twice the instructions, so it pays while the chip is not
+// full, longest where the chain is longest (the Gaussian's 42 contributors,
+// the double terms of the general pass). Whole steps in us, one thread / 4 /
+// 8 / 16 lanes, on dam breaks:
+//   double uniform   6.5k 54.5 46.9 41.1 40.0; 23k 56.0 48.9 44.9 51.5;
+//                    44k 57.4 53.3 58.0 68.3; 60k 58.9 65.4 67.4 80.8
+//   float uniform    6.5k 47.3 41.5 38.6 37.6; 71k 53.9 51.1; 118k 56.4 61.3
+//   double Gaussian  6.5k 114 52 44 41; 332k 254 229; 617k 388 391
+//   float Gaussian   6.5k 77 45 40 38; 169k 92 84; 251k 101 104
+//   double general   6.5k 71 51 46 45; 86k 85 80; 118k 89 94
+//   float general    6.5k 64 49 44 43; 138k 82 78; 251k 98 106
+inline int group_lanes(long long n, bool f64, bool uniform, int kernel) {
+    const bool gauss = kernel == SPH_KERNEL_GAUSSIAN;
+    const long long most = !uniform ? (f64 ? 100000 : 150000)
+                           : gauss  ? (f64 ? 450000 : 200000)
+                                    : (f64 ? 48000 : 80000);
+    return n > most ? 0 : (n <= 16384 ? 16 : (n <= 32768 ? 8 : 4));
+}
+// Host: calls f with the group's lanes as a compile-time constant.
+template <typename F>
+inline void with_group(int lanes, F &&f) {
+    if (lanes == 16)
+        f(std::integral_constant<int, 16>{});
+    else if (lanes == 4)
+        f(std::integral_constant<int, 4>{});
+    else
+        f(std::integral_constant<int, 8>{});
+}
 
 // Launchers implemented in the pair translation units (threads: workgroup
 // size of the pair pass, 64, 128 or 256; chosen by the autotuner).

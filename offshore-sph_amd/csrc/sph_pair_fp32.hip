@@ -76,6 +76,21 @@ hipError_t launch_pair_fp32u(const Ctrl *ctrl, PairIn in, PairOut out, const Uni
     const UniformArgs P = uniform_args(in, out, n);
     UniformConst K;
     uniform_const_fp32(u, &K);
+    if (const int lanes = group_lanes(n, false, true, kernel)) {
+        const int nb = xcd_blocks((long long)n * lanes, 256);
+        with_kernel(kernel, [&](auto kk) {
+            with_group(lanes, [&](auto gg) {
+                constexpr int KN = decltype(kk)::value, G = decltype(gg)::value;
+                if (out.mode == kContinuity)
+                    k_group_uniform<KN, kContinuity, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                else if (out.mode == kMomentum)
+                    k_group_uniform<KN, kMomentum, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                else
+                    k_group_uniform<KN, kFused, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+            });
+        });
+        return hipGetLastError();
+    }
     const int nb = xcd_blocks(n, 256);
     with_kernel(kernel, [&](auto kk) {
         constexpr int KN = decltype(kk)::value;
@@ -94,6 +109,15 @@ hipError_t launch_pair_fp32u_pec(Ctrl *ctrl, PairIn in, PairOut out, const Unifo
     const UniformArgs P = uniform_args(in, out, n);
     UniformConst K;
     uniform_const_fp32(u, &K);
+    if (const int lanes = group_lanes(n, false, true, kernel)) {
+        const int nb = xcd_blocks((long long)n * lanes, 256);
+        with_kernel(kernel, [&](auto kk) {
+            with_group(lanes, [&](auto gg) {
+                k_group_uniform_pec<decltype(kk)::value, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+            });
+        });
+        return hipGetLastError();
+    }
     const int nb = xcd_blocks(n, 256);  // its dt partials: one per workgroup
     with_kernel(kernel, [&](auto kk) {
         k_pair_uniform_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);

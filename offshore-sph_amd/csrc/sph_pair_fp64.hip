@@ -63,6 +63,21 @@ hipError_t launch_pair_fp64u(const Ctrl *ctrl, PairIn in, PairOut out, const Uni
     const Uniform64Args P = uniform64_args(in, out, n);
     Uniform64Const K;
     uniform_const_fp64(u, &K);
+    if (const int lanes = group_lanes(n, true, true, kernel)) {
+        const int nb = xcd_blocks((long long)n * lanes, 256);
+        with_kernel(kernel, [&](auto kk) {
+            with_group(lanes, [&](auto gg) {
+                constexpr int KN = decltype(kk)::value, G = decltype(gg)::value;
+                if (out.mode == kContinuity)
+                    k_group_uniform64<KN, kContinuity, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                else if (out.mode == kMomentum)
+                    k_group_uniform64<KN, kMomentum, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                else
+                    k_group_uniform64<KN, kFused, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+            });
+        });
+        return hipGetLastError();
+    }
     const int nb = xcd_blocks(n, 256);
     with_kernel(kernel, [&](auto kk) {
         constexpr int KN = decltype(kk)::value;
@@ -81,6 +96,15 @@ hipError_t launch_pair_fp64u_pec(Ctrl *ctrl, PairIn in, PairOut out, const Unifo
     const Uniform64Args P = uniform64_args(in, out, n);
     Uniform64Const K;
     uniform_const_fp64(u, &K);
+    if (const int lanes = group_lanes(n, true, true, kernel)) {
+        const int nb = xcd_blocks((long long)n * lanes, 256);
+        with_kernel(kernel, [&](auto kk) {
+            with_group(lanes, [&](auto gg) {
+                k_group_uniform64_pec<decltype(kk)::value, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+            });
+        });
+        return hipGetLastError();
+    }
     const int nb = xcd_blocks(n, 256);  // its dt partials: one per workgroup
     with_kernel(kernel, [&](auto kk) {
         k_pair_uniform64_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);

@@ -873,21 +873,5 @@ hipError_t launch_pair_batch(const BInst *inst, const int *instOf, const PairArg
     return hipGetLastError();
 }
 
-template <typename R, bool EXACT>
-hipError_t launch_pair(const Ctrl *ctrl, const PairArgs<R> &P, const Phys &ph, int threads, int mode, hipStream_t s) {
-    if (threads != 64 && threads != 128 && threads != 256) threads = kPairThreads;
-    const int nb = xcd_blocks(P.n, threads);
-    const bool xs = P.xsx != nullptr;  // XSPH velocity requested (fused and momentum passes only)
-    if (mode == kContinuity)
-        launch_pair_mode<R, EXACT, kContinuity>(ctrl, P, ph, nb, threads, s);
-    else if (mode == kMomentum)
-        xs ? launch_pair_mode<R, EXACT, kMomentum, true>(ctrl, P, ph, nb, threads, s)
-           : launch_pair_mode<R, EXACT, kMomentum>(ctrl, P, ph, nb, threads, s);
-    else
-        xs ? launch_pair_mode<R, EXACT, kFused, true>(ctrl, P, ph, nb, threads, s)
-           : launch_pair_mode<R, EXACT, kFused>(ctrl, P, ph, nb, threads, s);
-    return hipGetLastError();
-}
-
 }  // namespace
 }  // namespace hipsph

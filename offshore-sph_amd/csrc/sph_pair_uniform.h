@@ -31,6 +31,7 @@
 //     registers), and the list of contributors advances by pointer.
 #pragma once
 #include "sph_common.h"
+#include "sph_pair_group.h"
 
 namespace hipsph {
 namespace {
@@ -618,6 +619,132 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_pec(const BInst *ins
     }
     v.store(C.part, NC, c, lds);
     if (c == 0 && threadIdx.x == 0 && C.mark) *C.mark = 1;
+}
+
+// ---------------------------------------------------------------------------
+// G lanes per target (sph_pair_group.h)
+// ---------------------------------------------------------------------------
+template <int KERNEL, int MODE>
+struct UniformGroup {
+    using RecA = double2;
+    using Term = float;
+    struct Sum {  // each float term into a double sum, as uniform_rates
+        double s = 0.0;
+        __device__ void add(float v) { s += (double)v; }
+        __device__ double get() const { return s; }
+    };
+    static constexpr bool kDesc = false, kCount = false;
+    static constexpr int NQ = 3;  // drho, momentum and wall force along x and y
+    const UniformArgs &P;
+    const UniformConst &K;
+    double X, Y;
+    float4 bt;
+    __device__ __forceinline__ RecA load(unsigned u) const { return at32(P.A, u); }
+    __device__ __forceinline__ bool test(const RecA &a, unsigned, bool &) const {
+        const double dx = X - a.x, dy = Y - a.y;
+        const double r2 = dx * dx + dy * dy;
+        bool in = r2 <= K.lim2 && r2 > 0.0;
+        if (KERNEL == SPH_KERNEL_GAUSSIAN && in && !(r2 < K.lo)) in = exact_q_test(X, Y, K.hd, a.x, a.y, K.hd, 3.0);
+        return in;
+    }
+    __device__ __forceinline__ void terms(unsigned u, float *out) const {
+        const double2 a = at32(P.A, u);
+        const float4 b = at32(P.B, u);
+        const float3 f = uniform_terms<KERNEL>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
+        if constexpr (MODE != kMomentum) out[0] = f.x;
+        if constexpr (MODE != kContinuity) {
+            out[1] = f.y;
+            out[2] = f.z;
+        }
+    }
+};
+
+// The rates of target t by its G lanes, in every lane; false: it has no
+// neighbour (or walks is false).
+template <int KERNEL, int MODE, int G>
+__device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformConst &K, int ncx, int ncy, int t,
+                                           const float4 &bt, bool walks, int l,
+                                           GroupMem<UniformGroup<KERNEL, MODE>, G> &M, double &drho, double &ax,
+                                           double &ay) {
+    using UG = UniformGroup<KERNEL, MODE>;
+    double2 at = make_double2(0.0, 0.0);
+    int2 c = make_int2(0, 0);
+    if (walks) {
+        at = P.A[t];
+        c = P.cxy[t];
+    }
+    const UG ug{P, K, at.x, at.y, bt};
+    GroupSums<UG, G> acc;
+    int cnt;
+    group_sums<UG, G>(ug, P.cellStart, c, ncx, ncy, 0, walks, l, M, acc, cnt);
+    drho = acc.get(0);
+    ax = acc.get(1);
+    const double say = acc.get(2);
+    ay = MODE == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
+    if (!walks) return false;
+    const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;  // it finds itself: a neighbour
+    return inside || uniform_count(P, K, at.x, at.y, c, ncx, ncy, 0) != 0;  // SolverTools.py:166-169
+}
+
+template <int KERNEL, int MODE, int G>
+__global__ __launch_bounds__(256) void k_group_uniform(const Ctrl *ctrl, UniformArgs P, UniformConst K) {
+    __shared__ GroupMem<UniformGroup<KERNEL, MODE>, G> mem[256 / G];
+    if (!ctrl->active) return;
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid(bt.w);
+    const Grid &g = ctrl->grid;
+    double drho, ax, ay;
+    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i], drho,
+                                                          ax, ay);
+    if (!any || l != 0) return;
+    if constexpr (MODE != kMomentum) P.drho[t] = drho;
+    if constexpr (MODE != kContinuity) {
+        P.ax[t] = ax;
+        P.ay[t] = ay;
+    }
+}
+
+// k_pair_uniform_pec with G lanes per target; the group's first lane corrects.
+template <int KERNEL, int G>
+__global__ __launch_bounds__(256) void k_group_uniform_pec(Ctrl *ctrl, UniformArgs P, UniformConst K, PecArgs C) {
+    __shared__ GroupMem<UniformGroup<KERNEL, kFused>, G> mem[256 / G];
+    __shared__ double lds[kDtQ * 16];
+    if (!ctrl->active) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctrl->dt_parts = kDtSlots;
+        ctrl->pec_parts = 1;
+    }
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid(bt.w);
+    const Grid &g = ctrl->grid;
+    const double dt = ctrl->dt, damping = ctrl->damping;
+    const bool corrects = walks && l == 0;
+    PecStart p0{};
+    if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
+    double drho, ax, ay;
+    const bool any = uniform_group_rates<KERNEL, kFused, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+                                                            drho, ax, ay);
+    DtVars v;
+    if (corrects) {
+        if (any) {
+            P.drho[t] = drho;
+            P.ax[t] = ax;
+            P.ay[t] = ay;
+        } else {
+            drho = P.drho[t];
+            ax = P.ax[t];
+            ay = P.ay[t];
+        }
+        v.add(C.hc.on ? C.hc.h : C.s.h[t], ax, ay);
+        pec_finish(C, t, p0, ax, ay, drho, dt, damping);
+    }
+    v.publish_slots(C.dslots, lds);
 }
 
 }  // namespace

@@ -24,6 +24,7 @@
 //     loaded before they are tested.
 #pragma once
 #include "sph_common.h"
+#include "sph_pair_group.h"
 
 namespace hipsph {
 namespace {
@@ -408,6 +409,178 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *i
     }
     v.store(C.part, NC, c, lds);
     if (c == 0 && threadIdx.x == 0 && C.mark) *C.mark = 1;
+}
+
+// ---------------------------------------------------------------------------
+// G lanes per target (sph_pair_group.h)
+// ---------------------------------------------------------------------------
+template <int KERNEL, int MODE>
+struct Uniform64Group {
+    using RecA = double2;
+    using Term = double;
+    using Sum = PlainSum;
+    static constexpr bool kDesc = true, kCount = true;  // counts every neighbour of a target outside the grid
+    static constexpr int NQ = 5;  // drho, momentum and wall force along x and y
+    const Uniform64Args &P;
+    const Uniform64Const &K;
+    double X, Y;
+    const double4 &bt;
+    bool counts;
+    __device__ __forceinline__ RecA load(unsigned u) const { return at32(P.A, u); }
+    __device__ __forceinline__ bool test(const RecA &a, unsigned, bool &counted) const {
+        const double dx = X - a.x, dy = Y - a.y;
+        const double r2 = dx * dx + dy * dy;
+        if (counts) {  // SolverTools.py:166-169
+            const double lim = (K.qmax * K.h) * (K.qmax * K.h);
+            counted = r2 < lim * (1.0 - 1e-12);
+            if (!counted && !(r2 > lim * (1.0 + 1e-12))) counted = exact_q_test(X, Y, K.h, a.x, a.y, K.h, K.qmax);
+        }
+        return r2 <= K.lim2 && r2 > 0.0;
+    }
+    // uniform64_rates' expressions for one listed pair
+    __device__ __forceinline__ void terms(unsigned u, double *out) const {
+        const double2 a = at32(P.A, u);
+        const double4 b = at32(P.B, u);
+        const double dx = X - a.x, dy = Y - a.y;
+        const double xij2 = dx * dx + dy * dy;
+        const double r = sqrt(xij2);
+        if (!not_fluid64(b.w)) {
+            const double qq = r / K.h;
+            double dwx, dwy;
+            if (KERNEL == SPH_KERNEL_GAUSSIAN) {
+                const double tmp = r * K.h;
+                if (!(tmp > 1e-12 && qq <= 3)) return;
+                const double dwdq = -2 * qq * K.alpha_k * exp(-qq * qq);
+                const double f = dwdq / tmp;
+                dwx = f * dx;
+                dwy = f * dy;
+            } else {
+                double grad;
+                if (KERNEL == SPH_KERNEL_WENDLAND) {
+                    if ((qq >= 2.0) || (r < 1e-10)) return;
+                    const double inner = 1.0 - 0.5 * qq;
+                    grad = ipow(inner, 5.0) * (-14.0 / 3.0) * qq * (1 + 2.5 * qq);
+                } else {
+                    if ((qq > 2.0) || (r < 1e-10)) return;
+                    grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
+                }
+                const double norm = K.alpha_k * grad / (K.h * r);
+                dwx = norm * dx;
+                dwy = norm * dy;
+            }
+            const double vx = bt.x - b.x, vy = bt.y - b.y;
+            const double dot = vx * dwx + vy * dwy;
+            if constexpr (MODE != kMomentum) out[0] = K.m * dot;
+            if constexpr (MODE == kContinuity) return;
+            const double dv = vx * dx + vy * dy;
+            double PI_ij = 0.0;
+            if (dv < 0) {
+                const double rhoij = 0.5 * (bt.z + b.z);
+                const double muij = K.h * dv / (r * r + K.c01);
+                const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
+                PI_ij = ppij / rhoij;
+            }
+            const double factor = bt.w + b.w + PI_ij;
+            out[1] = -K.m * factor * dwx;
+            out[2] = -K.m * factor * dwy;
+        } else if (MODE != kContinuity && !(r > K.r0) && r > 1e-12) {
+            const double frac = K.r0 / r;
+            const double tmp = ipow(frac, K.p1) - ipow(frac, K.p2);
+            const double fac = K.D * tmp;
+            out[3] = fac * dx / (r * r);
+            out[4] = fac * dy / (r * r);
+        }
+    }
+};
+
+// The rates of target t by its G lanes, in every lane; false: it has no
+// neighbour (or walks is false).
+template <int KERNEL, int MODE, int G>
+__device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy, int t,
+                                             const double4 &bt, bool walks, int l,
+                                             GroupMem<Uniform64Group<KERNEL, MODE>, G> &M, double &drho, double &ax,
+                                             double &ay) {
+    using UG = Uniform64Group<KERNEL, MODE>;
+    double2 at = make_double2(0.0, 0.0);
+    int2 c = make_int2(0, 0);
+    if (walks) {
+        at = P.A[t];
+        c = P.cxy[t];
+    }
+    // a target whose own cell is in the grid finds itself (q = 0)
+    const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;
+    const UG ug{P, K, at.x, at.y, bt, !inside};
+    GroupSums<UG, G> acc;
+    int cnt;
+    group_sums<UG, G>(ug, P.cellStart, c, ncx, ncy, 0, walks, l, M, acc, cnt);
+    drho = acc.get(0);
+    const double a0 = acc.get(1), a1 = acc.get(2), f0 = acc.get(3), f1 = acc.get(4);
+    ax = a0 + f0;
+    ay = MODE == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
+    return walks && (inside || cnt != 0);  // SolverTools.py:166-169
+}
+
+template <int KERNEL, int MODE, int G>
+__global__ __launch_bounds__(256) void k_group_uniform64(const Ctrl *ctrl, Uniform64Args P, Uniform64Const K) {
+    __shared__ GroupMem<Uniform64Group<KERNEL, MODE>, G> mem[256 / G];
+    if (!ctrl->active) return;
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid64(bt.w);
+    const Grid &g = ctrl->grid;
+    double drho, ax, ay;
+    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+                                                            drho, ax, ay);
+    if (!any || l != 0) return;
+    if constexpr (MODE != kMomentum) P.drho[t] = drho;
+    if constexpr (MODE != kContinuity) {
+        P.ax[t] = ax;
+        P.ay[t] = ay;
+    }
+}
+
+// k_pair_uniform64_pec with G lanes per target; the group's first lane
+// corrects.
+template <int KERNEL, int G>
+__global__ __launch_bounds__(256) void k_group_uniform64_pec(Ctrl *ctrl, Uniform64Args P, Uniform64Const K,
+                                                             PecArgs C) {
+    __shared__ GroupMem<Uniform64Group<KERNEL, kFused>, G> mem[256 / G];
+    __shared__ double lds[kDtQ * 16];
+    if (!ctrl->active) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctrl->dt_parts = kDtSlots;
+        ctrl->pec_parts = 1;
+    }
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid64(bt.w);
+    const Grid &g = ctrl->grid;
+    const double dt = ctrl->dt, damping = ctrl->damping;
+    const bool corrects = walks && l == 0;
+    PecStart p0{};
+    if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
+    double drho, ax, ay;
+    const bool any = uniform64_group_rates<KERNEL, kFused, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+                                                              drho, ax, ay);
+    DtVars v;
+    if (corrects) {
+        if (any) {
+            P.drho[t] = drho;
+            P.ax[t] = ax;
+            P.ay[t] = ay;
+        } else {
+            drho = P.drho[t];
+            ax = P.ax[t];
+            ay = P.ay[t];
+        }
+        v.add(C.hc.on ? C.hc.h : C.s.h[t], ax, ay);
+        pec_finish(C, t, p0, ax, ay, drho, dt, damping);
+    }
+    v.publish_slots(C.dslots, lds);
 }
 
 }  // namespace
