@@ -27,6 +27,8 @@ struct sph_ctx {
     bool dt_fresh = false;  // part_d holds the dt partials of the current state (left by the corrector)
     bool loaded = false;    // a state was uploaded: every id indexes 0 .. n-1
     bool mid = false;       // a split step is open (sph_step_begin ran, sph_step_end not yet)
+    bool x0_same = false;   // x0 ... rho0 are the state itself and are not in memory
+    bool xs_zero = false;   // no XSPH, and the state was given without an XSPH velocity: it is 0 everywhere
     bool xs_fluid_zero = false;  // XSPH off and a reorder ran: the fluid's XSPH velocity reads as 0
     void *recA = nullptr, *recB = nullptr;  // packed pair-pass records (Rec<double> / Rec<float>)
     int *slot_of = nullptr;
@@ -41,6 +43,7 @@ struct sph_ctx {
     // one h and one mass for every particle (walls included) and no dynamic
     // h: both buffers hold them in every slot and nothing permutes them
     bool static_hm = false;
+    double static_m = 0.0;
     int rec_fmt = 0;  // format of the records the last reorder wrote
     // timing of the pair pass and of the neighbour update
     bool timing = false;

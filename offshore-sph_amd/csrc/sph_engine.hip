@@ -647,6 +647,9 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
 // the grid may find none and keep its previous rates (SolverTools.py:166-169).
 // The raw cell of each slot (for the pair pass's 3x3 walk) is formed again
 // from the position the keys were computed from.
+// carry: keep x0 ... rho0 with the state (between a predictor and its
+// corrector; skipped where they are still the state itself, which saves 80 of
+// 263 bytes per particle).
 // pred as for upd_pos; xs: carry the XSPH velocity with the state; dyn:
 // dynamic h for the fluid, formed here, after the keys were binned with the
 // previous h (Solver._compute: nn.update :238, then computeH :242-246) and
@@ -656,7 +659,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
 // (bin_place), and perm[t] records the source slot for the corrector.
 __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *perm, const int *cellStart,
                           const int *binflag, int2 *cxy_s, Phys ph, int n, int fmt, void *recA, void *recB, int pred,
-                          int strict, int lean, int xs, int dyn, HmConst hc) {
+                          int strict, int lean, int xs, int dyn, HmConst hc, int carry) {
     // An inactive step (halted, or past the duration) still flips the
     // buffers on the host, so copy the state unpermuted.
     const int act = ctrl->active;
@@ -704,7 +707,7 @@ __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *p
             b.vy0[t] = vy0;
             b.rho0[t] = rho0;
         }
-    } else {
+    } else if (carry) {
         b.x0[t] = a.x0[s];
         b.y0[t] = a.y0[s];
         b.vx0[t] = a.vx0[s];
@@ -803,11 +806,11 @@ __global__ void k_fill_hm(State st, int n, double h, double m) {
 __global__ void k_upload(State d, sph_state_t in, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    d.x[i] = d.x0[i] = in.x[i];
-    d.y[i] = d.y0[i] = in.y[i];
-    d.vx[i] = d.vx0[i] = in.vx[i];
-    d.vy[i] = d.vy0[i] = in.vy[i];
-    d.rho[i] = d.rho0[i] = in.rho[i];
+    d.x[i] = in.x[i];
+    d.y[i] = in.y[i];
+    d.vx[i] = in.vx[i];
+    d.vy[i] = in.vy[i];
+    d.rho[i] = in.rho[i];
     d.ax[i] = in.ax ? in.ax[i] : 0.0;
     d.ay[i] = in.ay ? in.ay[i] : 0.0;
     d.drho[i] = in.drho ? in.drho[i] : 0.0;
@@ -817,6 +820,18 @@ __global__ void k_upload(State d, sph_state_t in, int n) {
     d.xsphx[i] = in.xsphx ? in.xsphx[i] : 0.0;
     d.xsphy[i] = in.xsphy ? in.xsphy[i] : 0.0;
     d.id[i] = i;
+}
+
+// x0 ... rho0 from the state (what an upload leaves there), before something
+// changes the state without a predictor.
+__global__ void k_save_start(State s, int n) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    s.x0[j] = s.x[j];
+    s.y0[j] = s.y[j];
+    s.vx0[j] = s.vx[j];
+    s.vy0[j] = s.vy[j];
+    s.rho0[j] = s.rho[j];
 }
 
 // Clock and flags of a restored state (device side, so a restore needs no
@@ -837,24 +852,46 @@ __device__ inline double xs_read(const State &s, const double *v, int t, int fz)
     return fz && s.label[t] == kFluid ? 0.0 : v[t];
 }
 
-__global__ void k_download(State s, sph_state_t out, Phys ph, int n, int fz) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+// The state in reference order, kDownloadFields fields per blockIdx.y. The
+// writes scatter (a slot's neighbours in its cell lie a column apart in the
+// caller's order): each XCD takes one contiguous range of slots, so that a
+// line's parts meet in its L2, and few fields at a time keep the lines being
+// filled within it (1M dam break: 134 -> 79 us). Fields that hold one value
+// (hc; the XSPH velocity where no state ever had one, xz) are written in
+// order.
+constexpr int kDownloadFields = 4;
+__global__ void k_download(State s, sph_state_t out, Phys ph, int n, int fz, int xz, HmConst hc) {
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    int i = s.id[t];
-    if (out.x) out.x[i] = s.x[t];
-    if (out.y) out.y[i] = s.y[t];
-    if (out.vx) out.vx[i] = s.vx[t];
-    if (out.vy) out.vy[i] = s.vy[t];
-    if (out.rho) out.rho[i] = s.rho[t];
-    if (out.ax) out.ax[i] = s.ax[t];
-    if (out.ay) out.ay[i] = s.ay[t];
-    if (out.drho) out.drho[i] = s.drho[t];
-    if (out.m) out.m[i] = s.m[t];
-    if (out.h) out.h[i] = s.h[t];
-    if (out.label) out.label[i] = s.label[t];
-    if (out.xsphx) out.xsphx[i] = xs_read(s, s.xsphx, t, fz);
-    if (out.xsphy) out.xsphy[i] = xs_read(s, s.xsphy, t, fz);
-    if (out.p) out.p[i] = tait_p(s.rho[t], s.label[t], ph.gamma, ph.B, ph.rho0, ph.Pb);
+    const int i = s.id[t];
+    switch (blockIdx.y) {
+        case 0:
+            if (out.x) out.x[i] = s.x[t];
+            if (out.y) out.y[i] = s.y[t];
+            if (out.vx) out.vx[i] = s.vx[t];
+            if (out.vy) out.vy[i] = s.vy[t];
+            break;
+        case 1:
+            if (out.rho) out.rho[i] = s.rho[t];
+            if (out.p) out.p[i] = tait_p(s.rho[t], s.label[t], ph.gamma, ph.B, ph.rho0, ph.Pb);
+            if (out.ax) out.ax[i] = s.ax[t];
+            if (out.ay) out.ay[i] = s.ay[t];
+            break;
+        case 2:
+            if (out.drho) out.drho[i] = s.drho[t];
+            if (out.m) out.m[hc.on ? t : i] = hc.on ? hc.m : s.m[t];
+            if (out.h) out.h[hc.on ? t : i] = hc.on ? hc.h : s.h[t];
+            if (out.label) out.label[i] = s.label[t];
+            break;
+        default:
+            if (xz) {
+                if (out.xsphx) out.xsphx[t] = 0.0;
+                if (out.xsphy) out.xsphy[t] = 0.0;
+                break;
+            }
+            if (out.xsphx) out.xsphx[i] = xs_read(s, s.xsphx, t, fz);
+            if (out.xsphy) out.xsphy[i] = xs_read(s, s.xsphy, t, fz);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1170,6 +1207,7 @@ static int check_params(const sph_params_t *P) {
 }
 
 static int refresh_uniform(sph_ctx *c, hipStream_t s);
+static HmConst hm_const(const sph_ctx *c);
 
 static void ctrl_from_params(Ctrl &h, const sph_params_t &P) {
     h.nm = P.coupled_integrator == SPH_COUPLED_NEWMARK;
@@ -1377,6 +1415,8 @@ int sph_state_upload(sph_ctx_t *ctx, const sph_state_t *st, int32_t reset_clock,
     ctx->dt_fresh = false;
     ctx->mid = false;
     ctx->xs_fluid_zero = false;
+    ctx->xs_zero = !ctx->P.use_xsph && !st->xsphx && !st->xsphy;
+    ctx->x0_same = true;
     k_upload<<<nblk(ctx->n), kBlock, 0, s>>>(ctx->buf[0], *st, ctx->n);
     HIPCHK(hipGetLastError());
     ctx->loaded = true;
@@ -1406,6 +1446,8 @@ int sph_state_restore(sph_ctx_t *ctx, const sph_state_t *st, double t, void *str
     ctx->dt_fresh = false;
     ctx->mid = false;
     ctx->xs_fluid_zero = false;
+    ctx->xs_zero = !ctx->P.use_xsph && !st->xsphx && !st->xsphy;
+    ctx->x0_same = true;
     k_upload<<<nblk(ctx->n), kBlock, 0, s>>>(ctx->buf[0], *st, ctx->n);
     k_restore_ctrl<<<1, 1, 0, s>>>(ctx->ctrl, t);
     HIPCHK(hipGetLastError());
@@ -1416,8 +1458,9 @@ int sph_state_restore(sph_ctx_t *ctx, const sph_state_t *st, double t, void *str
 int sph_state_download(sph_ctx_t *ctx, const sph_state_t *st, void *stream) {
     if (!ctx || !st) return fail(SPH_EINVAL, "NULL argument");
     if (unloaded(ctx)) return SPH_ESTATE;
-    k_download<<<nblk(ctx->n), kBlock, 0, S(stream)>>>(ctx->buf[ctx->cur], *st, make_phys(ctx->P), ctx->n,
-                                                        ctx->xs_fluid_zero);
+    const dim3 grid(xcd_blocks(ctx->n, kBlock), (14 + kDownloadFields - 1) / kDownloadFields);
+    k_download<<<grid, kBlock, 0, S(stream)>>>(ctx->buf[ctx->cur], *st, make_phys(ctx->P), ctx->n, ctx->xs_fluid_zero,
+                                            ctx->xs_zero, hm_const(ctx));
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1462,6 +1505,7 @@ static int refresh_uniform(sph_ctx *c, hipStream_t s) {
     c->uni_h = v[0];
     c->uni_m = v[2];
     c->static_hm = !c->P.dynamic_h && v[0] == v[1] && v[4] == v[5];
+    c->static_m = v[4];
     if (c->static_hm) {  // both buffers, every slot: the reorder will not write them
         for (int k = 0; k < 2; ++k) k_fill_hm<<<nblk(c->n), kBlock, 0, s>>>(c->buf[k], c->n, v[0], v[4]);
         HIPCHK(hipGetLastError());
@@ -1474,7 +1518,7 @@ static HmConst hm_const(const sph_ctx *c) {
     HmConst hc{};
     hc.on = c->static_hm && !c->P.dynamic_h;
     hc.h = c->uni_h;
-    hc.m = c->uni_m;
+    hc.m = c->static_m;  // uni_m where there is fluid
     return hc;
 }
 
@@ -1512,6 +1556,15 @@ static void nn_launch(const NnWork &w, const State &a, int n, int pred, const Hm
                                        w.slots.b);
 }
 
+// x0 ... rho0 in memory, for what reads them or changes the state under them.
+static int save_start(sph_ctx *c, hipStream_t s) {
+    if (!c->x0_same) return 0;
+    k_save_start<<<nblk(c->n), kBlock, 0, s>>>(c->buf[c->cur], c->n);
+    HIPCHK(hipGetLastError());
+    c->x0_same = false;
+    return 0;
+}
+
 // pred != 0: the PEC predictor runs inside the update (bounds and keys see
 // the predicted positions, the reorder writes the predicted state). fold: the
 // update opens a step (dt from the partials of the current state).
@@ -1534,8 +1587,9 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
     c->rec_fmt = rec_format(c);
     k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, a, b, c->perm0, c->perm, c->cellStart, c->binflag, c->cxy_s,
                                          make_phys(c->P), n, c->rec_fmt, c->recA, c->recB, pred, c->P.strict, lean,
-                                         c->P.use_xsph, c->P.dynamic_h, hc);
+                                         c->P.use_xsph, c->P.dynamic_h, hc, pred == 0 && !c->x0_same);
     HIPCHK(hipGetLastError());
+    if (pred) c->x0_same = false;
     if (!c->P.use_xsph) c->xs_fluid_zero = true;
     if (c->timing) {
         int rc = ev_record(c, c->ev_nn, c->n_nn, s);
@@ -1591,6 +1645,8 @@ static int compute(sph_ctx *c, hipStream_t s, int *count = nullptr, int mode = 0
         return 0;
     }
     if (sd) {
+        int rc = save_start(c, s);  // the sum replaces rho
+        if (rc) return rc;
         const SdOut so{st.rho, st.drho, c->recB};
         hipError_t e = f32 ? launch_sumden_fp32c(c->ctrl, in, so, ph, c->n, c->pair_threads, s)
                            : launch_sumden_fp64(c->ctrl, in, so, ph, c->n, c->pair_threads, s);
@@ -1626,6 +1682,7 @@ static int dt_step(sph_ctx *c, hipStream_t s) {
 
 static int predict(sph_ctx *c, hipStream_t s) {
     if (c->P.integrator != SPH_INTEGRATOR_PEC) return 0;  // Euler.predict is a no-op
+    c->x0_same = false;
     k_pec_predict<<<nblk(c->n), kBlock, 0, s>>>(c->ctrl, c->buf[c->cur], c->n, c->P.strict, c->P.use_xsph);
     HIPCHK(hipGetLastError());
     return 0;
@@ -1634,6 +1691,8 @@ static int predict(sph_ctx *c, hipStream_t s) {
 // lean: the step's reorder ran lean (start-of-step values from the previous
 // buffer through perm).
 static int correct(sph_ctx *c, hipStream_t s, bool lean = false) {
+    int rc = save_start(c, s);
+    if (rc) return rc;
     k_correct<<<redblk(c->n), kBlock, 0, s>>>(c->ctrl, c->buf[c->cur], c->buf[1 - c->cur],
                                               lean ? c->perm : nullptr, c->n, c->P.integrator, c->P.strict,
                                               c->P.use_xsph, c->part_d, hm_const(c));
@@ -1876,6 +1935,7 @@ int sph_state_scatter(sph_ctx_t *ctx, const int64_t *ids, int64_t k, const sph_s
     hipStream_t s = S(stream);
     int rc = stage_ids(ctx, ids, k, true, s);
     if (rc || k == 0) return rc;
+    if ((rc = save_start(ctx, s))) return rc;
     k_scatter_ids<<<nblk(k), kBlock, 0, s>>>(ctx->buf[ctx->cur], ctx->slot_of, ctx->bin, (int)k, *st);
     HIPCHK(hipGetLastError());
     ctx->dt_fresh = false;  // h or a may have changed under the corrector's dt partials
