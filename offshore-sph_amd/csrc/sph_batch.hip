@@ -5,15 +5,16 @@
 // share one concatenated, cell-ordered state and one segmented cell grid, and
 // every stage of the step is ONE launch covering all instances:
 //   * instance k owns particle slots [off_k, off_k + n_k) for good (its
-//     particles only ever move among its own slots) and the bins
-//     [cellBase_k, cellBase_k + ncells_k] of the grid, rebased every step by
-//     a scan over the instances of (ncells_k + 1);
-//   * reductions (bounds, dt) run over fixed chunks of one instance each and a
-//     workgroup per instance folds them;
-//   * keys, the prefix scan, scatter, bin sort, reorder and the pair pass are
-//     the single-simulation kernels with a per-particle instance lookup
-//     (the scan/scatter/sort kernels are literally shared, over the union of
-//     the instances' bins);
+//     particles only ever move among its own slots) and room for its most
+//     cells from a fixed bin on, so each instance's offsets are scanned from
+//     off_k without the others;
+//   * every workgroup works on one instance (tiles of 256 slots, chunks of
+//     1,024 for the bounds), whose control block it reads once;
+//   * reductions (bounds, dt) leave partials per chunk or tile, and the
+//     kernel that needs the result folds its instance's in every workgroup,
+//     as the single engine's k_bounds and k_keys do (24 dam breaks, 0.72M
+//     particles: the update's six kernels take 55 us, against 72 with
+//     kernels of their own for the folds, the bins' bases and the bin sort);
 //   * every instance has its own control block (BInst): clock, dt, grid,
 //     halt flags and constants (alpha, c0, B, r0, D ...).
 // A step needs no host round trip, like the single simulation's. The
@@ -34,10 +35,9 @@ using namespace hipsph;
 namespace {
 
 // Two segmentations of the slots, each segment inside one instance: chunks
-// of kChunk for the bounds reduction, tiles of kTile for the dt reduction,
-// the corrector and the uniform pair pass with the corrector fused in (one
-// 256-thread workgroup per tile).
-constexpr int kChunk = 2048;
+// of kChunk for the bounds reduction (one workgroup of kChunkThreads), tiles
+// of kTile for everything else (one 256-thread workgroup per tile).
+constexpr int kChunk = 1024, kChunkThreads = 512;
 constexpr int kTile = 256;
 static_assert(kTile == 256, "the fused batch pair pass runs one 256-thread workgroup per tile");
 
@@ -61,66 +61,36 @@ __global__ void kb_dt_partial(const int *cs, const int *segInst, const BInst *in
     v.store(part, NC, c, lds);
 }
 
-// One workgroup per instance: fold its chunks, open or close its step, and
-// carry the instance's bounds of the border-cell path as k_dt_final does
-// (view->pec_parts: the partials come from the fused PEC pass).
-__global__ void kb_dt_final(BInst *inst, const int *chunk0, const double *part, int NC, const Ctrl *view) {
-    __shared__ double lds[4 * 16];
-    BInst &I = inst[blockIdx.x];
-    const int c0 = chunk0[blockIdx.x], c1 = chunk0[blockIdx.x + 1];
-    const int kind[4] = {0, 1, 2, 2};
-    double v[4] = {INFINITY, -INFINITY, 0.0, 0.0};
-    for (int c = c0 + threadIdx.x; c < c1; c += blockDim.x) {
-        const double a = part[0 * NC + c], b = part[1 * NC + c];
+// One workgroup's fold of its instance's dt partials (tiles [t0, t1) of NT);
+// the result is valid in thread 0. lds holds kDtQ * 16 doubles.
+__device__ inline void bdt_fold(const double *part, int NT, int t0, int t1, double (&v)[kDtQ], double *lds) {
+    const int kind[kDtQ] = {0, 1, 2, 2};
+    v[0] = INFINITY;
+    v[1] = -INFINITY;
+    v[2] = v[3] = 0.0;
+    for (int c = t0 + threadIdx.x; c < t1; c += blockDim.x) {
+        const double a = part[0 * NT + c], b = part[1 * NT + c];
         v[0] = a < v[0] ? a : v[0];
         v[1] = b > v[1] ? b : v[1];
-        v[2] += part[2 * NC + c];
-        v[3] += part[3 * NC + c];
+        v[2] += part[2 * NT + c];
+        v[3] += part[3 * NT + c];
     }
-    block_fold<4>(v, kind, lds);
-    if (threadIdx.x != 0) return;
-    const int pec = view->pec_parts;
-    const double dt0 = I.dt, V = I.vbound, A0 = I.abound;
-    I.disp = I.vbound = I.abound = INFINITY;
-    const double mn = v[0], mx = v[1], cnt = v[2], bad = v[3];
-    const unsigned halt = SPH_FLAG_CAPACITY | SPH_FLAG_NONFINITE | SPH_FLAG_NO_FLUID | SPH_FLAG_ZERO_DENSITY;
-    if ((I.flags & halt) || !(I.t < I.duration)) {
-        I.active = 0;
-        return;
-    }
-    if (cnt == 0) {
-        I.flags |= SPH_FLAG_NO_FLUID;
-        I.active = 0;
-        return;
-    }
-    if (bad != 0) I.flags |= SPH_FLAG_NONFINITE;
-    double dt, c, f;
-    if (I.fixed_dt > 0.0) {
-        dt = I.fixed_dt;
-        c = 0.0;
-        f = 0.0;
-    } else {
-        c = I.gamma_c * mn / I.co;
-        f = (mx < 1e-12) ? 1e10 : I.gamma_f * sqrt(mn / mx);
-        dt = (f < c) ? f : c;
-        if (dt < 1e-6) I.flags |= SPH_FLAG_DT_SMALL;
-    }
-    I.dt = dt;
-    I.dt_c = c;
-    I.dt_f = f;
-    if (I.advance_t) I.t = I.t + dt;
-    I.step = I.step + 1;
-    I.active = 1;
-    if (bad == 0) {
-        const double A1 = sqrt(mx);
-        I.abound = A1;
-        if (pec) {
-            const double V1 = V + dt0 * A1;
-            const double d = dt0 * (V + 0.5 * dt0 * A0) + 0.5 * dt0 * V + 0.5 * dt * V1;
-            if (d == d) I.disp = d;
-            I.vbound = V1;
-        }
-    }
+    block_fold<kDtQ>(v, kind, lds);
+}
+
+// The decision takes effect (dt_commit, for an instance).
+__device__ inline void bdt_commit(BInst &I, const DtNext &x) {
+    I.disp = x.disp;
+    I.vbound = x.vbound;
+    I.abound = x.abound;
+    if (x.flags) atomicOr(&I.flags, x.flags);
+    I.active = x.active;
+    if (!x.active) return;
+    I.dt = x.dt;
+    I.dt_c = x.dt_c;
+    I.dt_f = x.dt_f;
+    I.t = x.t;
+    I.step = x.step;
 }
 
 // ---------------------------------------------------------------------------
@@ -138,24 +108,46 @@ __device__ inline void bupd_pos(const State &a, int i, bool pred, double dt, dou
     }
 }
 
-// Per chunk of 2048 slots (one instance's): the bounds' partials. With PEC's
-// predictor the full scan also finds the largest |vx|, |vy| (kb_grid keeps it
-// as the instance's vbound). With cellStart (the fused PEC step) and an
-// instance whose carried bound allows it (as the single engine's k_bounds),
-// the instance's chunks share the walk of its border cells instead.
-__global__ void kb_bounds(const int *cs, const int *chunkInst, const int *chunk0, BInst *inst, State a, int pec,
-                          double *part, const int *cellStart, Ctrl *view) {
+// Per chunk of 1,024 slots (one instance's): the fold of the instance's dt
+// partials and its decision (every workgroup needs dt; the first chunk's
+// leaves it in I.nx for kb_keys), then the bounds' partials of the chunk,
+// part[c * kBoundsVQ + q]. With PEC's predictor the full scan also finds the
+// largest |vx|, |vy| (kb_keys keeps it as the instance's vbound). With
+// cellStart (the fused PEC step) and an instance whose carried bound allows
+// it (as the single engine's k_bounds), the instance's chunks share the walk
+// of its border cells instead.
+__global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const int *chunkInst, const int *chunk0,
+                                                           const int *tile0, BInst *inst, State a, int pec,
+                                                           const double *part_d, int NT, double *part,
+                                                           const int *cellStart, Ctrl *view) {
     __shared__ double lds[kBoundsVQ * 16];
-    const int c = blockIdx.x, NC = gridDim.x;
-    if (c == 0 && threadIdx.x == 0) view->pec_parts = 0;  // kb_dt_final has read it
+    __shared__ double s_dt, s_disp;
+    __shared__ int s_active;
+    const int c = blockIdx.x;
+    if (c == 0 && threadIdx.x == 0) view->epoch += 1;
     const int k = chunkInst[c];
     BInst &I = inst[k];
-    const bool pred = pec && I.active;
+    {
+        const DtIn in(I, view->pec_parts);
+        double v[kDtQ];
+        bdt_fold(part_d, NT, tile0[k], tile0[k + 1], v, lds);
+        if (threadIdx.x == 0) {
+            const DtNext x = dt_decide(in, v, I.gamma_c, I.gamma_f);
+            s_dt = x.dt;
+            s_disp = x.disp;
+            s_active = x.active;
+            if (c == chunk0[k]) I.nx = x;
+        }
+        __syncthreads();
+    }
+    if (!s_active) return;
+    const double dt = s_dt;
+    const bool pred = pec != 0;
     double xmn = INFINITY, xmx = -INFINITY, ymn = INFINITY, ymx = -INFINITY, hmn = INFINITY, hmx = -INFINITY;
     double bad = 0.0, vmx = -INFINITY;
     auto take = [&](int i) {
         double xi, yi;
-        bupd_pos(a, i, pred, I.dt, xi, yi);
+        bupd_pos(a, i, pred, dt, xi, yi);
         const double hi = I.uh_on ? I.uh : a.h[i];
         if (!(xi - xi == 0.0) || !(yi - yi == 0.0)) bad += 1.0;
         xmn = xi < xmn ? xi : xmn;
@@ -165,7 +157,7 @@ __global__ void kb_bounds(const int *cs, const int *chunkInst, const int *chunk0
         hmn = hi < hmn ? hi : hmn;
         hmx = hi > hmx ? hi : hmx;
     };
-    if (cellStart && pred && I.uh_on && border_margin_ok(I.grid, I.disp)) {
+    if (cellStart && pred && I.uh_on && border_margin_ok(I.grid, s_disp)) {
         const int j = c - chunk0[k], nck = chunk0[k + 1] - chunk0[k];
         if (j == 0 && threadIdx.x == 0) I.border_updates += 1;
         hmn = hmx = I.uh;
@@ -183,128 +175,89 @@ __global__ void kb_bounds(const int *cs, const int *chunkInst, const int *chunk0
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
     double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
-    block_partials<kBoundsVQ>(v, kind, lds, part, NC, c);
+    __syncthreads();  // lds held the dt fold
+    block_fold<kBoundsVQ>(v, kind, lds);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < kBoundsVQ; ++q) part[c * kBoundsVQ + q] = v[q];
 }
 
-// One workgroup per instance: its grid (_get_cell_size :103-110,
-// _get_number_of_cells :112-127). A finished or halted instance gets
-// ncells = 0 (its particles park in its one bin).
-__global__ void kb_grid(BInst *inst, const int *chunk0, const double *part, int NC) {
-    __shared__ double lds[kBoundsVQ * 16];
-    BInst &I = inst[blockIdx.x];
-    const int c0 = chunk0[blockIdx.x], c1 = chunk0[blockIdx.x + 1];
-    const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
-    double v[kBoundsVQ] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY, 0.0, -INFINITY};
-    for (int c = c0 + threadIdx.x; c < c1; c += blockDim.x) {
-#pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q) {
-            const double u = part[q * NC + c];
-            v[q] = kind[q] == 0 ? (u < v[q] ? u : v[q]) : kind[q] == 1 ? (u > v[q] ? u : v[q]) : v[q] + u;
-        }
+// _bin :129-141 with the instance's grid; rank by runs as k_keys does. One
+// tile per workgroup, which derives its instance's grid from the chunks'
+// partials itself (32 lanes per quantity); the instance's first tile moves the grid and the dt decision into
+// its control block, whose fields no workgroup reads here (they take I.nx and
+// their own grid). An instance that is not active is left where it is.
+__global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileInst, const int *tile0,
+                                                 const int *chunk0, BInst *inst, State a, int pec, const double *part,
+                                                 int *counts, int *bin, int *rank, int *binflag, Ctrl *view) {
+    __shared__ double s_v[kBoundsVQ];
+    __shared__ Grid s_g;
+    __shared__ unsigned s_halt;
+    const int c = blockIdx.x;
+    if (c == 0 && threadIdx.x == 0) view->pec_parts = 0;  // kb_bounds has read it
+    const int k = tileInst[c];
+    BInst &I = inst[k];
+    const bool first = c == tile0[k];
+    if (!I.nx.active) {
+        if (first && threadIdx.x == 0) bdt_commit(I, I.nx);
+        return;
     }
-    block_fold<kBoundsVQ>(v, kind, lds);
-    if (threadIdx.x != 0) return;
-    if (I.active && v[7] >= 0.0) I.vbound = v[7];  // a full scan's velocity bound
-    Grid g = I.grid;
-    g.ncells = 0;
-    if (I.active) {
-        const double xmn = v[0], xmx = v[1], ymn = v[2], ymx = v[3], hmn = v[4], hmx = v[5], bad = v[6];
-        double cell_size = hmn * I.scale;
-        if (cell_size < 1e-6) cell_size = 1.0;
-        const double cell_size1 = 1. / cell_size;
-        const double fx = ceil(cell_size1 * (xmx - xmn));
-        const double fy = ceil(cell_size1 * (ymx - ymn));
-        if (bad != 0.0 || !(fx < 2.0e9) || !(fy < 2.0e9)) {
-            I.flags |= SPH_FLAG_NONFINITE;
-            I.active = 0;
-        } else {
-            long long ncx = (long long)fx, ncy = (long long)fy;
-            if (ncx < 1) ncx = 1;
-            if (ncy < 1) ncy = 1;
-            if (ncx * ncy > I.cap) {
-                I.flags |= SPH_FLAG_CAPACITY;
+    const int epoch = view->epoch;
+    const int t = ts[c] + (int)threadIdx.x;
+    const bool in = t < ts[c + 1];
+    const int lane = threadIdx.x & 63;
+    double x = 0.0, y = 0.0;
+    int id = 0x7fffffff;
+    if (in) {
+        bupd_pos(a, t, pec != 0, I.nx.dt, x, y);
+        id = a.id[t];
+    }
+    {  // 32 lanes per quantity fold the instance's chunks
+        const int q = threadIdx.x >> 5;
+        const bool mn = q == 0 || q == 2 || q == 4, sum = q == 6;
+        double u = mn ? INFINITY : (sum ? 0.0 : -INFINITY);
+        for (int j = chunk0[k] + (threadIdx.x & 31); j < chunk0[k + 1]; j += 32) {
+            const double w = part[j * kBoundsVQ + q];
+            u = mn ? (w < u ? w : u) : sum ? u + w : (w > u ? w : u);
+        }
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) {
+            const double w = __shfl_xor(u, o, 64);
+            u = mn ? (w < u ? w : u) : sum ? u + w : (w > u ? w : u);
+        }
+        if ((threadIdx.x & 31) == 0) s_v[q] = u;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        Grid g;
+        const unsigned halt = derive_grid(s_v, I.scale, I.cap, g);
+        s_halt = halt;
+        s_g = g;
+        if (first) {
+            bdt_commit(I, I.nx);
+            if (s_v[7] >= 0.0) I.vbound = s_v[7];  // a full scan's velocity bound
+            if (halt) {
+                atomicOr(&I.flags, halt);
                 I.active = 0;
             } else {
-                g.xmin = xmn;
-                g.xmax = xmx;
-                g.ymin = ymn;
-                g.ymax = ymx;
-                g.cs = cell_size;
-                g.uniform_h = hmn == hmx;
-                g.ncx = ncx;
-                g.ncy = ncy;
-                g.ncells = ncx * ncy;
+                I.grid = g;
             }
         }
     }
-    I.grid = g;
-}
-
-// Rebase the instances' bins (exclusive scan of ncells + 1) and publish the
-// union as one grid for the shared scan / scatter / bin-sort kernels.
-__global__ void kb_bases(BInst *inst, int K, Ctrl *view, long long capBins) {
-    __shared__ long long lds[16];
-    long long carry = 0;
-    for (int b0 = 0; b0 < K; b0 += blockDim.x) {
-        const int k = b0 + threadIdx.x;
-        long long v = k < K ? inst[k].grid.ncells + 1 : 0;
-        // inclusive scan in the wave, then across waves
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-        long long sc = v;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const long long u = __shfl_up(sc, o, 64);
-            if (lane >= o) sc += u;
-        }
-        if (lane == 63) lds[w] = sc;
-        __syncthreads();
-        long long off = 0, tot = 0;
-        for (int q = 0; q < nw; ++q) {
-            if (q < w) off += lds[q];
-            tot += lds[q];
-        }
-        __syncthreads();
-        if (k < K) inst[k].cellBase = carry + off + sc - v;
-        carry += tot;
-    }
-    if (threadIdx.x == 0) {
-        view->active = carry <= capBins;
-        if (carry > capBins) {  // cannot happen with per-instance caps summed into capBins; kept as a guard
-            for (int k = 0; k < K; ++k) {
-                inst[k].flags |= SPH_FLAG_CAPACITY;
-                inst[k].active = 0;
-            }
-        }
-        view->grid.ncells = carry - 1;
-    }
-}
-
-// _bin :129-141 with the instance's grid; rank by runs as k_keys does.
-__global__ void kb_keys(BInst *inst, const int *instOf, State a, int n, int pec, int *counts, int *bin,
-                        int *rank, int *binflag, const Ctrl *view) {
-    if (!view->active) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
+    __syncthreads();
+    if (s_halt) return;
+    const Grid &g = s_g;
     int b = -1;
-    if (t < n) {
-        BInst &I = inst[instOf[t]];
-        const Grid g = I.grid;
-        if (I.active) {
-            double x, y;
-            bupd_pos(a, t, pec != 0, I.dt, x, y);
-            const int2 c = cell_of(x, y, g);
-            const long long key = (long long)c.x + g.ncx * (long long)c.y;
-            if (key >= 0 && key < g.ncells) {
-                b = (int)(I.cellBase + key);
-            } else {  // as k_keys: the overflow bin, and the instance's flag
-                b = (int)(I.cellBase + g.ncells);
-                atomicOr(&I.flags, (unsigned)SPH_FLAG_OOB_KEY);
-            }
-        } else {
-            b = (int)I.cellBase;  // parked: the instance's single bin
+    if (in) {
+        const int2 cc = cell_of(x, y, g);
+        const long long key = (long long)cc.x + g.ncx * (long long)cc.y;
+        if (key >= 0 && key < g.ncells) {
+            b = (int)(I.cellBase + key);
+        } else {  // as k_keys: the overflow bin, and the instance's flag
+            b = (int)(I.cellBase + g.ncells);
+            atomicOr(&I.flags, (unsigned)SPH_FLAG_OOB_KEY);
         }
     }
-    const int id = t < n ? a.id[t] : 0x7fffffff;
     const int prev = __shfl_up(b, 1, 64);
     const int prev_id = __shfl_up(id, 1, 64);
     const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
@@ -315,13 +268,47 @@ __global__ void kb_keys(BInst *inst, const int *instOf, State a, int n, int pec,
     int base = 0;
     if (lane == leader && b >= 0) {
         base = atomicAdd(&counts[b], next - leader);
-        if (base != 0) binflag[b] = 1;
+        if (base != 0) binflag[b] = epoch;
     }
     base = __shfl(base, leader, 64);
-    if (t < n) {
+    if (in) {
         bin[t] = b;
         rank[t] = base + (lane - leader);
     }
+}
+
+// Each instance's offsets, scanned from its first slot by a number of
+// workgroups (scan_share): 8, or as many more as it takes to give each CU two
+// in a small batch (every workgroup reads the counts before its share again).
+inline int scan_shares(int K) { return K >= 64 ? 8 : (K >= 16 ? 16 : 32); }
+__global__ __launch_bounds__(kScanThreads) void kb_scan(const BInst *inst, const int *counts, int *cellStart) {
+    __shared__ int lds[16];
+    const BInst &I = inst[blockIdx.y];
+    if (!I.active) return;
+    const long long nbins = I.grid.ncells + 1;
+    int sum;
+    if (scan_share(counts + I.cellBase, cellStart + I.cellBase, nbins, blockIdx.x, gridDim.x, I.off, lds, sum) &&
+        threadIdx.x == 0)
+        cellStart[I.cellBase + nbins] = sum;
+}
+
+// Each particle's place (k_place); an instance that is not active keeps its
+// order. Also zeroes the instance's counts for the next update.
+__global__ __launch_bounds__(kTile) void kb_place(const int *ts, const int *tileInst, const int *tile0,
+                                                  const BInst *inst, const int *cellStart, const int *bin,
+                                                  const int *rank, int *perm0, int *counts) {
+    const int c = blockIdx.x, k = tileInst[c];
+    const BInst &I = inst[k];
+    const int t = ts[c] + (int)threadIdx.x;
+    const bool in = t < ts[c + 1];
+    if (!I.active) {
+        if (in) perm0[t] = t;
+        return;
+    }
+    const int j = c - tile0[k], nt = tile0[k + 1] - tile0[k];
+    for (long long b = j * kTile + (int)threadIdx.x; b <= I.grid.ncells; b += (long long)nt * kTile)
+        counts[I.cellBase + b] = 0;
+    if (in) perm0[cellStart[bin[t]] + rank[t]] = t;
 }
 
 // Permute the state into the new order with the PEC predictor of active
@@ -331,13 +318,16 @@ __global__ void kb_keys(BInst *inst, const int *instOf, State a, int n, int pec,
 // x, y, vx, vy, rho (kb_correct forms the half-step velocity again and
 // overwrites the rest), no rates of a particle inside its instance's grid
 // (written by the pair pass).
-__global__ void kb_reorder(BInst *inst, const int *instOf, State a, State b, const int *perm, int2 *cxy_s,
-                           int n, int fmt, void *recA, void *recB, int pec) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int k = instOf[t];  // slots never change instance
+__global__ __launch_bounds__(kTile) void kb_reorder(const int *ts, const int *tileInst, BInst *inst, State a, State b,
+                                                    const int *perm0, int *perm, const int *cellStart,
+                                                    const int *binflag, int2 *cxy_s, int fmt, void *recA, void *recB,
+                                                    int pec, const Ctrl *view) {
+    const int c = blockIdx.x, k = tileInst[c];
+    int t = ts[c] + (int)threadIdx.x;
+    if (t >= ts[c + 1]) return;
     const BInst &I = inst[k];
-    const int s = perm[t];
+    const int s = perm0[t];
+    const int id = a.id[s];
     const bool hs = I.uh_on;  // m and h stay in place (and m is not read: the uniform records have none)
     double x = a.x[s], y = a.y[s], vx = a.vx[s], vy = a.vy[s], rho = a.rho[s];
     const double m = hs ? 0.0 : a.m[s], h = hs ? I.uh : a.h[s];
@@ -353,9 +343,16 @@ __global__ void kb_reorder(BInst *inst, const int *instOf, State a, State b, con
         rho = pec_half_rho(rho, drho, dt, I.strict);
     }
     // x0 ... rho0 are not kept: nothing in a batch step reads them
-    // the raw cell the keys used (parked particles of an inactive instance: 0, 0)
+    // the raw cell the keys used (0, 0 in an inactive instance)
     const Grid &g = I.grid;
-    const int2 cc = I.active ? cell_of(x, y, g) : make_int2(0, 0);
+    int2 cc = make_int2(0, 0);
+    if (I.active) {
+        cc = cell_of(x, y, g);
+        const long long key = (long long)cc.x + g.ncx * (long long)cc.y;  // kb_keys' bin
+        t = bin_place(t, id, I.cellBase + (key >= 0 && key < g.ncells ? key : g.ncells), cellStart, binflag, view->epoch,
+                      perm0, a.id);
+    }
+    perm[t] = s;
     if (!skip) {
         b.x[t] = x;
         b.y[t] = y;
@@ -368,7 +365,7 @@ __global__ void kb_reorder(BInst *inst, const int *instOf, State a, State b, con
         b.h[t] = h;
     }
     b.label[t] = lab;
-    b.id[t] = a.id[s];
+    b.id[t] = id;
     if (!skip || !(cc.x >= 0 && cc.x < g.ncx && cc.y >= 0 && cc.y < g.ncy && h > 0.0 && I.qmax >= 0.0)) {
         b.ax[t] = ax;
         b.ay[t] = ay;
@@ -485,6 +482,10 @@ __global__ void kb_download(State s, sph_state_t out, const BInst *inst, const i
     if (out.p) out.p[i] = tait_p(s.rho[t], s.label[t], I.gamma, I.B, I.rho0, I.Pb);
 }
 
+// The bins an instance of at most cap cells needs, with the overflow bin and
+// the end of its slots, in whole 16-byte rows of counts.
+inline long long bin_room(long long cap) { return (cap + 2 + 3) / 4 * 4; }
+
 inline int nblk_b(long long n, int bs = kBlock) {
     long long b = (n + bs - 1) / bs;
     return (int)(b < 1 ? 1 : b);
@@ -507,9 +508,9 @@ struct sph_batch {
     int *instOf = nullptr, *cs = nullptr, *chunkInst = nullptr, *chunk0 = nullptr;
     int NT = 0;  // tiles: starts ts (NT + 1), instance of each, first tile of each instance (K + 1)
     int *ts = nullptr, *tileInst = nullptr, *tile0 = nullptr;
-    int *bin = nullptr, *rank = nullptr, *perm = nullptr, *permKey = nullptr;
+    int *bin = nullptr, *rank = nullptr, *perm0 = nullptr, *perm = nullptr;
     int2 *cxy_s = nullptr;
-    int *counts = nullptr, *cellStart = nullptr, *tileSums = nullptr, *binflag = nullptr;
+    int *counts = nullptr, *cellStart = nullptr, *binflag = nullptr;
     double *part_b = nullptr, *part_d = nullptr;
     void *recA = nullptr, *recB = nullptr;
     long long capBins = 0;
@@ -543,7 +544,7 @@ void free_batch(sph_batch *b) {
     }
     void *ptrs[] = {b->inst, b->view, b->instOf, b->cs, b->chunkInst, b->chunk0, b->ts, b->tileInst, b->tile0,
                     b->bin, b->rank, b->perm,
-                    b->permKey, b->cxy_s, b->counts, b->cellStart, b->tileSums, b->binflag,
+                    b->perm0, b->cxy_s, b->counts, b->cellStart, b->binflag,
                     b->part_b, b->part_d, b->recA, b->recB, b->queue, b->uniK, b->hm};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -564,37 +565,25 @@ void size_queue(sph_batch *b) {
     b->queue_grid = (b->cus > 0 ? b->cus : kXcds) * per;
 }
 
-int b_dt(sph_batch *b, hipStream_t s) {
-    if (!b->dt_fresh)
-        kb_dt_partial<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->inst, b->buf[b->cur], b->part_d, b->view);
-    kb_dt_final<<<b->K, kBlock, 0, s>>>(b->inst, b->tile0, b->part_d, b->NT, b->view);
-    HIPCHK(hipGetLastError());
-    return 0;
-}
-
 int b_nn(sph_batch *b, hipStream_t s) {
-    const int n = b->n, pec = b->integrator == SPH_INTEGRATOR_PEC;
+    const int pec = b->integrator == SPH_INTEGRATOR_PEC;
     State a = b->buf[b->cur], c = b->buf[1 - b->cur];
+    if (!b->dt_fresh)
+        kb_dt_partial<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->inst, a, b->part_d, b->view);
     // the border-cell bounds only in the fused PEC step's update
     const bool fused = b->uni && !b->persistent && pec;
-    kb_bounds<<<b->NC, kBlock, 0, s>>>(b->cs, b->chunkInst, b->chunk0, b->inst, a, pec, b->part_b,
-                                       fused && b->border_bounds ? b->cellStart : nullptr, b->view);
-    kb_grid<<<b->K, kBlock, 0, s>>>(b->inst, b->chunk0, b->part_b, b->NC);
-    kb_bases<<<1, 1024, 0, s>>>(b->inst, b->K, b->view, b->capBins);
-    kb_keys<<<nblk_b(n), kBlock, 0, s>>>(b->inst, b->instOf, a, n, pec, b->counts, b->bin, b->rank, b->binflag,
-                                         b->view);
-    long long tiles_cap = (b->capBins + kScanTile - 1) / kScanTile;
-    int tiles = (int)(tiles_cap < 1024 ? tiles_cap : 1024);
-    k_scan_reduce<<<tiles, kBlock, 0, s>>>(b->view, b->counts, b->tileSums);
-    k_scan_apply<<<tiles, kBlock, 0, s>>>(b->view, b->counts, b->tileSums, b->cellStart);
-    k_scatter<<<nblk_b(n), kBlock, 0, s>>>(b->view, b->cellStart, b->bin, b->rank, a.id, b->perm, b->permKey, n);
-    long long cb = (b->capBins + kBlock - 1) / kBlock;
-    k_cellsort<<<(int)(cb < kRedBlocks ? (cb < 1 ? 1 : cb) : kRedBlocks), kBlock, 0, s>>>(
-        b->view, b->cellStart, b->perm, b->permKey, b->binflag, b->bin, b->rank);
+    kb_bounds<<<b->NC, kChunkThreads, 0, s>>>(b->cs, b->chunkInst, b->chunk0, b->tile0, b->inst, a, pec, b->part_d,
+                                              b->NT, b->part_b, fused && b->border_bounds ? b->cellStart : nullptr,
+                                              b->view);
+    kb_keys<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->chunk0, b->inst, a, pec, b->part_b, b->counts,
+                                    b->bin, b->rank, b->binflag, b->view);
+    kb_scan<<<dim3(scan_shares(b->K), b->K), kScanThreads, 0, s>>>(b->inst, b->counts, b->cellStart);
+    kb_place<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->inst, b->cellStart, b->bin, b->rank, b->perm0,
+                                     b->counts);
     const int fmt = b->precision == SPH_PREC_FP32C ? (b->uni ? kRecUniform : kRecFp32)
                                                    : (b->uni ? kRecUniform64 : kRecFp64);
-    kb_reorder<<<nblk_b(n), kBlock, 0, s>>>(b->inst, b->instOf, a, c, b->perm, b->cxy_s, n, fmt, b->recA, b->recB,
-                                            pec);
+    kb_reorder<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->inst, a, c, b->perm0, b->perm, b->cellStart, b->binflag,
+                                       b->cxy_s, fmt, b->recA, b->recB, pec, b->view);
     HIPCHK(hipGetLastError());
     b->cur = 1 - b->cur;
     return 0;
@@ -649,7 +638,6 @@ int b_pair_pec(sph_batch *b, hipStream_t s) {
 
 int b_step(sph_batch *b, hipStream_t s) {
     int rc;
-    if ((rc = b_dt(b, s))) return rc;
     if ((rc = b_nn(b, s))) return rc;
     // timed: the pair pass and the corrector, fused or apart
     if (b->timing && (rc = b_mark(b, s))) return rc;
@@ -695,7 +683,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
             return fail(SPH_EINVAL, "instance %d: scale, qmax and rho0 must be positive", k);
         ntot += P.n;
         const long long cap = P.cell_capacity > 0 ? P.cell_capacity : P.n * 8 + 4096;
-        capTot += cap + 1;
+        capTot += bin_room(cap);
     }
     if (ntot > (1LL << 30)) return fail(SPH_EINVAL, "%lld particles in the batch (max 2^30)", ntot);
     if (capTot > (1LL << 31) - 16) return fail(SPH_EINVAL, "too many cells in the batch");
@@ -712,7 +700,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     // chunk and tile tables
     std::vector<int> cs, chunkInst, chunk0, ts, tileInst, tile0;
     std::vector<BInst> hI(ninst);
-    long long off = 0;
+    long long off = 0, base = 0;
     for (int k = 0; k < ninst; ++k) {
         const sph_params_t &P = params[k];
         chunk0.push_back((int)cs.size());
@@ -733,6 +721,8 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         I.active = 1;
         I.advance_t = 1;
         I.cap = P.cell_capacity > 0 ? P.cell_capacity : P.n * 8 + 4096;
+        I.cellBase = base;
+        base += bin_room(I.cap);
         I.duration = P.duration;
         I.fixed_dt = P.fixed_dt;
         I.damping = P.damping;
@@ -785,7 +775,6 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         p += n * sizeof(int);
         b->buf[k].label = (int8_t *)p;
     }
-    const long long tiles = (capTot + kScanTile - 1) / kScanTile;
     const size_t ra = b->precision == SPH_PREC_FP32C ? sizeof(Rec<float>::A) : sizeof(Rec<double>::A);
     // the uniform forms' records (16-B A, float4 / double4 B) fit in these
     const size_t rb = b->precision == SPH_PREC_FP32C ? sizeof(float4) : sizeof(Rec<double>::B);
@@ -802,11 +791,10 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMalloc(&b->tileInst, sizeof(int) * tileInst.size()) == hipSuccess &&
          hipMalloc(&b->tile0, sizeof(int) * tile0.size()) == hipSuccess &&
          hipMalloc(&b->bin, sizeof(int) * n) == hipSuccess && hipMalloc(&b->rank, sizeof(int) * n) == hipSuccess &&
-         hipMalloc(&b->perm, sizeof(int) * n) == hipSuccess && hipMalloc(&b->permKey, sizeof(int) * n) == hipSuccess &&
+         hipMalloc(&b->perm, sizeof(int) * n) == hipSuccess && hipMalloc(&b->perm0, sizeof(int) * n) == hipSuccess &&
          hipMalloc(&b->cxy_s, sizeof(int2) * n) == hipSuccess &&
          hipMalloc(&b->counts, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMalloc(&b->cellStart, sizeof(int) * (capTot + 2)) == hipSuccess &&
-         hipMalloc(&b->tileSums, sizeof(int) * (tiles + 1)) == hipSuccess &&
          hipMalloc(&b->binflag, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMalloc(&b->part_b, sizeof(double) * kBoundsVQ * b->NC) == hipSuccess &&
          hipMalloc(&b->part_d, sizeof(double) * kDtQ * b->NT) == hipSuccess &&

@@ -206,6 +206,109 @@ struct DtVars {
         }
     }
 };
+// Solver._minTimeStep (src/Solver.py:210-230): courant (TimeStep.py:47-49),
+// force (:51-56), min(c, f) (:45), from the folded fluid reduction v. Also
+// opens the step: the reference's loop condition `while self.t <
+// self.duration` (src/Solver.py:366) and `self.t += self.dt` (:409) move
+// here, so a step needs no host. It also bounds how far
+// this step's predictor puts any particle from where the last update binned
+// it (disp, for the border-cell bounds): after the fused PEC pass of the last
+// step (ctrl->pec_parts; dt0 its dt, V = ctrl->vbound its velocity bound at the
+// start, A0 = ctrl->abound its predictor's rates, A1 this fold's), a fluid
+// particle binned at x + dt0 v / 2 was corrected to x + dt0 vh, with |vh| <=
+// V + dt0 A0 / 2 (damping only shrinks it), and its new velocity v' has
+// |v'| <= V + dt0 A1, so per axis it now lies within dt0 (V + dt0 A0 / 2) +
+// dt0 V / 2 of where it was binned and this step's predictor moves it dt |v'|
+// / 2 further; V + dt0 A1 bounds the next step's start. Anything else (other
+// partials, non-finite rates, a halted step, a second call on the same
+// partials) leaves +inf: the next update scans every particle. Changes nothing
+// itself. C: the control block, or a batch instance with its ensemble's
+// pec_parts.
+struct DtIn {  // the control fields of the decision, loaded before the fold
+    double t, dt, dt_c, dt_f, duration, fixed_dt, co, V, A0;
+    long long step;
+    unsigned flags;
+    int advance_t, pec;
+    template <typename C>
+    __device__ DtIn(const C &c, int pec_parts)
+        : t(c.t), dt(c.dt), dt_c(c.dt_c), dt_f(c.dt_f), duration(c.duration), fixed_dt(c.fixed_dt), co(c.co),
+          V(c.vbound), A0(c.abound), step(c.step), flags(c.flags), advance_t(c.advance_t), pec(pec_parts) {}
+};
+__device__ inline DtNext dt_decide(const DtIn &in, const double *v, double gamma_c, double gamma_f) {
+    DtNext x;
+    x.t = in.t;
+    x.dt = in.dt;
+    x.dt_c = in.dt_c;
+    x.dt_f = in.dt_f;
+    x.step = in.step;
+    x.disp = x.vbound = x.abound = INFINITY;
+    x.flags = 0;
+    x.active = 0;
+    const double mn = v[0], mx = v[1], cnt = v[2], bad = v[3];
+    const unsigned halt = SPH_FLAG_CAPACITY | SPH_FLAG_NONFINITE | SPH_FLAG_NO_FLUID | SPH_FLAG_ZERO_DENSITY;
+    if ((in.flags & halt) || !(x.t < in.duration)) return x;
+    if (cnt == 0) {
+        x.flags = SPH_FLAG_NO_FLUID;
+        return x;
+    }
+    if (bad != 0) x.flags |= SPH_FLAG_NONFINITE;
+    double dt, c, f;
+    if (in.fixed_dt > 0.0) {
+        dt = in.fixed_dt;  // src/Solver.py:370-372
+        c = 0.0;
+        f = 0.0;
+    } else {
+        const double max_c = in.co;  // c = co for every fluid particle (WCSPH.py:110-129)
+        c = gamma_c * mn / max_c;
+        f = (mx < 1e-12) ? 1e10 : gamma_f * sqrt(mn / mx);
+        dt = (f < c) ? f : c;
+        if (dt < 1e-6) x.flags |= SPH_FLAG_DT_SMALL;  // src/Solver.py:220-224
+    }
+    const double dt0 = x.dt;
+    x.dt = dt;
+    x.dt_c = c;
+    x.dt_f = f;
+    if (in.advance_t) x.t = x.t + dt;
+    x.step = x.step + 1;
+    x.active = 1;
+    if (bad == 0) {
+        const double A1 = sqrt(mx);
+        x.abound = A1;
+        if (in.pec) {
+            const double V1 = in.V + dt0 * A1;
+            const double d = dt0 * (in.V + 0.5 * dt0 * in.A0) + 0.5 * dt0 * in.V + 0.5 * dt * V1;
+            if (d == d) x.disp = d;  // NaN: +inf
+            x.vbound = V1;
+        }
+    }
+    return x;
+}
+
+// _get_cell_size :103-110 and _get_number_of_cells :112-127 from the folded
+// bounds. Returns the halt flag (0: the grid is valid).
+__device__ inline unsigned derive_grid(const double *v, double scale, long long cap, Grid &g) {
+    const double xmn = v[0], xmx = v[1], ymn = v[2], ymx = v[3], hmn = v[4], hmx = v[5], bad = v[6];
+    g.xmin = xmn;
+    g.xmax = xmx;
+    g.ymin = ymn;
+    g.ymax = ymx;
+    double cell_size = hmn * scale;
+    if (cell_size < 1e-6) cell_size = 1.0;
+    g.cs = cell_size;
+    g.uniform_h = hmn == hmx;
+    double cell_size1 = 1. / cell_size;
+    double fx = ceil(cell_size1 * (xmx - xmn));
+    double fy = ceil(cell_size1 * (ymx - ymn));
+    if (bad != 0.0 || !(fx < 2.0e9) || !(fy < 2.0e9)) return SPH_FLAG_NONFINITE;
+    long long ncx = (long long)fx, ncy = (long long)fy;
+    if (ncx < 1) ncx = 1;
+    if (ncy < 1) ncy = 1;
+    g.ncx = ncx;
+    g.ncy = ncy;
+    g.ncells = ncx * ncy;
+    return g.ncells > cap ? SPH_FLAG_CAPACITY : 0u;
+}
+
 __device__ inline double pec_half_rho(double rho, double drho, double dt, int strict) {
     double r = rho + 0.5 * dt * drho;
     if (strict && r < 0.0) r = 0.0;
@@ -299,20 +402,16 @@ __global__ void k_scan_apply(const Ctrl *ctrl, int *counts, const int *tileSums,
     }
 }
 
-// The scan in one kernel of kScanBlocks workgroups, for a state small enough
-// that a launch costs more than reading counts again: workgroup i sums every
-// count before its share itself (nbins / 2 counts on average, from L2; 25k
-// bins of a 50k-particle tank: 3 loads of 16 bytes per thread), then scans its
-// share. counts is cleared by the next kernel (k_place): other workgroups
-// still read it here.
-constexpr int kScanBlocks = 64, kScanThreads = 1024;
-__global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, const int *counts, int *cellStart) {
-    if (!ctrl->active) return;
-    const long long nbins = ctrl->grid.ncells + 1;
-    __shared__ int lds[16];
-    const long long share = ((nbins + gridDim.x - 1) / gridDim.x + 3) / 4 * 4;
-    const long long b0 = blockIdx.x * share;
-    if (b0 >= nbins) return;
+// Share i of S of the exclusive scan of counts[0 .. nbins) (16-byte aligned)
+// into cellStart, from `first` on: the workgroup sums every count before its
+// share itself, then scans its share, four bins per thread. Returns whether
+// the share holds the last bin; sum is then the scan's total. lds holds 16
+// ints.
+__device__ inline bool scan_share(const int *counts, int *cellStart, long long nbins, int i, int S, int first, int *lds,
+                                  int &sum) {
+    const long long share = ((nbins + S - 1) / S + 3) / 4 * 4;
+    const long long b0 = i * share;
+    if (b0 >= nbins) return false;
     const long long b1 = b0 + share < nbins ? b0 + share : nbins;
     int pre = 0;
     constexpr int U = 8;  // loads in flight per thread
@@ -327,14 +426,37 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, con
     }
     int run, tot;
     block_scan_excl(pre, lds, &run);  // run: the sum before the share
-    for (long long b = b0; b < b1; b += blockDim.x) {
-        const long long k = b + threadIdx.x;
-        const int v = k < b1 ? counts[k] : 0;
-        const int ex = block_scan_excl(v, lds, &tot) + run;
-        if (k < b1) cellStart[k] = ex;
+    run += first;
+    for (long long b = b0; b < b1; b += step) {
+        const long long k = b + 4 * (long long)threadIdx.x;
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = k + u < b1 ? counts[k + u] : 0;
+        int ex = block_scan_excl(v[0] + v[1] + v[2] + v[3], lds, &tot) + run;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k + u < b1) cellStart[k + u] = ex;
+            ex += v[u];
+        }
         run += tot;
     }
-    if (b1 == nbins && threadIdx.x == 0) cellStart[nbins] = run;
+    sum = run;
+    return b1 == nbins;
+}
+
+// The scan in one kernel of kScanBlocks workgroups, for a state small enough
+// that a launch costs more than reading counts again (nbins / 2 counts per
+// workgroup on average, from L2; 25k bins of a 50k-particle tank: 3 loads of
+// 16 bytes per thread). counts is cleared by the next kernel (k_place): other
+// workgroups still read it here.
+constexpr int kScanBlocks = 64, kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, const int *counts, int *cellStart) {
+    if (!ctrl->active) return;
+    __shared__ int lds[16];
+    const long long nbins = ctrl->grid.ncells + 1;
+    int sum;
+    if (scan_share(counts, cellStart, nbins, blockIdx.x, gridDim.x, 0, lds, sum) && threadIdx.x == 0)
+        cellStart[nbins] = sum;
 }
 
 // Each particle's place from its bin's offset and its rank there: perm0 maps
@@ -396,108 +518,6 @@ __device__ inline int bin_place(int t, int my, long long b, const int *cellStart
     }
     for (; j < e; ++j) r += id[perm0[j]] < my;
     return s + r;
-}
-
-__global__ void k_scatter(const Ctrl *ctrl, const int *cellStart, const int *bin, const int *rank, const int *id,
-                          int *perm, int *permKey, int n) {
-    if (!ctrl->active) return;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    int pos = cellStart[bin[t]] + rank[t];
-    perm[pos] = t;
-    permKey[pos] = id[t];
-}
-
-// Sort the slots [s, e) of one bin by key (the reference index; keys are
-// distinct) with one wavefront: each element's destination is the number of
-// smaller keys in the bin. Bins of up to 64 sort in registers (one load and
-// one store round); larger ones rank through global memory and stage the
-// result in tmpKey/tmpVal before copying it back.
-__device__ void wave_sort_bin(int s, int e, int *perm, int *permKey, int *tmpKey, int *tmpVal) {
-    const int lane = threadIdx.x & 63;
-    const int len = e - s;
-    if (len <= 64) {
-        const int key = lane < len ? permKey[s + lane] : 0x7fffffff;
-        const int val = lane < len ? perm[s + lane] : 0;
-        int r = 0;
-        for (int j = 0; j < len; ++j) r += __shfl(key, j, 64) < key;
-        if (lane < len) {
-            permKey[s + r] = key;
-            perm[s + r] = val;
-        }
-        return;
-    }
-    for (int i = s + lane; i < e; i += 64) {
-        const int key = permKey[i];
-        int r = 0;
-        for (int j = s; j < e; ++j) r += permKey[j] < key;
-        tmpKey[s + r] = key;
-        tmpVal[s + r] = perm[i];
-    }
-    __threadfence_block();
-    for (int i = s + lane; i < e; i += 64) {
-        permKey[i] = tmpKey[i];
-        perm[i] = tmpVal[i];
-    }
-}
-
-// Order each bin by the reference index, which is what the reference's
-// head-inserted lists are ordered by (descending there; the pair pass walks
-// the bin backwards). Only bins flagged by k_keys (filled by more than one
-// run) can be out of order; most of them are cells whose run crossed a
-// wavefront boundary in k_keys. Each wavefront reads the flags of 64
-// consecutive bins and clears them; every lane sorts its own flagged bin.
-constexpr int kLaneSort = 16;  // bins up to this size are sorted by one lane
-
-__global__ void k_cellsort(const Ctrl *ctrl, const int *cellStart, int *perm, int *permKey, int *binflag,
-                           int *tmpKey, int *tmpVal) {
-    if (!ctrl->active) return;
-    const long long nbins = ctrl->grid.ncells + 1;
-    const int lane = threadIdx.x & 63;
-    const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
-    for (long long b0 = wave * 64; b0 < nbins; b0 += nwaves * 64) {
-        const long long bl = b0 + lane;
-        int f = 0;
-        if (bl < nbins) {
-            f = binflag[bl];
-            if (f) binflag[bl] = 0;
-        }
-        // Each lane sorts its own flagged bin of up to kLaneSort slots in
-        // registers (rank = number of smaller keys; cells hold ~3-9
-        // particles); longer bins go to the whole wavefront afterwards.
-        const bool own = f != 0;
-        int s = 0, len = 0;
-        if (own) {
-            s = cellStart[bl];
-            len = cellStart[bl + 1] - s;
-        }
-        if (own && len <= kLaneSort) {
-            int key[kLaneSort], val[kLaneSort];
-#pragma unroll
-            for (int i = 0; i < kLaneSort; ++i) {
-                key[i] = i < len ? permKey[s + i] : 0x7fffffff;
-                val[i] = i < len ? perm[s + i] : 0;
-            }
-#pragma unroll
-            for (int i = 0; i < kLaneSort; ++i) {
-                int r = 0;
-#pragma unroll
-                for (int j = 0; j < kLaneSort; ++j) r += key[j] < key[i];
-                if (i < len) {
-                    permKey[s + r] = key[i];
-                    perm[s + r] = val[i];
-                }
-            }
-        }
-        unsigned long long m = __ballot(own && len > kLaneSort);
-        while (m) {
-            const int k = __ffsll((long long)m) - 1;
-            m &= m - 1;
-            const long long b = b0 + k;
-            wave_sort_bin(cellStart[b], cellStart[b + 1], perm, permKey, tmpKey, tmpVal);
-        }
-    }
 }
 
 // _bin's cell of a position (src/Tools/NNLinkedList.py:146-176): floor of

@@ -75,82 +75,6 @@ __global__ void k_dt_partial(Ctrl *ctrl, const int8_t *label, const double *h, c
     v.publish(part, lds);
 }
 
-// Solver._minTimeStep (src/Solver.py:210-230): courant (TimeStep.py:47-49),
-// force (:51-56), min(c, f) (:45), from the folded fluid reduction v. Also
-// opens the step: the reference's loop condition `while self.t <
-// self.duration` (src/Solver.py:366) and `self.t += self.dt` (:409) move
-// here, so a step needs no host. It also bounds how far
-// this step's predictor puts any particle from where the last update binned
-// it (disp, for the border-cell bounds): after the fused PEC pass of the last
-// step (ctrl->pec_parts; dt0 its dt, V = ctrl->vbound its velocity bound at the
-// start, A0 = ctrl->abound its predictor's rates, A1 this fold's), a fluid
-// particle binned at x + dt0 v / 2 was corrected to x + dt0 vh, with |vh| <=
-// V + dt0 A0 / 2 (damping only shrinks it), and its new velocity v' has
-// |v'| <= V + dt0 A1, so per axis it now lies within dt0 (V + dt0 A0 / 2) +
-// dt0 V / 2 of where it was binned and this step's predictor moves it dt |v'|
-// / 2 further; V + dt0 A1 bounds the next step's start. Anything else (other
-// partials, non-finite rates, a halted step, a second call on the same
-// partials) leaves +inf: the next update scans every particle. Reads the
-// control block and changes nothing (dt_commit does).
-struct DtIn {  // the control fields of the decision, loaded before the fold
-    double t, dt, dt_c, dt_f, duration, fixed_dt, co, V, A0;
-    long long step;
-    unsigned flags;
-    int advance_t, pec;
-    __device__ explicit DtIn(const Ctrl *c)
-        : t(c->t), dt(c->dt), dt_c(c->dt_c), dt_f(c->dt_f), duration(c->duration), fixed_dt(c->fixed_dt), co(c->co),
-          V(c->vbound), A0(c->abound), step(c->step), flags(c->flags), advance_t(c->advance_t), pec(c->pec_parts) {}
-};
-__device__ inline DtNext dt_decide(const DtIn &in, const double *v, double gamma_c, double gamma_f) {
-    DtNext x;
-    x.t = in.t;
-    x.dt = in.dt;
-    x.dt_c = in.dt_c;
-    x.dt_f = in.dt_f;
-    x.step = in.step;
-    x.disp = x.vbound = x.abound = INFINITY;
-    x.flags = 0;
-    x.active = 0;
-    const double mn = v[0], mx = v[1], cnt = v[2], bad = v[3];
-    const unsigned halt = SPH_FLAG_CAPACITY | SPH_FLAG_NONFINITE | SPH_FLAG_NO_FLUID | SPH_FLAG_ZERO_DENSITY;
-    if ((in.flags & halt) || !(x.t < in.duration)) return x;
-    if (cnt == 0) {
-        x.flags = SPH_FLAG_NO_FLUID;
-        return x;
-    }
-    if (bad != 0) x.flags |= SPH_FLAG_NONFINITE;
-    double dt, c, f;
-    if (in.fixed_dt > 0.0) {
-        dt = in.fixed_dt;  // src/Solver.py:370-372
-        c = 0.0;
-        f = 0.0;
-    } else {
-        const double max_c = in.co;  // c = co for every fluid particle (WCSPH.py:110-129)
-        c = gamma_c * mn / max_c;
-        f = (mx < 1e-12) ? 1e10 : gamma_f * sqrt(mn / mx);
-        dt = (f < c) ? f : c;
-        if (dt < 1e-6) x.flags |= SPH_FLAG_DT_SMALL;  // src/Solver.py:220-224
-    }
-    const double dt0 = x.dt;
-    x.dt = dt;
-    x.dt_c = c;
-    x.dt_f = f;
-    if (in.advance_t) x.t = x.t + dt;
-    x.step = x.step + 1;
-    x.active = 1;
-    if (bad == 0) {
-        const double A1 = sqrt(mx);
-        x.abound = A1;
-        if (in.pec) {
-            const double V1 = in.V + dt0 * A1;
-            const double d = dt0 * (in.V + 0.5 * dt0 * in.A0) + 0.5 * dt0 * in.V + 0.5 * dt * V1;
-            if (d == d) x.disp = d;  // NaN: +inf
-            x.vbound = V1;
-        }
-    }
-    return x;
-}
-
 // The decision takes effect: clock, dt, bounds, flags and the dt series.
 __device__ inline void dt_commit(Ctrl *ctrl, const DtNext &x, double *hist) {
     ctrl->pec_parts = 0;  // these partials are used once
@@ -225,7 +149,7 @@ __global__ void k_dt_final(Ctrl *ctrl, double gamma_c, double gamma_f, double *h
                            const unsigned long long *dslots, double h1) {
     __shared__ double lds[kDtQ * 16];
     double v[kDtQ];
-    const DtIn in(ctrl);
+    const DtIn in(*ctrl, ctrl->pec_parts);
     dt_fold(ctrl->dt_parts, part, dslots, h1, v, lds);
     if (threadIdx.x == 0) dt_commit(ctrl, dt_decide(in, v, gamma_c, gamma_f), hist);
 }
@@ -428,7 +352,7 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
     double dt, disp;
     if (D.on) {
         double v[kDtQ];
-        const DtIn in(ctrl);
+        const DtIn in(*ctrl, ctrl->pec_parts);
         dt_fold(ctrl->dt_parts, D.part, D.dslots, D.h1, v, lds);
         if (threadIdx.x == 0) {
             const DtNext x = dt_decide(in, v, D.gamma_c, D.gamma_f);
@@ -497,31 +421,6 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
 #pragma unroll
         for (int q = 0; q < kBoundsVQ; ++q) atomicMax(p + q, order_key(v[q]));
     }
-}
-
-// _get_cell_size :103-110 and _get_number_of_cells :112-127 from the folded
-// bounds. Returns the halt flag (0: the grid is valid).
-__device__ inline unsigned derive_grid(const double *v, double scale, long long cap, Grid &g) {
-    const double xmn = v[0], xmx = v[1], ymn = v[2], ymx = v[3], hmn = v[4], hmx = v[5], bad = v[6];
-    g.xmin = xmn;
-    g.xmax = xmx;
-    g.ymin = ymn;
-    g.ymax = ymx;
-    double cell_size = hmn * scale;
-    if (cell_size < 1e-6) cell_size = 1.0;
-    g.cs = cell_size;
-    g.uniform_h = hmn == hmx;
-    double cell_size1 = 1. / cell_size;
-    double fx = ceil(cell_size1 * (xmx - xmn));
-    double fy = ceil(cell_size1 * (ymx - ymn));
-    if (bad != 0.0 || !(fx < 2.0e9) || !(fy < 2.0e9)) return SPH_FLAG_NONFINITE;
-    long long ncx = (long long)fx, ncy = (long long)fy;
-    if (ncx < 1) ncx = 1;
-    if (ncy < 1) ncy = 1;
-    g.ncx = ncx;
-    g.ncy = ncy;
-    g.ncells = ncx * ncy;
-    return g.ncells > cap ? SPH_FLAG_CAPACITY : 0u;
 }
 
 // _bin :129-141: cid = floor((x - xmin) / cs) per axis (:146-176), flat key

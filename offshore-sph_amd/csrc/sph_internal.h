@@ -306,9 +306,9 @@ hipError_t launch_sumden_fp32c(const Ctrl *ctrl, PairIn in, SdOut out, Phys ph, 
 
 // One simulation of a batched ensemble (device array, one per instance).
 // Instance k owns the particle slots [off, off + n) of the concatenated
-// cell-ordered state and the bins [cellBase, cellBase + grid.ncells] of the
-// segmented cell grid (the last one collects keys outside its grid; an
-// inactive instance has ncells = 0 and parks every particle there).
+// cell-ordered state and, from its fixed cellBase, room for its most cells:
+// the bins [cellBase, cellBase + grid.ncells] (the last one collects keys
+// outside its grid) and the end of the last one's slots.
 struct BInst {
     double t, dt, dt_c, dt_f;
     long long step;
@@ -330,6 +330,7 @@ struct BInst {
     // the bounds of the border-cell path, as Ctrl's disp, vbound, abound
     double disp, vbound, abound;
     long long border_updates;
+    DtNext nx;  // as Ctrl's
 };
 
 __host__ __device__ inline Phys inst_phys(const BInst &I) {
