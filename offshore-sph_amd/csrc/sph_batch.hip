@@ -524,6 +524,7 @@ struct sph_batch {
     // allows the uniform pass (found at upload): records kRecUniform(64) and
     // the uniform pair pass, each instance's constants in uniK
     bool uni = false;
+    bool whole = true;  // every instance's wall force exponents are whole numbers
     void *uniK = nullptr;
     double *hm = nullptr;  // per-instance h and fluid-mass ranges (4 per instance)
     int *queue = nullptr;  // its counters (9 x 32 ints), zero between launches
@@ -629,9 +630,9 @@ int b_pair_pec(sph_batch *b, hipStream_t s) {
     const PecArgs pec{st, b->buf[1 - b->cur], b->perm, b->part_d, nullptr, HmConst{}, 0, &b->view->pec_parts};
     hipError_t e = b->precision == SPH_PREC_FP32C
                        ? launch_pair_batch_fp32u_pec(b->inst, b->ts, b->tileInst, b->NT, in, out, b->uniK, b->kernel,
-                                                     b->n, pec, s)
+                                                     b->n, b->whole, pec, s)
                        : launch_pair_batch_fp64u_pec(b->inst, b->ts, b->tileInst, b->NT, in, out, b->uniK, b->kernel,
-                                                     b->n, pec, s);
+                                                     b->n, b->whole, pec, s);
     if (e != hipSuccess) return fail(SPH_EHIP, "batch pair launch: %s", hipGetErrorString(e));
     return 0;
 }
@@ -743,6 +744,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         I.gamma_c = P.gamma_c;
         I.gamma_f = P.gamma_f;
         I.strict = P.strict;
+        b->whole = b->whole && whole_exponent(P.p1) && whole_exponent(P.p2);
         I.kernel = P.kernel;
         b->offs.push_back((int)off);
         off += P.n;

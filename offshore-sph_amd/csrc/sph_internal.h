@@ -156,6 +156,13 @@ struct PecArgs {
 // The equations of a pair pass: all of them (continuity, momentum, wall
 // force, gravity), the continuity equation alone (drho) or the rest (ax, ay).
 constexpr int kFused = 0, kContinuity = 1, kMomentum = 2;
+// A pass's compile-time mode may carry kIntPow: the wall force's exponents p1
+// and p2 are whole numbers of 0 to 16 (the reference's 4 and 2), so the kernel
+// holds no pow(), whose inlined code otherwise sets the pass's registers
+// (double fused cubic pass: 117 vector registers and 39 spilled scalar ones
+// with it, 75 and 2 without; 500k particles, step 139 -> 131 us).
+constexpr int kIntPow = 8, kEquations = 3;  // MODE & kEquations: which equations
+inline bool whole_exponent(double p) { return p >= 0.0 && p <= 16.0 && p == (double)(int)p; }
 
 // Record formats written by the reorder: the double pass's, the general
 // float pass's, and the float pass's for one h and one fluid mass
@@ -239,6 +246,14 @@ inline int group_lanes(long long n, bool f64, bool uniform, int kernel) {
                                     : (f64 ? 48000 : 80000);
     return n > most ? 0 : (n <= 16384 ? 16 : (n <= 32768 ? 8 : 4));
 }
+// Host: calls f with kIntPow or 0 as a compile-time constant.
+template <typename F>
+inline void with_pow(bool whole, F &&f) {
+    if (whole)
+        f(std::integral_constant<int, kIntPow>{});
+    else
+        f(std::integral_constant<int, 0>{});
+}
 // Host: calls f with the group's lanes as a compile-time constant.
 template <typename F>
 inline void with_group(int lanes, F &&f) {
@@ -291,13 +306,14 @@ hipError_t launch_pair_batch_fp64u(const BInst *inst, const int *instOf, PairIn 
 // fused in: one 256-thread workgroup per chunk of one instance (slots
 // cs[c] .. cs[c + 1], c < NC, at most 256 each; chunkInst: the chunk's
 // instance); the partials go to pec.part[q * NC + c] (pec.strict is unused:
-// each instance's own).
+// each instance's own). whole: every instance's wall force exponents are
+// whole numbers (whole_exponent).
 hipError_t launch_pair_batch_fp32u_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC, PairIn in,
-                                       PairOut out, const void *Ks, int kernel, int n, const PecArgs &pec,
-                                       hipStream_t s);
+                                       PairOut out, const void *Ks, int kernel, int n, bool whole,
+                                       const PecArgs &pec, hipStream_t s);
 hipError_t launch_pair_batch_fp64u_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC, PairIn in,
-                                       PairOut out, const void *Ks, int kernel, int n, const PecArgs &pec,
-                                       hipStream_t s);
+                                       PairOut out, const void *Ks, int kernel, int n, bool whole,
+                                       const PecArgs &pec, hipStream_t s);
 int pair_batch_uniform_occupancy_fp32(int kernel);
 int pair_batch_uniform_occupancy_fp64(int kernel);
 // Summation density before the pair pass (src/Tools/SolverTools.py:129-140).
@@ -424,6 +440,19 @@ __device__ inline R ipow(R x, R p) {
     }
     if (p == R(0)) return R(1);
     return pow(x, p);
+}
+
+// ipow for the wall force of a pass of mode MODE.
+template <int MODE, typename R>
+__device__ inline R wall_pow(R x, R p) {
+    if constexpr ((MODE & kIntPow) != 0) {
+        const int n = (int)p;
+        R r = n > 0 ? x : R(1);
+        for (int k = 1; k < n; ++k) r = r * x;
+        return r;
+    } else {
+        return ipow(x, p);
+    }
 }
 
 }  // namespace hipsph

@@ -76,31 +76,32 @@ hipError_t launch_pair_fp32u(const Ctrl *ctrl, PairIn in, PairOut out, const Uni
     const UniformArgs P = uniform_args(in, out, n);
     UniformConst K;
     uniform_const_fp32(u, &K);
-    if (const int lanes = group_lanes(n, false, true, kernel)) {
+    const bool whole = whole_exponent(u.p1) && whole_exponent(u.p2);
+    if (const int lanes = whole ? group_lanes(n, false, true, kernel) : 0) {
         const int nb = xcd_blocks((long long)n * lanes, 256);
         with_kernel(kernel, [&](auto kk) {
             with_group(lanes, [&](auto gg) {
                 constexpr int KN = decltype(kk)::value, G = decltype(gg)::value;
                 if (out.mode == kContinuity)
-                    k_group_uniform<KN, kContinuity, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform<KN, kContinuity | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
                 else if (out.mode == kMomentum)
-                    k_group_uniform<KN, kMomentum, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform<KN, kMomentum | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
                 else
-                    k_group_uniform<KN, kFused, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform<KN, kFused | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
             });
         });
         return hipGetLastError();
     }
     const int nb = xcd_blocks(n, 256);
-    with_kernel(kernel, [&](auto kk) {
-        constexpr int KN = decltype(kk)::value;
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        constexpr int KN = decltype(kk)::value, W = decltype(ww)::value;
         if (out.mode == kContinuity)
-            k_pair_uniform<KN, kContinuity><<<nb, 256, 0, s>>>(ctrl, P, K);
+            k_pair_uniform<KN, kContinuity | W><<<nb, 256, 0, s>>>(ctrl, P, K);
         else if (out.mode == kMomentum)
-            k_pair_uniform<KN, kMomentum><<<nb, 256, 0, s>>>(ctrl, P, K);
+            k_pair_uniform<KN, kMomentum | W><<<nb, 256, 0, s>>>(ctrl, P, K);
         else
-            k_pair_uniform<KN, kFused><<<nb, 256, 0, s>>>(ctrl, P, K);
-    });
+            k_pair_uniform<KN, kFused | W><<<nb, 256, 0, s>>>(ctrl, P, K);
+    }); });
     return hipGetLastError();
 }
 
@@ -109,19 +110,20 @@ hipError_t launch_pair_fp32u_pec(Ctrl *ctrl, PairIn in, PairOut out, const Unifo
     const UniformArgs P = uniform_args(in, out, n);
     UniformConst K;
     uniform_const_fp32(u, &K);
-    if (const int lanes = group_lanes(n, false, true, kernel)) {
+    const bool whole = whole_exponent(u.p1) && whole_exponent(u.p2);
+    if (const int lanes = whole ? group_lanes(n, false, true, kernel) : 0) {
         const int nb = xcd_blocks((long long)n * lanes, 256);
         with_kernel(kernel, [&](auto kk) {
             with_group(lanes, [&](auto gg) {
-                k_group_uniform_pec<decltype(kk)::value, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+                k_group_uniform_pec<decltype(kk)::value, kFused | kIntPow, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
             });
         });
         return hipGetLastError();
     }
     const int nb = xcd_blocks(n, 256);  // its dt partials: one per workgroup
-    with_kernel(kernel, [&](auto kk) {
-        k_pair_uniform_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
-    });
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        k_pair_uniform_pec<decltype(kk)::value, kFused | decltype(ww)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+    }); });
     return hipGetLastError();
 }
 
@@ -159,13 +161,15 @@ int pair_batch_queue_occupancy_fp32c(int kernel, int list, int threads) {
 }
 
 hipError_t launch_pair_batch_fp32u_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC, PairIn in, PairOut out,
-                                       const void *Ks, int kernel, int n, const PecArgs &pec, hipStream_t s) {
+                                       const void *Ks, int kernel, int n, bool whole, const PecArgs &pec,
+                                       hipStream_t s) {
     const UniformArgs P = uniform_args(in, out, n);
     const UniformConst *K = (const UniformConst *)Ks;
     const int nb = (NC + kXcds - 1) / kXcds * kXcds;  // xcd_remap maps [0, nb) onto itself
-    with_kernel(kernel, [&](auto kk) {
-        k_pair_batch_uniform_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(inst, cs, chunkInst, NC, P, K, pec);
-    });
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        k_pair_batch_uniform_pec<decltype(kk)::value, kFused | decltype(ww)::value><<<nb, 256, 0, s>>>(
+            inst, cs, chunkInst, NC, P, K, pec);
+    }); });
     return hipGetLastError();
 }
 

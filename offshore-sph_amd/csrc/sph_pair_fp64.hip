@@ -42,6 +42,8 @@ void uniform_const_fp64(const UniformParams &u, void *out) {
     K.p2 = u.p2;
     K.g = u.g;
     K.qmax = u.qmax;
+    K.ih2 = 1.0 / (u.h * u.h);
+    K.g2 = -2.0 * u.alpha_k * K.ih2;
     *(Uniform64Const *)out = K;
 }
 
@@ -63,31 +65,32 @@ hipError_t launch_pair_fp64u(const Ctrl *ctrl, PairIn in, PairOut out, const Uni
     const Uniform64Args P = uniform64_args(in, out, n);
     Uniform64Const K;
     uniform_const_fp64(u, &K);
-    if (const int lanes = group_lanes(n, true, true, kernel)) {
+    const bool whole = whole_exponent(u.p1) && whole_exponent(u.p2);
+    if (const int lanes = whole ? group_lanes(n, true, true, kernel) : 0) {
         const int nb = xcd_blocks((long long)n * lanes, 256);
         with_kernel(kernel, [&](auto kk) {
             with_group(lanes, [&](auto gg) {
                 constexpr int KN = decltype(kk)::value, G = decltype(gg)::value;
                 if (out.mode == kContinuity)
-                    k_group_uniform64<KN, kContinuity, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform64<KN, kContinuity | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
                 else if (out.mode == kMomentum)
-                    k_group_uniform64<KN, kMomentum, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform64<KN, kMomentum | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
                 else
-                    k_group_uniform64<KN, kFused, G><<<nb, 256, 0, s>>>(ctrl, P, K);
+                    k_group_uniform64<KN, kFused | kIntPow, G><<<nb, 256, 0, s>>>(ctrl, P, K);
             });
         });
         return hipGetLastError();
     }
     const int nb = xcd_blocks(n, 256);
-    with_kernel(kernel, [&](auto kk) {
-        constexpr int KN = decltype(kk)::value;
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        constexpr int KN = decltype(kk)::value, W = decltype(ww)::value;
         if (out.mode == kContinuity)
-            k_pair_uniform64<KN, kContinuity><<<nb, 256, 0, s>>>(ctrl, P, K);
+            k_pair_uniform64<KN, kContinuity | W><<<nb, 256, 0, s>>>(ctrl, P, K);
         else if (out.mode == kMomentum)
-            k_pair_uniform64<KN, kMomentum><<<nb, 256, 0, s>>>(ctrl, P, K);
+            k_pair_uniform64<KN, kMomentum | W><<<nb, 256, 0, s>>>(ctrl, P, K);
         else
-            k_pair_uniform64<KN, kFused><<<nb, 256, 0, s>>>(ctrl, P, K);
-    });
+            k_pair_uniform64<KN, kFused | W><<<nb, 256, 0, s>>>(ctrl, P, K);
+    }); });
     return hipGetLastError();
 }
 
@@ -96,19 +99,20 @@ hipError_t launch_pair_fp64u_pec(Ctrl *ctrl, PairIn in, PairOut out, const Unifo
     const Uniform64Args P = uniform64_args(in, out, n);
     Uniform64Const K;
     uniform_const_fp64(u, &K);
-    if (const int lanes = group_lanes(n, true, true, kernel)) {
+    const bool whole = whole_exponent(u.p1) && whole_exponent(u.p2);
+    if (const int lanes = whole ? group_lanes(n, true, true, kernel) : 0) {
         const int nb = xcd_blocks((long long)n * lanes, 256);
         with_kernel(kernel, [&](auto kk) {
             with_group(lanes, [&](auto gg) {
-                k_group_uniform64_pec<decltype(kk)::value, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+                k_group_uniform64_pec<decltype(kk)::value, kFused | kIntPow, decltype(gg)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
             });
         });
         return hipGetLastError();
     }
     const int nb = xcd_blocks(n, 256);  // its dt partials: one per workgroup
-    with_kernel(kernel, [&](auto kk) {
-        k_pair_uniform64_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
-    });
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        k_pair_uniform64_pec<decltype(kk)::value, kFused | decltype(ww)::value><<<nb, 256, 0, s>>>(ctrl, P, K, pec);
+    }); });
     return hipGetLastError();
 }
 
@@ -157,13 +161,15 @@ int pair_batch_queue_occupancy_fp64(int kernel, int list, int threads) {
 }
 
 hipError_t launch_pair_batch_fp64u_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC, PairIn in, PairOut out,
-                                       const void *Ks, int kernel, int n, const PecArgs &pec, hipStream_t s) {
+                                       const void *Ks, int kernel, int n, bool whole, const PecArgs &pec,
+                                       hipStream_t s) {
     const Uniform64Args P = uniform64_args(in, out, n);
     const Uniform64Const *K = (const Uniform64Const *)Ks;
     const int nb = (NC + kXcds - 1) / kXcds * kXcds;  // xcd_remap maps [0, nb) onto itself
-    with_kernel(kernel, [&](auto kk) {
-        k_pair_batch_uniform64_pec<decltype(kk)::value><<<nb, 256, 0, s>>>(inst, cs, chunkInst, NC, P, K, pec);
-    });
+    with_kernel(kernel, [&](auto kk) { with_pow(whole, [&](auto ww) {
+        k_pair_batch_uniform64_pec<decltype(kk)::value, kFused | decltype(ww)::value><<<nb, 256, 0, s>>>(
+            inst, cs, chunkInst, NC, P, K, pec);
+    }); });
     return hipGetLastError();
 }
 

@@ -218,7 +218,7 @@ struct GeneralGroup {
             counted = in;
         }
         const bool apart = XS ? (r2 > R(0) || (int)u != T.slot) : r2 > R(0);
-        return in && apart && !(r2 > sup2) && (MODE != kContinuity || a.w >= R(0));
+        return in && apart && !(r2 > sup2) && ((MODE & kEquations) != kContinuity || a.w >= R(0));
     }
     __device__ __forceinline__ void terms(unsigned u, R *out) const {
         Sums<R> S;
@@ -277,8 +277,8 @@ __global__ __launch_bounds__(256) void k_pair_group(const Ctrl *ctrl, PairArgs<R
     }
     if (!walks || l != 0) return;
     if (!implied && cnt == 0) return;  // SolverTools.py:166-169: no neighbours, keep the previous values
-    if constexpr (MODE != kMomentum) P.drho[t] = arho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = arho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = a0 + f0;
         P.ay[t] = (a1 - ph.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
     }
@@ -303,28 +303,32 @@ void launch_group_mode(const Ctrl *ctrl, const PairArgs<R> &P, const Phys &ph, i
 template <typename R, bool EXACT>
 hipError_t launch_pair(const Ctrl *ctrl, const PairArgs<R> &P, const Phys &ph, int threads, int mode, hipStream_t s) {
     const bool xs = P.xsx != nullptr;  // XSPH velocity requested (fused and momentum passes only)
-    const int lanes = P.count ? 0 : group_lanes(P.n, sizeof(R) == 8, false, ph.kernel);
+    const bool whole = whole_exponent(ph.p1) && whole_exponent(ph.p2);
+    const int lanes = P.count || !whole ? 0 : group_lanes(P.n, sizeof(R) == 8, false, ph.kernel);
     if (lanes) {
         if (mode == kContinuity)
-            launch_group_mode<R, kContinuity>(ctrl, P, ph, lanes, s);
+            launch_group_mode<R, kContinuity | kIntPow>(ctrl, P, ph, lanes, s);
         else if (mode == kMomentum)
-            xs ? launch_group_mode<R, kMomentum, true>(ctrl, P, ph, lanes, s)
-               : launch_group_mode<R, kMomentum>(ctrl, P, ph, lanes, s);
+            xs ? launch_group_mode<R, kMomentum | kIntPow, true>(ctrl, P, ph, lanes, s)
+               : launch_group_mode<R, kMomentum | kIntPow>(ctrl, P, ph, lanes, s);
         else
-            xs ? launch_group_mode<R, kFused, true>(ctrl, P, ph, lanes, s)
-               : launch_group_mode<R, kFused>(ctrl, P, ph, lanes, s);
+            xs ? launch_group_mode<R, kFused | kIntPow, true>(ctrl, P, ph, lanes, s)
+               : launch_group_mode<R, kFused | kIntPow>(ctrl, P, ph, lanes, s);
         return hipGetLastError();
     }
     if (threads != 64 && threads != 128 && threads != 256) threads = kPairThreads;
     const int nb = xcd_blocks(P.n, threads);
-    if (mode == kContinuity)
-        launch_pair_mode<R, EXACT, kContinuity>(ctrl, P, ph, nb, threads, s);
-    else if (mode == kMomentum)
-        xs ? launch_pair_mode<R, EXACT, kMomentum, true>(ctrl, P, ph, nb, threads, s)
-           : launch_pair_mode<R, EXACT, kMomentum>(ctrl, P, ph, nb, threads, s);
-    else
-        xs ? launch_pair_mode<R, EXACT, kFused, true>(ctrl, P, ph, nb, threads, s)
-           : launch_pair_mode<R, EXACT, kFused>(ctrl, P, ph, nb, threads, s);
+    with_pow(whole, [&](auto ww) {
+        constexpr int W = decltype(ww)::value;
+        if (mode == kContinuity)
+            launch_pair_mode<R, EXACT, kContinuity | W>(ctrl, P, ph, nb, threads, s);
+        else if (mode == kMomentum)
+            xs ? launch_pair_mode<R, EXACT, kMomentum | W, true>(ctrl, P, ph, nb, threads, s)
+               : launch_pair_mode<R, EXACT, kMomentum | W>(ctrl, P, ph, nb, threads, s);
+        else
+            xs ? launch_pair_mode<R, EXACT, kFused | W, true>(ctrl, P, ph, nb, threads, s)
+               : launch_pair_mode<R, EXACT, kFused | W>(ctrl, P, ph, nb, threads, s);
+    });
     return hipGetLastError();
 }
 

@@ -138,18 +138,47 @@ __device__ inline bool cutoff_implied(const int *count, double qmax, int2 c, int
            h > 0.0;
 }
 
+// The reference's neighbour test in double (src/Tools/NNLinkedList.py:63-71),
+// contraction off whatever the translation unit's default.
+__device__ inline bool exact_q_test(double xi, double yi, double hi, double xj, double yj, double hj, double qmax) {
+#pragma clang fp contract(off)
+    const double dx = xi - xj, dy = yi - yj;
+    const double xij2 = dx * dx + dy * dy;
+    const double r = sqrt(xij2);
+    const double h_ij = 0.5 * (hi + hj);
+    const double q = r / h_ij;
+    return q <= qmax;
+}
+
+// The Gaussian's gradient factor f, grad W = f (dx, dy) (src/Kernels/
+// Gaussian.py:39-60): dW/dq / (r h) = -2 q alpha exp(-q^2) / (r h) with q = r /
+// h is -2 alpha / h^2 exp(-r^2 / h^2), which needs no square root and no
+// division per pair (ih2 = 1 / h^2, g2 = -2 alpha / h^2). The reference's
+// conditions, q <= 3 and r h > 1e-12, take its expressions where r^2 is
+// within rounding of the limit, so they decide as it does.
+__device__ inline bool gauss_factor(double r2, double h, double ih2, double g2, double &f) {
+    const double q2 = r2 * ih2;
+    if (!(q2 <= 9.0 * (1.0 - 1e-12))) {
+        if (!(q2 <= 9.0 * (1.0 + 1e-12))) return false;
+        if (!(sqrt(r2) / h <= 3)) return false;
+    }
+    if (r2 * (h * h) < 4e-24 && !(sqrt(r2) * h > 1e-12)) return false;
+    f = g2 * exp(-q2);
+    return true;
+}
+
 // Double gradient in the reference's expression order
 // (src/Kernels/CubicSpline.py:38-70, Gaussian.py:39-60, Wendland.py:32-64),
 // with h = h_ij, r = r_ij and q = r / h (the reference recomputes q = r / h in
 // the kernel: the same value). Returns false where the reference returns 0.
+// The Gaussian's is gauss_factor's instead: no order of its operations can
+// match the reference's bits, whose exp is another library's.
 template <int KERNEL>
-__device__ inline bool grad_exact(double dx, double dy, double r, double q, double h, double &dwx, double &dwy) {
+__device__ inline bool grad_exact(double dx, double dy, double r2, double r, double q, double h, double &dwx,
+                                  double &dwy) {
     if (KERNEL == SPH_KERNEL_GAUSSIAN) {
-        double tmp = r * h;
-        if (!(tmp > 1e-12 && q <= 3)) return false;
-        double alpha_c = (1.0 / kPI) / (h * h);
-        double dwdq = -2 * q * alpha_c * exp(-q * q);
-        double f = dwdq / tmp;
+        double f;
+        if (!gauss_factor(r2, h, 1.0 / (h * h), -2.0 * ((1.0 / kPI) / (h * h)) * (1.0 / (h * h)), f)) return false;
         dwx = f * dx;
         dwy = f * dy;
         return true;
@@ -190,18 +219,6 @@ __device__ inline float grad_norm_f(float r, float rinv, float q, float hinv) {
         const float grad = (q > 1.0f) ? -0.75f * (2.0f - q) * (2.0f - q) : -3.0f * q * (1.0f - 0.75f * q);
         return (float)(10.0 / (7.0 * kPI)) * hinv * hinv * grad * hinv * rinv;
     }
-}
-
-// The reference's neighbour test in double (src/Tools/NNLinkedList.py:63-71),
-// contraction off whatever the translation unit's default.
-__device__ inline bool exact_q_test(double xi, double yi, double hi, double xj, double yj, double hj, double qmax) {
-#pragma clang fp contract(off)
-    const double dx = xi - xj, dy = yi - yj;
-    const double xij2 = dx * dx + dy * dy;
-    const double r = sqrt(xij2);
-    const double h_ij = 0.5 * (hi + hj);
-    const double q = r / h_ij;
-    return q <= qmax;
 }
 
 template <typename R>
@@ -291,31 +308,32 @@ __device__ inline void contribute(const PairArgs<R> &P, const Target<R> &T, cons
         if (a.w >= 0) {
             const double q = r / hij;
             double dwx, dwy;
-            if (!grad_exact<KERNEL>(dx, dy, r, q, hij, dwx, dwy)) return;  // the reference adds exactly +-0
+            if (!grad_exact<KERNEL>(dx, dy, xij2, r, q, hij, dwx, dwy)) return;  // the reference adds exactly +-0
             const typename Rec<R>::B b = P.B[u];
             const double vx = (double)T.vx - (double)rec_vx(a, b), vy = (double)T.vy - (double)rec_vy(a, b);
             const double mj = (double)a.w;
-            if constexpr (MODE != kMomentum) {
+            if constexpr ((MODE & kEquations) != kMomentum) {
                 const double dot = vx * dwx + vy * dwy;
                 S.arho.add((R)(mj * dot));
             }
-            if constexpr (MODE == kContinuity) return;
+            if constexpr ((MODE & kEquations) == kContinuity) return;
             const double dv = vx * dx + vy * dy;
             double PI_ij = 0.0;
             if (dv < 0) {
                 const double hm = 0.5 * ((double)T.h + hij);
                 const double cij = 0.5 * (ph.co + 0.0);  // c_j is never filled: c_ij = c_i / 2
                 const double rhoij = 0.5 * ((double)T.rho + (double)b.rho);
-                const double muij = hm * dv / (r * r + 0.01 * hm * hm);
+                const double rr = KERNEL == SPH_KERNEL_GAUSSIAN ? xij2 : r * r;
+                const double muij = hm * dv / (rr + 0.01 * hm * hm);
                 const double ppij = muij * (ph.beta * muij - ph.alpha * cij);
                 PI_ij = ppij / rhoij;
             }
             const double factor = (double)T.slf + (double)b.prs + PI_ij;
             S.a0.add((R)(-mj * factor * dwx));
             S.a1.add((R)(-mj * factor * dwy));
-        } else if (MODE != kContinuity && !(r > ph.r0) && r > 1e-12) {
+        } else if ((MODE & kEquations) != kContinuity && !(r > ph.r0) && r > 1e-12) {
             const double frac = ph.r0 / r;
-            const double tmp = ipow(frac, ph.p1) - ipow(frac, ph.p2);
+            const double tmp = wall_pow<MODE>(frac, ph.p1) - wall_pow<MODE>(frac, ph.p2);
             const double fac = ph.D * tmp;
             S.f0.add((R)(fac * dx / (r * r)));
             S.f1.add((R)(fac * dy / (r * r)));
@@ -344,8 +362,8 @@ __device__ inline void contribute(const PairArgs<R> &P, const Target<R> &T, cons
             const float dwx = norm * dx, dwy = norm * dy;
             const float vx = (float)T.vx - (float)rec_vx(a, b), vy = (float)T.vy - (float)rec_vy(a, b);
             const float mj = (float)a.w;
-            if constexpr (MODE != kMomentum) S.arho.add(mj * (vx * dwx + vy * dwy));
-            if constexpr (MODE == kContinuity) return;
+            if constexpr ((MODE & kEquations) != kMomentum) S.arho.add(mj * (vx * dwx + vy * dwy));
+            if constexpr ((MODE & kEquations) == kContinuity) return;
             const float dv = vx * dx + vy * dy;
             float PI_ij = 0.0f;
             if (dv < 0.f) {
@@ -361,9 +379,9 @@ __device__ inline void contribute(const PairArgs<R> &P, const Target<R> &T, cons
             const float fm = -mj * ((float)T.slf + (float)b.prs + PI_ij);
             S.a0.add(fm * dwx);
             S.a1.add(fm * dwy);
-        } else if (MODE != kContinuity && !(r > (float)ph.r0) && r > 1e-12f) {
+        } else if ((MODE & kEquations) != kContinuity && !(r > (float)ph.r0) && r > 1e-12f) {
             const float frac = (float)ph.r0 * rinv;
-            const float tmp = ipow(frac, (float)ph.p1) - ipow(frac, (float)ph.p2);
+            const float tmp = wall_pow<MODE>(frac, (float)ph.p1) - wall_pow<MODE>(frac, (float)ph.p2);
             const float fac = (float)ph.D * tmp * (rinv * rinv);
             S.f0.add(fac * dx);
             S.f1.add(fac * dy);
@@ -454,7 +472,7 @@ __device__ inline int scan_cell(const PairArgs<R> &P, const Target<R> &T, const 
         // r = 0 pairs contribute exactly nothing (to XSPH they do, W(0) != 0,
         // unless it is the target itself); walls add nothing to continuity
         const bool apart = XS ? (r2 > R(0) || (int)u != T.slot) : r2 > R(0);
-        if (in && apart && !(r2 > sup2) && (MODE != kContinuity || a.w >= R(0))) {
+        if (in && apart && !(r2 > sup2) && ((MODE & kEquations) != kContinuity || a.w >= R(0))) {
             list[nlist * blockDim.x] = (unsigned)u;
             ++nlist;
             if constexpr (KERNEL != SPH_KERNEL_GAUSSIAN) {
@@ -545,8 +563,8 @@ __device__ inline void pair_target(const PairArgs<R> &P, const Phys &ph, int ncx
     flush<R, KERNEL, MODE>(P, T, ph, list, nlist, S);
     if (P.count) P.count[t] = cnt;
     if (!implied && cnt == 0) return;  // SolverTools.py:166-169: no neighbours, keep the previous values
-    if constexpr (MODE != kMomentum) P.drho[t] = S.arho.get();
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = S.arho.get();
+    if constexpr ((MODE & kEquations) != kContinuity) {
         const double a0 = S.a0.get(), a1 = S.a1.get(), f0 = S.f0.get(), f1 = S.f1.get();
         P.ax[t] = a0 + f0;
         P.ay[t] = (a1 - ph.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
@@ -589,8 +607,8 @@ __global__ __launch_bounds__(kPairThreads) void k_pair(const Ctrl *ctrl, PairArg
     flush<R, KERNEL, MODE, XS>(P, T, ph, list, nlist, S);
     if (P.count) P.count[t] = cnt;
     if (!implied && cnt == 0) return;  // SolverTools.py:166-169: no neighbours, keep the previous values
-    if constexpr (MODE != kMomentum) P.drho[t] = S.arho.get();
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = S.arho.get();
+    if constexpr ((MODE & kEquations) != kContinuity) {
         const double a0 = S.a0.get(), a1 = S.a1.get(), f0 = S.f0.get(), f1 = S.f1.get();
         P.ax[t] = a0 + f0;
         P.ay[t] = (a1 - ph.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171

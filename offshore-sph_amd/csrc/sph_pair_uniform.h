@@ -126,7 +126,7 @@ __device__ inline float grad_q(float q) {
 // The terms of one listed pair (dx, dy: x_i - x_j): (m v_ij . grad W,
 // momentum + viscosity along x and y) for a fluid neighbour, (0, the
 // Lennard-Jones force) for a wall within r0, zero otherwise.
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __device__ inline float3 uniform_terms(const UniformConst &K, float dx, float dy, float vxi, float vyi, float rhoi,
                                        float slf, const float4 &b) {
     const float r2 = dx * dx + dy * dy;
@@ -162,7 +162,7 @@ __device__ inline float3 uniform_terms(const UniformConst &K, float dx, float dy
     }
     if (r <= K.r0 && r > 1e-12f) {
         const float frac = K.r0 * rinv;
-        const float tmp = ipow(frac, K.p1) - ipow(frac, K.p2);
+        const float tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
         const float fac = K.D * tmp * (rinv * rinv);
         return make_float3(0.0f, fac * dx, fac * dy);
     }
@@ -216,9 +216,9 @@ __device__ inline bool uniform_rates(const UniformArgs &P, const UniformConst &K
             const unsigned u = *q;
             const double2 a = at32(P.A, u);
             const float4 b = at32(P.B, u);
-            const float3 f = uniform_terms<KERNEL>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
-            if constexpr (MODE != kMomentum) srho += (double)f.x;
-            if constexpr (MODE != kContinuity) {
+            const float3 f = uniform_terms<KERNEL, MODE>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
+            if constexpr ((MODE & kEquations) != kMomentum) srho += (double)f.x;
+            if constexpr ((MODE & kEquations) != kContinuity) {
                 sax += (double)f.y;
                 say += (double)f.z;
             }
@@ -270,7 +270,7 @@ __device__ inline bool uniform_rates(const UniformArgs &P, const UniformConst &K
     if (!inside && uniform_count(P, K, X, Y, c, ncx, ncy, base) == 0) return false;  // SolverTools.py:166-169
     drho = srho;
     ax = sax;
-    ay = MODE == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
     return true;
 }
 
@@ -301,9 +301,9 @@ __device__ inline bool uniform_rates_staged(const UniformArgs &P, const UniformC
             const double2 a = sA[i];
             const int shi = i >= S.off[2] ? sh2 : (i >= S.off[1] ? sh1 : sh0);
             const float4 b = at32(P.B, (unsigned)(i - shi));
-            const float3 f = uniform_terms<KERNEL>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
-            if constexpr (MODE != kMomentum) srho += (double)f.x;
-            if constexpr (MODE != kContinuity) {
+            const float3 f = uniform_terms<KERNEL, MODE>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
+            if constexpr ((MODE & kEquations) != kMomentum) srho += (double)f.x;
+            if constexpr ((MODE & kEquations) != kContinuity) {
                 sax += (double)f.y;
                 say += (double)f.z;
             }
@@ -349,7 +349,7 @@ __device__ inline bool uniform_rates_staged(const UniformArgs &P, const UniformC
     if (!inside && uniform_count(P, K, X, Y, c, ncx, ncy, base) == 0) return false;  // SolverTools.py:166-169
     drho = srho;
     ax = sax;
-    ay = MODE == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
     return true;
 }
 
@@ -411,8 +411,8 @@ __device__ inline void uniform_target(const UniformArgs &P, const UniformConst &
     double drho, ax, ay;
     if (!uniform_rates<KERNEL, MODE, uniform_batch_list<KERNEL>()>(P, K, ncx, ncy, base, t, bt, s_list, drho, ax, ay))
         return;
-    if constexpr (MODE != kMomentum) P.drho[t] = drho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = ax;
         P.ay[t] = ay;
     }
@@ -433,8 +433,8 @@ __global__ __launch_bounds__(256) void k_pair_uniform(const Ctrl *ctrl, UniformA
     StagedWalk<KERNEL, MODE, LIST> W(P, K, g, ncx, ncy, 0, t, walks, s_mem, s_red);
     double drho, ax, ay;
     if (!walks || !W.rates(P, K, ncx, ncy, t, bt, drho, ax, ay)) return;
-    if constexpr (MODE != kMomentum) P.drho[t] = drho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = ax;
         P.ay[t] = ay;
     }
@@ -471,7 +471,7 @@ __device__ inline void uniform_target_batch(const BInst *inst, const int *instOf
 // workgroup stages its walk's records in LDS first (see stage_plan); a
 // workgroup whose ranges exceed the stage, or K.stage = 0, walks global
 // memory. The sums are the same either way.
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_uniform_pec(Ctrl *ctrl, UniformArgs P, UniformConst K, PecArgs C) {
     constexpr int LIST = uniform_list<KERNEL>();
     __shared__ __align__(16) unsigned char s_mem[stage_bytes<LIST>()];
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(256) void k_pair_uniform_pec(Ctrl *ctrl, UniformArg
     float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
     if (t < P.n) bt = P.B[t];
     const bool walks = t < P.n && !not_fluid(bt.w);
-    StagedWalk<KERNEL, kFused, LIST> W(P, K, g, ncx, ncy, 0, t, walks, s_mem, s_red);
+    StagedWalk<KERNEL, MODE, LIST> W(P, K, g, ncx, ncy, 0, t, walks, s_mem, s_red);
     DtVars v;
     if (t < P.n) {
         if (walks) {
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_queue(const BInst *i
 // that is not active keeps its state; its fluid still enters the partials.
 // The tile's walk is staged in LDS as the single-simulation pass's (one
 // instance per tile: its grid and bins).
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_batch_uniform_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC,
                                                        UniformArgs P, const UniformConst *Ks, PecArgs C) {
     constexpr int LIST = uniform_list<KERNEL>();
@@ -584,7 +584,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_pec(const BInst *ins
     const bool in = t < cs[c + 1];
     float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
     if (in) bt = P.B[t];
-    StagedWalk<KERNEL, kFused, LIST> W(P, Ks[k], g, ncx, ncy, I.cellBase, t, in && I.active && !not_fluid(bt.w),
+    StagedWalk<KERNEL, MODE, LIST> W(P, Ks[k], g, ncx, ncy, I.cellBase, t, in && I.active && !not_fluid(bt.w),
                                        s_mem, s_red);
     DtVars v;
     if (in) {
@@ -650,9 +650,9 @@ struct UniformGroup {
     __device__ __forceinline__ void terms(unsigned u, float *out) const {
         const double2 a = at32(P.A, u);
         const float4 b = at32(P.B, u);
-        const float3 f = uniform_terms<KERNEL>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
-        if constexpr (MODE != kMomentum) out[0] = f.x;
-        if constexpr (MODE != kContinuity) {
+        const float3 f = uniform_terms<KERNEL, MODE>(K, (float)(X - a.x), (float)(Y - a.y), bt.x, bt.y, bt.z, bt.w, b);
+        if constexpr ((MODE & kEquations) != kMomentum) out[0] = f.x;
+        if constexpr ((MODE & kEquations) != kContinuity) {
             out[1] = f.y;
             out[2] = f.z;
         }
@@ -680,7 +680,7 @@ __device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformCo
     drho = acc.get(0);
     ax = acc.get(1);
     const double say = acc.get(2);
-    ay = MODE == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
     if (!walks) return false;
     const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;  // it finds itself: a neighbour
     return inside || uniform_count(P, K, at.x, at.y, c, ncx, ncy, 0) != 0;  // SolverTools.py:166-169
@@ -700,17 +700,17 @@ __global__ __launch_bounds__(256) void k_group_uniform(const Ctrl *ctrl, Uniform
     const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i], drho,
                                                           ax, ay);
     if (!any || l != 0) return;
-    if constexpr (MODE != kMomentum) P.drho[t] = drho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = ax;
         P.ay[t] = ay;
     }
 }
 
 // k_pair_uniform_pec with G lanes per target; the group's first lane corrects.
-template <int KERNEL, int G>
+template <int KERNEL, int MODE, int G>
 __global__ __launch_bounds__(256) void k_group_uniform_pec(Ctrl *ctrl, UniformArgs P, UniformConst K, PecArgs C) {
-    __shared__ GroupMem<UniformGroup<KERNEL, kFused>, G> mem[256 / G];
+    __shared__ GroupMem<UniformGroup<KERNEL, MODE>, G> mem[256 / G];
     __shared__ double lds[kDtQ * 16];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(256) void k_group_uniform_pec(Ctrl *ctrl, UniformAr
     PecStart p0{};
     if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
     double drho, ax, ay;
-    const bool any = uniform_group_rates<KERNEL, kFused, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
                                                             drho, ax, ay);
     DtVars v;
     if (corrects) {

@@ -37,26 +37,15 @@ namespace {
 #define HIPSPH_UNIFORM64_UNROLL 4
 #endif
 #ifndef HIPSPH_UNIFORM64_LIST
-#define HIPSPH_UNIFORM64_LIST 32
+#define HIPSPH_UNIFORM64_LIST 30
 #endif
-// The Gaussian's lists (about 42 contributors) fill at least once: the
-// longest list that keeps the 4 workgroups per CU its registers allow (40 KB
-// of LDS each; 38 beside the corrector's 512 B) flushes least often (on a 4M
-// jittered lattice 40 entries take 1.59 ms, 32 1.84 ms, 24 1.96 ms).
-#ifndef HIPSPH_UNIFORM64_GAUSS_LIST
-#define HIPSPH_UNIFORM64_GAUSS_LIST 40
-#endif
-#ifndef HIPSPH_UNIFORM64_GAUSS_PEC_LIST
-#define HIPSPH_UNIFORM64_GAUSS_PEC_LIST 38
-#endif
-constexpr int kUniform64List = HIPSPH_UNIFORM64_LIST;  // contributor-list entries per thread (4 B each)
+// contributor-list entries per thread (4 B each): 30 for five workgroups per
+// CU (500k particles, 30 steps: 4.04 ms against 4.14 with 32, 4.06 with 25)
+constexpr int kUniform64List = HIPSPH_UNIFORM64_LIST;
+// the Gaussian's pass keeps no list (uniform64_rates_direct)
 template <int KERNEL>
 __host__ __device__ constexpr int uniform64_list() {
-    return KERNEL == SPH_KERNEL_GAUSSIAN ? HIPSPH_UNIFORM64_GAUSS_LIST : kUniform64List;
-}
-template <int KERNEL>
-__host__ __device__ constexpr int uniform64_pec_list() {
-    return KERNEL == SPH_KERNEL_GAUSSIAN ? HIPSPH_UNIFORM64_GAUSS_PEC_LIST : kUniform64List;
+    return KERNEL == SPH_KERNEL_GAUSSIAN ? 1 : kUniform64List;
 }
 
 struct Uniform64Args {
@@ -73,10 +62,37 @@ struct Uniform64Const {
     double h, m, alpha_k;  // alpha_k: the kernel normalisation 10 / (7 pi) / (h h) (Wendland: 9 / (4 pi) / (h h))
     double c01;            // 0.01 h h, in the reference's order (0.01 h) h
     double cij, alpha, beta;
+    double ih2, g2;        // the Gaussian's 1 / h^2 and -2 alpha_k / h^2 (gauss_factor)
     double r0, D, p1, p2, g, qmax;
 };
 
 __device__ inline bool not_fluid64(double prs) { return prs != prs; }
+
+// Whether the target at (X, Y) in cell c has a neighbour: one whose own cell
+// is in the grid finds itself (q = 0); one outside looks (SolverTools.py:
+// 166-169).
+__device__ inline bool uniform64_has_neighbour(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
+                                               long long base, double X, double Y, int2 c) {
+    if (c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy) return true;
+    const double lim = (K.qmax * K.h) * (K.qmax * K.h);
+    for (int da = -1; da <= 1; ++da) {
+        const int cx = c.x + da;
+        if (!(ncx > cx && cx > -1)) continue;
+        for (int db = -1; db <= 1; ++db) {
+            const int cy = c.y + db;
+            if (!(ncy > cy && cy > -1)) continue;
+            const long long cell = base + cx + (long long)ncx * cy;
+            for (int k = P.cellStart[cell]; k < P.cellStart[cell + 1]; ++k) {
+                const double2 a = at32(P.A, (unsigned)k);
+                const double ddx = X - a.x, ddy = Y - a.y;
+                const double r2 = ddx * ddx + ddy * ddy;
+                if (r2 < lim * (1.0 - 1e-12)) return true;
+                if (!(r2 > lim * (1.0 + 1e-12)) && exact_q_test(X, Y, K.h, a.x, a.y, K.h, K.qmax)) return true;
+            }
+        }
+    }
+    return false;
+}
 
 // The rates of fluid target t (bt: its B record) over a grid of ncx x ncy
 // cells starting at bin `base` (0 for a single simulation, the instance's
@@ -84,8 +100,8 @@ __device__ inline bool not_fluid64(double prs) { return prs != prs; }
 // previous rates. MODE kContinuity sums drho only, kMomentum ax and ay only
 // (the other outputs are then zero); each sum keeps the order of the fused
 // pass, so the split passes give its bits.
-template <int KERNEL, int MODE = kFused, int LIST = uniform64_list<KERNEL>()>
-__device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
+template <int KERNEL, int MODE = kFused>
+__device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
                                        long long base, int t, const double4 &bt, unsigned *s_list, double &drho,
                                        double &ax, double &ay) {
     const double2 at = P.A[t];
@@ -109,31 +125,22 @@ __device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Co
             if (!not_fluid64(b.w)) {
                 const double qq = r / K.h;
                 double dwx, dwy;
-                if (KERNEL == SPH_KERNEL_GAUSSIAN) {
-                    const double tmp = r * K.h;
-                    if (!(tmp > 1e-12 && qq <= 3)) continue;
-                    const double dwdq = -2 * qq * K.alpha_k * exp(-qq * qq);
-                    const double f = dwdq / tmp;
-                    dwx = f * dx;
-                    dwy = f * dy;
+                double grad;
+                if (KERNEL == SPH_KERNEL_WENDLAND) {
+                    if ((qq >= 2.0) || (r < 1e-10)) continue;
+                    const double inner = 1.0 - 0.5 * qq;
+                    grad = ipow(inner, 5.0) * (-14.0 / 3.0) * qq * (1 + 2.5 * qq);
                 } else {
-                    double grad;
-                    if (KERNEL == SPH_KERNEL_WENDLAND) {
-                        if ((qq >= 2.0) || (r < 1e-10)) continue;
-                        const double inner = 1.0 - 0.5 * qq;
-                        grad = ipow(inner, 5.0) * (-14.0 / 3.0) * qq * (1 + 2.5 * qq);
-                    } else {
-                        if ((qq > 2.0) || (r < 1e-10)) continue;
-                        grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
-                    }
-                    const double norm = K.alpha_k * grad / (K.h * r);
-                    dwx = norm * dx;
-                    dwy = norm * dy;
+                    if ((qq > 2.0) || (r < 1e-10)) continue;
+                    grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
                 }
+                const double norm = K.alpha_k * grad / (K.h * r);
+                dwx = norm * dx;
+                dwy = norm * dy;
                 const double vx = bt.x - b.x, vy = bt.y - b.y;
                 const double dot = vx * dwx + vy * dwy;
-                if constexpr (MODE != kMomentum) arho += K.m * dot;
-                if constexpr (MODE == kContinuity) continue;
+                if constexpr ((MODE & kEquations) != kMomentum) arho += K.m * dot;
+                if constexpr ((MODE & kEquations) == kContinuity) continue;
                 const double dv = vx * dx + vy * dy;
                 double PI_ij = 0.0;
                 if (dv < 0) {
@@ -145,9 +152,9 @@ __device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Co
                 const double factor = bt.w + b.w + PI_ij;
                 a0 += -K.m * factor * dwx;
                 a1 += -K.m * factor * dwy;
-            } else if (MODE != kContinuity && !(r > K.r0) && r > 1e-12) {
+            } else if ((MODE & kEquations) != kContinuity && !(r > K.r0) && r > 1e-12) {
                 const double frac = K.r0 / r;
-                const double tmp = ipow(frac, K.p1) - ipow(frac, K.p2);
+                const double tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
                 const double fac = K.D * tmp;
                 f0 += fac * dx / (r * r);
                 f1 += fac * dy / (r * r);
@@ -155,15 +162,10 @@ __device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Co
         }
         lp = list0;
     };
-    constexpr int U = HIPSPH_UNIFORM64_UNROLL;
+    constexpr int U = HIPSPH_UNIFORM64_UNROLL, LIST = kUniform64List;
     static_assert(U >= 1 && U < LIST, "unroll within the list");
     unsigned *const full = list0 + (LIST - U) * stride;  // past this, U appends could overflow
-    // the Gaussian's lists all fill: every active lane flushes when one must,
-    // one flush loop for the wave instead of one per lane
-    auto overflow = [&]() {
-        if constexpr (KERNEL == SPH_KERNEL_GAUSSIAN) return __ballot(lp > full) != 0;
-        return lp > full;
-    };
+    auto overflow = [&]() { return lp > full; };
     auto test = [&](double2 a, int k) {
         const double dx = X - a.x, dy = Y - a.y;
         const double r2 = dx * dx + dy * dy;
@@ -198,34 +200,99 @@ __device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Co
         }
     }
     flush();
-    // a target whose own cell is in the grid finds itself (q = 0): it has a
-    // neighbour; one outside counts them (SolverTools.py:166-169)
-    if (!(c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy)) {
-        const double lim = (K.qmax * K.h) * (K.qmax * K.h);
-        int cnt = 0;
-        for (int da = -1; da <= 1; ++da) {
-            const int cx = c.x + da;
-            if (!(ncx > cx && cx > -1)) continue;
-            for (int db = -1; db <= 1; ++db) {
-                const int cy = c.y + db;
-                if (!(ncy > cy && cy > -1)) continue;
-                const long long cell = base + cx + (long long)ncx * cy;
-                for (int k = P.cellStart[cell]; k < P.cellStart[cell + 1]; ++k) {
-                    const double2 a = at32(P.A, (unsigned)k);
-                    const double ddx = X - a.x, ddy = Y - a.y;
-                    const double r2 = ddx * ddx + ddy * ddy;
-                    bool in = r2 < lim * (1.0 - 1e-12);
-                    if (!in && !(r2 > lim * (1.0 + 1e-12))) in = exact_q_test(X, Y, K.h, a.x, a.y, K.h, K.qmax);
-                    cnt += in;
+    if (!uniform64_has_neighbour(P, K, ncx, ncy, base, X, Y, c)) return false;
+    drho = arho;
+    ax = a0 + f0;
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
+    return true;
+}
+
+// The Gaussian's pass: the same walk, each candidate's terms formed as it is
+// met, its records and the next one's in flight. About 42 of 61 candidates
+// contribute; listing them first left lanes idle in the flushes of lists that
+// filled at different candidates, fetched every contributor's records a second
+// time from scattered places, and its 40 KB of lists kept the pass at 4
+// wavefronts per SIMD (1M particles: continuity 394 -> 178 us, momentum 456 ->
+// 330 us; the cubic spline, 21 of 61, keeps the lists).
+template <int MODE>
+__device__ inline bool uniform64_rates_direct(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
+                                              long long base, int t, const double4 &bt, double &drho, double &ax,
+                                              double &ay) {
+    const double2 at = P.A[t];
+    const double X = at.x, Y = at.y;
+    const int2 c = P.cxy[t];
+    double arho = 0.0, a0 = 0.0, a1 = 0.0, f0 = 0.0, f1 = 0.0;
+    for (int da = -1; da <= 1; ++da) {
+        const int cx = c.x + da;
+        if (!(ncx > cx && cx > -1)) continue;
+        for (int db = -1; db <= 1; ++db) {
+            const int cy = c.y + db;
+            if (!(ncy > cy && cy > -1)) continue;
+            const long long cell = base + cx + (long long)ncx * cy;
+            const int s = P.cellStart[cell], e = P.cellStart[cell + 1];
+            double2 an{};
+            double4 bn{};
+            if (s < e) {
+                an = at32(P.A, (unsigned)(e - 1));
+                bn = at32(P.B, (unsigned)(e - 1));
+            }
+            for (int k = e - 1; k >= s; --k) {
+                const double2 a = an;
+                const double4 b = bn;
+                if (k > s) {
+                    an = at32(P.A, (unsigned)(k - 1));
+                    bn = at32(P.B, (unsigned)(k - 1));
+                }
+                const double dx = X - a.x, dy = Y - a.y;
+                const double xij2 = dx * dx + dy * dy;
+                if (!(xij2 <= K.lim2 && xij2 > 0.0)) continue;
+                if (!not_fluid64(b.w)) {
+                    double f;
+                    if (!gauss_factor(xij2, K.h, K.ih2, K.g2, f)) continue;
+                    const double dwx = f * dx, dwy = f * dy;
+                    const double vx = bt.x - b.x, vy = bt.y - b.y;
+                    const double dot = vx * dwx + vy * dwy;
+                    if constexpr ((MODE & kEquations) != kMomentum) arho += K.m * dot;
+                    if constexpr ((MODE & kEquations) == kContinuity) continue;
+                    const double dv = vx * dx + vy * dy;
+                    double PI_ij = 0.0;
+                    if (dv < 0) {
+                        const double rhoij = 0.5 * (bt.z + b.z);
+                        const double muij = K.h * dv / (xij2 + K.c01);
+                        const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
+                        PI_ij = ppij / rhoij;
+                    }
+                    const double factor = bt.w + b.w + PI_ij;
+                    a0 += -K.m * factor * dwx;
+                    a1 += -K.m * factor * dwy;
+                } else if ((MODE & kEquations) != kContinuity) {
+                    const double r = sqrt(xij2);
+                    if (!(r > K.r0) && r > 1e-12) {
+                        const double frac = K.r0 / r;
+                        const double tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
+                        const double fac = K.D * tmp;
+                        f0 += fac * dx / (r * r);
+                        f1 += fac * dy / (r * r);
+                    }
                 }
             }
         }
-        if (cnt == 0) return false;
     }
+    if (!uniform64_has_neighbour(P, K, ncx, ncy, base, X, Y, c)) return false;
     drho = arho;
     ax = a0 + f0;
-    ay = MODE == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
     return true;
+}
+
+template <int KERNEL, int MODE = kFused>
+__device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
+                                       long long base, int t, const double4 &bt, unsigned *s_list, double &drho,
+                                       double &ax, double &ay) {
+    if constexpr (KERNEL == SPH_KERNEL_GAUSSIAN)
+        return uniform64_rates_direct<MODE>(P, K, ncx, ncy, base, t, bt, drho, ax, ay);
+    else
+        return uniform64_rates_listed<KERNEL, MODE>(P, K, ncx, ncy, base, t, bt, s_list, drho, ax, ay);
 }
 
 // One target t of the pass: its rates, or nothing for a wall or a target
@@ -237,8 +304,8 @@ __device__ inline void uniform64_target(const Uniform64Args &P, const Uniform64C
     if (not_fluid64(bt.w)) return;  // walls are not targets
     double drho, ax, ay;
     if (!uniform64_rates<KERNEL, MODE>(P, K, ncx, ncy, base, t, bt, s_list, drho, ax, ay)) return;
-    if constexpr (MODE != kMomentum) P.drho[t] = drho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = ax;
         P.ay[t] = ay;
     }
@@ -277,10 +344,10 @@ __device__ inline void uniform64_target_batch(const BInst *inst, const int *inst
 // The pass with PEC's corrector and the next dt's partials fused in, as the
 // float pass's k_pair_uniform_pec (the corrector's arithmetic is the
 // engine's, bit for bit).
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_uniform64_pec(Ctrl *ctrl, Uniform64Args P, Uniform64Const K,
                                                             PecArgs C) {
-    __shared__ unsigned s_list[uniform64_pec_list<KERNEL>() * 256];
+    __shared__ unsigned s_list[uniform64_list<KERNEL>() * 256];
     __shared__ double lds[kDtQ * 16];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -298,7 +365,7 @@ __global__ __launch_bounds__(256) void k_pair_uniform64_pec(Ctrl *ctrl, Uniform6
             const PecStart p0 = pec_start(C, t, dt, damping);
 #endif
             double drho, ax, ay;
-            if (uniform64_rates<KERNEL, kFused, uniform64_pec_list<KERNEL>()>(P, K, (int)g.ncx, (int)g.ncy, 0, t, bt,
+            if (uniform64_rates<KERNEL, MODE>(P, K, (int)g.ncx, (int)g.ncy, 0, t, bt,
                                                                               s_list, drho, ax, ay)) {
                 P.drho[t] = drho;
                 P.ax[t] = ax;
@@ -364,10 +431,10 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_queue(const BInst 
 // same for the whole workgroup. The chunk's dt partials go to
 // C.part[q * NC + c], where the batch's corrector stores them. An instance
 // that is not active keeps its state; its fluid still enters the partials.
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC,
                                                        Uniform64Args P, const Uniform64Const *Ks, PecArgs C) {
-    __shared__ unsigned s_list[uniform64_pec_list<KERNEL>() * 256];
+    __shared__ unsigned s_list[uniform64_list<KERNEL>() * 256];
     __shared__ double lds[kDtQ * 16];
     const int c = xcd_remap(blockIdx.x, gridDim.x);
     if (c >= NC) return;  // the whole workgroup
@@ -386,7 +453,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *i
 #if HIPSPH_PEC64_EARLY
                 const PecStart p0 = pec_start(Ci, t, dt, damping);
 #endif
-                if (uniform64_rates<KERNEL, kFused, uniform64_pec_list<KERNEL>()>(
+                if (uniform64_rates<KERNEL, MODE>(
                         P, Ks[k], (int)I.grid.ncx, (int)I.grid.ncy, I.cellBase, t, bt, s_list, drho, ax, ay)) {
                     P.drho[t] = drho;
                     P.ax[t] = ax;
@@ -448,10 +515,8 @@ struct Uniform64Group {
             const double qq = r / K.h;
             double dwx, dwy;
             if (KERNEL == SPH_KERNEL_GAUSSIAN) {
-                const double tmp = r * K.h;
-                if (!(tmp > 1e-12 && qq <= 3)) return;
-                const double dwdq = -2 * qq * K.alpha_k * exp(-qq * qq);
-                const double f = dwdq / tmp;
+                double f;
+                if (!gauss_factor(xij2, K.h, K.ih2, K.g2, f)) return;
                 dwx = f * dx;
                 dwy = f * dy;
             } else {
@@ -470,22 +535,23 @@ struct Uniform64Group {
             }
             const double vx = bt.x - b.x, vy = bt.y - b.y;
             const double dot = vx * dwx + vy * dwy;
-            if constexpr (MODE != kMomentum) out[0] = K.m * dot;
-            if constexpr (MODE == kContinuity) return;
+            if constexpr ((MODE & kEquations) != kMomentum) out[0] = K.m * dot;
+            if constexpr ((MODE & kEquations) == kContinuity) return;
             const double dv = vx * dx + vy * dy;
             double PI_ij = 0.0;
             if (dv < 0) {
                 const double rhoij = 0.5 * (bt.z + b.z);
-                const double muij = K.h * dv / (r * r + K.c01);
+                const double rr = KERNEL == SPH_KERNEL_GAUSSIAN ? xij2 : r * r;
+                const double muij = K.h * dv / (rr + K.c01);
                 const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
                 PI_ij = ppij / rhoij;
             }
             const double factor = bt.w + b.w + PI_ij;
             out[1] = -K.m * factor * dwx;
             out[2] = -K.m * factor * dwy;
-        } else if (MODE != kContinuity && !(r > K.r0) && r > 1e-12) {
+        } else if ((MODE & kEquations) != kContinuity && !(r > K.r0) && r > 1e-12) {
             const double frac = K.r0 / r;
-            const double tmp = ipow(frac, K.p1) - ipow(frac, K.p2);
+            const double tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
             const double fac = K.D * tmp;
             out[3] = fac * dx / (r * r);
             out[4] = fac * dy / (r * r);
@@ -516,7 +582,7 @@ __device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Unifo
     drho = acc.get(0);
     const double a0 = acc.get(1), a1 = acc.get(2), f0 = acc.get(3), f1 = acc.get(4);
     ax = a0 + f0;
-    ay = MODE == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
     return walks && (inside || cnt != 0);  // SolverTools.py:166-169
 }
 
@@ -534,8 +600,8 @@ __global__ __launch_bounds__(256) void k_group_uniform64(const Ctrl *ctrl, Unifo
     const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
                                                             drho, ax, ay);
     if (!any || l != 0) return;
-    if constexpr (MODE != kMomentum) P.drho[t] = drho;
-    if constexpr (MODE != kContinuity) {
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
         P.ax[t] = ax;
         P.ay[t] = ay;
     }
@@ -543,10 +609,10 @@ __global__ __launch_bounds__(256) void k_group_uniform64(const Ctrl *ctrl, Unifo
 
 // k_pair_uniform64_pec with G lanes per target; the group's first lane
 // corrects.
-template <int KERNEL, int G>
+template <int KERNEL, int MODE, int G>
 __global__ __launch_bounds__(256) void k_group_uniform64_pec(Ctrl *ctrl, Uniform64Args P, Uniform64Const K,
                                                              PecArgs C) {
-    __shared__ GroupMem<Uniform64Group<KERNEL, kFused>, G> mem[256 / G];
+    __shared__ GroupMem<Uniform64Group<KERNEL, MODE>, G> mem[256 / G];
     __shared__ double lds[kDtQ * 16];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -564,7 +630,7 @@ __global__ __launch_bounds__(256) void k_group_uniform64_pec(Ctrl *ctrl, Uniform
     PecStart p0{};
     if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
     double drho, ax, ay;
-    const bool any = uniform64_group_rates<KERNEL, kFused, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
                                                               drho, ax, ay);
     DtVars v;
     if (corrects) {
