@@ -229,21 +229,21 @@ struct BInst;
 // Lanes per target of the single-simulation pair passes (sph_pair_group.h) for
 // n particles; 0: one thread per target. A group shortens a target's serial
 // chain at about twice the instructions, so it pays while the chip is not
-// full, longest where the chain is longest (the Gaussian's 42 contributors,
-// the double terms of the general pass). Whole steps in us, one thread / 4 /
-// 8 / 16 lanes, on dam breaks:
-//   double uniform   6.5k 54.5 46.9 41.1 40.0; 23k 56.0 48.9 44.9 51.5;
-//                    44k 57.4 53.3 58.0 68.3; 60k 58.9 65.4 67.4 80.8
-//   float uniform    6.5k 47.3 41.5 38.6 37.6; 71k 53.9 51.1; 118k 56.4 61.3
-//   double Gaussian  6.5k 114 52 44 41; 332k 254 229; 617k 388 391
-//   float Gaussian   6.5k 77 45 40 38; 169k 92 84; 251k 101 104
-//   double general   6.5k 71 51 46 45; 86k 85 80; 118k 89 94
-//   float general    6.5k 64 49 44 43; 138k 82 78; 251k 98 106
+// full, longest where the chain is longest (the float Gaussian's lists of 42
+// contributors, the general pass). Whole steps in us, one thread / 4 / 8 / 16
+// lanes, on dam breaks:
+//   double uniform   6.5k 52.0 45.1 39.7 38.9; 23k 53.3 47.3 43.6 48.7;
+//                    49k 55.3 52.1 55.3 64.0; 61k 55.8 56.3 61.3 72.5
+//   float uniform    6.5k 46.9 40.7 37.5 36.4; 86k 53.8 52.4; 118k 54.9 59.1
+//   double Gaussian  6.5k 71 51 43 41; 61k 74 76 71; 86k 87 89 85
+//   float Gaussian   6.5k 75 44 39 37; 169k 90 78; 332k 119 113; 617k 171 197
+//   double general   6.5k 69 50 45 43; 86k 84 76; 118k 88 87; 169k 99 104
+//   float general    6.5k 62 48 44 42; 118k 74 71; 169k 81 81; 332k 117 119
 inline int group_lanes(long long n, bool f64, bool uniform, int kernel) {
     const bool gauss = kernel == SPH_KERNEL_GAUSSIAN;
-    const long long most = !uniform ? (f64 ? 100000 : 150000)
-                           : gauss  ? (f64 ? 450000 : 200000)
-                                    : (f64 ? 48000 : 80000);
+    const long long most = !uniform ? (f64 ? 115000 : 160000)
+                           : gauss  ? (f64 ? 80000 : 400000)
+                                    : (f64 ? 60000 : 96000);
     return n > most ? 0 : (n <= 16384 ? 16 : (n <= 32768 ? 8 : 4));
 }
 // Host: calls f with kIntPow or 0 as a compile-time constant.

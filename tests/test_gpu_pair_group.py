@@ -99,7 +99,7 @@ def test_group_lists_that_fill(precision):
 
 
 def test_staged_walk_above_the_group_sizes():
-    sc = scenarios.stress_lattice(nside=300, hfac=3.0)
+    sc = scenarios.stress_lattice(nside=340, hfac=3.0)
     out = []
     for staging in (True, False):
         say('staged walk', len(sc.pA), staging)
