@@ -37,6 +37,7 @@
 
 #include "sph_ctx.h"
 #include "sph_common.h"
+#include "sph_pair_group.h"
 
 using namespace hipsph;
 
@@ -181,13 +182,14 @@ __device__ inline void pair_vjp2(double rx, double ry, double d, double G, doubl
 
 // Adjoint of the Lennard-Jones wall term of fluid i, wall j
 // (src/Equations/BoundaryForce.py:31-41): f = D ((r0/d)^p1 - (r0/d)^p2) r / d^2.
+template <int MODE>
 __device__ inline void wall_vjp(double rx, double ry, double lamx, double lamy, const Phys &ph, double &gx,
                                 double &gy) {
     const double d2 = rx * rx + ry * ry;
     const double d = sqrt(d2);
     if (d > ph.r0 || !(d > 1e-12)) return;
     const double fr = ph.r0 / d;
-    const double t1 = ipow(fr, ph.p1), t2 = ipow(fr, ph.p2);
+    const double t1 = wall_pow<MODE>(fr, ph.p1), t2 = wall_pow<MODE>(fr, ph.p2);
     const double phi = ph.D * (t1 - t2) / d2;
     const double dphi = ph.D / (d2 * d) * (-(ph.p1 + 2.0) * t1 + (ph.p2 + 2.0) * t2);
     const double lr = (lamx * rx + lamy * ry) * dphi / d;
@@ -232,33 +234,12 @@ __global__ void k_tape_static(State s, int n, int8_t *label) {
 }
 
 // Argmax of |a_prev|^2 over the fluid at the start of a step, with the
-// engine's expression (contraction off): per-workgroup (value, id), then one
-// workgroup folds. Ties go to the smaller id.
+// engine's expression (contraction off): per-workgroup (value, id) of each
+// recorded step, folded by k_adj_final. Ties go to the smaller id.
 __device__ inline void amax_merge(double &v, int &i, double v2, int i2) {
     if (v2 > v || (v2 == v && i2 < i)) {
         v = v2;
         i = i2;
-    }
-}
-
-__global__ void k_tape_amax_final(const double *pv, const int *pi, int R, TapeHdr *hdr) {
-    double v = -1.0;
-    int id = 0x7fffffff;
-    for (int b = threadIdx.x; b < R; b += blockDim.x) amax_merge(v, id, pv[b], pi[b]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax_merge(v, id, __shfl_xor(v, o, 64), __shfl_xor(id, o, 64));
-    __shared__ double lv[16];
-    __shared__ int li[16];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if (lane == 0) {
-        lv[w] = v;
-        li[w] = id;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < nw; ++k) amax_merge(v, id, lv[k], li[k]);
-        hdr->amax2 = v;
-        hdr->amax_id = id;
     }
 }
 
@@ -418,25 +399,30 @@ __global__ void k_adj_correct(const TapeHdr *hdr, TapeSlot T, const int8_t *labe
 }
 
 // Pair pass, reversed: gather over the step's cells, kAdjLanes lanes per
-// particle (cell order of the step). Lane l of a particle's group takes the
-// candidates l, l + kAdjLanes, ... of each row of three cells (consecutive
-// bins: one run of slots, ~20 candidates, instead of nine cells of ~7 that
-// left most lanes idle); the group then
-// folds its sums with a fixed xor-shuffle tree, so the result does not depend
-// on scheduling. (A thread per particle leaves most of the chip idle at the
-// particle counts the adjoint is used for, and each pair costs two adjoint
-// evaluations.)
+// particle (cell order of the step), as the forward's passes for small states
+// (sph_pair_group.h; a thread per particle leaves most of the chip idle at the
+// particle counts the adjoint is used for). The lanes test the candidates
+// of the three row runs side by side and list, by ballot, those inside the
+// kernel's support or a wall's range; then each takes every kAdjLanes-th
+// listed pair, whose two adjoint evaluations are the pass's cost (about 450
+// instructions). Evaluating candidates as they were met ran that code for
+// every round of the walk with a third of the lanes in it (20k particles: 41
+// us and 171 registers, pow() among them; listed, and without the pow(): 25
+// us, 162). The group folds its sums with
+// a fixed xor-shuffle tree, so the result does not depend on scheduling.
 constexpr int kAdjLanes = 8;
+constexpr int kAdjList = 64;  // entries per particle; emptied when kAdjLanes more might not fit
 
 // The group's first lane then reverses the predictor for its particle (PEC;
 // for Euler the pair inputs are the start state), which needs nothing of
 // any other particle: the half-step adjoint goes straight into A, and the
 // predictor's dt term into this workgroup's partial 0.
-template <int KERNEL>
+template <int KERNEL, int MODE>
 __global__ __launch_bounds__(kAdjBlock) void k_adj_pair(const TapeHdr *hdr, TapeSlot T, int n, Phys ph,
                                                          const double4 *lk, Adj A, const double *vbx,
                                                          const double *vby, double damping, int euler,
                                                          double *part) {
+    __shared__ unsigned s_list[kAdjBlock / kAdjLanes][kAdjList];
     double red[kAdjQ] = {0.0, 0.0, 0.0, 0.0};
     const long long gt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int t = (int)(gt / kAdjLanes);  // uniform within a lane group
@@ -448,43 +434,71 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pair(const TapeHdr *hdr, Tape
         k = T.id[t];
         ak = T.pa[t];
     }
+    const bool walks = live && ak.w >= 0.0;
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // xbar, ybar, vxbar, vybar, rhobar
-    if (live && ak.w >= 0.0) {
-        const Grid g = hdr->grid;
-        const int ncx = (int)g.ncx, ncy = (int)g.ncy;
-        const double4 bk = T.pb[t], sk = T.ps[t], lmk = lk[t];
+    {
+        double4 bk = make_double4(0.0, 0.0, 0.0, 0.0), sk = bk, lmk = bk;
+        int2 c = make_int2(0, 0);
+        if (walks) {
+            bk = T.pb[t];
+            sk = T.ps[t];
+            lmk = lk[t];
+            c = T.cxy[t];
+        }
         const double xk = ak.x, yk = ak.y, hk = ak.z, vxk = bk.x, vyk = bk.y;
         const Side K{hk, bk.z, bk.w, sk.x, sk.y, sk.z};
         double ga = 0.0, gc = 0.0;
-        const int2 c = T.cxy[t];
-        const double qmax = ph.qmax;
-        const int lo = c.x - 1 > 0 ? c.x - 1 : 0;
-        const int hi = c.x + 1 < ncx - 1 ? c.x + 1 : ncx - 1;
-        for (int db = -1; db <= 1 && lo <= hi; ++db) {
-            const int cy = c.y + db;
-            if (!(ncy > cy && cy > -1)) continue;
-            {
-                const int row = ncx * cy;
-                const int s0 = T.cellStart[row + lo], s1 = T.cellStart[row + hi + 1];
-                for (int u = s0 + l; u < s1; u += kAdjLanes) {
-                    if (u == t) continue;
-                    const double4 aj = T.pa[u];
-                    const double rx = xk - aj.x, ry = yk - aj.y;
-                    const double d = sqrt(rx * rx + ry * ry);
-                    const double hh = 0.5 * (hk + aj.z);
-                    if (!(d / hh <= qmax)) continue;  // the forward's neighbour rule
-                    if (aj.w < 0.0) {
-                        wall_vjp(rx, ry, lmk.x, lmk.y, ph, acc[0], acc[1]);
-                        continue;
-                    }
-                    double G, Gp;
-                    if (!grad_factor<KERNEL>(d, hh, G, Gp)) continue;  // outside the support
-                    const double4 bj = T.pb[u], sj = T.ps[u], lmj = lk[u];
-                    const Side J{aj.z, bj.z, bj.w, sj.x, sj.y, sj.z};
-                    pair_vjp2(rx, ry, d, G, Gp, vxk - bj.x, vyk - bj.y, K, J, lmk.x, lmk.y, lmk.z, lmj.x, lmj.y,
-                              lmj.z, ph, acc, ga, gc);
-                }
+        const Candidates<false> S(T.cellStart, c, (int)hdr->grid.ncx, (int)hdr->grid.ncy, 0, walks);
+        unsigned *list = s_list[threadIdx.x / kAdjLanes];
+        const int shift = (threadIdx.x & 63) - l;
+        const unsigned below = (1u << l) - 1u, mask = (1u << kAdjLanes) - 1u;
+        const double r0sq = ph.r0 * ph.r0;
+        constexpr double sup = KERNEL == SPH_KERNEL_GAUSSIAN ? 3.0 : 2.0;
+        int nl = 0;
+        unsigned u0 = S.slot(l);
+        double4 a0 = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (l < S.n) a0 = T.pa[u0];
+        for (int i0 = 0;; i0 += kAdjLanes) {
+            const bool more = __ballot(i0 < S.n) != 0;
+            if (more) {
+                const double4 aj = a0;
+                const unsigned u = u0;
+                const int i = i0 + l;
+                u0 = S.slot(i + kAdjLanes);
+                if (i + kAdjLanes < S.n) a0 = T.pa[u0];
+                const double rx = xk - aj.x, ry = yk - aj.y;
+                const double r2 = rx * rx + ry * ry;
+                const double sh = sup * (0.5 * (hk + aj.z));
+                // a superset of the contributors; the terms decide
+                const bool in = i < S.n && (int)u != t && r2 <= (aj.w < 0.0 ? r0sq : sh * sh) * (1.0 + 1e-9);
+                const unsigned m = (unsigned)(__ballot(in) >> shift) & mask;
+                if (in) list[nl + __popc(m & below)] = u;
+                nl += __popc(m);
             }
+            if (more && __ballot(nl > kAdjList - kAdjLanes) == 0) continue;
+            wave_sync();
+            for (int q = l; __ballot(q - l < nl) != 0; q += kAdjLanes) {
+                if (q >= nl) continue;
+                const unsigned u = list[q];
+                const double4 aj = T.pa[u];
+                const double rx = xk - aj.x, ry = yk - aj.y;
+                const double d = sqrt(rx * rx + ry * ry);
+                const double hh = 0.5 * (hk + aj.z);
+                if (!(d / hh <= ph.qmax)) continue;  // the forward's neighbour rule
+                if (aj.w < 0.0) {
+                    wall_vjp<MODE>(rx, ry, lmk.x, lmk.y, ph, acc[0], acc[1]);
+                    continue;
+                }
+                double G, Gp;
+                if (!grad_factor<KERNEL>(d, hh, G, Gp)) continue;  // outside the support
+                const double4 bj = T.pb[u], sj = T.ps[u], lmj = lk[u];
+                const Side J{aj.z, bj.z, bj.w, sj.x, sj.y, sj.z};
+                pair_vjp2(rx, ry, d, G, Gp, vxk - bj.x, vyk - bj.y, K, J, lmk.x, lmk.y, lmk.z, lmj.x, lmj.y, lmj.z, ph,
+                          acc, ga, gc);
+            }
+            wave_sync();
+            nl = 0;
+            if (!more) break;
         }
         red[1] = ga;
         red[2] = gc;
@@ -528,9 +542,11 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pair(const TapeHdr *hdr, Tape
 // pass's dL/dalpha, dL/dc0 and the predictor's dt term); add this step's
 // dL/dalpha and dL/dc0. One workgroup.
 __global__ void k_adj_final(const TapeHdr *hdr, TapeSlot T, Adj A, const double *p1, int R1, const double *p2,
-                            int R2, double co, double fixed_dt, double *g_alpha, double *g_co, int *force_steps) {
+                            int R2, const double *pv, const int *pi, int R3, double co, double fixed_dt,
+                            double *g_alpha, double *g_co, int *force_steps) {
     if (!hdr->active) return;
-    __shared__ double lds[3 * 16];
+    __shared__ double lds[4 * 16];
+    __shared__ int li[16];
     double dtb = 0.0, ga = 0.0, gc = 0.0;
     for (int b = threadIdx.x; b < R1; b += blockDim.x) dtb += p1[b];
     for (int b = threadIdx.x; b < R2; b += blockDim.x) {
@@ -538,6 +554,12 @@ __global__ void k_adj_final(const TapeHdr *hdr, TapeSlot T, Adj A, const double 
         ga += p2[1 * R2 + b];
         gc += p2[2 * R2 + b];
     }
+    // the particle attaining max |a_prev|^2 over the fluid
+    double av = -1.0;
+    int ai = 0x7fffffff;
+    for (int b = threadIdx.x; b < R3; b += blockDim.x) amax_merge(av, ai, pv[b], pi[b]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) amax_merge(av, ai, __shfl_xor(av, o, 64), __shfl_xor(ai, o, 64));
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     dtb = wave_sum(dtb);
     ga = wave_sum(ga);
@@ -546,6 +568,8 @@ __global__ void k_adj_final(const TapeHdr *hdr, TapeSlot T, Adj A, const double 
         lds[w] = dtb;
         lds[16 + w] = ga;
         lds[32 + w] = gc;
+        lds[48 + w] = av;
+        li[w] = ai;
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
@@ -554,16 +578,17 @@ __global__ void k_adj_final(const TapeHdr *hdr, TapeSlot T, Adj A, const double 
         dtb += lds[k];
         ga += lds[16 + k];
         gc += lds[32 + k];
+        amax_merge(av, ai, lds[48 + k], li[k]);
     }
     // dt = min(courant, force) (src/Equations/TimeStep.py:40-45): the Courant
     // value gamma_c h_min / c0 is taken unless force < courant.
     if (!(fixed_dt > 0.0)) {
         if (!(hdr->dt_f < hdr->dt_c)) {
             gc += dtb * (-hdr->dt / co);
-        } else if (hdr->amax2 >= 1e-12 && hdr->amax_id >= 0 && hdr->amax_id < 0x7fffffff) {
+        } else if (av >= 1e-12 && ai >= 0 && ai < 0x7fffffff) {
             // dt = gamma_f sqrt(h_min / a2max): d dt / d a_k = -dt a_k / a2max
-            const int k = hdr->amax_id;
-            const double coef = -dtb * hdr->dt / hdr->amax2;
+            const int k = ai;
+            const double coef = -dtb * hdr->dt / av;
             A.ax[k] += coef * T.axp[k];
             A.ay[k] += coef * T.ayp[k];
             atomicAdd(force_steps, 1);
@@ -591,9 +616,8 @@ int hipsph::tape_record_pair(sph_ctx *c, sph_tape *t, int slot, hipStream_t s, b
     const int R = nblk_(c->n, kAdjBlock);
     k_tape_pair<<<R, kAdjBlock, 0, s>>>(c->ctrl, c->buf[c->cur], c->buf[1 - c->cur], c->perm, c->cxy_s,
                                         c->cellStart, c->n, t->slot[slot], t->hdr + slot, t->cells,
-                                        make_phys(c->P), t->amax_v, t->amax_i, lean,
+                                        make_phys(c->P), t->amax_v + (size_t)R * slot, t->amax_i + (size_t)R * slot, lean,
                                         c->P.strict && c->P.integrator == SPH_INTEGRATOR_PEC);
-    k_tape_amax_final<<<1, 1024, 0, s>>>(t->amax_v, t->amax_i, R, t->hdr + slot);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -639,7 +663,7 @@ int sph_tape_create(sph_ctx_t *ctx, int32_t nslots, sph_tape_t **out) {
                        (size_t)t->cells * sizeof(int) + 20 * 256;
     const size_t npart = (size_t)kAdjQ * (kRedBlocks + nblk_((long long)ctx->n * kAdjLanes, kAdjBlock));
     const size_t fixed = n + n * 2 * sizeof(double) + n * sizeof(double4) + npart * sizeof(double) +
-                         sizeof(TapeHdr) * nslots + nblk_(ctx->n, kAdjBlock) * (sizeof(double) + sizeof(int)) + 20 * 256 + 4096;
+                         sizeof(TapeHdr) * nslots + (size_t)nblk_(ctx->n, kAdjBlock) * nslots * (sizeof(double) + sizeof(int)) + 20 * 256 + 4096;
     if (hipMalloc(&t->arena, per * nslots + fixed) != hipSuccess) {
         delete t;
         return fail(SPH_ENOMEM, "tape allocation of %zu bytes failed", per * nslots + fixed);
@@ -654,8 +678,8 @@ int sph_tape_create(sph_ctx_t *ctx, int32_t nslots, sph_tape_t **out) {
     t->hdr = (TapeHdr *)take(sizeof(TapeHdr) * nslots);
     t->part = (double *)take(npart * sizeof(double));
     t->force_steps = (int *)take(sizeof(int));
-    t->amax_v = (double *)take(nblk_(ctx->n, kAdjBlock) * sizeof(double));
-    t->amax_i = (int *)take(nblk_(ctx->n, kAdjBlock) * sizeof(int));
+    t->amax_v = (double *)take((size_t)nblk_(ctx->n, kAdjBlock) * nslots * sizeof(double));
+    t->amax_i = (int *)take((size_t)nblk_(ctx->n, kAdjBlock) * nslots * sizeof(int));
     t->label = (int8_t *)take(n);
     double **scr[] = {&t->vbx, &t->vby};
     for (double **d : scr) *d = (double *)take(n * sizeof(double));
@@ -737,21 +761,16 @@ int hipsph::adjoint_launch(sph_ctx *ctx, sph_tape *tape, int slot, const sph_adj
     const int euler = ctx->P.integrator == SPH_INTEGRATOR_EULER;
     k_adj_correct<<<R, kAdjBlock, 0, s>>>(H, T, tape->label, n, A, ctx->P.damping, euler, tape->lk, tape->vbx,
                                            tape->vby, p1);
-    const double dmp = ctx->P.damping;
-    switch (ctx->P.kernel) {
-        case SPH_KERNEL_GAUSSIAN:
-            k_adj_pair<SPH_KERNEL_GAUSSIAN><<<Rp, kAdjBlock, 0, s>>>(H, T, n, ph, tape->lk, A, tape->vbx, tape->vby,
-                                                                     dmp, euler, p2);
-            break;
-        case SPH_KERNEL_WENDLAND:
-            k_adj_pair<SPH_KERNEL_WENDLAND><<<Rp, kAdjBlock, 0, s>>>(H, T, n, ph, tape->lk, A, tape->vbx, tape->vby,
-                                                                     dmp, euler, p2);
-            break;
-        default:
-            k_adj_pair<SPH_KERNEL_CUBIC><<<Rp, kAdjBlock, 0, s>>>(H, T, n, ph, tape->lk, A, tape->vbx, tape->vby,
-                                                                  dmp, euler, p2);
-    }
-    k_adj_final<<<1, 1024, 0, s>>>(H, T, A, p1, R, p2, Rp, ctx->P.co, ctx->P.fixed_dt, adj->g_alpha, adj->g_co,
+    const bool whole = whole_exponent(ph.p1) && whole_exponent(ph.p2);
+    with_kernel(ctx->P.kernel, [&](auto kk) {
+        with_pow(whole, [&](auto ww) {
+            k_adj_pair<decltype(kk)::value, decltype(ww)::value><<<Rp, kAdjBlock, 0, s>>>(
+                H, T, n, ph, tape->lk, A, tape->vbx, tape->vby, ctx->P.damping, euler, p2);
+        });
+    });
+    const int Ra = nblk_(n, kAdjBlock);  // the argmax partials of the recording
+    k_adj_final<<<1, 1024, 0, s>>>(H, T, A, p1, R, p2, Rp, tape->amax_v + (size_t)Ra * slot,
+                                   tape->amax_i + (size_t)Ra * slot, Ra, ctx->P.co, ctx->P.fixed_dt, adj->g_alpha, adj->g_co,
                                    tape->force_steps);
     HIPCHK(hipGetLastError());
     return 0;

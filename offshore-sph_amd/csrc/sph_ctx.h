@@ -57,8 +57,6 @@ namespace hipsph {
 struct TapeHdr {
     Grid grid;
     double dt, dt_c, dt_f;
-    double amax2;  // max |a_prev|^2 over the fluid (the force criterion's argument)
-    int amax_id;   // a fluid particle attaining it (smallest id)
     int active;
 };
 
@@ -98,7 +96,9 @@ struct sph_tape {
     double *vbx = nullptr, *vby = nullptr;
     double4 *lk = nullptr;
     double *part = nullptr;  // reduction partials
-    double *amax_v = nullptr;  // argmax partials (value, id) per workgroup
+    // per slot and workgroup: max |a_prev|^2 over the fluid (the force
+    // criterion's argument) and a fluid particle attaining it (smallest id)
+    double *amax_v = nullptr;
     int *amax_i = nullptr;
     int *force_steps = nullptr;  // device counter: reversed steps whose dt came from the force criterion
 };
