@@ -258,13 +258,8 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
             atomicOr(&I.flags, (unsigned)SPH_FLAG_OOB_KEY);
         }
     }
-    const int prev = __shfl_up(b, 1, 64);
-    const int prev_id = __shfl_up(id, 1, 64);
-    const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
-    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-    const int leader = 63 - __clzll(heads & upto);
-    const unsigned long long after = heads & ~upto;
-    const int next = after ? __ffsll((long long)after) - 1 : 64;
+    int leader, next;
+    bin_run(b, id, leader, next);
     int base = 0;
     if (lane == leader && b >= 0) {
         base = atomicAdd(&counts[b], next - leader);

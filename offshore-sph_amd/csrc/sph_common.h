@@ -459,6 +459,22 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, con
         cellStart[nbins] = sum;
 }
 
+// Runs of equal bins in lane order. A run also breaks where the reference
+// index drops (consecutive slots from two old cells), so every run is in
+// reference-index order; a bin that receives two runs is flagged for
+// bin_place. leader: the first lane of this lane's run; next: the lane after
+// its last.
+__device__ inline void bin_run(int b, int id, int &leader, int &next) {
+    const int lane = threadIdx.x & 63;
+    const int prev = __shfl_up(b, 1, 64);
+    const int prev_id = __shfl_up(id, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
+    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+    leader = 63 - __clzll(heads & upto);
+    const unsigned long long after = heads & ~upto;
+    next = after ? __ffsll((long long)after) - 1 : 64;
+}
+
 // Each particle's place from its bin's offset and its rank there: perm0 maps
 // places to slots. Inside a bin the order is that of the ranks' atomics;
 // bin_place orders it. clear (after k_scan_one): also zeroes the counts for

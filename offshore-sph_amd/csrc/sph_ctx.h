@@ -21,6 +21,7 @@ struct sph_ctx {
     unsigned long long *slots = nullptr;  // reduction slots (Slots)
     int2 *cxy_s = nullptr;  // raw cell (cx, cy) of each slot in cell order
     int *counts = nullptr, *cellStart = nullptr, *tileSums = nullptr, *binflag = nullptr;
+    int *members = nullptr;  // the bins' first indices (k_reorder_scan); null: the update of a larger state
     double *part_b = nullptr, *part_d = nullptr;  // per-workgroup partials: bounds, dt
     double *part_k = nullptr;                     // kinetic-energy partials + result
     long long cap_cells = 0;

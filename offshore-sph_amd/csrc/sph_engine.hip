@@ -345,8 +345,12 @@ constexpr int kBoundsBlocks = 1024;
 // break, against 9.6 with all 1,024 and 10.1 with 64)
 constexpr int kBorderBlocks = 256;
 __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const int *cellStart, DtFold D,
-                         unsigned long long *bslots) {
+                         unsigned long long *bslots, int *clear, int nclear) {
     __shared__ double lds[kBoundsVQ * 16];
+    if (clear) {  // the last update's counts, all of whose readers (k_reorder_scan) are done
+        const int m = ctrl->counted < nclear ? ctrl->counted : nclear;
+        for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < m; b += gridDim.x * blockDim.x) clear[b] = 0;
+    }
     __shared__ double s_dt, s_disp;
     __shared__ int s_active;
     double dt, disp;
@@ -423,6 +427,8 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
     }
 }
 
+// The least number of a bin's indices that k_keys lists for k_reorder_scan.
+constexpr int kBinMembers = 16;
 // _bin :129-141: cid = floor((x - xmin) / cs) per axis (:146-176), flat key
 // cx + ncx * cy (:200-208). Counts per bin; the rank inside a bin comes from
 // one atomic per run of equal bins within a wavefront (the state is already
@@ -437,7 +443,7 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
 // slots that k_bounds has folded.
 __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double scale, long long cap,
                        const unsigned long long *bslots, unsigned long long *dslots, double *hist, int *counts, int *bin,
-                       int *rank, int *binflag) {
+                       int *rank, int *binflag, int *members, int most) {
     if (!(fold ? ctrl->nx.active : ctrl->active)) {
         if (fold && blockIdx.x == 0 && threadIdx.x == 0) dt_commit(ctrl, ctrl->nx, hist);
         return;
@@ -505,17 +511,9 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
             atomicOr(&ctrl->flags, (unsigned)SPH_FLAG_OOB_KEY);
         }
     }
-    // Runs of equal bins in lane order, one atomic per run. A run also breaks
-    // where the reference index drops (consecutive slots from two old cells),
-    // so every run is in reference-index order; a bin that receives two runs
-    // is flagged for bin_place below.
-    const int prev = __shfl_up(b, 1, 64);
-    const int prev_id = __shfl_up(id, 1, 64);
-    const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
-    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-    const int leader = 63 - __clzll(heads & upto);
-    const unsigned long long after = heads & ~upto;
-    const int next = after ? __ffsll((long long)after) - 1 : 64;
+    // one atomic per run of equal bins
+    int leader, next;
+    bin_run(b, id, leader, next);
     int base = 0;
     if (lane == leader && b >= 0) {
         base = atomicAdd(&counts[b], next - leader);
@@ -527,8 +525,10 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
     }
     base = __shfl(base, leader, 64);
     if (t < n) {
+        const int r = base + (lane - leader);
         bin[t] = b;
-        rank[t] = base + (lane - leader);
+        rank[t] = r;
+        if (members && r < most) members[(size_t)b * most + r] = id;  // for k_reorder_scan
     }
 }
 
@@ -556,32 +556,48 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
 // perm0 gives the source slot of each place, in any order inside a bin; the
 // slot t that a thread writes is the place of its particle in index order
 // (bin_place), and perm[t] records the source slot for the corrector.
-__global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *perm, const int *cellStart,
-                          const int *binflag, int2 *cxy_s, Phys ph, int n, int fmt, void *recA, void *recB, int pred,
-                          int strict, int lean, int xs, int dyn, HmConst hc, int carry) {
-    // An inactive step (halted, or past the duration) still flips the
-    // buffers on the host, so copy the state unpermuted.
-    const int act = ctrl->active;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    if (t == 0 && act) ctrl->nn_valid = 1;
-    const int s = act ? perm0[t] : t;
-    const int id = a.id[s];
+struct Moved {  // one particle on its way
+    double x, y, vx, vy, rho, m, h, ax, ay, drho, x0, y0, vx0, vy0, rho0;
+    int id;
+    int8_t lab;
+    bool skip, moved;
+};
+struct ReorderArgs {
+    State a, b;
+    int *perm;
+    const int *cellStart, *binflag;
+    int2 *cxy_s;
+    Phys ph;
+    int n, fmt;
+    void *recA, *recB;
+    int pred, strict, lean, xs, dyn;
+    HmConst hc;
+    int carry;
+};
+__device__ inline Moved reorder_load(const Ctrl *ctrl, const ReorderArgs &A, int act, int s) {
+    const State &a = A.a;
+    Moved p;
+    p.id = a.id[s];
     double x = a.x[s], y = a.y[s], vx = a.vx[s], vy = a.vy[s], rho = a.rho[s];
-    double m = hc.on ? hc.m : a.m[s], h = hc.on ? hc.h : a.h[s];
+    p.m = A.hc.on ? A.hc.m : a.m[s];
+    p.h = A.hc.on ? A.hc.h : a.h[s];
     const double ax = a.ax[s], ay = a.ay[s], drho = a.drho[s];
-    int8_t lab = a.label[s];
-    const bool skip = lean && act && pred && lab == kFluid;
-    const bool moved = act && pred && lab == kFluid;
-    const double x0 = x, y0 = y, vx0 = vx, vy0 = vy, rho0 = rho;
-    if (moved) {
+    const int8_t lab = a.label[s];
+    p.skip = A.lean && act && A.pred && lab == kFluid;
+    p.moved = act && A.pred && lab == kFluid;
+    p.x0 = x;
+    p.y0 = y;
+    p.vx0 = vx;
+    p.vy0 = vy;
+    p.rho0 = rho;
+    if (p.moved) {
         // PEC.predict (src/Integrators/PEC.py:32-59) fused into the permutation
         const double dt = ctrl->dt, damping = ctrl->damping;
-        x = pec_half_pos(x, pred == 2 ? a.xsphx[s] : vx, dt);
-        y = pec_half_pos(y, pred == 2 ? a.xsphy[s] : vy, dt);
+        x = pec_half_pos(x, A.pred == 2 ? a.xsphx[s] : vx, dt);
+        y = pec_half_pos(y, A.pred == 2 ? a.xsphy[s] : vy, dt);
         vx = pec_half_vel(vx, ax, dt, damping);
         vy = pec_half_vel(vy, ay, dt, damping);
-        rho = pec_half_rho(rho, drho, dt, strict);
+        rho = pec_half_rho(rho, drho, dt, A.strict);
     } else if (act && lab == kCoupled && ctrl->nm) {
         // NewmarkBeta.predict (src/Integrators/NewmarkBeta.py:41-52), src/Solver.py:381-382
         const double dt = ctrl->dt, nb = ctrl->nm_beta, ng = ctrl->nm_gamma;
@@ -590,23 +606,37 @@ __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *p
         vx = nm_pred_vel(vx, ax, ng, dt);
         vy = nm_pred_vel(vy, ay, ng, dt);
     }
+    p.x = x;
+    p.y = y;
+    p.vx = vx;
+    p.vy = vy;
+    p.rho = rho;
+    p.ax = ax;
+    p.ay = ay;
+    p.drho = drho;
+    p.lab = lab;
+    return p;
+}
+// k_keys' bin
+__device__ inline long long reorder_bin(const Grid &g, int2 cc) {
+    const long long key = (long long)cc.x + g.ncx * (long long)cc.y;
+    return key >= 0 && key < g.ncells ? key : g.ncells;
+}
+// p, of slot s, into place t
+__device__ inline void reorder_store(Ctrl *ctrl, const ReorderArgs &A, int act, int s, int t, int2 cc, const Moved &p) {
+    const State &a = A.a, &b = A.b;
     const Grid &g = ctrl->grid;
-    int2 cc = make_int2(0, 0);
-    if (act) {
-        cc = cell_of(x, y, g);
-        const long long key = (long long)cc.x + g.ncx * (long long)cc.y;  // k_keys' bin
-        t = bin_place(t, id, key >= 0 && key < g.ncells ? key : g.ncells, cellStart, binflag, ctrl->epoch, perm0, a.id);
-        perm[t] = s;
-    }
-    if (moved) {
-        if (!skip) {
-            b.x0[t] = x0;
-            b.y0[t] = y0;
-            b.vx0[t] = vx0;
-            b.vy0[t] = vy0;
-            b.rho0[t] = rho0;
+    const int8_t lab = p.lab;
+    double h = p.h;
+    if (p.moved) {
+        if (!p.skip) {
+            b.x0[t] = p.x0;
+            b.y0[t] = p.y0;
+            b.vx0[t] = p.vx0;
+            b.vy0[t] = p.vy0;
+            b.rho0[t] = p.rho0;
         }
-    } else if (carry) {
+    } else if (A.carry) {
         b.x0[t] = a.x0[s];
         b.y0[t] = a.y0[s];
         b.vx0[t] = a.vx0[s];
@@ -615,33 +645,268 @@ __global__ void k_reorder(Ctrl *ctrl, State a, State b, const int *perm0, int *p
     }
     // SolverTools.computeH :106-118, sigma 1.3, d = 2 (the reference's fastmath
     // (m / rho) ** 0.5 is the square root)
-    if (dyn && act && lab == kFluid) h = rho > 1e-12 ? 1.3 * sqrt(m / rho) : 0.0;
-    if (!skip) {
-        b.x[t] = x;
-        b.y[t] = y;
-        b.vx[t] = vx;
-        b.vy[t] = vy;
-        b.rho[t] = rho;
+    if (A.dyn && act && lab == kFluid) h = p.rho > 1e-12 ? 1.3 * sqrt(p.m / p.rho) : 0.0;
+    if (!p.skip) {
+        b.x[t] = p.x;
+        b.y[t] = p.y;
+        b.vx[t] = p.vx;
+        b.vy[t] = p.vy;
+        b.rho[t] = p.rho;
     }
-    if (!hc.on) {  // else both buffers hold the one m and h in every slot
-        b.m[t] = m;
+    if (!A.hc.on) {  // else both buffers hold the one m and h in every slot
+        b.m[t] = p.m;
         b.h[t] = h;
     }
     b.label[t] = lab;
-    b.id[t] = id;
-    if (xs || lab != kFluid) {  // without XSPH the fluid's is 0 after every loop (WCSPH.py:187-189)
+    b.id[t] = p.id;
+    if (A.xs || lab != kFluid) {  // without XSPH the fluid's is 0 after every loop (WCSPH.py:187-189)
         b.xsphx[t] = a.xsphx[s];
         b.xsphy[t] = a.xsphy[s];
     }
-    if (!skip || !(cc.x >= 0 && cc.x < g.ncx && cc.y >= 0 && cc.y < g.ncy && h > 0.0 && ph.qmax >= 0.0)) {
-        b.ax[t] = ax;
-        b.ay[t] = ay;
-        b.drho[t] = drho;
+    if (!p.skip || !(cc.x >= 0 && cc.x < g.ncx && cc.y >= 0 && cc.y < g.ncy && h > 0.0 && A.ph.qmax >= 0.0)) {
+        b.ax[t] = p.ax;
+        b.ay[t] = p.ay;
+        b.drho[t] = p.drho;
     }
     if (!act) return;
-    cxy_s[t] = cc;
-    const double pr = write_pair_records(t, x, y, vx, vy, rho, m, h, lab, ph, fmt, recA, recB);
+    A.cxy_s[t] = cc;
+    const double pr = write_pair_records(t, p.x, p.y, p.vx, p.vy, p.rho, p.m, h, lab, A.ph, A.fmt, A.recA, A.recB);
     if (lab == kFluid && !isfinite(pr)) atomicOr(&ctrl->flags, (unsigned)SPH_FLAG_ZERO_DENSITY);
+}
+__global__ void k_reorder(Ctrl *ctrl, ReorderArgs A, const int *perm0) {
+    // An inactive step (halted, or past the duration) still flips the
+    // buffers on the host, so copy the state unpermuted.
+    const int act = ctrl->active;
+    int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= A.n) return;
+    if (t == 0 && act) ctrl->nn_valid = 1;
+    const int s = act ? perm0[t] : t;
+    const Moved p = reorder_load(ctrl, A, act, s);
+    int2 cc = make_int2(0, 0);
+    if (act) {
+        cc = cell_of(p.x, p.y, ctrl->grid);
+        t = bin_place(t, p.id, reorder_bin(ctrl->grid, cc), A.cellStart, A.binflag, ctrl->epoch, perm0, A.a.id);
+        A.perm[t] = s;
+    }
+    reorder_store(ctrl, A, act, s, t, cc, p);
+}
+
+// The scan, the places and the reorder in one kernel, for a state of at most
+// kReorderScanMax particles: slot s goes to its bin's offset plus the number
+// of smaller indices in the bin (k_keys has listed the bin's first `most`;
+// crowded_ranks counts in a bin of more). The first kReorderShares workgroups
+// write cellStart (scan_share); each of the others scans the bins of its
+// SLOTS slots for itself and sums the counts before them, with 1,024 threads of
+// which SLOTS carry a slot. Launches, drains and dependent trips to memory are
+// what a small state's update costs: every load is issued in one of two
+// rounds, the bins and states, then the counts and members. Steps in us, by
+// k_scan_one (two kernels above 65,536), k_place and k_reorder and by this:
+//     FP64, 6.5k particles 38.9, 33.5; 39k 51.6, 45.7; 112k 66.6, 60.8
+//     FP32C, 53k 46.7, 40.5; 112k 55.1, 50.6
+// and the same on grids of up to 18 cells per particle (6.5k: 40.5, 37.0).
+// One round of workgroups on the chip: 256 slots each to 57,344 particles
+// (60k: 53.3 against 56.8 before, then 61.3 against 61.1 at 66k), 512 to 114,688.
+constexpr int kReorderShares = 32;
+constexpr int kScanBins = 1 << 13;  // bins in LDS at a time
+constexpr int kReorderScanMax = (256 - kReorderShares) * 512;
+constexpr long long kReorderScanCap = 1 << 20;  // most cells
+constexpr size_t kMembersBytes = 128u << 20;
+// Indices per bin that k_keys lists: a bin of a water column holds 7, of
+// walls without h (cells of 1 m, whatever the spacing) or a wider scale more.
+inline int bin_members(long long cap) {
+    int m = 256;
+    while (m > kBinMembers && sizeof(int) * m * (size_t)(cap + 1) > kMembersBytes) m /= 2;
+    return m;
+}
+
+// For every slot of the workgroup whose bin holds more than are listed (key
+// >= 0), the number of smaller indices in the bin, from all particles' bins:
+// tiles of kCrowdTile staged in LDS, the workgroup's threads sharing each
+// slot's tile.
+constexpr int kCrowdTile = kScanBins / 2;
+template <int SLOTS>
+__device__ inline int crowded_ranks(int key, int id, int n, const int *bin, const int *ids, int *s_tile) {
+    __shared__ int s_key[SLOTS], s_id[SLOTS], s_cnt[SLOTS];
+    const int tid = threadIdx.x, q = tid % SLOTS, part = tid / SLOTS;
+    constexpr int parts = kScanThreads / SLOTS, len = kCrowdTile / parts;
+    if (tid < SLOTS) {
+        s_key[tid] = key;
+        s_id[tid] = id;
+        s_cnt[tid] = 0;
+    }
+    __syncthreads();
+    const int k = s_key[q], my = s_id[q];
+    int r = 0;
+    for (int u0 = 0; u0 < n; u0 += kCrowdTile) {
+        for (int j = tid; j < kCrowdTile; j += kScanThreads) {
+            s_tile[j] = u0 + j < n ? bin[u0 + j] : -1;
+            s_tile[kCrowdTile + j] = u0 + j < n ? ids[u0 + j] : 0;
+        }
+        __syncthreads();
+        if (k >= 0)
+            for (int j = part * len; j < (part + 1) * len; j += 4) {
+                const int4 b = *reinterpret_cast<const int4 *>(s_tile + j);
+                if (b.x != k && b.y != k && b.z != k && b.w != k) continue;
+                const int4 c = *reinterpret_cast<const int4 *>(s_tile + kCrowdTile + j);
+                r += (b.x == k && c.x < my) + (b.y == k && c.y < my) + (b.z == k && c.z < my) + (b.w == k && c.w < my);
+            }
+        __syncthreads();
+    }
+    if (r) atomicAdd(&s_cnt[q], r);
+    __syncthreads();
+    return tid < SLOTS ? s_cnt[tid] : 0;
+}
+
+template <int SLOTS>
+__global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, ReorderArgs A, const int *counts,
+                                                               int *cellStart, const int *bin, const int *rank,
+                                                               const int *members, int most,
+                                                               unsigned long long *bslots) {
+    __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
+    __shared__ int lds[16], s_lo[SLOTS / 64], s_hi[SLOTS / 64];
+    constexpr bool kPacked = SLOTS <= kBlock;  // n < 65,536
+    const int act = ctrl->active, n = A.n, tid = threadIdx.x;
+    if (blockIdx.x < kReorderShares) {
+        if (blockIdx.x == 0 && tid < kBoundsSlots * kBoundsStride) bslots[tid] = 0;  // as k_place
+        if (!act) return;
+        const int nbins = (int)ctrl->grid.ncells + 1;
+        int sum;
+        scan_share(counts, cellStart, nbins, blockIdx.x, kReorderShares, 0, lds, sum);
+        if (blockIdx.x == 0 && tid == 0) {
+            ctrl->nn_valid = 1;
+            ctrl->counted = nbins;
+            cellStart[nbins] = n;
+        }
+        return;
+    }
+    const int s = ((int)blockIdx.x - kReorderShares) * SLOTS + tid;
+    const bool live = tid < SLOTS && s < n;
+    Moved p{};
+    int t = s, key = -1, r = 0, begin = 0, end = 0;
+    if (live) {
+        key = act ? bin[s] : 0;
+        r = rank[s];
+        p = reorder_load(ctrl, A, act, s);
+    }
+    if (act) {
+        if (tid < SLOTS) {
+            int lo = live ? key : 0x7fffffff, hi = key;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const int l2 = __shfl_xor(lo, o, 64), h2 = __shfl_xor(hi, o, 64);
+                lo = l2 < lo ? l2 : lo;
+                hi = h2 > hi ? h2 : hi;
+            }
+            if ((tid & 63) == 0) {
+                s_lo[tid >> 6] = lo;
+                s_hi[tid >> 6] = hi;
+            }
+        }
+        __syncthreads();
+        bool flagged = false;
+        int4 mem[kBinMembers / 4];
+        if (live) {
+            flagged = A.binflag[key] == ctrl->epoch;
+#pragma unroll
+            for (int j = 0; j < kBinMembers / 4; ++j)
+                mem[j] = *reinterpret_cast<const int4 *>(members + (size_t)key * most + 4 * j);
+        }
+        int lo = s_lo[0], hi = s_hi[0];
+#pragma unroll
+        for (int j = 1; j < SLOTS / 64; ++j) {
+            lo = s_lo[j] < lo ? s_lo[j] : lo;
+            hi = s_hi[j] > hi ? s_hi[j] : hi;
+        }
+        // rows of four bins; the counts past the last bin's row are not read
+        const int from0 = lo & ~3, to = (hi | 3) + 1;
+        unsigned pre = 0;
+        {
+            constexpr int U = 4;  // loads in flight per thread
+            for (int j = 4 * tid; j < from0; j += 4 * U * kScanThreads) {
+                int4 c[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int q = j + 4 * u * kScanThreads;
+                    c[u] = q < from0 ? *reinterpret_cast<const int4 *>(counts + q) : make_int4(0, 0, 0, 0);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) pre += (unsigned)(c[u].x + c[u].y + c[u].z + c[u].w);
+            }
+        }
+        int run = 0;
+        for (int from = from0; from < to; from += kScanBins) {
+            const int m = to - from < kScanBins ? to - from : kScanBins;
+            constexpr int U = kScanBins / (4 * kScanThreads);
+            const int rows = (m + 4 * kScanThreads - 1) / (4 * kScanThreads);
+            int4 c[U];
+            unsigned sum = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int j = 4 * (tid * rows + u);
+                c[u] = u < rows && j < m ? *reinterpret_cast<const int4 *>(counts + from + j) : make_int4(0, 0, 0, 0);
+                sum += (unsigned)(c[u].x + c[u].y + c[u].z + c[u].w);
+            }
+            int tot, ex;
+            if (kPacked) {  // the stretch's sum below, that of the counts before it above
+                const unsigned both = (unsigned)block_scan_excl((int)(sum | pre << 16), lds, &tot);
+                run += (int)((unsigned)tot >> 16);
+                ex = run + (int)(both & 0xffff);
+                run += (int)((unsigned)tot & 0xffff);
+            } else {
+                if (from == from0) {
+                    block_scan_excl((int)pre, lds, &tot);
+                    run += tot;
+                }
+                ex = run + block_scan_excl((int)sum, lds, &tot);
+                run += tot;
+            }
+            pre = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int j = 4 * (tid * rows + u);
+                if (u >= rows || j >= m) continue;
+                const int4 e = make_int4(ex, ex + c[u].x, ex + c[u].x + c[u].y, ex + c[u].x + c[u].y + c[u].z);
+                *reinterpret_cast<int4 *>(s_start + j) = e;
+                ex = e.w + c[u].w;
+            }
+            __syncthreads();
+            const int k = key - from;
+            if (live && k >= 0 && k < m) {
+                begin = s_start[k];
+                end = k + 1 < m ? s_start[k + 1] : run;
+            }
+            __syncthreads();
+        }
+        const int cnt = end - begin;
+        if (flagged) {
+            r = 0;
+#pragma unroll
+            for (int j = 0; j < kBinMembers / 4; ++j) {
+                r += 4 * j < cnt && mem[j].x < p.id;
+                r += 4 * j + 1 < cnt && mem[j].y < p.id;
+                r += 4 * j + 2 < cnt && mem[j].z < p.id;
+                r += 4 * j + 3 < cnt && mem[j].w < p.id;
+            }
+            if (cnt > kBinMembers && cnt <= most)
+                for (int j = kBinMembers; j < cnt; j += 4) {
+                    const int4 c = *reinterpret_cast<const int4 *>(members + (size_t)key * most + j);
+                    r += c.x < p.id;
+                    r += j + 1 < cnt && c.y < p.id;
+                    r += j + 2 < cnt && c.z < p.id;
+                    r += j + 3 < cnt && c.w < p.id;
+                }
+        }
+        const bool crowded = flagged && cnt > most;
+        if (__syncthreads_or(crowded)) {
+            const int rc = crowded_ranks<SLOTS>(crowded ? key : -1, p.id, n, bin, A.a.id, s_start);
+            if (crowded) r = rc;
+        }
+        if (live) {
+            t = begin + r;
+            A.perm[t] = s;
+        }
+    }
+    if (live) reorder_store(ctrl, A, act, s, t, act ? cell_of(p.x, p.y, ctrl->grid) : make_int2(0, 0), p);
 }
 
 // The records of the current cell-ordered state in format fmt (after a
@@ -1052,7 +1317,7 @@ static void free_ctx(sph_ctx *c) {
         if (c->arena[k]) hipFree(c->arena[k]);
     }
     void *ptrs[] = {c->ctrl, c->dt_hist, c->bin, c->rank, c->perm, c->perm0, c->slots, c->cxy_s,
-                    c->counts, c->cellStart, c->tileSums, c->binflag, c->part_b, c->part_d, c->part_k, c->recA, c->recB,
+                    c->counts, c->cellStart, c->tileSums, c->binflag, c->members, c->part_b, c->part_d, c->part_k, c->recA, c->recB,
                     c->slot_of};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -1066,18 +1331,26 @@ static int alloc_cells(sph_ctx *c, long long cap) {
     if (c->cellStart) hipFree(c->cellStart);
     if (c->tileSums) hipFree(c->tileSums);
     if (c->binflag) hipFree(c->binflag);
+    if (c->members) hipFree(c->members);
     c->counts = nullptr;
     c->cellStart = nullptr;
     c->tileSums = nullptr;
     c->binflag = nullptr;
+    c->members = nullptr;
     long long tiles = (cap + 1 + kScanTile - 1) / kScanTile;
-    HIPCHK(hipMalloc(&c->counts, sizeof(int) * (cap + 1)));
+    const size_t rows = ((size_t)cap + 1 + 3) / 4;  // counts are read in rows of four bins
+    HIPCHK(hipMalloc(&c->counts, sizeof(int) * 4 * rows));
     HIPCHK(hipMalloc(&c->cellStart, sizeof(int) * (cap + 2)));
     HIPCHK(hipMalloc(&c->tileSums, sizeof(int) * (tiles + 1)));
-    HIPCHK(hipMemset(c->counts, 0, sizeof(int) * (cap + 1)));
+    HIPCHK(hipMemset(c->counts, 0, sizeof(int) * 4 * rows));
     HIPCHK(hipMemset(c->cellStart, 0, sizeof(int) * (cap + 2)));
     HIPCHK(hipMalloc(&c->binflag, sizeof(int) * (cap + 1)));
     HIPCHK(hipMemset(c->binflag, 0, sizeof(int) * (cap + 1)));
+    if (c->n <= kReorderScanMax && cap <= kReorderScanCap &&
+        hipMalloc(&c->members, sizeof(int) * bin_members(cap) * (cap + 1)) != hipSuccess) {
+        c->members = nullptr;  // the update of a larger state needs none
+        (void)hipGetLastError();
+    }
     c->cap_cells = cap;
     return 0;
 }
@@ -1434,14 +1707,18 @@ struct NnWork {
     Ctrl *ctrl;
     Slots slots;
     int *counts, *cellStart, *tileSums, *binflag, *bin, *rank, *perm0;
+    int *members;  // not null: k_reorder_scan follows (then no places, and the counts stay until the next k_bounds)
+    int most;      // members per bin
     long long cap;
 };
 static void nn_launch(const NnWork &w, const State &a, int n, int pred, const HmConst &hc, const int *border,
                       double scale, const DtFold &D, hipStream_t s) {
     const int R = redblk(n) < kBoundsBlocks ? redblk(n) : kBoundsBlocks;
-    k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b);
+    k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b, w.members ? w.counts : nullptr,
+                                 (int)w.cap + 1);
     k_keys<<<nblk(n), kBlock, 0, s>>>(w.ctrl, a, n, pred, D.on, scale, w.cap, w.slots.b, w.slots.d, D.hist, w.counts,
-                                      w.bin, w.rank, w.binflag);
+                                      w.bin, w.rank, w.binflag, w.members, w.most);
+    if (w.members) return;  // k_reorder_scan does the rest
     const bool one = n <= kScanOneMax;
     if (one) {
         k_scan_one<<<kScanBlocks, kScanThreads, 0, s>>>(w.ctrl, w.counts, w.cellStart);
@@ -1480,13 +1757,22 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
     const int *border = c->border_bounds && pred == 1 ? c->cellStart : nullptr;
     const HmConst hc = hm_const(c);
     const Slots sl = slots_of(c->slots);
-    const NnWork w{c->ctrl, sl, c->counts, c->cellStart, c->tileSums, c->binflag, c->bin, c->rank, c->perm0, c->cap_cells};
+    const NnWork w{c->ctrl, sl, c->counts, c->cellStart, c->tileSums, c->binflag, c->bin, c->rank, c->perm0,
+                   c->members, bin_members(c->cap_cells), c->cap_cells};
     nn_launch(w, a, n, pred, hc, border, c->P.scale,
               DtFold{fold, c->P.gamma_c, c->P.gamma_f, c->uni_h, c->dt_hist, c->part_d, sl.d}, s);
     c->rec_fmt = rec_format(c);
-    k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, a, b, c->perm0, c->perm, c->cellStart, c->binflag, c->cxy_s,
-                                         make_phys(c->P), n, c->rec_fmt, c->recA, c->recB, pred, c->P.strict, lean,
-                                         c->P.use_xsph, c->P.dynamic_h, hc, pred == 0 && !c->x0_same);
+    const ReorderArgs ra{a, b, c->perm, c->cellStart, c->binflag, c->cxy_s, make_phys(c->P), n, c->rec_fmt, c->recA,
+                         c->recB, pred, c->P.strict, lean, c->P.use_xsph, c->P.dynamic_h, hc,
+                         pred == 0 && !c->x0_same};
+    if (!w.members)
+        k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, ra, c->perm0);
+    else if (n <= kReorderScanMax / 2)
+        k_reorder_scan<256><<<kReorderShares + nblk(n, 256), kScanThreads, 0, s>>>(
+            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, w.most, sl.b);
+    else
+        k_reorder_scan<512><<<kReorderShares + nblk(n, 512), kScanThreads, 0, s>>>(
+            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, w.most, sl.b);
     HIPCHK(hipGetLastError());
     if (pred) c->x0_same = false;
     if (!c->P.use_xsph) c->xs_fluid_zero = true;
@@ -2293,7 +2579,7 @@ extern "C" int sph_loop_noalloc(const sph_params_t *params, const sph_state_t *s
     a.id = id;
     const long long ninit = (kNaCells + 1 > n ? kNaCells + 1 : n);
     k_na_init<<<nblk(ninit), kBlock, 0, s>>>(ctrl, slots, counts, binflag, id, nn, kNaCells);
-    const NnWork nw{ctrl, slots_of(slots), counts, cellStart, tileSums, binflag, bin, rank, perm0, kNaCells};
+    const NnWork nw{ctrl, slots_of(slots), counts, cellStart, tileSums, binflag, bin, rank, perm0, nullptr, 0, kNaCells};
     nn_launch(nw, a, nn, 0, HmConst{}, nullptr, params->scale, DtFold{}, s);
     const bool f32 = params->precision == SPH_PREC_FP32C;
     const Phys ph = make_phys(*params);
