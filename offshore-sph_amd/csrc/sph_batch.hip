@@ -157,12 +157,15 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
         hmn = hi < hmn ? hi : hmn;
         hmx = hi > hmx ? hi : hmx;
     };
-    if (cellStart && pred && I.uh_on && border_margin_ok(I.grid, s_disp)) {
+    if (cellStart && pred && I.uh_on && I.grid.ncx >= 3 && I.grid.ncy >= 3 && border_margin_ok(I.grid, s_disp)) {
         const int j = c - chunk0[k], nck = chunk0[k + 1] - chunk0[k];
         if (j == 0 && threadIdx.x == 0) I.border_updates += 1;
         hmn = hmx = I.uh;
-        border_walk(cellStart, I.cellBase, I.grid, j * (int)blockDim.x + (int)threadIdx.x, nck * (int)blockDim.x,
-                    take);
+        const BorderWalk W(cellStart, I.cellBase, I.grid, j * (int)blockDim.x + (int)threadIdx.x,
+                           nck * (int)blockDim.x);
+        if (W.first_row() >= 0) take(W.first_row());
+        if (W.first_run() >= 0) take(W.first_run());
+        W.rest(take);
     } else {
         for (int i = cs[c] + threadIdx.x; i < cs[c + 1]; i += blockDim.x) {
             take(i);

@@ -156,8 +156,7 @@ __device__ inline void pec_correct(const State &s, int j, double x0, double y0, 
 struct PecStart {
     double x0, y0, vx0, vy0, rho0, vxh, vyh;
 };
-__device__ inline PecStart pec_start(const PecArgs &C, int j, double dt, double damping) {
-    const int q = C.perm[j];
+__device__ inline PecStart pec_start_from(const PecArgs &C, int q, double dt, double damping) {
     PecStart p;
     p.x0 = C.o.x[q];
     p.y0 = C.o.y[q];
@@ -167,6 +166,9 @@ __device__ inline PecStart pec_start(const PecArgs &C, int j, double dt, double 
     p.vxh = pec_half_vel(p.vx0, C.o.ax[q], dt, damping);
     p.vyh = pec_half_vel(p.vy0, C.o.ay[q], dt, damping);
     return p;
+}
+__device__ inline PecStart pec_start(const PecArgs &C, int j, double dt, double damping) {
+    return pec_start_from(C, C.perm[j], dt, damping);
 }
 __device__ inline void pec_finish(const PecArgs &C, int j, const PecStart &p, double ax, double ay, double drho,
                                   double dt, double damping) {
@@ -549,12 +551,11 @@ __device__ inline int2 cell_of(double x, double y, const Grid &g) {
     return make_int2((int)(long long)fx, (int)(long long)fy);
 }
 
-// The border-cell bounds (after a fused PEC step; see border_bounds_ok in
+// The border-cell bounds (after a fused PEC step; see border_bounds_may in
 // the engine): the margin test, 2 disp under the cell size by far more than
 // the rounding of positions and cell arithmetic (false for +inf and NaN), on
-// a grid of at least 3 x 3 cells.
+// a grid of at least 3 x 3 cells (the caller's test).
 __device__ inline bool border_margin_ok(const Grid &g, double disp) {
-    if (g.ncx < 3 || g.ncy < 3) return false;
     const double slack = 1e-12 * (fabs(g.xmin) + fabs(g.xmax) + fabs(g.ymin) + fabs(g.ymax));
     return 2.0 * disp * (1.0 + 1e-6) + slack < g.cs * (1.0 - 1e-6);
 }
@@ -567,20 +568,40 @@ __device__ inline bool border_margin_ok(const Grid &g, double disp) {
 // ncx - 1 of row r and column 0 of row r + 1 (consecutive keys: one slot
 // range, one wavefront; it also holds what a flat key carries past the last
 // column into the next row). take(slot) for each.
-template <class F>
-__device__ inline void border_walk(const int *cellStart, long long cb, const Grid &g, int tid, int nthreads,
-                                   F &&take) {
-    const long long ncx = g.ncx, ncy = g.ncy;
-    const int a0 = cellStart[cb], a1 = cellStart[cb + ncx];
-    const int b0 = cellStart[cb + (ncy - 2) * ncx], b1 = cellStart[cb + g.ncells + 1];
-    const int la = a1 - a0, lab = la + (b1 - b0);
-    for (int j = tid; j < lab; j += nthreads) take(j < la ? a0 + j : b0 + (j - la));
-    const int lane = tid & 63;
-    for (long long r = tid >> 6; r <= ncy - 3; r += nthreads >> 6) {
-        const int s0 = cellStart[cb + r * ncx + ncx - 2], s1 = cellStart[cb + (r + 1) * ncx + 1];
-        for (int i = s0 + lane; i < s1; i += 64) take(i);
+// The first slot of each kind is known on construction (-1: none), so that
+// a caller can load it while it still decides; rest takes the others.
+struct BorderWalk {
+    const int *start;
+    long long ncx, ncy, cb;
+    int tid, nthreads, a0, la, b0, lab, s0 = 0, s1 = 0;
+    __device__ BorderWalk(const int *cellStart, long long cb_, const Grid &g, int tid_, int nthreads_)
+        : start(cellStart), ncx(g.ncx), ncy(g.ncy), cb(cb_), tid(tid_), nthreads(nthreads_) {
+        a0 = start[cb];
+        const int a1 = start[cb + ncx], b1 = start[cb + g.ncells + 1];
+        b0 = start[cb + (ncy - 2) * ncx];
+        if ((tid >> 6) <= ncy - 3) run(tid >> 6, s0, s1);
+        la = a1 - a0;
+        lab = la + (b1 - b0);
     }
-}
+    __device__ void run(long long r, int &x0, int &x1) const {
+        x0 = start[cb + r * ncx + ncx - 2];
+        x1 = start[cb + (r + 1) * ncx + 1];
+    }
+    __device__ int at(int j) const { return j < la ? a0 + j : b0 + (j - la); }
+    __device__ int first_row() const { return tid < lab ? at(tid) : -1; }
+    __device__ int first_run() const { return s0 + (tid & 63) < s1 ? s0 + (tid & 63) : -1; }
+    template <class F>
+    __device__ void rest(F &&take) const {
+        for (int j = tid + nthreads; j < lab; j += nthreads) take(at(j));
+        const int lane = tid & 63;
+        for (int i = s0 + lane + 64; i < s1; i += 64) take(i);
+        for (long long r = (tid + nthreads) >> 6; r <= ncy - 3; r += nthreads >> 6) {
+            int x0, x1;
+            run(r, x0, x1);
+            for (int i = x0 + lane; i < x1; i += 64) take(i);
+        }
+    }
+};
 
 // Tait pressure + Pb (src/Equations/TaitEOS.py:6-31; WCSPH.py:131-149).
 __device__ inline double tait_p(double rho, int8_t label, double gamma, double B, double rho0, double Pb) {

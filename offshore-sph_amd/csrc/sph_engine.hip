@@ -221,10 +221,13 @@ __global__ void k_correct(Ctrl *ctrl, State s, State o, const int *perm, int n, 
     const int nm = ctrl->nm;
     DtVars v;
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+        // loaded with the label, not after it
         const int8_t lab = s.label[j];
+        const double ax = s.ax[j], ay = s.ay[j];
+        const int q = perm ? perm[j] : j;
         if (lab != kFluid) {
             if (nm && lab == kCoupled) {
-                const double nb = ctrl->nm_beta, ng = ctrl->nm_gamma, ax = s.ax[j], ay = s.ay[j];
+                const double nb = ctrl->nm_beta, ng = ctrl->nm_gamma;
                 s.x[j] = nm_corr_pos(s.x[j], ax, nb, dt);
                 s.y[j] = nm_corr_pos(s.y[j], ay, nb, dt);
                 s.vx[j] = nm_corr_vel(s.vx[j], ax, ng, dt);
@@ -232,14 +235,12 @@ __global__ void k_correct(Ctrl *ctrl, State s, State o, const int *perm, int n, 
             }
             continue;
         }
-        const double ax = s.ax[j], ay = s.ay[j];
         v.add(hc.on ? hc.h : s.h[j], ax, ay);
         if (integrator == SPH_INTEGRATOR_PEC) {
             double x0, y0, vx0, vy0, rho0, vxh, vyh;
             if (perm) {
                 // the half-step velocity again from the same inputs (the
                 // predictor's expression, as in k_reorder)
-                const int q = perm[j];
                 x0 = o.x[q];
                 y0 = o.y[q];
                 vx0 = o.vx[q];
@@ -278,18 +279,24 @@ __global__ void k_correct(Ctrl *ctrl, State s, State o, const int *perm, int n, 
 // pred: 0 none, 1 PEC, 2 PEC moving x by the XSPH velocity (PEC.py:43-48).
 // With Newmark-beta on (ctrl->nm) the coupled particles' predicted position
 // (NewmarkBeta.py:46-47).
-__device__ inline void upd_pos(const Ctrl *ctrl, const State &a, int i, int pred, double dt, double &x,
-                               double &y) {
-    x = a.x[i];
-    y = a.y[i];
+struct PosIn {  // what it is formed from, loaded before dt is known
+    double x, y, vx, vy;
+    int8_t lab;
+};
+__device__ inline PosIn pos_load(const State &a, int i, int pred) {
+    PosIn p{a.x[i], a.y[i], 0.0, 0.0, a.label[i]};
     if (pred) {
-        // the velocity is loaded with the label, not after it, and selected
-        const double vx = pred == 2 ? a.xsphx[i] : a.vx[i], vy = pred == 2 ? a.xsphy[i] : a.vy[i];
-        const bool f = a.label[i] == kFluid;
-        x = f ? pec_half_pos(x, vx, dt) : x;
-        y = f ? pec_half_pos(y, vy, dt) : y;
+        p.vx = pred == 2 ? a.xsphx[i] : a.vx[i];
+        p.vy = pred == 2 ? a.xsphy[i] : a.vy[i];
     }
-    if (ctrl->nm && a.label[i] == kCoupled) {
+    return p;
+}
+__device__ inline void upd_pos(const Ctrl *ctrl, const State &a, int i, const PosIn &p, int pred, double dt, double &x,
+                               double &y) {
+    const bool f = pred && p.lab == kFluid;
+    x = f ? pec_half_pos(p.x, p.vx, dt) : p.x;
+    y = f ? pec_half_pos(p.y, p.vy, dt) : p.y;
+    if (ctrl->nm && p.lab == kCoupled) {
         const double b = ctrl->nm_beta;
         x = nm_pred_pos(x, a.vx[i], a.ax[i], b, dt);
         y = nm_pred_pos(y, a.vy[i], a.ay[i], b, dt);
@@ -308,10 +315,9 @@ __device__ inline void upd_pos(const Ctrl *ctrl, const State &a, int i, int pred
 // binned at the old maximum x lies beyond ncx - 1 cells and one of a column
 // <= ncx - 3 within ncx - 2, so the maximum lies in columns ncx - 2 or
 // ncx - 1; y likewise with rows 0, ncy - 2 and ncy - 1.
-__device__ inline bool border_bounds_ok(const Ctrl *ctrl, const int *cellStart, int pred, const HmConst &hc,
-                                        double disp) {
-    if (!cellStart || pred != 1 || !hc.on || ctrl->nm || !ctrl->nn_valid) return false;
-    return border_margin_ok(ctrl->grid, disp);
+// border_bounds_may: all of it but the displacement, which the dt fold gives.
+__device__ inline bool border_bounds_may(const Ctrl *ctrl, const int *cellStart, int pred, const HmConst &hc) {
+    return cellStart && pred == 1 && hc.on && !ctrl->nm && ctrl->nn_valid && ctrl->grid.ncx >= 3 && ctrl->grid.ncy >= 3;
 }
 
 // What k_bounds takes to fold the dt partials itself (a step's update);
@@ -335,8 +341,8 @@ struct DtFold {
 // their loads issued together (one workgroup per 256 particles measured 40 %
 // slower, the per-workgroup fold paid in more rounds; 2048 workgroups with
 // one particle per round 3 % slower). With cellStart (the fused PEC step)
-// and border_bounds_ok, only the particles of the border cells
-// (border_walk), over the first kBorderBlocks workgroups. The extremes are
+// and border_bounds_may, only the particles of the border cells
+// (BorderWalk), over the first kBorderBlocks workgroups. The extremes are
 // the same values the full scan finds. With PEC's
 // predictor the full scan also finds the largest |vx|, |vy| (k_keys keeps it
 // as ctrl->vbound; +inf if one is not finite).
@@ -353,6 +359,28 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
     }
     __shared__ double s_dt, s_disp;
     __shared__ int s_active;
+    // the first particles of either scan, in flight under the dt fold
+    const int stride = gridDim.x * blockDim.x;
+    const int gt = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool may = border_bounds_may(ctrl, cellStart, pred, hc);
+    const int fblocks = kBorderBlocks < (int)gridDim.x ? kBorderBlocks : (int)gridDim.x;
+    constexpr int U = 4;
+    PosIn p[U];
+    int slot[U];
+    Grid g;
+    if (may) {
+        g = ctrl->grid;
+        const BorderWalk W(cellStart, 0, g, gt, fblocks * blockDim.x);
+        slot[0] = (int)blockIdx.x < fblocks ? W.first_row() : -1;
+        slot[1] = (int)blockIdx.x < fblocks ? W.first_run() : -1;
+        slot[2] = slot[3] = -1;
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) slot[u] = gt + u * stride < n ? gt + u * stride : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (slot[u] >= 0) p[u] = pos_load(a, slot[u], pred);
     double dt, disp;
     if (D.on) {
         double v[kDtQ];
@@ -377,9 +405,9 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
     if (blockIdx.x == 0 && threadIdx.x == 0) ctrl->epoch += 1;
     double xmn = INFINITY, xmx = -INFINITY, ymn = INFINITY, ymx = -INFINITY, hmn = INFINITY, hmx = -INFINITY;
     double bad = 0.0, vmx = -INFINITY;
-    auto take = [&](int i) {
+    auto take = [&](int i, const PosIn &q) {
         double xi, yi;
-        upd_pos(ctrl, a, i, pred, dt, xi, yi);
+        upd_pos(ctrl, a, i, q, pred, dt, xi, yi);
         const double hi = hc.on ? hc.h : a.h[i];
         if (!(xi - xi == 0.0) || !(yi - yi == 0.0)) bad += 1.0;  // NaN or Inf
         xmn = xi < xmn ? xi : xmn;
@@ -389,28 +417,41 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
         hmn = hi < hmn ? hi : hmn;
         hmx = hi > hmx ? hi : hmx;
     };
-    const int stride = gridDim.x * blockDim.x;
-    const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-    if (border_bounds_ok(ctrl, cellStart, pred, hc, disp)) {
-        if (blockIdx.x >= kBorderBlocks) return;
-        const int fstride = (kBorderBlocks < (int)gridDim.x ? kBorderBlocks : (int)gridDim.x) * blockDim.x;
-        if (gt == 0) ctrl->border_updates += 1;
-        hmn = hmx = hc.h;  // every particle's h
-        border_walk(cellStart, 0, ctrl->grid, gt, fstride, take);
-    } else {
-        for (int i0 = gt; i0 < n; i0 += 4 * stride) {
+    const bool border = may && border_margin_ok(g, disp);
+    if (border && (int)blockIdx.x >= fblocks) return;
+    if (border) hmn = hmx = hc.h;  // every particle's h
+    int i0 = gt;
+    if (!may || border) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = i0 + u * stride;
-                if (i < n) {
-                    take(i);
-                    if (pred == 1) {
-                        const double ux = fabs(a.vx[i]), uy = fabs(a.vy[i]);
-                        const double w = (isfinite(ux) && isfinite(uy)) ? (ux > uy ? ux : uy) : INFINITY;
-                        vmx = w > vmx ? w : vmx;
-                    }
+        for (int u = 0; u < U; ++u)
+            if (slot[u] >= 0) take(slot[u], p[u]);
+    }
+    if (border) {
+        if (gt == 0) ctrl->border_updates += 1;
+        BorderWalk(cellStart, 0, g, gt, fblocks * blockDim.x).rest([&](int i) { take(i, pos_load(a, i, pred)); });
+    } else {
+        auto speed = [&](const PosIn &q) {
+            if (pred != 1) return;
+            const double ux = fabs(q.vx), uy = fabs(q.vy);
+            const double w = (isfinite(ux) && isfinite(uy)) ? (ux > uy ? ux : uy) : INFINITY;
+            vmx = w > vmx ? w : vmx;
+        };
+        if (!may) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (slot[u] >= 0) speed(p[u]);
+            i0 += U * stride;
+        }
+        for (; i0 < n; i0 += U * stride) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * stride < n) p[u] = pos_load(a, i0 + u * stride, pred);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * stride < n) {
+                    take(i0 + u * stride, p[u]);
+                    speed(p[u]);
                 }
-            }
         }
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
@@ -444,26 +485,27 @@ constexpr int kBinMembers = 16;
 __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double scale, long long cap,
                        const unsigned long long *bslots, unsigned long long *dslots, double *hist, int *counts, int *bin,
                        int *rank, int *binflag, int *members, int most) {
+    __shared__ double s_v[kBoundsVQ];
+    __shared__ Grid s_g;
+    __shared__ unsigned s_halt;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    // loaded together with the control block
+    const int t0 = t < n ? t : n - 1;
+    const PosIn p = pos_load(a, t0, pred);
+    const int id = t < n ? a.id[t0] : 0x7fffffff;
+    const int bq = threadIdx.x / kBoundsSlots % kBoundsVQ, bk = threadIdx.x % kBoundsSlots;
+    unsigned long long m = bslots[bk * kBoundsStride + bq];
     if (!(fold ? ctrl->nx.active : ctrl->active)) {
         if (fold && blockIdx.x == 0 && threadIdx.x == 0) dt_commit(ctrl, ctrl->nx, hist);
         return;
     }
-    __shared__ double s_v[kBoundsVQ];
-    __shared__ Grid s_g;
-    __shared__ unsigned s_halt;
     const double dt = fold ? ctrl->nx.dt : ctrl->dt;
     const int epoch = ctrl->epoch;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    double x = 0.0, y = 0.0;
-    int id = 0x7fffffff;
-    if (t < n) {
-        upd_pos(ctrl, a, t, pred, dt, x, y);
-        id = a.id[t];
-    }
+    double x, y;
+    upd_pos(ctrl, a, t0, p, pred, dt, x, y);
     if (threadIdx.x < kBoundsVQ * kBoundsSlots) {
-        const int q = threadIdx.x / kBoundsSlots, k = threadIdx.x % kBoundsSlots;
-        unsigned long long m = bslots[k * kBoundsStride + q];
+        const int q = bq, k = bk;
 #pragma unroll
         for (int o = kBoundsSlots / 2; o > 0; o >>= 1) {
             const unsigned long long m2 = __shfl_xor(m, o, 64);
@@ -784,7 +826,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
     Moved p{};
     int t = s, key = -1, r = 0, begin = 0, end = 0;
     if (live) {
-        key = act ? bin[s] : 0;
+        key = bin[s];  // as the ranks, not this update's unless it is active
         r = rank[s];
         p = reorder_load(ctrl, A, act, s);
     }

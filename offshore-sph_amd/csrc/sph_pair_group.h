@@ -239,32 +239,28 @@ template <typename R, int KERNEL, int MODE, bool XS, int G>
 __global__ __launch_bounds__(256) void k_pair_group(const Ctrl *ctrl, PairArgs<R> P, Phys ph) {
     using GG = GeneralGroup<R, KERNEL, MODE, XS>;
     __shared__ GroupMem<GG, G> mem[256 / G];
-    if (!ctrl->active) return;
     const int i = threadIdx.x / G, l = threadIdx.x % G;
     const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    const int t0 = t < P.n ? t : P.n - 1;
+    const typename Rec<R>::A at = P.A[t0];  // the target's records together with the control block
+    const typename Rec<R>::B bt = P.B[t0];
+    const int2 c = P.cxy[t0];
+    const double H = sizeof(R) == 8 ? (double)at.h : P.H[t0];
+    if (!ctrl->active) return;
     const Grid &g = ctrl->grid;
     const int ncx = (int)g.ncx, ncy = (int)g.ncy;
-    typename Rec<R>::A at{};
-    at.w = R(-1);
-    if (t < P.n) at = P.A[t];
     const bool walks = t < P.n && at.w >= R(0);  // walls are not targets
-    Target<R> T{};
-    int2 c = make_int2(0, 0);
-    bool implied = true;
-    if (walks) {
-        const typename Rec<R>::B bt = P.B[t];
-        T.X = at.x;
-        T.Y = at.y;
-        T.H = sizeof(R) == 8 ? (double)at.h : P.H[t];
-        T.h = (R)at.h;
-        T.vx = (R)rec_vx(at, bt);
-        T.vy = (R)rec_vy(at, bt);
-        T.rho = (R)bt.rho;
-        T.slf = (R)bt.prs;
-        T.slot = t;
-        c = P.cxy[t];
-        implied = cutoff_implied<KERNEL>(nullptr, ph.qmax, c, ncx, ncy, T.H);
-    }
+    Target<R> T;
+    T.X = at.x;
+    T.Y = at.y;
+    T.H = H;
+    T.h = (R)at.h;
+    T.vx = (R)rec_vx(at, bt);
+    T.vy = (R)rec_vy(at, bt);
+    T.rho = (R)bt.rho;
+    T.slf = (R)bt.prs;
+    T.slot = t;
+    const bool implied = !walks || cutoff_implied<KERNEL>(nullptr, ph.qmax, c, ncx, ncy, T.H);
     const GG gg{P, T, ph, implied};
     GroupSums<GG, G> acc;
     int cnt = 0;

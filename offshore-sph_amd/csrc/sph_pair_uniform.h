@@ -662,17 +662,11 @@ struct UniformGroup {
 // The rates of target t by its G lanes, in every lane; false: it has no
 // neighbour (or walks is false).
 template <int KERNEL, int MODE, int G>
-__device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformConst &K, int ncx, int ncy, int t,
-                                           const float4 &bt, bool walks, int l,
+__device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformConst &K, int ncx, int ncy,
+                                           const double2 &at, int2 c, const float4 &bt, bool walks, int l,
                                            GroupMem<UniformGroup<KERNEL, MODE>, G> &M, double &drho, double &ax,
                                            double &ay) {
     using UG = UniformGroup<KERNEL, MODE>;
-    double2 at = make_double2(0.0, 0.0);
-    int2 c = make_int2(0, 0);
-    if (walks) {
-        at = P.A[t];
-        c = P.cxy[t];
-    }
     const UG ug{P, K, at.x, at.y, bt};
     GroupSums<UG, G> acc;
     int cnt;
@@ -689,15 +683,17 @@ __device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformCo
 template <int KERNEL, int MODE, int G>
 __global__ __launch_bounds__(256) void k_group_uniform(const Ctrl *ctrl, UniformArgs P, UniformConst K) {
     __shared__ GroupMem<UniformGroup<KERNEL, MODE>, G> mem[256 / G];
-    if (!ctrl->active) return;
     const int i = threadIdx.x / G, l = threadIdx.x % G;
     const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
-    float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
-    if (t < P.n) bt = P.B[t];
+    const int t0 = t < P.n ? t : P.n - 1;
+    const float4 bt = P.B[t0];  // the target's records together with the control block
+    const double2 at = P.A[t0];
+    const int2 c = P.cxy[t0];
+    if (!ctrl->active) return;
     const bool walks = t < P.n && !not_fluid(bt.w);
     const Grid &g = ctrl->grid;
     double drho, ax, ay;
-    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i], drho,
+    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, at, c, bt, walks, l, mem[i], drho,
                                                           ax, ay);
     if (!any || l != 0) return;
     if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
@@ -712,23 +708,26 @@ template <int KERNEL, int MODE, int G>
 __global__ __launch_bounds__(256) void k_group_uniform_pec(Ctrl *ctrl, UniformArgs P, UniformConst K, PecArgs C) {
     __shared__ GroupMem<UniformGroup<KERNEL, MODE>, G> mem[256 / G];
     __shared__ double lds[kDtQ * 16];
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    const int t0 = t < P.n ? t : P.n - 1;
+    const float4 bt = P.B[t0];  // the target's records together with the control block
+    const double2 at = P.A[t0];
+    const int2 c = P.cxy[t0];
+    const int q = C.perm[t0];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctrl->dt_parts = kDtSlots;
         ctrl->pec_parts = 1;
     }
-    const int i = threadIdx.x / G, l = threadIdx.x % G;
-    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
-    float4 bt = make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
-    if (t < P.n) bt = P.B[t];
     const bool walks = t < P.n && !not_fluid(bt.w);
     const Grid &g = ctrl->grid;
     const double dt = ctrl->dt, damping = ctrl->damping;
     const bool corrects = walks && l == 0;
     PecStart p0{};
-    if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
+    if (corrects) p0 = pec_start_from(C, q, dt, damping);  // in flight under the walk
     double drho, ax, ay;
-    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+    const bool any = uniform_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, at, c, bt, walks, l, mem[i],
                                                             drho, ax, ay);
     DtVars v;
     if (corrects) {

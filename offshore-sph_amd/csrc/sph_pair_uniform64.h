@@ -562,17 +562,11 @@ struct Uniform64Group {
 // The rates of target t by its G lanes, in every lane; false: it has no
 // neighbour (or walks is false).
 template <int KERNEL, int MODE, int G>
-__device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy, int t,
-                                             const double4 &bt, bool walks, int l,
+__device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
+                                             const double2 &at, int2 c, const double4 &bt, bool walks, int l,
                                              GroupMem<Uniform64Group<KERNEL, MODE>, G> &M, double &drho, double &ax,
                                              double &ay) {
     using UG = Uniform64Group<KERNEL, MODE>;
-    double2 at = make_double2(0.0, 0.0);
-    int2 c = make_int2(0, 0);
-    if (walks) {
-        at = P.A[t];
-        c = P.cxy[t];
-    }
     // a target whose own cell is in the grid finds itself (q = 0)
     const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;
     const UG ug{P, K, at.x, at.y, bt, !inside};
@@ -589,15 +583,17 @@ __device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Unifo
 template <int KERNEL, int MODE, int G>
 __global__ __launch_bounds__(256) void k_group_uniform64(const Ctrl *ctrl, Uniform64Args P, Uniform64Const K) {
     __shared__ GroupMem<Uniform64Group<KERNEL, MODE>, G> mem[256 / G];
-    if (!ctrl->active) return;
     const int i = threadIdx.x / G, l = threadIdx.x % G;
     const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
-    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
-    if (t < P.n) bt = P.B[t];
+    const int t0 = t < P.n ? t : P.n - 1;
+    const double4 bt = P.B[t0];  // the target's records together with the control block
+    const double2 at = P.A[t0];
+    const int2 c = P.cxy[t0];
+    if (!ctrl->active) return;
     const bool walks = t < P.n && !not_fluid64(bt.w);
     const Grid &g = ctrl->grid;
     double drho, ax, ay;
-    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, at, c, bt, walks, l, mem[i],
                                                             drho, ax, ay);
     if (!any || l != 0) return;
     if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
@@ -614,23 +610,26 @@ __global__ __launch_bounds__(256) void k_group_uniform64_pec(Ctrl *ctrl, Uniform
                                                              PecArgs C) {
     __shared__ GroupMem<Uniform64Group<KERNEL, MODE>, G> mem[256 / G];
     __shared__ double lds[kDtQ * 16];
+    const int i = threadIdx.x / G, l = threadIdx.x % G;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
+    const int t0 = t < P.n ? t : P.n - 1;
+    const double4 bt = P.B[t0];  // the target's records together with the control block
+    const double2 at = P.A[t0];
+    const int2 c = P.cxy[t0];
+    const int q = C.perm[t0];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctrl->dt_parts = kDtSlots;
         ctrl->pec_parts = 1;
     }
-    const int i = threadIdx.x / G, l = threadIdx.x % G;
-    const int t = xcd_remap(blockIdx.x, gridDim.x) * (256 / G) + i;
-    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
-    if (t < P.n) bt = P.B[t];
     const bool walks = t < P.n && !not_fluid64(bt.w);
     const Grid &g = ctrl->grid;
     const double dt = ctrl->dt, damping = ctrl->damping;
     const bool corrects = walks && l == 0;
     PecStart p0{};
-    if (corrects) p0 = pec_start(C, t, dt, damping);  // in flight under the walk
+    if (corrects) p0 = pec_start_from(C, q, dt, damping);  // in flight under the walk
     double drho, ax, ay;
-    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, t, bt, walks, l, mem[i],
+    const bool any = uniform64_group_rates<KERNEL, MODE, G>(P, K, (int)g.ncx, (int)g.ncy, at, c, bt, walks, l, mem[i],
                                                               drho, ax, ay);
     DtVars v;
     if (corrects) {
