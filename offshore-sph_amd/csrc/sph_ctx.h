@@ -1,6 +1,7 @@
 // sph_ctx.h — the context and tape objects behind the C ABI, shared by the
 // engine and the adjoint translation units.
 #pragma once
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -15,6 +16,8 @@ struct sph_ctx {
     void *arena[2] = {nullptr, nullptr};
     int cur = 0;
     hipsph::Ctrl *ctrl = nullptr;
+    hipsph::Ctrl *pinned = nullptr;  // where the host reads ctrl (read_ctrl), under its lock
+    std::mutex pinned_lock;
     double *dt_hist = nullptr;
     // perm0: the source slot of each place before the bins are ordered; perm: after
     int *bin = nullptr, *rank = nullptr, *perm0 = nullptr, *perm = nullptr;

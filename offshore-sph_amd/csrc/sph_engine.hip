@@ -1422,9 +1422,19 @@ static void free_ctx(sph_ctx *c) {
                     c->slot_of};
     for (void *p : ptrs)
         if (p) hipFree(p);
+    if (c->pinned) hipHostFree(c->pinned);
     for (auto e : c->ev_pair) hipEventDestroy(e);
     for (auto e : c->ev_nn) hipEventDestroy(e);
     delete c;
+}
+
+// The control block when s has come to it: one copy to pinned memory.
+static int read_ctrl(sph_ctx *c, hipStream_t s, Ctrl &h) {
+    std::lock_guard<std::mutex> hold(c->pinned_lock);
+    HIPCHK(hipMemcpyAsync(c->pinned, c->ctrl, sizeof h, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    h = *c->pinned;
+    return 0;
 }
 
 static int alloc_cells(sph_ctx *c, long long cap) {
@@ -1607,6 +1617,7 @@ int sph_ctx_create(const sph_params_t *params, sph_ctx_t **out) {
         c->buf[k].label = (int8_t *)p;
     }
     bool ok = hipMalloc(&c->ctrl, sizeof(Ctrl)) == hipSuccess &&
+              hipHostMalloc(&c->pinned, sizeof(Ctrl), hipHostMallocDefault) == hipSuccess &&
               hipMalloc(&c->dt_hist, sizeof(double) * 3 * SPH_DT_HISTORY) == hipSuccess &&
               hipMalloc(&c->bin, sizeof(int) * n) == hipSuccess && hipMalloc(&c->rank, sizeof(int) * n) == hipSuccess &&
               hipMalloc(&c->perm, sizeof(int) * n) == hipSuccess &&
@@ -2177,10 +2188,10 @@ int sph_step_end(sph_ctx_t *ctx, void *stream) {
 // Stage `ids` (host, validated) in ctx->bin and map every reference index to
 // its slot of the current buffer in ctx->slot_of. bin is scratch outside the
 // neighbour update.
-static int stage_ids(sph_ctx *c, const int64_t *ids, int64_t k, bool distinct, hipStream_t s) {
+static int stage_ids(sph_ctx *c, const int64_t *ids, int64_t k, bool distinct, std::vector<int> &v, hipStream_t s) {
     if (k < 0 || k > c->n) return fail(SPH_EINVAL, "k=%lld out of range (0 .. n=%d)", (long long)k, c->n);
     if (k > 0 && !ids) return fail(SPH_EINVAL, "ids is NULL");
-    std::vector<int> v((size_t)k);
+    v.resize((size_t)k);
     for (int64_t j = 0; j < k; ++j) {
         if (ids[j] < 0 || ids[j] >= c->n)
             return fail(SPH_EINVAL, "ids[%lld]=%lld outside 0 .. n-1=%d", (long long)j, (long long)ids[j], c->n - 1);
@@ -2195,7 +2206,6 @@ static int stage_ids(sph_ctx *c, const int64_t *ids, int64_t k, bool distinct, h
     HIPCHK(hipMemcpyAsync(c->bin, v.data(), sizeof(int) * k, hipMemcpyHostToDevice, s));
     k_inverse<<<nblk(c->n), kBlock, 0, s>>>(c->buf[c->cur].id, c->slot_of, c->n);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s));  // v is freed on return
     return 0;
 }
 
@@ -2203,7 +2213,8 @@ int sph_state_gather(sph_ctx_t *ctx, const int64_t *ids, int64_t k, const sph_st
     if (!ctx || !st) return fail(SPH_EINVAL, "NULL argument");
     if (unloaded(ctx)) return SPH_ESTATE;
     hipStream_t s = S(stream);
-    int rc = stage_ids(ctx, ids, k, false, s);
+    std::vector<int> v;  // until the stream has been waited for
+    int rc = stage_ids(ctx, ids, k, false, v, s);
     if (rc || k == 0) return rc;
     k_gather_ids<<<nblk(k), kBlock, 0, s>>>(ctx->buf[ctx->cur], ctx->slot_of, ctx->bin, (int)k, *st,
                                             make_phys(ctx->P), ctx->xs_fluid_zero);
@@ -2219,7 +2230,8 @@ int sph_state_scatter(sph_ctx_t *ctx, const int64_t *ids, int64_t k, const sph_s
     if (!ctx->P.use_xsph && (st->xsphx || st->xsphy))
         return fail(SPH_EUNSUPPORTED, "without XSPH the XSPH velocity is not kept on the device");
     hipStream_t s = S(stream);
-    int rc = stage_ids(ctx, ids, k, true, s);
+    std::vector<int> v;  // until the stream has been waited for
+    int rc = stage_ids(ctx, ids, k, true, v, s);
     if (rc || k == 0) return rc;
     if ((rc = save_start(ctx, s))) return rc;
     k_scatter_ids<<<nblk(k), kBlock, 0, s>>>(ctx->buf[ctx->cur], ctx->slot_of, ctx->bin, (int)k, *st);
@@ -2284,9 +2296,8 @@ int sph_probe_pressure(sph_ctx_t *ctx, int64_t npts, const double *x, const doub
 
 int sph_status(sph_ctx_t *ctx, double out_d[4], int64_t out_i[2], void *stream) {
     if (!ctx) return fail(SPH_EINVAL, "ctx is NULL");
-    HIPCHK(hipStreamSynchronize(S(stream)));
     Ctrl h;
-    HIPCHK(hipMemcpy(&h, ctx->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (int rc = read_ctrl(ctx, S(stream), h)) return rc;
     if (out_d) {
         out_d[0] = h.t;
         out_d[1] = h.dt;
@@ -2327,25 +2338,23 @@ int sph_kinetic_energy(sph_ctx_t *ctx, double *out, void *stream) {
 int sph_dt_history(sph_ctx_t *ctx, double *out3, int64_t count, void *stream) {
     if (!ctx || !out3) return fail(SPH_EINVAL, "NULL argument");
     if (count < 0 || count > SPH_DT_HISTORY) return fail(SPH_EINVAL, "count out of range");
-    HIPCHK(hipStreamSynchronize(S(stream)));
     Ctrl h;
-    HIPCHK(hipMemcpy(&h, ctx->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (int rc = read_ctrl(ctx, S(stream), h)) return rc;
     if (count > h.step) return fail(SPH_EINVAL, "only %lld steps taken", (long long)h.step);
-    std::vector<double> ring(3 * (size_t)SPH_DT_HISTORY);
-    HIPCHK(hipMemcpy(ring.data(), ctx->dt_hist, sizeof(double) * ring.size(), hipMemcpyDeviceToHost));
-    for (int64_t k = 0; k < count; ++k) {
-        long long step = h.step - count + k;
-        long long slot = step % SPH_DT_HISTORY;
-        for (int c = 0; c < 3; ++c) out3[3 * k + c] = ring[3 * slot + c];
-    }
+    // the slots asked for: one stretch of the ring, or its end and its start
+    const int64_t first = (h.step - count) % SPH_DT_HISTORY;
+    const int64_t tail = first + count > SPH_DT_HISTORY ? first + count - SPH_DT_HISTORY : 0;
+    const size_t row = 3 * sizeof(double);
+    if (count > tail)
+        HIPCHK(hipMemcpy(out3, ctx->dt_hist + 3 * first, row * (count - tail), hipMemcpyDeviceToHost));
+    if (tail > 0) HIPCHK(hipMemcpy(out3 + 3 * (count - tail), ctx->dt_hist, row * tail, hipMemcpyDeviceToHost));
     return 0;
 }
 
 int sph_nn_grid(sph_ctx_t *ctx, double out_d[5], int64_t out_i[3], void *stream) {
     if (!ctx) return fail(SPH_EINVAL, "ctx is NULL");
-    HIPCHK(hipStreamSynchronize(S(stream)));
     Ctrl h;
-    HIPCHK(hipMemcpy(&h, ctx->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (int rc = read_ctrl(ctx, S(stream), h)) return rc;
     if (!h.nn_valid) return fail(SPH_ESTATE, "no valid neighbour update (flags=0x%x)", h.flags);
     if (out_d) {
         out_d[0] = h.grid.xmin;
@@ -2474,9 +2483,8 @@ int sph_ctx_set_border_bounds(sph_ctx_t *ctx, int32_t on) {
 
 int sph_nn_border_count(sph_ctx_t *ctx, int64_t *count, void *stream) {
     if (!ctx || !count) return fail(SPH_EINVAL, "NULL argument");
-    HIPCHK(hipStreamSynchronize(S(stream)));
     Ctrl h;
-    HIPCHK(hipMemcpy(&h, ctx->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (int rc = read_ctrl(ctx, S(stream), h)) return rc;
     *count = h.border_updates;
     return 0;
 }

@@ -208,7 +208,7 @@ class Solver:
     def _pull(self, e):
         """Device state -> active records of particleArray."""
         d = e.download()
-        idx = np.nonzero(self.indexes)[0]
+        idx = slice(None) if self.indexes.all() else np.nonzero(self.indexes)[0]
         for k in ('x', 'y', 'vx', 'vy', 'rho', 'ax', 'ay', 'drho', 'p', 'xsphx', 'xsphy', 'h', 'm'):
             self.particleArray[k][idx] = d[k]
         for f, (rows, vals) in self._host_hook.items():  # the last coupling hook's values stand
@@ -218,7 +218,7 @@ class Solver:
         """Launch n device steps; returns the steps actually taken."""
         if self.coupling is not None:
             return sum(self._coupled_step(e) for _ in range(n))
-        before = e.status()['steps']
+        before = self._hist_seen  # the steps of this engine so far
         e.step(n, graph=self.graph and n > 1)
         st = e.status()
         bad = st['flags'] & _HALT_FLAGS
@@ -242,7 +242,7 @@ class Solver:
         active records goes back to the device before the correctors. The
         hook's pressures (and, without XSPH, XSPH velocities) are kept on the
         host: the device derives p from rho and keeps no XSPH velocity then."""
-        before = e.status()['steps']
+        before = self._hist_seen  # the steps of this engine so far
         e.step_begin()
         st = e.status()
         taken = st['steps'] - before

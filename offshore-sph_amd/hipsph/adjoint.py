@@ -116,7 +116,7 @@ class SPHRun:
 
     def _upload_initial(self, v0):
         import torch
-        st = {k: v.clone() for k, v in self._base.items()}
+        st = {k: v.clone() if k in ('vx', 'vy') else v for k, v in self._base.items()}
         v0 = v0.to(device=self.device, dtype=torch.float64)
         st['vx'][self.fluid] = v0[:, 0]
         st['vy'][self.fluid] = v0[:, 1]
