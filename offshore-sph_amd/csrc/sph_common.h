@@ -328,10 +328,52 @@ __device__ inline double nm_pred_vel(double v, double a, double gamma, double dt
 __device__ inline double nm_corr_pos(double x, double a, double beta, double dt) { return x + a * beta * (dt * dt); }
 __device__ inline double nm_corr_vel(double v, double a, double gamma, double dt) { return v + a * gamma * dt; }
 
+// Runs of equal bins in lane order. A run also breaks where the reference
+// index drops (consecutive slots from two old cells), so every run is in
+// reference-index order; a bin that receives two runs is flagged for
+// bin_place. leader: the first lane of this lane's run; next: the lane after
+// its last.
+__device__ inline void bin_run(int b, int id, int &leader, int &next) {
+    const int lane = threadIdx.x & 63;
+    const int prev = __shfl_up(b, 1, 64);
+    const int prev_id = __shfl_up(id, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
+    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+    leader = 63 - __clzll(heads & upto);
+    const unsigned long long after = heads & ~upto;
+    next = after ? __ffsll((long long)after) - 1 : 64;
+}
+
 // Exclusive prefix scan of counts[0 .. ncells] into cellStart, in tiles of
-// kScanTile bins: the tile sums, then each tile's scan offset by the sum of
-// the tile sums before it (a few hundred integers, read by that tile's
-// workgroup: no separate pass over the tile sums).
+// kScanTile bins: the keys kernels add their particles to their tiles' sums
+// as well, so each tile's workgroup reads the sums before it and its own
+// counts in one round of loads. (A kernel of its own for the tile sums took
+// 4.6 us and its launch.) A workgroup's particles lie in one tile or two: those
+// of its first particle's tile are added up in LDS, and the sums
+// lie kTileStride apart, since the atomics of a line go one after another
+// (one per wavefront on packed sums: the 1M dam break's keys take 41 us instead of
+// 16). Called by the whole workgroup; b: the thread's bin, or -1.
+constexpr int kTileStride = 4;
+__device__ inline void tile_add(int *tileSums, int b) {
+    __shared__ int s_tile, s_sum;
+    if (threadIdx.x == 0) {
+        s_tile = b / kScanTile;  // the first thread has a particle
+        s_sum = 0;
+    }
+    __syncthreads();
+    const int tile = b < 0 ? -1 : b / kScanTile;
+    const unsigned long long same = __ballot(tile == s_tile);
+    if ((threadIdx.x & 63) == 0 && same) atomicAdd(&s_sum, __popcll(same));
+    const int other = tile == s_tile ? -1 : tile;
+    if (__ballot(other >= 0)) {
+        int leader, next;
+        bin_run(other, 0, leader, next);
+        if ((int)(threadIdx.x & 63) == leader && other >= 0)
+            atomicAdd(&tileSums[(size_t)other * kTileStride], next - leader);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&tileSums[(size_t)s_tile * kTileStride], s_sum);
+}
 __device__ inline int block_scan_excl(int v, int *lds, int *total) {
     // inclusive scan inside each wave
     int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -355,53 +397,45 @@ __device__ inline int block_scan_excl(int v, int *lds, int *total) {
     return off + s - v;
 }
 
-__global__ void k_scan_reduce(const Ctrl *ctrl, const int *counts, int *tileSums) {
-    if (!ctrl->active) return;
-    long long nbins = ctrl->grid.ncells + 1;
-    long long ntiles = (nbins + kScanTile - 1) / kScanTile;
-    __shared__ double lds[8];
-    for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        long long base = tile * kScanTile;
-        double s = 0.0;
-        for (int k = 0; k < kScanItems; ++k) {
-            long long b = base + (long long)threadIdx.x * kScanItems + k;
-            if (b < nbins) s += (double)counts[b];
-        }
-        s = block_reduce(s, AddOp(), lds);
-        if (threadIdx.x == 0) tileSums[tile] = (int)s;
+// Tile `tile` of the scan of nbins counts, from `first` on (workgroups of
+// kBlock threads, four bins each; counts and cellStart from a multiple of four bins,
+// with whole rows of four). Clears its counts for the next update. lds holds 16 ints.
+__device__ inline void scan_tile(int *counts, const int *tileSums, int *cellStart, long long nbins, long long tile,
+                                 int first, int *lds) {
+    const long long b0 = tile * kScanTile + (long long)threadIdx.x * kScanItems;
+    int4 c = b0 < nbins ? *reinterpret_cast<const int4 *>(counts + b0) : make_int4(0, 0, 0, 0);
+    int pre = 0;
+    constexpr int U = 4;  // loads in flight
+    for (long long j = threadIdx.x; j < tile; j += U * kBlock) {
+        int t[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[u] = j + u * kBlock < tile ? tileSums[(j + u * kBlock) * kTileStride] : 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) pre += t[u];
     }
+    int tot, sum;
+    block_scan_excl(pre, lds, &tot);
+    if (b0 + 1 >= nbins) c.y = 0;  // past the last bin
+    if (b0 + 2 >= nbins) c.z = 0;
+    if (b0 + 3 >= nbins) c.w = 0;
+    const int v[kScanItems] = {c.x, c.y, c.z, c.w};
+    int ex = block_scan_excl(c.x + c.y + c.z + c.w, lds, &sum) + tot + first;
+    if (b0 < nbins) *reinterpret_cast<int4 *>(counts + b0) = make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (b0 + k < nbins) cellStart[b0 + k] = ex;
+        ex += v[k];
+    }
+    // the end of the last bin
+    if (b0 < nbins && b0 + kScanItems >= nbins) cellStart[nbins] = ex;
 }
 
-__global__ void k_scan_apply(const Ctrl *ctrl, int *counts, const int *tileSums, int *cellStart) {
+__global__ __launch_bounds__(kBlock) void k_scan(const Ctrl *ctrl, int *counts, const int *tileSums, int *cellStart) {
     if (!ctrl->active) return;
-    long long nbins = ctrl->grid.ncells + 1;
-    long long ntiles = (nbins + kScanTile - 1) / kScanTile;
     __shared__ int lds[16];
-    for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        long long base = tile * kScanTile;
-        int v[kScanItems];
-        int sum = 0;
-        long long b0 = base + (long long)threadIdx.x * kScanItems;
-        for (int k = 0; k < kScanItems; ++k) {
-            long long b = b0 + k;
-            v[k] = b < nbins ? counts[b] : 0;
-            sum += v[k];
-        }
-        int pre = 0;
-        for (long long j = threadIdx.x; j < tile; j += blockDim.x) pre += tileSums[j];
-        int tot;
-        block_scan_excl(pre, lds, &pre);
-        int ex = block_scan_excl(sum, lds, &tot) + pre;
-        for (int k = 0; k < kScanItems; ++k) {
-            long long b = b0 + k;
-            if (b < nbins) {
-                cellStart[b] = ex;
-                counts[b] = 0;  // ready for the next update (no memset node in a graph)
-            }
-            ex += v[k];
-        }
-        if (tile == ntiles - 1 && threadIdx.x == blockDim.x - 1) cellStart[nbins] = ex;
-    }
+    const long long nbins = ctrl->grid.ncells + 1;
+    for (long long tile = blockIdx.x; tile * kScanTile < nbins; tile += gridDim.x)
+        scan_tile(counts, tileSums, cellStart, nbins, tile, 0, lds);
 }
 
 // Share i of S of the exclusive scan of counts[0 .. nbins) (16-byte aligned)
@@ -446,51 +480,19 @@ __device__ inline bool scan_share(const int *counts, int *cellStart, long long n
     return b1 == nbins;
 }
 
-// The scan in one kernel of kScanBlocks workgroups, for a state small enough
-// that a launch costs more than reading counts again (nbins / 2 counts per
-// workgroup on average, from L2; 25k bins of a 50k-particle tank: 3 loads of
-// 16 bytes per thread). counts is cleared by the next kernel (k_place): other
-// workgroups still read it here.
-constexpr int kScanBlocks = 64, kScanThreads = 1024;
-__global__ __launch_bounds__(kScanThreads) void k_scan_one(const Ctrl *ctrl, const int *counts, int *cellStart) {
-    if (!ctrl->active) return;
-    __shared__ int lds[16];
-    const long long nbins = ctrl->grid.ncells + 1;
-    int sum;
-    if (scan_share(counts, cellStart, nbins, blockIdx.x, gridDim.x, 0, lds, sum) && threadIdx.x == 0)
-        cellStart[nbins] = sum;
-}
-
-// Runs of equal bins in lane order. A run also breaks where the reference
-// index drops (consecutive slots from two old cells), so every run is in
-// reference-index order; a bin that receives two runs is flagged for
-// bin_place. leader: the first lane of this lane's run; next: the lane after
-// its last.
-__device__ inline void bin_run(int b, int id, int &leader, int &next) {
-    const int lane = threadIdx.x & 63;
-    const int prev = __shfl_up(b, 1, 64);
-    const int prev_id = __shfl_up(id, 1, 64);
-    const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
-    const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-    leader = 63 - __clzll(heads & upto);
-    const unsigned long long after = heads & ~upto;
-    next = after ? __ffsll((long long)after) - 1 : 64;
-}
+constexpr int kScanThreads = 1024;  // of the kernels that use scan_share
 
 // Each particle's place from its bin's offset and its rank there: perm0 maps
 // places to slots. Inside a bin the order is that of the ranks' atomics;
-// bin_place orders it. clear (after k_scan_one): also zeroes the counts for
-// the next update. The bounds slots, folded by now, are cleared for the next
+// bin_place orders it. Also zeroes the tile sums for the next update. The bounds slots, folded by now, are cleared for the next
 // update too, active or not (a halted step's k_bounds may have filled them).
 __global__ void k_place(const Ctrl *ctrl, const int *cellStart, const int *bin, const int *rank, int *perm0, int n,
-                        int *clear, unsigned long long *bslots) {
+                        int *tiles, unsigned long long *bslots) {
     if (blockIdx.x == 0 && threadIdx.x < kBoundsSlots * kBoundsStride) bslots[threadIdx.x] = 0;
     if (!ctrl->active) return;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (clear) {
-        const long long nbins = ctrl->grid.ncells + 1;
-        for (long long b = t; b < nbins; b += (long long)gridDim.x * blockDim.x) clear[b] = 0;
-    }
+    for (long long j = t; j * kScanTile <= ctrl->grid.ncells; j += (long long)gridDim.x * blockDim.x)
+        tiles[j * kTileStride] = 0;
     if (t < n) perm0[cellStart[bin[t]] + rank[t]] = t;
 }
 

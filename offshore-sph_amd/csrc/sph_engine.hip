@@ -485,7 +485,7 @@ constexpr int kBinMembers = 16;
 // slots that k_bounds has folded.
 __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double scale, long long cap,
                        const unsigned long long *bslots, unsigned long long *dslots, double *hist, int *counts, int *bin,
-                       int *rank, int *binflag, int *members, int most) {
+                       int *rank, int *binflag, int *tiles, int *members, int most) {
     __shared__ double s_v[kBoundsVQ];
     __shared__ Grid s_g;
     __shared__ unsigned s_halt;
@@ -566,6 +566,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         // flagged; the store is idempotent, so no atomic is needed.
         if (base != 0) binflag[b] = epoch;
     }
+    if (tiles) tile_add(tiles, b);
     base = __shfl(base, leader, 64);
     if (t < n) {
         const int r = base + (lane - leader);
@@ -1452,8 +1453,9 @@ static int alloc_cells(sph_ctx *c, long long cap) {
     const size_t rows = ((size_t)cap + 1 + 3) / 4;  // counts are read in rows of four bins
     HIPCHK(hipMalloc(&c->counts, sizeof(int) * 4 * rows));
     HIPCHK(hipMalloc(&c->cellStart, sizeof(int) * (cap + 2)));
-    HIPCHK(hipMalloc(&c->tileSums, sizeof(int) * (tiles + 1)));
+    HIPCHK(hipMalloc(&c->tileSums, sizeof(int) * kTileStride * (tiles + 1)));
     HIPCHK(hipMemset(c->counts, 0, sizeof(int) * 4 * rows));
+    HIPCHK(hipMemset(c->tileSums, 0, sizeof(int) * kTileStride * (tiles + 1)));
     HIPCHK(hipMemset(c->cellStart, 0, sizeof(int) * (cap + 2)));
     HIPCHK(hipMalloc(&c->binflag, sizeof(int) * (cap + 1)));
     HIPCHK(hipMemset(c->binflag, 0, sizeof(int) * (cap + 1)));
@@ -1808,11 +1810,6 @@ static HmConst hm_const(const sph_ctx *c) {
 
 static Slots slots_of(unsigned long long *w) { return Slots{w, w + (size_t)kBoundsSlots * kBoundsStride}; }
 
-// The scan's form: one kernel up to kScanOneMax particles, else two. Measured
-// per step: 4.7 us against 3.1 + 3.6 us and a launch gap at 5k particles
-// (4.6k bins), 8.0 against 2.9 + 3.9 us and the gap at 90k (72k bins).
-constexpr int kScanOneMax = 1 << 16;
-
 // The neighbour update's kernels on the state a of n particles: bounds, keys,
 // scan, places (perm0, cellStart, binflag). D.on: the dt fold in the bounds.
 struct NnWork {
@@ -1829,19 +1826,11 @@ static void nn_launch(const NnWork &w, const State &a, int n, int pred, const Hm
     k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b, w.members ? w.counts : nullptr,
                                  (int)w.cap + 1);
     k_keys<<<nblk(n), kBlock, 0, s>>>(w.ctrl, a, n, pred, D.on, scale, w.cap, w.slots.b, w.slots.d, D.hist, w.counts,
-                                      w.bin, w.rank, w.binflag, w.members, w.most);
+                                      w.bin, w.rank, w.binflag, w.members ? nullptr : w.tileSums, w.members, w.most);
     if (w.members) return;  // k_reorder_scan does the rest
-    const bool one = n <= kScanOneMax;
-    if (one) {
-        k_scan_one<<<kScanBlocks, kScanThreads, 0, s>>>(w.ctrl, w.counts, w.cellStart);
-    } else {
-        const long long tiles_cap = (w.cap + 1 + kScanTile - 1) / kScanTile;
-        const int tiles = (int)(tiles_cap < 1024 ? tiles_cap : 1024);
-        k_scan_reduce<<<tiles, kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums);
-        k_scan_apply<<<tiles, kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums, w.cellStart);
-    }
-    k_place<<<nblk(n), kBlock, 0, s>>>(w.ctrl, w.cellStart, w.bin, w.rank, w.perm0, n, one ? w.counts : nullptr,
-                                       w.slots.b);
+    const long long tiles = (w.cap + 1 + kScanTile - 1) / kScanTile;
+    k_scan<<<(int)(tiles < 2048 ? tiles : 2048), kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums, w.cellStart);
+    k_place<<<nblk(n), kBlock, 0, s>>>(w.ctrl, w.cellStart, w.bin, w.rank, w.perm0, n, w.tileSums, w.slots.b);
 }
 
 // x0 ... rho0 in memory, for what reads them or changes the state under them.
@@ -2569,7 +2558,7 @@ constexpr size_t kNaOffCounts = kNaOffDrho + al256(8 * kNaParticles);
 constexpr size_t kNaOffCellStart = kNaOffCounts + al256(4 * (kNaCells + 1));
 constexpr size_t kNaOffBinflag = kNaOffCellStart + al256(4 * (kNaCells + 2));
 constexpr size_t kNaOffTiles = kNaOffBinflag + al256(4 * (kNaCells + 1));
-constexpr size_t kNaBytes = kNaOffTiles + al256(4 * ((kNaCells + 1 + kScanTile - 1) / kScanTile + 1));
+constexpr size_t kNaBytes = kNaOffTiles + al256(4 * kTileStride * ((kNaCells + 1 + kScanTile - 1) / kScanTile + 1));
 }  // namespace
 
 static __device__ __align__(256) unsigned char scratch[kNaBytes];
@@ -2600,8 +2589,8 @@ static int na_workspace(unsigned char **out) {
 // no coupled integrator; the cell counts and bin flags cleared over the whole
 // capacity (the workspace keeps the last call's contents); the identity as
 // each particle's reference index.
-__global__ void k_na_init(Ctrl *ctrl, unsigned long long *slots, int *counts, int *binflag, int *id, int n,
-                          long long ncap) {
+__global__ void k_na_init(Ctrl *ctrl, unsigned long long *slots, int *counts, int *binflag, int *tileSums, int *id,
+                          int n, long long ncap) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         Ctrl c{};
@@ -2613,6 +2602,7 @@ __global__ void k_na_init(Ctrl *ctrl, unsigned long long *slots, int *counts, in
         counts[i] = 0;
         binflag[i] = 0;
     }
+    if (i * kScanTile <= ncap) tileSums[i * kTileStride] = 0;
     if (i < n) id[i] = (int)i;
 }
 
@@ -2689,7 +2679,7 @@ extern "C" int sph_loop_noalloc(const sph_params_t *params, const sph_state_t *s
     a.label = st->label;
     a.id = id;
     const long long ninit = (kNaCells + 1 > n ? kNaCells + 1 : n);
-    k_na_init<<<nblk(ninit), kBlock, 0, s>>>(ctrl, slots, counts, binflag, id, nn, kNaCells);
+    k_na_init<<<nblk(ninit), kBlock, 0, s>>>(ctrl, slots, counts, binflag, tileSums, id, nn, kNaCells);
     const NnWork nw{ctrl, slots_of(slots), counts, cellStart, tileSums, binflag, bin, rank, perm0, nullptr, 0, kNaCells};
     nn_launch(nw, a, nn, 0, HmConst{}, nullptr, params->scale, DtFold{}, s);
     const bool f32 = params->precision == SPH_PREC_FP32C;
