@@ -96,16 +96,17 @@ __device__ inline void bdt_commit(BInst &I, const DtNext &x) {
 // ---------------------------------------------------------------------------
 // neighbour update over the segmented grid (src/Tools/NNLinkedList.py)
 // ---------------------------------------------------------------------------
-__device__ inline void bupd_pos(const State &a, int i, bool pred, double dt, double &x, double &y) {
-    x = a.x[i];
-    y = a.y[i];
-    if (pred) {
-        // the velocity is loaded with the label, not after it, and selected
-        const double vx = a.vx[i], vy = a.vy[i];
-        const bool f = a.label[i] == kFluid;
-        x = f ? pec_half_pos(x, vx, dt) : x;
-        y = f ? pec_half_pos(y, vy, dt) : y;
-    }
+struct BPos {  // what it is formed from, loaded before dt is known
+    double x, y, vx, vy;
+    int8_t lab;
+};
+__device__ inline BPos bpos_load(const State &a, int i, bool pred) {
+    return BPos{a.x[i], a.y[i], pred ? a.vx[i] : 0.0, pred ? a.vy[i] : 0.0, a.label[i]};
+}
+__device__ inline void bupd_pos(const BPos &p, bool pred, double dt, double &x, double &y) {
+    const bool f = pred && p.lab == kFluid;
+    x = f ? pec_half_pos(p.x, p.vx, dt) : p.x;
+    y = f ? pec_half_pos(p.y, p.vy, dt) : p.y;
 }
 
 // Per chunk of 1,024 slots (one instance's): the fold of the instance's dt
@@ -127,6 +128,30 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
     if (c == 0 && threadIdx.x == 0) view->epoch += 1;
     const int k = chunkInst[c];
     BInst &I = inst[k];
+    const bool pred = pec != 0;
+    // the first particles of either scan, in flight under the dt fold
+    const Grid g = I.grid;
+    const bool may = cellStart && pred && I.uh_on && g.ncx >= 3 && g.ncy >= 3;
+    const int tid = (c - chunk0[k]) * (int)blockDim.x + (int)threadIdx.x;
+    const int nthreads = (chunk0[k + 1] - chunk0[k]) * (int)blockDim.x;
+    constexpr int U = kChunk / kChunkThreads;
+    int slot[U];
+    BPos p[U];
+    if (may) {
+        static_assert(U == 2, "the border's rows and runs");
+        const BorderWalk W(cellStart, I.cellBase, g, tid, nthreads);
+        slot[0] = W.first_row();
+        slot[1] = W.first_run();
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = cs[c] + (int)threadIdx.x + u * kChunkThreads;
+            slot[u] = i < cs[c + 1] ? i : -1;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (slot[u] >= 0) p[u] = bpos_load(a, slot[u], pred);
     {
         const DtIn in(I, view->pec_parts);
         double v[kDtQ];
@@ -142,12 +167,11 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
     }
     if (!s_active) return;
     const double dt = s_dt;
-    const bool pred = pec != 0;
     double xmn = INFINITY, xmx = -INFINITY, ymn = INFINITY, ymx = -INFINITY, hmn = INFINITY, hmx = -INFINITY;
     double bad = 0.0, vmx = -INFINITY;
-    auto take = [&](int i) {
+    auto take = [&](int i, const BPos &q) {
         double xi, yi;
-        bupd_pos(a, i, pred, dt, xi, yi);
+        bupd_pos(q, pred, dt, xi, yi);
         const double hi = I.uh_on ? I.uh : a.h[i];
         if (!(xi - xi == 0.0) || !(yi - yi == 0.0)) bad += 1.0;
         xmn = xi < xmn ? xi : xmn;
@@ -157,20 +181,22 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
         hmn = hi < hmn ? hi : hmn;
         hmx = hi > hmx ? hi : hmx;
     };
-    if (cellStart && pred && I.uh_on && I.grid.ncx >= 3 && I.grid.ncy >= 3 && border_margin_ok(I.grid, s_disp)) {
-        const int j = c - chunk0[k], nck = chunk0[k + 1] - chunk0[k];
-        if (j == 0 && threadIdx.x == 0) I.border_updates += 1;
+    if (may && border_margin_ok(g, s_disp)) {
+        if (c == chunk0[k] && threadIdx.x == 0) I.border_updates += 1;
         hmn = hmx = I.uh;
-        const BorderWalk W(cellStart, I.cellBase, I.grid, j * (int)blockDim.x + (int)threadIdx.x,
-                           nck * (int)blockDim.x);
-        if (W.first_row() >= 0) take(W.first_row());
-        if (W.first_run() >= 0) take(W.first_run());
-        W.rest(take);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (slot[u] >= 0) take(slot[u], p[u]);
+        BorderWalk(cellStart, I.cellBase, g, tid, nthreads).rest([&](int i) { take(i, bpos_load(a, i, pred)); });
     } else {
-        for (int i = cs[c] + threadIdx.x; i < cs[c + 1]; i += blockDim.x) {
-            take(i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = cs[c] + (int)threadIdx.x + u * kChunkThreads;
+            if (i >= cs[c + 1]) continue;
+            if (may) p[u] = bpos_load(a, i, pred);
+            take(i, p[u]);
             if (pred) {
-                const double ux = fabs(a.vx[i]), uy = fabs(a.vy[i]);
+                const double ux = fabs(p[u].vx), uy = fabs(p[u].vy);
                 const double w = (isfinite(ux) && isfinite(uy)) ? (ux > uy ? ux : uy) : INFINITY;
                 vmx = w > vmx ? w : vmx;
             }
@@ -192,7 +218,7 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
 // their own grid). An instance that is not active is left where it is.
 __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileInst, const int *tile0,
                                                  const int *chunk0, BInst *inst, State a, int pec, const double *part,
-                                                 int *counts, int *bin, int *rank, int *binflag, Ctrl *view) {
+                                                 int *counts, int *bin, int *rank, int *binflag, int *tileSums, Ctrl *view) {
     __shared__ double s_v[kBoundsVQ];
     __shared__ Grid s_g;
     __shared__ unsigned s_halt;
@@ -201,20 +227,20 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     const int k = tileInst[c];
     BInst &I = inst[k];
     const bool first = c == tile0[k];
+    // loaded together with the instance's control block
+    const int t = ts[c] + (int)threadIdx.x;
+    const bool in = t < ts[c + 1];
+    const int lane = threadIdx.x & 63;
+    const int t0 = in ? t : ts[c];
+    const BPos p = bpos_load(a, t0, pec != 0);
+    const int id = in ? a.id[t0] : 0x7fffffff;
     if (!I.nx.active) {
         if (first && threadIdx.x == 0) bdt_commit(I, I.nx);
         return;
     }
     const int epoch = view->epoch;
-    const int t = ts[c] + (int)threadIdx.x;
-    const bool in = t < ts[c + 1];
-    const int lane = threadIdx.x & 63;
-    double x = 0.0, y = 0.0;
-    int id = 0x7fffffff;
-    if (in) {
-        bupd_pos(a, t, pec != 0, I.nx.dt, x, y);
-        id = a.id[t];
-    }
+    double x, y;
+    bupd_pos(p, pec != 0, I.nx.dt, x, y);
     {  // 32 lanes per quantity fold the instance's chunks
         const int q = threadIdx.x >> 5;
         const bool mn = q == 0 || q == 2 || q == 4, sum = q == 6;
@@ -268,6 +294,7 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
         base = atomicAdd(&counts[b], next - leader);
         if (base != 0) binflag[b] = epoch;
     }
+    tile_add(tileSums, b < 0 ? -1 : I.tileBase + (b - (int)I.cellBase) / kScanTile);
     base = __shfl(base, leader, 64);
     if (in) {
         bin[t] = b;
@@ -275,26 +302,24 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     }
 }
 
-// Each instance's offsets, scanned from its first slot by a number of
-// workgroups (scan_share): 8, or as many more as it takes to give each CU two
-// in a small batch (every workgroup reads the counts before its share again).
-inline int scan_shares(int K) { return K >= 64 ? 8 : (K >= 16 ? 16 : 32); }
-__global__ __launch_bounds__(kScanThreads) void kb_scan(const BInst *inst, const int *counts, int *cellStart) {
+// Each instance's offsets, scanned from its first slot, up to scan_tiles(K)
+// tiles at a time.
+inline int scan_tiles(int K) { return K >= 256 ? 8 : (K >= 64 ? 16 : 64); }
+__global__ __launch_bounds__(kBlock) void kb_scan(const BInst *inst, int *counts, const int *tileSums, int *cellStart) {
     __shared__ int lds[16];
     const BInst &I = inst[blockIdx.y];
     if (!I.active) return;
     const long long nbins = I.grid.ncells + 1;
-    int sum;
-    if (scan_share(counts + I.cellBase, cellStart + I.cellBase, nbins, blockIdx.x, gridDim.x, I.off, lds, sum) &&
-        threadIdx.x == 0)
-        cellStart[I.cellBase + nbins] = sum;
+    for (long long tile = blockIdx.x; tile * kScanTile < nbins; tile += gridDim.x)
+        scan_tile(counts + I.cellBase, tileSums + (size_t)I.tileBase * kTileStride, cellStart + I.cellBase, nbins,
+                  tile, I.off, lds);
 }
 
 // Each particle's place (k_place); an instance that is not active keeps its
-// order. Also zeroes the instance's counts for the next update.
+// order. Also zeroes the instance's tile sums for the next update.
 __global__ __launch_bounds__(kTile) void kb_place(const int *ts, const int *tileInst, const int *tile0,
                                                   const BInst *inst, const int *cellStart, const int *bin,
-                                                  const int *rank, int *perm0, int *counts) {
+                                                  const int *rank, int *perm0, int *tileSums) {
     const int c = blockIdx.x, k = tileInst[c];
     const BInst &I = inst[k];
     const int t = ts[c] + (int)threadIdx.x;
@@ -304,8 +329,8 @@ __global__ __launch_bounds__(kTile) void kb_place(const int *ts, const int *tile
         return;
     }
     const int j = c - tile0[k], nt = tile0[k + 1] - tile0[k];
-    for (long long b = j * kTile + (int)threadIdx.x; b <= I.grid.ncells; b += (long long)nt * kTile)
-        counts[I.cellBase + b] = 0;
+    for (long long q = j * kTile + (int)threadIdx.x; q * kScanTile <= I.grid.ncells; q += (long long)nt * kTile)
+        tileSums[(I.tileBase + q) * kTileStride] = 0;
     if (in) perm0[cellStart[bin[t]] + rank[t]] = t;
 }
 
@@ -481,8 +506,9 @@ __global__ void kb_download(State s, sph_state_t out, const BInst *inst, const i
 }
 
 // The bins an instance of at most cap cells needs, with the overflow bin and
-// the end of its slots, in whole 16-byte rows of counts.
+// the end of its slots, in whole 16-byte rows of counts; and its scan tiles.
 inline long long bin_room(long long cap) { return (cap + 2 + 3) / 4 * 4; }
+inline long long tile_room(long long cap) { return (cap + 1 + kScanTile - 1) / kScanTile; }
 
 inline int nblk_b(long long n, int bs = kBlock) {
     long long b = (n + bs - 1) / bs;
@@ -508,7 +534,7 @@ struct sph_batch {
     int *ts = nullptr, *tileInst = nullptr, *tile0 = nullptr;
     int *bin = nullptr, *rank = nullptr, *perm0 = nullptr, *perm = nullptr;
     int2 *cxy_s = nullptr;
-    int *counts = nullptr, *cellStart = nullptr, *binflag = nullptr;
+    int *counts = nullptr, *cellStart = nullptr, *binflag = nullptr, *tileSums = nullptr;
     double *part_b = nullptr, *part_d = nullptr;
     void *recA = nullptr, *recB = nullptr;
     long long capBins = 0;
@@ -543,7 +569,7 @@ void free_batch(sph_batch *b) {
     }
     void *ptrs[] = {b->inst, b->view, b->instOf, b->cs, b->chunkInst, b->chunk0, b->ts, b->tileInst, b->tile0,
                     b->bin, b->rank, b->perm,
-                    b->perm0, b->cxy_s, b->counts, b->cellStart, b->binflag,
+                    b->perm0, b->cxy_s, b->counts, b->cellStart, b->binflag, b->tileSums,
                     b->part_b, b->part_d, b->recA, b->recB, b->queue, b->uniK, b->hm};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -575,10 +601,10 @@ int b_nn(sph_batch *b, hipStream_t s) {
                                               b->NT, b->part_b, fused && b->border_bounds ? b->cellStart : nullptr,
                                               b->view);
     kb_keys<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->chunk0, b->inst, a, pec, b->part_b, b->counts,
-                                    b->bin, b->rank, b->binflag, b->view);
-    kb_scan<<<dim3(scan_shares(b->K), b->K), kScanThreads, 0, s>>>(b->inst, b->counts, b->cellStart);
+                                    b->bin, b->rank, b->binflag, b->tileSums, b->view);
+    kb_scan<<<dim3(scan_tiles(b->K), b->K), kBlock, 0, s>>>(b->inst, b->counts, b->tileSums, b->cellStart);
     kb_place<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->inst, b->cellStart, b->bin, b->rank, b->perm0,
-                                     b->counts);
+                                     b->tileSums);
     const int fmt = b->precision == SPH_PREC_FP32C ? (b->uni ? kRecUniform : kRecFp32)
                                                    : (b->uni ? kRecUniform64 : kRecFp64);
     kb_reorder<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->inst, a, c, b->perm0, b->perm, b->cellStart, b->binflag,
@@ -664,7 +690,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     if (!params || !out) return fail(SPH_EINVAL, "NULL argument");
     *out = nullptr;
     if (ninst < 1 || ninst > (1 << 20)) return fail(SPH_EINVAL, "ninst=%d out of range", ninst);
-    long long ntot = 0, capTot = 0;
+    long long ntot = 0, capTot = 0, tiles = 0;
     for (int k = 0; k < ninst; ++k) {
         const sph_params_t &P = params[k];
         if (P.n <= 0) return fail(SPH_EINVAL, "instance %d: n=%lld", k, (long long)P.n);
@@ -683,6 +709,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         ntot += P.n;
         const long long cap = P.cell_capacity > 0 ? P.cell_capacity : P.n * 8 + 4096;
         capTot += bin_room(cap);
+        tiles += tile_room(cap);
     }
     if (ntot > (1LL << 30)) return fail(SPH_EINVAL, "%lld particles in the batch (max 2^30)", ntot);
     if (capTot > (1LL << 31) - 16) return fail(SPH_EINVAL, "too many cells in the batch");
@@ -700,6 +727,7 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     std::vector<int> cs, chunkInst, chunk0, ts, tileInst, tile0;
     std::vector<BInst> hI(ninst);
     long long off = 0, base = 0;
+    int tbase = 0;
     for (int k = 0; k < ninst; ++k) {
         const sph_params_t &P = params[k];
         chunk0.push_back((int)cs.size());
@@ -721,6 +749,8 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         I.advance_t = 1;
         I.cap = P.cell_capacity > 0 ? P.cell_capacity : P.n * 8 + 4096;
         I.cellBase = base;
+        I.tileBase = tbase;
+        tbase += (int)tile_room(I.cap);
         base += bin_room(I.cap);
         I.duration = P.duration;
         I.fixed_dt = P.fixed_dt;
@@ -796,6 +826,8 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMalloc(&b->counts, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMalloc(&b->cellStart, sizeof(int) * (capTot + 2)) == hipSuccess &&
          hipMalloc(&b->binflag, sizeof(int) * (capTot + 1)) == hipSuccess &&
+         hipMalloc(&b->tileSums, sizeof(int) * kTileStride * tiles) == hipSuccess &&
+         hipMemset(b->tileSums, 0, sizeof(int) * kTileStride * tiles) == hipSuccess &&
          hipMalloc(&b->part_b, sizeof(double) * kBoundsVQ * b->NC) == hipSuccess &&
          hipMalloc(&b->part_d, sizeof(double) * kDtQ * b->NT) == hipSuccess &&
          hipMalloc(&b->recA, ra * n) == hipSuccess && hipMalloc(&b->recB, rb * n) == hipSuccess &&

@@ -352,16 +352,16 @@ __device__ inline void bin_run(int b, int id, int &leader, int &next) {
 // of its first particle's tile are added up in LDS, and the sums
 // lie kTileStride apart, since the atomics of a line go one after another
 // (one per wavefront on packed sums: the 1M dam break's keys take 41 us instead of
-// 16). Called by the whole workgroup; b: the thread's bin, or -1.
+// 16). Called by the whole workgroup;
+// tile: that of the thread's particle, or -1 (not the first thread's).
 constexpr int kTileStride = 4;
-__device__ inline void tile_add(int *tileSums, int b) {
+__device__ inline void tile_add(int *tileSums, int tile) {
     __shared__ int s_tile, s_sum;
     if (threadIdx.x == 0) {
-        s_tile = b / kScanTile;  // the first thread has a particle
+        s_tile = tile;
         s_sum = 0;
     }
     __syncthreads();
-    const int tile = b < 0 ? -1 : b / kScanTile;
     const unsigned long long same = __ballot(tile == s_tile);
     if ((threadIdx.x & 63) == 0 && same) atomicAdd(&s_sum, __popcll(same));
     const int other = tile == s_tile ? -1 : tile;

@@ -566,7 +566,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         // flagged; the store is idempotent, so no atomic is needed.
         if (base != 0) binflag[b] = epoch;
     }
-    if (tiles) tile_add(tiles, b);
+    if (tiles) tile_add(tiles, b < 0 ? -1 : b / kScanTile);
     base = __shfl(base, leader, 64);
     if (t < n) {
         const int r = base + (lane - leader);

@@ -333,6 +333,7 @@ struct BInst {
     unsigned flags;
     Grid grid;
     long long cellBase;
+    int tileBase;  // the first of its bins' scan tiles
     int off, n;
     int advance_t;
     int nfluid;
