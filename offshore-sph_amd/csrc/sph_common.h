@@ -59,46 +59,105 @@ struct AddOp {
     __device__ double operator()(double a, double b) const { return a + b; }
 };
 
-__device__ inline double fold_op(int kind, double a, double b) {
-    return kind == 0 ? (b < a ? b : a) : kind == 1 ? (b > a ? b : a) : a + b;
+__device__ inline double max_of(double a, double b) { return b > a ? b : a; }
+
+// x of another lane of the same row of 16 lanes (a DPP control), and the upper
+// lanes of a exchanged with the lower ones of b, over the wavefront's halves
+// (ROWS 32) or each half's rows (16): cross-lane moves of the vector ALU.
+template <int CTRL>
+__device__ inline double row_move(double x) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+template <int ROWS>
+__device__ inline void row_swap(double &a, double &b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+    unsigned long long p = 0, q = 0;
+#pragma unroll
+    for (int w = 0; w < 64; w += 32) {
+        if constexpr (ROWS == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap((unsigned)(x >> w), (unsigned)(y >> w), false, false);
+            p |= (unsigned long long)r[0] << w;
+            q |= (unsigned long long)r[1] << w;
+        } else {
+            const auto r = __builtin_amdgcn_permlane16_swap((unsigned)(x >> w), (unsigned)(y >> w), false, false);
+            p |= (unsigned long long)r[0] << w;
+            q |= (unsigned long long)r[1] << w;
+        }
+    }
+    a = __longlong_as_double((long long)p);
+    b = __longlong_as_double((long long)q);
+}
+constexpr int kRor8 = 0x128, kRor4 = 0x124, kRor2 = 0x122, kRor1 = 0x121;       // rotations of a row
+constexpr int kHalfMirror = 0x141, kQuadXor2 = 0x4e, kQuadXor1 = 0xb1;
+
+// The maximum over each group of 64 / P lanes, in all of them (P: 4 or 8).
+template <int P>
+__device__ inline double group_max(double x) {
+    if constexpr (P == 8) {
+        x = max_of(x, row_move<kHalfMirror>(x));
+        x = max_of(x, row_move<kQuadXor2>(x));
+        return max_of(x, row_move<kQuadXor1>(x));
+    } else {
+        x = max_of(x, row_move<kRor8>(x));
+        x = max_of(x, row_move<kRor4>(x));
+        x = max_of(x, row_move<kRor2>(x));
+        return max_of(x, row_move<kRor1>(x));
+    }
 }
 
-// Fold NQ quantities over a whole workgroup (up to 16 wavefronts): a shuffle
-// tree inside each wavefront, one LDS round, then wavefront 0 folds the
-// per-wave values of four quantities at a time, one quantity per group of 16
-// lanes (the single-workgroup finalisers are latency-bound: no serial loop
-// over the waves). kind: 0 min, 1 max, 2 sum; every sum folded here is a
-// count, exact in any order. The result is valid in thread 0. lds holds
-// NQ * 16 doubles.
+// Fold NQ (at most 8) quantities over a whole workgroup (up to 16
+// wavefronts). kind: 0 min, 1 max, 2 a count of which only zero or not is
+// kept: all are taken as maxima. Inside a wavefront each exchange halves the
+// quantities a lane carries, so eight of them take 10 exchanges instead of 48,
+// all in the vector ALU (as 96 LDS permutes per wavefront they kept a CU's LDS
+// pipe busy for 3 us in the bounds kernels); one LDS round, then wavefront 0
+// folds the wavefronts' values, a group of lanes per quantity. The result is valid
+// in wavefront 0. lds holds P * 16 doubles, P the next of 4 and 8.
 template <int NQ>
 __device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double *lds) {
+    constexpr int P = NQ <= 4 ? 4 : 8, L = 64 / P;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double m[P];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
+    for (int q = 0; q < P; ++q) m[q] = q < NQ ? (kind[q < NQ ? q : 0] == 0 ? -v[q < NQ ? q : 0] : v[q < NQ ? q : 0]) : -INFINITY;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v[q] = fold_op(kind[q], v[q], __shfl_xor(v[q], o, 64));
-        if (lane == 0) lds[q * 16 + w] = v[q];
+    for (int q = 0; q < P / 2; ++q) {
+        row_swap<32>(m[q], m[q + P / 2]);
+        m[q] = max_of(m[q], m[q + P / 2]);
     }
+#pragma unroll
+    for (int q = 0; q < P / 4; ++q) {
+        row_swap<16>(m[q], m[q + P / 4]);
+        m[q] = max_of(m[q], m[q + P / 4]);
+    }
+    if constexpr (P == 8) {
+        const bool up = lane & 8;
+        const double mine = up ? m[1] : m[0], other = up ? m[0] : m[1];
+        m[0] = max_of(mine, row_move<kRor8>(other));
+    }
+    m[0] = group_max<P>(m[0]);
+    if (lane % L == 0) lds[(lane / L) * 16 + w] = m[0];
     __syncthreads();
     if (w != 0) return;
+    double x = -INFINITY;
 #pragma unroll
-    for (int q0 = 0; q0 < NQ; q0 += 4) {
-        const int q = q0 + (lane >> 4), ww = lane & 15;
-        int kd = 2;
+    for (int u = 0; u < 16; u += L)
+        if (u + lane % L < nw) x = max_of(x, lds[(lane / L) * 16 + u + lane % L]);
+    x = group_max<P>(x);
+    const long long bits = __double_as_longlong(x);
 #pragma unroll
-        for (int j = 0; j < NQ; ++j) kd = q == j ? kind[j] : kd;
-        double x = kd == 0 ? INFINITY : (kd == 1 ? -INFINITY : 0.0);
-        if (q < NQ && ww < nw) x = lds[q * 16 + ww];
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) x = fold_op(kd, x, __shfl_xor(x, o, 64));
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (q0 + j < NQ) v[q0 + j] = __shfl(x, j * 16, 64);
+    for (int q = 0; q < NQ; ++q) {
+        const int lo = __builtin_amdgcn_readlane((int)bits, q * L), hi = __builtin_amdgcn_readlane((int)(bits >> 32), q * L);
+        const double r = __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+        v[q] = kind[q] == 0 ? -r : r;
     }
 }
 
 // Per-workgroup partials of NQ quantities in one LDS round (block_fold):
-// thread 0 stores part[q * R + k]. lds holds NQ * 16 doubles.
+// thread 0 stores part[q * R + k]. lds as block_fold's.
 template <int NQ>
 __device__ inline void block_partials(double (&v)[NQ], const int (&kind)[NQ], double *lds, double *part, int R,
                                       int k) {
@@ -196,7 +255,7 @@ struct DtVars {
     }
     __device__ void publish(double *part, double *lds) { store(part, gridDim.x, blockIdx.x, lds); }
     // into the dt slots (one h for every particle: min h is not folded).
-    // |a|^2 >= 0 orders as its bits. lds holds 3 * 16 doubles.
+    // |a|^2 >= 0 orders as its bits. lds holds 4 * 16 doubles.
     __device__ void publish_slots(unsigned long long *d, double *lds) {
         const int kind[3] = {1, 2, 2};
         double v[3] = {mx, cnt, bad};

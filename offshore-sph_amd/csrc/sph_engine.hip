@@ -967,7 +967,7 @@ __global__ void k_records(const Ctrl *ctrl, State st, Phys ph, int n, int fmt, v
 // all particles (upload, restore and scatter only): per-workgroup partials
 // part[q * gridDim.x + b] (grid-stride), folded by k_hm_final into out[0..5].
 __global__ void k_hm_range(State st, int n, double *part) {
-    __shared__ double lds[6 * 16];
+    __shared__ double lds[8 * 16];
     double v[6] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const double h = st.h[i], m = st.m[i];
@@ -986,7 +986,7 @@ __global__ void k_hm_range(State st, int n, double *part) {
 
 // The R partials of k_hm_range into out[0..5]. One workgroup.
 __global__ void k_hm_final(const double *part, int R, double *out) {
-    __shared__ double lds[6 * 16];
+    __shared__ double lds[8 * 16];
     const int kind[6] = {0, 1, 0, 1, 0, 1};
     double v[6] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY};
     for (int k = threadIdx.x; k < R; k += blockDim.x)
