@@ -198,9 +198,7 @@ __device__ inline void wall_vjp(double rx, double ry, double lamx, double lamy, 
 }
 
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_fold(v, [](double a, double b) { return a + b; });
 }
 
 // Sum NQ values over the workgroup into part[q * R + blockIdx.x].
@@ -241,6 +239,26 @@ __device__ inline void amax_merge(double &v, int &i, double v2, int i2) {
         v = v2;
         i = i2;
     }
+}
+template <int CTRL>
+__device__ inline void amax_row(double &v, int &i) {
+    amax_merge(v, i, row_move<CTRL>(v), row_move<CTRL>(i));
+}
+__device__ inline void amax_wave(double &v, int &i) {  // over the wavefront, in every lane
+    double v2 = v;
+    int i2 = i;
+    row_swap<32>(v, v2);
+    row_swap<32>(i, i2);
+    amax_merge(v, i, v2, i2);
+    v2 = v;
+    i2 = i;
+    row_swap<16>(v, v2);
+    row_swap<16>(i, i2);
+    amax_merge(v, i, v2, i2);
+    amax_row<kRor8>(v, i);
+    amax_row<kRor4>(v, i);
+    amax_row<kRor2>(v, i);
+    amax_row<kRor1>(v, i);
 }
 
 // After the pair pass, everything the reverse step needs: in id order the
@@ -331,8 +349,7 @@ __global__ void k_tape_pair(const Ctrl *ctrl, State s, State o, const int *perm,
             }
         }
     }
-#pragma unroll
-    for (int o2 = 32; o2 > 0; o2 >>= 1) amax_merge(v, id, __shfl_xor(v, o2, 64), __shfl_xor(id, o2, 64));
+    amax_wave(v, id);
     __shared__ double lv[16];
     __shared__ int li[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -409,7 +426,7 @@ __global__ void k_adj_correct(const TapeHdr *hdr, TapeSlot T, const int8_t *labe
 // every round of the walk with a third of the lanes in it (20k particles: 41
 // us and 171 registers, pow() among them; listed, and without the pow(): 25
 // us, 162). The group folds its sums with
-// a fixed xor-shuffle tree, so the result does not depend on scheduling.
+// a fixed tree of lane moves, so the result does not depend on scheduling.
 constexpr int kAdjLanes = 8;
 constexpr int kAdjList = 64;  // entries per particle; emptied when kAdjLanes more might not fit
 
@@ -504,10 +521,13 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_pair(const TapeHdr *hdr, Tape
         red[2] = gc;
     }
     // fold the group (lanes of one particle are kAdjLanes consecutive lanes)
+    static_assert(kAdjLanes == 8, "the moves below");
 #pragma unroll
-    for (int o = kAdjLanes / 2; o > 0; o >>= 1)
-#pragma unroll
-        for (int q = 0; q < 5; ++q) acc[q] += __shfl_xor(acc[q], o, 64);
+    for (int q = 0; q < 5; ++q) {
+        acc[q] += row_move<kQuadXor1>(acc[q]);
+        acc[q] += row_move<kQuadXor2>(acc[q]);
+        acc[q] += row_move<kHalfMirror>(acc[q]);
+    }
     if (live && l == 0 && ak.w >= 0.0) {
         const double dt = hdr->dt, e = 1.0 + 0.5 * damping;
         // a predicted density the strict clamp set to 0 passes no adjoint back
@@ -558,8 +578,7 @@ __global__ void k_adj_final(const TapeHdr *hdr, TapeSlot T, Adj A, const double 
     double av = -1.0;
     int ai = 0x7fffffff;
     for (int b = threadIdx.x; b < R3; b += blockDim.x) amax_merge(av, ai, pv[b], pi[b]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax_merge(av, ai, __shfl_xor(av, o, 64), __shfl_xor(ai, o, 64));
+    amax_wave(av, ai);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     dtb = wave_sum(dtb);
     ga = wave_sum(ga);

@@ -241,20 +241,18 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     const int epoch = view->epoch;
     double x, y;
     bupd_pos(p, pec != 0, I.nx.dt, x, y);
-    {  // 32 lanes per quantity fold the instance's chunks
+    {  // 32 lanes per quantity fold the instance's chunks, all as maxima (the count: zero or not)
         const int q = threadIdx.x >> 5;
-        const bool mn = q == 0 || q == 2 || q == 4, sum = q == 6;
-        double u = mn ? INFINITY : (sum ? 0.0 : -INFINITY);
+        const bool mn = q == 0 || q == 2 || q == 4;
+        double u = q == 6 ? 0.0 : -INFINITY;
         for (int j = chunk0[k] + (threadIdx.x & 31); j < chunk0[k + 1]; j += 32) {
             const double w = part[j * kBoundsVQ + q];
-            u = mn ? (w < u ? w : u) : sum ? u + w : (w > u ? w : u);
+            u = max_of(u, mn ? -w : w);
         }
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) {
-            const double w = __shfl_xor(u, o, 64);
-            u = mn ? (w < u ? w : u) : sum ? u + w : (w > u ? w : u);
-        }
-        if ((threadIdx.x & 31) == 0) s_v[q] = u;
+        double u2 = u;
+        row_swap<16>(u, u2);
+        u = group_max<4>(max_of(u, u2));
+        if ((threadIdx.x & 31) == 0) s_v[q] = mn ? -u : u;
     }
     __syncthreads();
     if (threadIdx.x == 0) {

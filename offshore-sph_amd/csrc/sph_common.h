@@ -59,70 +59,116 @@ struct AddOp {
     __device__ double operator()(double a, double b) const { return a + b; }
 };
 
-__device__ inline double max_of(double a, double b) { return b > a ? b : a; }
+template <class T>
+__device__ inline T max_of(T a, T b) {
+    return b > a ? b : a;
+}
 
-// x of another lane of the same row of 16 lanes (a DPP control), and the upper
-// lanes of a exchanged with the lower ones of b, over the wavefront's halves
-// (ROWS 32) or each half's rows (16): cross-lane moves of the vector ALU.
-template <int CTRL>
-__device__ inline double row_move(double x) {
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+// Cross-lane moves of the vector ALU (an LDS permute each otherwise), for types of 4
+// and 8 bytes: x of another lane of the same row of 16 lanes (a DPP control), and
+// the upper lanes of a exchanged with the lower ones of b, over the
+// wavefront's halves (ROWS 32) or each half's rows (16).
+template <class T, class F>
+__device__ inline T by_words(T x, F &&f) {
+    if constexpr (sizeof(T) == 4) {
+        const unsigned r = f(__builtin_bit_cast(unsigned, x));
+        return __builtin_bit_cast(T, r);
+    } else {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+        const unsigned lo = f((unsigned)b), hi = f((unsigned)(b >> 32));
+        return __builtin_bit_cast(T, (unsigned long long)hi << 32 | lo);
+    }
+}
+template <int CTRL, class T>
+__device__ inline T row_move(T x) {
+    return by_words(x, [](unsigned w) { return (unsigned)__builtin_amdgcn_mov_dpp((int)w, CTRL, 0xf, 0xf, false); });
 }
 template <int ROWS>
-__device__ inline void row_swap(double &a, double &b) {
-    const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
-    unsigned long long p = 0, q = 0;
-#pragma unroll
-    for (int w = 0; w < 64; w += 32) {
-        if constexpr (ROWS == 32) {
-            const auto r = __builtin_amdgcn_permlane32_swap((unsigned)(x >> w), (unsigned)(y >> w), false, false);
-            p |= (unsigned long long)r[0] << w;
-            q |= (unsigned long long)r[1] << w;
-        } else {
-            const auto r = __builtin_amdgcn_permlane16_swap((unsigned)(x >> w), (unsigned)(y >> w), false, false);
-            p |= (unsigned long long)r[0] << w;
-            q |= (unsigned long long)r[1] << w;
-        }
+__device__ inline void row_swap(unsigned &a, unsigned &b) {
+    if constexpr (ROWS == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
     }
-    a = __longlong_as_double((long long)p);
-    b = __longlong_as_double((long long)q);
 }
-constexpr int kRor8 = 0x128, kRor4 = 0x124, kRor2 = 0x122, kRor1 = 0x121;       // rotations of a row
+template <int ROWS, class T>
+__device__ inline void row_swap(T &a, T &b) {
+    if constexpr (sizeof(T) == 4) {
+        unsigned x = __builtin_bit_cast(unsigned, a), y = __builtin_bit_cast(unsigned, b);
+        row_swap<ROWS>(x, y);
+        a = __builtin_bit_cast(T, x);
+        b = __builtin_bit_cast(T, y);
+    } else {
+        const auto x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+        unsigned x0 = (unsigned)x, x1 = (unsigned)(x >> 32), y0 = (unsigned)y, y1 = (unsigned)(y >> 32);
+        row_swap<ROWS>(x0, y0);
+        row_swap<ROWS>(x1, y1);
+        a = __builtin_bit_cast(T, (unsigned long long)x1 << 32 | x0);
+        b = __builtin_bit_cast(T, (unsigned long long)y1 << 32 | y0);
+    }
+}
+constexpr int kRor8 = 0x128, kRor4 = 0x124, kRor2 = 0x122, kRor1 = 0x121;  // rotations of a row
 constexpr int kHalfMirror = 0x141, kQuadXor2 = 0x4e, kQuadXor1 = 0xb1;
+template <class T>
+__device__ inline T lane_value(T x, int lane) {  // of a lane that is the same for the wavefront
+    return by_words(x, [&](unsigned w) { return (unsigned)__builtin_amdgcn_readlane((int)w, lane); });
+}
+// Of the lane before (lane 0: its own).
+__device__ inline int lane_before(int x) { return __builtin_amdgcn_update_dpp(x, x, 0x138, 0xf, 0xf, false); }
+// The sum over the lanes up to this one.
+__device__ inline int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // within the rows
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // a row's last lane into the next row
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // the lower half's into the upper
+    return x;
+}
+
+// f over the values of all lanes, in all of them: the pairs of an xor tree of
+// 32, 16, ... 1 (f commutes), so a sum has that tree's bits.
+template <class T, class F>
+__device__ inline T row_fold(T x, F &&f) {
+    x = f(x, row_move<kRor8>(x));
+    x = f(x, row_move<kRor4>(x));
+    x = f(x, row_move<kRor2>(x));
+    return f(x, row_move<kRor1>(x));
+}
+template <class T, class F>
+__device__ inline T wave_fold(T x, F &&f) {
+    T y = x;
+    row_swap<32>(x, y);
+    x = f(x, y);
+    y = x;
+    row_swap<16>(x, y);
+    return row_fold(f(x, y), f);
+}
+template <class T>
+__device__ inline T wave_max(T x) {
+    return wave_fold(x, [](T a, T b) { return max_of(a, b); });
+}
 
 // The maximum over each group of 64 / P lanes, in all of them (P: 4 or 8).
-template <int P>
-__device__ inline double group_max(double x) {
+template <int P, class T>
+__device__ inline T group_max(T x) {
     if constexpr (P == 8) {
         x = max_of(x, row_move<kHalfMirror>(x));
         x = max_of(x, row_move<kQuadXor2>(x));
         return max_of(x, row_move<kQuadXor1>(x));
     } else {
-        x = max_of(x, row_move<kRor8>(x));
-        x = max_of(x, row_move<kRor4>(x));
-        x = max_of(x, row_move<kRor2>(x));
-        return max_of(x, row_move<kRor1>(x));
+        return row_fold(x, [](T a, T b) { return max_of(a, b); });
     }
 }
-
-// Fold NQ (at most 8) quantities over a whole workgroup (up to 16
-// wavefronts). kind: 0 min, 1 max, 2 a count of which only zero or not is
-// kept: all are taken as maxima. Inside a wavefront each exchange halves the
-// quantities a lane carries, so eight of them take 10 exchanges instead of 48,
-// all in the vector ALU (as 96 LDS permutes per wavefront they kept a CU's LDS
-// pipe busy for 3 us in the bounds kernels); one LDS round, then wavefront 0
-// folds the wavefronts' values, a group of lanes per quantity. The result is valid
-// in wavefront 0. lds holds P * 16 doubles, P the next of 4 and 8.
-template <int NQ>
-__device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double *lds) {
-    constexpr int P = NQ <= 4 ? 4 : 8, L = 64 / P;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    double m[P];
-#pragma unroll
-    for (int q = 0; q < P; ++q) m[q] = q < NQ ? (kind[q < NQ ? q : 0] == 0 ? -v[q < NQ ? q : 0] : v[q < NQ ? q : 0]) : -INFINITY;
+// The maxima over the wavefront of P quantities (4 or 8): that of quantity q in
+// the q-th group of 64 / P lanes. Each exchange halves the quantities a lane
+// carries: eight take 10 exchanges instead of 48.
+template <int P, class T>
+__device__ inline T wave_maxima(T (&m)[P]) {
 #pragma unroll
     for (int q = 0; q < P / 2; ++q) {
         row_swap<32>(m[q], m[q + P / 2]);
@@ -134,12 +180,29 @@ __device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double
         m[q] = max_of(m[q], m[q + P / 4]);
     }
     if constexpr (P == 8) {
-        const bool up = lane & 8;
-        const double mine = up ? m[1] : m[0], other = up ? m[0] : m[1];
+        const bool up = threadIdx.x & 8;
+        const T mine = up ? m[1] : m[0], other = up ? m[0] : m[1];
         m[0] = max_of(mine, row_move<kRor8>(other));
     }
-    m[0] = group_max<P>(m[0]);
-    if (lane % L == 0) lds[(lane / L) * 16 + w] = m[0];
+    return group_max<P>(m[0]);
+}
+
+// Fold NQ (at most 8) quantities over a whole workgroup (up to 16
+// wavefronts). kind: 0 min, 1 max, 2 a count of which only zero or not is
+// kept: all are taken as maxima, inside a wavefront by wave_maxima (as 96 LDS
+// permutes per wavefront they kept a CU's LDS pipe busy for 3 us in the bounds
+// kernels); one LDS round, then wavefront 0
+// folds the wavefronts' values, a group of lanes per quantity. The result is valid
+// in wavefront 0. lds holds P * 16 doubles, P the next of 4 and 8.
+template <int NQ>
+__device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double *lds) {
+    constexpr int P = NQ <= 4 ? 4 : 8, L = 64 / P;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double m[P];
+#pragma unroll
+    for (int q = 0; q < P; ++q) m[q] = q < NQ ? (kind[q < NQ ? q : 0] == 0 ? -v[q < NQ ? q : 0] : v[q < NQ ? q : 0]) : -INFINITY;
+    const double top = wave_maxima<P>(m);
+    if (lane % L == 0) lds[(lane / L) * 16 + w] = top;
     __syncthreads();
     if (w != 0) return;
     double x = -INFINITY;
@@ -147,11 +210,9 @@ __device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double
     for (int u = 0; u < 16; u += L)
         if (u + lane % L < nw) x = max_of(x, lds[(lane / L) * 16 + u + lane % L]);
     x = group_max<P>(x);
-    const long long bits = __double_as_longlong(x);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int lo = __builtin_amdgcn_readlane((int)bits, q * L), hi = __builtin_amdgcn_readlane((int)(bits >> 32), q * L);
-        const double r = __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+        const double r = lane_value(x, q * L);
         v[q] = kind[q] == 0 ? -r : r;
     }
 }
@@ -394,8 +455,7 @@ __device__ inline double nm_corr_vel(double v, double a, double gamma, double dt
 // its last.
 __device__ inline void bin_run(int b, int id, int &leader, int &next) {
     const int lane = threadIdx.x & 63;
-    const int prev = __shfl_up(b, 1, 64);
-    const int prev_id = __shfl_up(id, 1, 64);
+    const int prev = lane_before(b), prev_id = lane_before(id);
     const unsigned long long heads = __ballot(lane == 0 || b != prev || id < prev_id);
     const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
     leader = 63 - __clzll(heads & upto);
@@ -434,14 +494,8 @@ __device__ inline void tile_add(int *tileSums, int tile) {
     if (threadIdx.x == 0) atomicAdd(&tileSums[(size_t)s_tile * kTileStride], s_sum);
 }
 __device__ inline int block_scan_excl(int v, int *lds, int *total) {
-    // inclusive scan inside each wave
-    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int s = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int u = __shfl_up(s, o, 64);
-        if (lane >= o) s += u;
-    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int s = wave_scan(v);
     if (lane == 63) lds[w] = s;
     __syncthreads();
     int nw = blockDim.x >> 6;
@@ -780,26 +834,17 @@ struct Stage {
 // the workgroup's ranges. Ends with a barrier; every thread returns the same
 // plan.
 __device__ inline Stage stage_plan(const int rs[3], const int re[3], int *s_red) {
-    int v[6];
+    int v[8];  // all as maxima
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const bool any = rs[d] < re[d];
-        v[d] = any ? rs[d] : 0x7fffffff;
+        v[d] = any ? -rs[d] : -0x7fffffff;
         v[3 + d] = any ? re[d] : -0x7fffffff;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const int a = __shfl_xor(v[d], o, 64), b = __shfl_xor(v[3 + d], o, 64);
-            v[d] = a < v[d] ? a : v[d];
-            v[3 + d] = b > v[3 + d] ? b : v[3 + d];
-        }
-    }
+    v[6] = v[7] = -0x7fffffff;
+    const int top = wave_maxima<8>(v);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < 6; ++q) s_red[q * 4 + w] = v[q];
+    if (lane % 8 == 0 && lane < 48) s_red[(lane / 8) * 4 + w] = lane < 24 ? -top : top;
     __syncthreads();
     Stage S;
     int off = 0;

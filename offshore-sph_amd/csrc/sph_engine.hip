@@ -110,16 +110,11 @@ __device__ inline void dt_fold(int R, const double *part, const unsigned long lo
     unsigned long long a = p[0], f = p[1];  // in flight together with R
     if (R == kDtSlots) {
         if (threadIdx.x < kDtSlotCount) {  // one wavefront
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const unsigned long long a2 = __shfl_xor(a, o, 64);
-                a = a2 > a ? a2 : a;
-                f |= __shfl_xor(f, o, 64);
-            }
+            const double top = wave_max(__longlong_as_double((long long)a));  // |a|^2 >= 0
             v[0] = h1;
-            v[1] = __longlong_as_double((long long)a);
-            v[2] = f & kDtAny ? 1.0 : 0.0;
-            v[3] = f & kDtBad ? 1.0 : 0.0;
+            v[1] = top;
+            v[2] = __ballot(f & kDtAny) ? 1.0 : 0.0;
+            v[3] = __ballot(f & kDtBad) ? 1.0 : 0.0;
         }
         return;
     }
@@ -507,11 +502,8 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
     upd_pos(ctrl, a, t0, p, pred, dt, x, y);
     if (threadIdx.x < kBoundsVQ * kBoundsSlots) {
         const int q = bq, k = bk;
-#pragma unroll
-        for (int o = kBoundsSlots / 2; o > 0; o >>= 1) {
-            const unsigned long long m2 = __shfl_xor(m, o, 64);
-            m = m2 > m ? m2 : m;
-        }
+        static_assert(kBoundsSlots == 16, "a row of lanes");
+        m = group_max<4>(m);
         if (k == 0) {
             const double u = order_value(m);
             s_v[q] = q == 0 || q == 2 || q == 4 ? -u : u;
@@ -834,13 +826,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
     }
     if (act) {
         if (tid < SLOTS) {
-            int lo = live ? key : 0x7fffffff, hi = key;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const int l2 = __shfl_xor(lo, o, 64), h2 = __shfl_xor(hi, o, 64);
-                lo = l2 < lo ? l2 : lo;
-                hi = h2 > hi ? h2 : hi;
-            }
+            const int lo = -wave_max(live ? -key : -0x7fffffff), hi = wave_max(live ? key : -1);
             if ((tid & 63) == 0) {
                 s_lo[tid >> 6] = lo;
                 s_hi[tid >> 6] = hi;

@@ -98,9 +98,14 @@ template <class P, int G>
 struct GroupSums {
     static constexpr int N = (P::NQ + G - 1) / G;
     typename P::Sum s[N];
-    // quantity q (a constant), in every lane of the group
-    __device__ __forceinline__ double get(int q) const {
-        return __shfl(s[q / G].get(), (int)((threadIdx.x & 63) / G * G) + q % G, 64);
+    // quantity Q, in the group's first lane
+    template <int Q>
+    __device__ __forceinline__ double get() const {
+        const double v = s[Q / G].get();
+        if constexpr (Q % G == 0)
+            return v;
+        else
+            return row_move<0x100 | Q % G>(v);  // of the lane Q % G further on
     }
 };
 
@@ -265,11 +270,12 @@ __global__ __launch_bounds__(256) void k_pair_group(const Ctrl *ctrl, PairArgs<R
     GroupSums<GG, G> acc;
     int cnt = 0;
     group_sums<GG, G>(gg, P.cellStart, c, ncx, ncy, 0, walks, l, mem[i], acc, cnt);
-    const double arho = acc.get(0), a0 = acc.get(1), a1 = acc.get(2), f0 = acc.get(3), f1 = acc.get(4);
+    const double arho = acc.template get<0>(), a0 = acc.template get<1>(), a1 = acc.template get<2>();
+    const double f0 = acc.template get<3>(), f1 = acc.template get<4>();
     double xs0 = 0.0, xs1 = 0.0;
     if constexpr (XS) {
-        xs0 = acc.get(5);
-        xs1 = acc.get(6);
+        xs0 = acc.template get<5>();
+        xs1 = acc.template get<6>();
     }
     if (!walks || l != 0) return;
     if (!implied && cnt == 0) return;  // SolverTools.py:166-169: no neighbours, keep the previous values

@@ -659,7 +659,7 @@ struct UniformGroup {
     }
 };
 
-// The rates of target t by its G lanes, in every lane; false: it has no
+// The rates of target t by its G lanes, in the first of them; false: it has no
 // neighbour (or walks is false).
 template <int KERNEL, int MODE, int G>
 __device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformConst &K, int ncx, int ncy,
@@ -671,9 +671,9 @@ __device__ inline bool uniform_group_rates(const UniformArgs &P, const UniformCo
     GroupSums<UG, G> acc;
     int cnt;
     group_sums<UG, G>(ug, P.cellStart, c, ncx, ncy, 0, walks, l, M, acc, cnt);
-    drho = acc.get(0);
-    ax = acc.get(1);
-    const double say = acc.get(2);
+    drho = acc.template get<0>();
+    ax = acc.template get<1>();
+    const double say = acc.template get<2>();
     ay = (MODE & kEquations) == kContinuity ? 0.0 : say - K.g;  // WCSPH.py:169
     if (!walks) return false;
     const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;  // it finds itself: a neighbour

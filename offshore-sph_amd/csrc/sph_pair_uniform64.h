@@ -559,7 +559,7 @@ struct Uniform64Group {
     }
 };
 
-// The rates of target t by its G lanes, in every lane; false: it has no
+// The rates of target t by its G lanes, in the first of them; false: it has no
 // neighbour (or walks is false).
 template <int KERNEL, int MODE, int G>
 __device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy,
@@ -573,8 +573,9 @@ __device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Unifo
     GroupSums<UG, G> acc;
     int cnt;
     group_sums<UG, G>(ug, P.cellStart, c, ncx, ncy, 0, walks, l, M, acc, cnt);
-    drho = acc.get(0);
-    const double a0 = acc.get(1), a1 = acc.get(2), f0 = acc.get(3), f1 = acc.get(4);
+    drho = acc.template get<0>();
+    const double a0 = acc.template get<1>(), a1 = acc.template get<2>();
+    const double f0 = acc.template get<3>(), f1 = acc.template get<4>();
     ax = a0 + f0;
     ay = (MODE & kEquations) == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
     return walks && (inside || cnt != 0);  // SolverTools.py:166-169
