@@ -59,6 +59,7 @@ struct Uniform64Args {
 
 struct Uniform64Const {
     double lim2;           // max((2h)^2, r0^2) (1 + 1e-12): the listed pairs
+    double hinv, hinv2;    // 1 / h, 2 / h
     double h, m, alpha_k;  // alpha_k: the kernel normalisation 10 / (7 pi) / (h h) (Wendland: 9 / (4 pi) / (h h))
     double c01;            // 0.01 h h, in the reference's order (0.01 h) h
     double cij, alpha, beta;
@@ -66,7 +67,44 @@ struct Uniform64Const {
     double r0, D, p1, p2, g, qmax;
 };
 
+constexpr double kPairNone = 1e-280;  // a pair at this r^2 or less adds nothing
 __device__ inline bool not_fluid64(double prs) { return prs != prs; }
+
+// Square roots and quotients of the pair terms with the bits of sqrt() and /,
+// without what those spend on the ends of the exponent range (scaling before
+// and after, 6 of a root's 16 instructions and 3 of a quotient's 11): the
+// launcher takes this pass for 1e-100 < h < 1e100 only and the walk lists no
+// pair with r^2 <= 1e-280, which adds nothing anywhere (r < 1e-12). Newton steps
+// on the hardware's estimates, then one correction by the exact remainder,
+// which rounds a quotient as / does when the reciprocal is itself the rounded
+// one (P. Markstein, IBM J. Res. Dev. 34, 1990).
+//
+// root(a) also leaves half = 0.5 / root(a) to about 2^-50, from which the
+// quotient by h root(a) needs no estimate of its own.
+__device__ inline double pair_root(double a, double &half) {
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y;
+    half = 0.5 * y;
+    const double e = __builtin_fma(-half, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    half = __builtin_fma(half, e, half);
+    g = __builtin_fma(__builtin_fma(-g, g, a), half, g);
+    return __builtin_fma(__builtin_fma(-g, g, a), half, g);
+}
+// a / b from y, the rounded 1 / b
+__device__ inline double pair_quotient(double a, double b, double y) {
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// 1 / b from an estimate y
+__device__ inline double pair_recip(double b, double y) {
+    return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+}
+// a / b, any a (a zero or non-finite a or b as /)
+__device__ inline double pair_divide(double a, double b) {
+    const double y = pair_recip(b, pair_recip(b, __builtin_amdgcn_rcp(b)));
+    return __builtin_amdgcn_div_fixup(pair_quotient(a, b, y), b, a);
+}
 
 // Whether the target at (X, Y) in cell c has a neighbour: one whose own cell
 // is in the grid finds itself (q = 0); one outside looks (SolverTools.py:
@@ -121,9 +159,10 @@ __device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Unif
             const double4 b = at32(P.B, u);
             const double dx = X - a.x, dy = Y - a.y;
             const double xij2 = dx * dx + dy * dy;
-            const double r = sqrt(xij2);
+            double half;
+            const double r = pair_root(xij2, half);
             if (!not_fluid64(b.w)) {
-                const double qq = r / K.h;
+                const double qq = pair_quotient(r, K.h, K.hinv);
                 double dwx, dwy;
                 double grad;
                 if (KERNEL == SPH_KERNEL_WENDLAND) {
@@ -134,7 +173,8 @@ __device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Unif
                     if ((qq > 2.0) || (r < 1e-10)) continue;
                     grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
                 }
-                const double norm = K.alpha_k * grad / (K.h * r);
+                const double hr = K.h * r;
+                const double norm = pair_quotient(K.alpha_k * grad, hr, pair_recip(hr, half * K.hinv2));
                 dwx = norm * dx;
                 dwy = norm * dy;
                 const double vx = bt.x - b.x, vy = bt.y - b.y;
@@ -145,9 +185,9 @@ __device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Unif
                 double PI_ij = 0.0;
                 if (dv < 0) {
                     const double rhoij = 0.5 * (bt.z + b.z);
-                    const double muij = K.h * dv / (r * r + K.c01);
+                    const double muij = pair_divide(K.h * dv, r * r + K.c01);
                     const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                    PI_ij = ppij / rhoij;
+                    PI_ij = pair_divide(ppij, rhoij);
                 }
                 const double factor = bt.w + b.w + PI_ij;
                 a0 += -K.m * factor * dwx;
@@ -172,7 +212,7 @@ __device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Unif
         // written whether or not it is kept (within the list's bounds either
         // way): no branch per candidate
         *lp = (unsigned)k;
-        lp += (r2 <= K.lim2 && r2 > 0.0) ? stride : 0u;
+        lp += (r2 <= K.lim2 && r2 > kPairNone) ? stride : 0u;
     };
     // src/Tools/NNLinkedList.py:50-56: x shift outer, y shift inner, cells at
     // the grid's edge dropped; each cell from its highest slot down (:129-141)
@@ -245,7 +285,7 @@ __device__ inline bool uniform64_rates_direct(const Uniform64Args &P, const Unif
                 }
                 const double dx = X - a.x, dy = Y - a.y;
                 const double xij2 = dx * dx + dy * dy;
-                if (!(xij2 <= K.lim2 && xij2 > 0.0)) continue;
+                if (!(xij2 <= K.lim2 && xij2 > kPairNone)) continue;
                 if (!not_fluid64(b.w)) {
                     double f;
                     if (!gauss_factor(xij2, K.h, K.ih2, K.g2, f)) continue;
@@ -258,9 +298,9 @@ __device__ inline bool uniform64_rates_direct(const Uniform64Args &P, const Unif
                     double PI_ij = 0.0;
                     if (dv < 0) {
                         const double rhoij = 0.5 * (bt.z + b.z);
-                        const double muij = K.h * dv / (xij2 + K.c01);
+                        const double muij = pair_divide(K.h * dv, xij2 + K.c01);
                         const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                        PI_ij = ppij / rhoij;
+                        PI_ij = pair_divide(ppij, rhoij);
                     }
                     const double factor = bt.w + b.w + PI_ij;
                     a0 += -K.m * factor * dwx;
@@ -491,7 +531,7 @@ struct Uniform64Group {
     const Uniform64Args &P;
     const Uniform64Const &K;
     double X, Y;
-    const double4 &bt;
+    double vx0, vy0, rho0, prs;  // the target's B record
     bool counts;
     __device__ __forceinline__ RecA load(unsigned u) const { return at32(P.A, u); }
     __device__ __forceinline__ bool test(const RecA &a, unsigned, bool &counted) const {
@@ -502,17 +542,30 @@ struct Uniform64Group {
             counted = r2 < lim * (1.0 - 1e-12);
             if (!counted && !(r2 > lim * (1.0 + 1e-12))) counted = exact_q_test(X, Y, K.h, a.x, a.y, K.h, K.qmax);
         }
-        return r2 <= K.lim2 && r2 > 0.0;
+        return r2 <= K.lim2 && r2 > kPairNone;
     }
-    // uniform64_rates' expressions for one listed pair
+    // uniform64_rates' expressions for one listed pair. All five quantities are
+    // returned together: stores into out from the fluid's and the
+    // wall's branch became stores through a selected address, and out
+    // 32 bytes of scratch memory.
     __device__ __forceinline__ void terms(unsigned u, double *out) const {
+        double d = 0.0, a0 = 0.0, a1 = 0.0, f0 = 0.0, f1 = 0.0;
+        pair(u, d, a0, a1, f0, f1);
+        out[0] = d;
+        out[1] = a0;
+        out[2] = a1;
+        out[3] = f0;
+        out[4] = f1;
+    }
+    __device__ __forceinline__ void pair(unsigned u, double &d, double &a0, double &a1, double &f0, double &f1) const {
         const double2 a = at32(P.A, u);
         const double4 b = at32(P.B, u);
         const double dx = X - a.x, dy = Y - a.y;
         const double xij2 = dx * dx + dy * dy;
-        const double r = sqrt(xij2);
+        double half;
+        const double r = pair_root(xij2, half);
         if (!not_fluid64(b.w)) {
-            const double qq = r / K.h;
+            const double qq = pair_quotient(r, K.h, K.hinv);
             double dwx, dwy;
             if (KERNEL == SPH_KERNEL_GAUSSIAN) {
                 double f;
@@ -529,32 +582,33 @@ struct Uniform64Group {
                     if ((qq > 2.0) || (r < 1e-10)) return;
                     grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
                 }
-                const double norm = K.alpha_k * grad / (K.h * r);
+                const double hr = K.h * r;
+                const double norm = pair_quotient(K.alpha_k * grad, hr, pair_recip(hr, half * K.hinv2));
                 dwx = norm * dx;
                 dwy = norm * dy;
             }
-            const double vx = bt.x - b.x, vy = bt.y - b.y;
+            const double vx = vx0 - b.x, vy = vy0 - b.y;
             const double dot = vx * dwx + vy * dwy;
-            if constexpr ((MODE & kEquations) != kMomentum) out[0] = K.m * dot;
+            if constexpr ((MODE & kEquations) != kMomentum) d = K.m * dot;
             if constexpr ((MODE & kEquations) == kContinuity) return;
             const double dv = vx * dx + vy * dy;
             double PI_ij = 0.0;
             if (dv < 0) {
-                const double rhoij = 0.5 * (bt.z + b.z);
+                const double rhoij = 0.5 * (rho0 + b.z);
                 const double rr = KERNEL == SPH_KERNEL_GAUSSIAN ? xij2 : r * r;
-                const double muij = K.h * dv / (rr + K.c01);
+                const double muij = pair_divide(K.h * dv, rr + K.c01);
                 const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                PI_ij = ppij / rhoij;
+                PI_ij = pair_divide(ppij, rhoij);
             }
-            const double factor = bt.w + b.w + PI_ij;
-            out[1] = -K.m * factor * dwx;
-            out[2] = -K.m * factor * dwy;
+            const double factor = prs + b.w + PI_ij;
+            a0 = -K.m * factor * dwx;
+            a1 = -K.m * factor * dwy;
         } else if ((MODE & kEquations) != kContinuity && !(r > K.r0) && r > 1e-12) {
             const double frac = K.r0 / r;
             const double tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
             const double fac = K.D * tmp;
-            out[3] = fac * dx / (r * r);
-            out[4] = fac * dy / (r * r);
+            f0 = fac * dx / (r * r);
+            f1 = fac * dy / (r * r);
         }
     }
 };
@@ -569,7 +623,7 @@ __device__ inline bool uniform64_group_rates(const Uniform64Args &P, const Unifo
     using UG = Uniform64Group<KERNEL, MODE>;
     // a target whose own cell is in the grid finds itself (q = 0)
     const bool inside = c.x >= 0 && c.x < ncx && c.y >= 0 && c.y < ncy;
-    const UG ug{P, K, at.x, at.y, bt, !inside};
+    const UG ug{P, K, at.x, at.y, bt.x, bt.y, bt.z, bt.w, !inside};
     GroupSums<UG, G> acc;
     int cnt;
     group_sums<UG, G>(ug, P.cellStart, c, ncx, ncy, 0, walks, l, M, acc, cnt);
