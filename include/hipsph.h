@@ -345,9 +345,9 @@ int sph_tait_eos(int64_t n, double gamma, double B, double rho0, double Pb, cons
  * autotuner (offshore-sph_amd/hipsph/autotune.py). */
 int sph_ctx_set_tuning(sph_ctx_t *ctx, int32_t pair_threads);
 int sph_ctx_get_tuning(sph_ctx_t *ctx, int32_t *pair_threads);
-/* No reference counterpart: whether the uniform float pair passes (FP32C,
- * one h, one fluid mass; sph_compute, the split passes and the step's fused
- * pass) stage each workgroup's neighbour records in LDS before the walk (1,
+/* No reference counterpart: whether the uniform pair passes (one h, one
+ * fluid mass; sph_compute, the split passes and the step's fused pass; not
+ * the Gaussian in FP64) stage each workgroup's neighbour records in LDS before the walk (1,
  * the default) or read them from global memory (0). Results are
  * bit-identical either way; for tests and tuning. */
 int sph_ctx_set_pair_staging(sph_ctx_t *ctx, int32_t on);

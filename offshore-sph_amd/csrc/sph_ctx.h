@@ -37,7 +37,7 @@ struct sph_ctx {
     void *recA = nullptr, *recB = nullptr;  // packed pair-pass records (Rec<double> / Rec<float>)
     int *slot_of = nullptr;
     int pair_threads = 256;
-    int pair_staging = 1;  // the uniform float pair passes stage each workgroup's records in LDS
+    int pair_staging = 1;  // the uniform pair passes stage each workgroup's records in LDS
     int border_bounds = 1;  // the fused PEC step's bounds from the border cells when the displacement allows
     // one h for every particle and one mass for every fluid particle in the
     // current state (found at upload, restore and scatter): the fused float

@@ -42,6 +42,7 @@ void uniform_const_fp64(const UniformParams &u, void *out) {
     K.p2 = u.p2;
     K.g = u.g;
     K.qmax = u.qmax;
+    K.stage = u.stage;
     K.hinv = 1.0 / u.h;
     K.hinv2 = 2.0 * K.hinv;
     K.ih2 = 1.0 / (u.h * u.h);

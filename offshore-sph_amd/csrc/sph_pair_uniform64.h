@@ -21,7 +21,8 @@
 //     p / rho^2 for particles that are not fluid;
 //   * the walk visits the reference's nine cells in its order (x shift outer,
 //     y shift inner, each cell from its highest slot down), UNROLL records
-//     loaded before they are tested.
+//     loaded before they are tested; a thread-per-target workgroup stages the
+//     records of its targets' cells in LDS first (StagedWalk64).
 #pragma once
 #include "sph_common.h"
 #include "sph_pair_group.h"
@@ -30,7 +31,7 @@ namespace hipsph {
 namespace {
 
 #ifndef HIPSPH_PEC64_EARLY
-#define HIPSPH_PEC64_EARLY 0  // 1: the corrector's gathers before the walk (137 VGPRs, 3 waves: 10 % slower)
+#define HIPSPH_PEC64_EARLY 0  // 1: the corrector's gathers before the walk (97 VGPRs instead of 83, 4 waves: no faster)
 #endif
 
 #ifndef HIPSPH_UNIFORM64_UNROLL
@@ -39,8 +40,8 @@ namespace {
 #ifndef HIPSPH_UNIFORM64_LIST
 #define HIPSPH_UNIFORM64_LIST 30
 #endif
-// contributor-list entries per thread (4 B each): 30 for five workgroups per
-// CU (500k particles, 30 steps: 4.04 ms against 4.14 with 32, 4.06 with 25)
+// contributor-list entries per thread (4 B each, 2 B in a staged walk): 30, with
+// which either walk's LDS leaves five workgroups per CU
 constexpr int kUniform64List = HIPSPH_UNIFORM64_LIST;
 // the Gaussian's pass keeps no list (uniform64_rates_direct)
 template <int KERNEL>
@@ -65,6 +66,7 @@ struct Uniform64Const {
     double cij, alpha, beta;
     double ih2, g2;        // the Gaussian's 1 / h^2 and -2 alpha_k / h^2 (gauss_factor)
     double r0, D, p1, p2, g, qmax;
+    int stage;             // stage the candidates' records in LDS
 };
 
 constexpr double kPairNone = 1e-280;  // a pair at this r^2 or less adds nothing
@@ -335,6 +337,159 @@ __device__ inline bool uniform64_rates(const Uniform64Args &P, const Uniform64Co
         return uniform64_rates_listed<KERNEL, MODE>(P, K, ncx, ncy, base, t, bt, s_list, drho, ax, ay);
 }
 
+// The same walk over A records staged in LDS (stage_plan: the three row ranges
+// of the workgroup's targets), with a 16-bit list. Walking them in
+// global memory kept the vector memory path 66 % busy (500k particles; VALU 53 %),
+// as 61 candidates and 21 contributors are 16-byte gathers each: 89 us, 83 staged
+// (30 steps 3.74 -> 3.62 ms; 3 instead of 4 records per round 3.66).
+template <int KERNEL, int MODE = kFused>
+__device__ inline bool uniform64_rates_staged(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy, int t,
+                                              const double4 &bt, const Stage &S, const double2 *sA,
+                                              unsigned short *s_list, double &drho, double &ax, double &ay) {
+    const double2 at = P.A[t];
+    const double X = at.x, Y = at.y;
+    const int2 c = P.cxy[t];
+    const unsigned stride = blockDim.x;
+    unsigned short *const list0 = s_list + threadIdx.x;
+    unsigned short *lp = list0;
+    // LDS record i holds slot i - sh of the row it lies in
+    const int off1 = S.off[1], off2 = S.off[2];
+    const int sh0 = S.off[0] - S.smin[0], sh1 = off1 - S.smin[1], sh2 = off2 - S.smin[2];
+    double arho = 0.0, a0 = 0.0, a1 = 0.0, f0 = 0.0, f1 = 0.0;
+    // The reference's expressions (Continuity.py:13-16, Momentum.py:36-56,
+    // BoundaryForce.py:31-41, CubicSpline.py:53-70 / Gaussian.py:41-60 /
+    // Wendland.py:32-64) for each listed pair, in listing order.
+    auto flush = [&]() {
+        for (unsigned short *q = list0; q != lp; q += stride) {
+            const int i = *q;
+            const double2 a = sA[i];
+            const double4 b = at32(P.B, (unsigned)(i - (i >= off2 ? sh2 : (i >= off1 ? sh1 : sh0))));
+            const double dx = X - a.x, dy = Y - a.y;
+            const double xij2 = dx * dx + dy * dy;
+            double half;
+            const double r = pair_root(xij2, half);
+            if (!not_fluid64(b.w)) {
+                const double qq = pair_quotient(r, K.h, K.hinv);
+                double dwx, dwy;
+                double grad;
+                if (KERNEL == SPH_KERNEL_WENDLAND) {
+                    if ((qq >= 2.0) || (r < 1e-10)) continue;
+                    const double inner = 1.0 - 0.5 * qq;
+                    grad = ipow(inner, 5.0) * (-14.0 / 3.0) * qq * (1 + 2.5 * qq);
+                } else {
+                    if ((qq > 2.0) || (r < 1e-10)) continue;
+                    grad = (qq > 1.0) ? -0.75 * ((2.0 - qq) * (2.0 - qq)) : -3.0 * qq * (1.0 - 0.75 * qq);
+                }
+                const double hr = K.h * r;
+                const double norm = pair_quotient(K.alpha_k * grad, hr, pair_recip(hr, half * K.hinv2));
+                dwx = norm * dx;
+                dwy = norm * dy;
+                const double vx = bt.x - b.x, vy = bt.y - b.y;
+                const double dot = vx * dwx + vy * dwy;
+                if constexpr ((MODE & kEquations) != kMomentum) arho += K.m * dot;
+                if constexpr ((MODE & kEquations) == kContinuity) continue;
+                const double dv = vx * dx + vy * dy;
+                double PI_ij = 0.0;
+                if (dv < 0) {
+                    const double rhoij = 0.5 * (bt.z + b.z);
+                    const double muij = pair_divide(K.h * dv, r * r + K.c01);
+                    const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
+                    PI_ij = pair_divide(ppij, rhoij);
+                }
+                const double factor = bt.w + b.w + PI_ij;
+                a0 += -K.m * factor * dwx;
+                a1 += -K.m * factor * dwy;
+            } else if ((MODE & kEquations) != kContinuity && !(r > K.r0) && r > 1e-12) {
+                const double frac = K.r0 / r;
+                const double tmp = wall_pow<MODE>(frac, K.p1) - wall_pow<MODE>(frac, K.p2);
+                const double fac = K.D * tmp;
+                f0 += fac * dx / (r * r);
+                f1 += fac * dy / (r * r);
+            }
+        }
+        lp = list0;
+    };
+    constexpr int U = HIPSPH_UNIFORM64_UNROLL, LIST = kUniform64List;
+    static_assert(U >= 1 && U < LIST, "unroll within the list");
+    unsigned short *const full = list0 + (LIST - U) * stride;  // past this, U appends could overflow
+    auto overflow = [&]() { return lp > full; };
+    auto test = [&](double2 a, int k) {
+        const double dx = X - a.x, dy = Y - a.y;
+        const double r2 = dx * dx + dy * dy;
+        // written whether or not it is kept (within the list's bounds either
+        // way): no branch per candidate
+        *lp = (unsigned short)k;
+        lp += (r2 <= K.lim2 && r2 > kPairNone) ? stride : 0u;
+    };
+    // the cells in uniform64_rates_listed's order
+    for (int da = -1; da <= 1; ++da) {
+        const int cx = c.x + da;
+        if (!(ncx > cx && cx > -1)) continue;
+        for (int db = -1; db <= 1; ++db) {
+            const int cy = c.y + db;
+            if (!(ncy > cy && cy > -1)) continue;
+            const long long cell = cx + (long long)ncx * cy;
+            const int sh = db < 0 ? sh0 : (db == 0 ? sh1 : sh2);
+            const int s = P.cellStart[cell] + sh, e = P.cellStart[cell + 1] + sh;
+            int k = e - 1;
+            for (; k - U + 1 >= s; k -= U) {
+                if (overflow()) flush();
+                double2 a[U];
+#pragma unroll
+                for (int j = 0; j < U; ++j) a[j] = sA[k - j];
+#pragma unroll
+                for (int j = 0; j < U; ++j) test(a[j], k - j);
+            }
+            if (k >= s) {
+                if (overflow()) flush();
+                for (; k >= s; --k) test(sA[k], k);  // fewer than U
+            }
+        }
+    }
+    flush();
+    if (!uniform64_has_neighbour(P, K, ncx, ncy, 0, X, Y, c)) return false;
+    drho = arho;
+    ax = a0 + f0;
+    ay = (MODE & kEquations) == kContinuity ? 0.0 : (a1 - K.g) + f1;  // WCSPH.py:169, then SolverTools.py:170-171
+    return true;
+}
+
+// LDS of a pass that stages: the records and a 16-bit list, or (a workgroup
+// whose ranges exceed the stage) a 32-bit list.
+template <int KERNEL>
+__host__ __device__ constexpr int stage_bytes64() {
+    constexpr int global = uniform64_list<KERNEL>() * 256 * 4;
+    constexpr int staged = kStageCap * 16 + uniform64_list<KERNEL>() * 256 * 2;
+    return KERNEL == SPH_KERNEL_GAUSSIAN || global > staged ? global : staged;
+}
+template <int KERNEL>
+struct StagedWalk64 {
+    unsigned char *mem;
+    Stage S{};
+    bool staged = false;
+    __device__ StagedWalk64(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy, int t, bool walks,
+                            unsigned char *s_mem, int *s_red)
+        : mem(s_mem) {
+        if (KERNEL == SPH_KERNEL_GAUSSIAN || !K.stage) return;  // uniform over the workgroup
+        int rs[3] = {0, 0, 0}, re[3] = {0, 0, 0};
+        if (walks) row_runs(P, ncx, ncy, 0, P.cxy[t], 0u, rs, re);
+        S = stage_plan(rs, re, s_red);
+        staged = S.total <= kStageCap;
+        if (staged) stage_copy(P, S, reinterpret_cast<double2 *>(mem));
+    }
+    template <int MODE>
+    __device__ bool rates(const Uniform64Args &P, const Uniform64Const &K, int ncx, int ncy, int t, const double4 &bt,
+                          double &drho, double &ax, double &ay) {
+        if constexpr (KERNEL != SPH_KERNEL_GAUSSIAN)
+            if (staged)
+                return uniform64_rates_staged<KERNEL, MODE>(P, K, ncx, ncy, t, bt, S,
+                                                            reinterpret_cast<const double2 *>(mem),
+                                                            reinterpret_cast<unsigned short *>(mem + kStageCap * 16),
+                                                            drho, ax, ay);
+        return uniform64_rates<KERNEL, MODE>(P, K, ncx, ncy, 0, t, bt, reinterpret_cast<unsigned *>(mem), drho, ax, ay);
+    }
+};
+
 // One target t of the pass: its rates, or nothing for a wall or a target
 // that keeps its previous rates; MODE selects the rates written.
 template <int KERNEL, int MODE = kFused>
@@ -353,12 +508,23 @@ __device__ inline void uniform64_target(const Uniform64Args &P, const Uniform64C
 
 template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_uniform64(const Ctrl *ctrl, Uniform64Args P, Uniform64Const K) {
-    __shared__ unsigned s_list[uniform64_list<KERNEL>() * 256];
+    __shared__ __align__(16) unsigned char s_mem[stage_bytes64<KERNEL>()];
+    __shared__ int s_red[6 * 4];
     if (!ctrl->active) return;
     const int t = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (t >= P.n) return;
     const Grid &g = ctrl->grid;
-    uniform64_target<KERNEL, MODE>(P, K, (int)g.ncx, (int)g.ncy, 0, t, s_list);
+    const int ncx = (int)g.ncx, ncy = (int)g.ncy;
+    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid64(bt.w);  // walls are not targets
+    StagedWalk64<KERNEL> W(P, K, ncx, ncy, t, walks, s_mem, s_red);
+    double drho, ax, ay;
+    if (!walks || !W.template rates<MODE>(P, K, ncx, ncy, t, bt, drho, ax, ay)) return;
+    if constexpr ((MODE & kEquations) != kMomentum) P.drho[t] = drho;
+    if constexpr ((MODE & kEquations) != kContinuity) {
+        P.ax[t] = ax;
+        P.ay[t] = ay;
+    }
 }
 
 // A batch target t: its instance's grid and constants. The lanes of a wave
@@ -387,40 +553,42 @@ __device__ inline void uniform64_target_batch(const BInst *inst, const int *inst
 template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_uniform64_pec(Ctrl *ctrl, Uniform64Args P, Uniform64Const K,
                                                             PecArgs C) {
-    __shared__ unsigned s_list[uniform64_list<KERNEL>() * 256];
+    __shared__ __align__(16) unsigned char s_mem[stage_bytes64<KERNEL>()];
     __shared__ double lds[kDtQ * 16];
+    __shared__ int s_red[6 * 4];
     if (!ctrl->active) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctrl->dt_parts = kDtSlots;
         ctrl->pec_parts = 1;
     }
     const int t = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const Grid &g = ctrl->grid;
+    const int ncx = (int)g.ncx, ncy = (int)g.ncy;
+    double4 bt = make_double4(0.0, 0.0, 0.0, __builtin_nan(""));
+    if (t < P.n) bt = P.B[t];
+    const bool walks = t < P.n && !not_fluid64(bt.w);
+    StagedWalk64<KERNEL> W(P, K, ncx, ncy, t, walks, s_mem, s_red);
     DtVars v;
-    if (t < P.n) {
-        const double4 bt = P.B[t];
-        if (!not_fluid64(bt.w)) {
-            const Grid &g = ctrl->grid;
-            const double dt = ctrl->dt, damping = ctrl->damping;
+    if (walks) {
+        const double dt = ctrl->dt, damping = ctrl->damping;
 #if HIPSPH_PEC64_EARLY
-            const PecStart p0 = pec_start(C, t, dt, damping);
+        const PecStart p0 = pec_start(C, t, dt, damping);
 #endif
-            double drho, ax, ay;
-            if (uniform64_rates<KERNEL, MODE>(P, K, (int)g.ncx, (int)g.ncy, 0, t, bt,
-                                                                              s_list, drho, ax, ay)) {
-                P.drho[t] = drho;
-                P.ax[t] = ax;
-                P.ay[t] = ay;
-            } else {
-                drho = P.drho[t];
-                ax = P.ax[t];
-                ay = P.ay[t];
-            }
-            v.add(C.hc.on ? C.hc.h : C.s.h[t], ax, ay);
-#if !HIPSPH_PEC64_EARLY
-            const PecStart p0 = pec_start(C, t, dt, damping);
-#endif
-            pec_finish(C, t, p0, ax, ay, drho, dt, damping);
+        double drho, ax, ay;
+        if (W.template rates<MODE>(P, K, ncx, ncy, t, bt, drho, ax, ay)) {
+            P.drho[t] = drho;
+            P.ax[t] = ax;
+            P.ay[t] = ay;
+        } else {
+            drho = P.drho[t];
+            ax = P.ax[t];
+            ay = P.ay[t];
         }
+        v.add(C.hc.on ? C.hc.h : C.s.h[t], ax, ay);
+#if !HIPSPH_PEC64_EARLY
+        const PecStart p0 = pec_start(C, t, dt, damping);
+#endif
+        pec_finish(C, t, p0, ax, ay, drho, dt, damping);
     }
     v.publish_slots(C.dslots, lds);
 }

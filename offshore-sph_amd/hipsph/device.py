@@ -416,7 +416,7 @@ class Engine:
         return out
 
     def set_pair_staging(self, on):
-        """Whether the uniform float pair passes stage each workgroup's
+        """Whether the uniform pair passes stage each workgroup's
         neighbour records in LDS (the default) or walk global memory; the
         results are bit-identical either way."""
         call('sph_ctx_set_pair_staging', self._ctx, int(bool(on)))
