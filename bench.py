@@ -449,7 +449,7 @@ def _short(name):
 def _pair_prec(name):
     if 'k_pair' not in name or 'batch' in name:
         return None
-    return 'fp64' if ('uniform64' in name or 'k_pair<double' in name) else 'fp32c'
+    return 'fp64' if ('uniform64' in name or '<double' in name) else 'fp32c'
 
 
 def summarize(raw, launches=5):
@@ -557,8 +557,8 @@ def summarize(raw, launches=5):
     return traffic, valu, phases, build
 
 
-NN_KERNELS = ('k_bounds', 'k_grid', 'k_keys', 'k_scan_reduce', 'k_scan_apply', 'k_scatter', 'k_cellsort', 'k_reorder')
-STEP_KERNELS = NN_KERNELS + ('k_correct', 'k_dt_final')
+NN_KERNELS = ('k_bounds', 'k_keys', 'k_scan', 'k_place', 'k_reorder')
+STEP_KERNELS = NN_KERNELS + ('k_correct',)
 PROFILE_COMMANDS = """    cd /tmp && export TMPDIR=/tmp      # OUT: an output directory, R: the repository
     rocprofv3 --kernel-trace --stats -f csv -d OUT/kt_pp -o kt -- python3 -u R/bench.py --profile-pair 5 2> OUT/kt_pp.log
     rocprofv3 --pmc TCC_EA0_RDREQ_sum TCC_EA0_RDREQ_32B_sum TCC_BUBBLE_sum TCC_EA0_RDREQ_DRAM_sum -f csv \\
@@ -675,7 +675,7 @@ STATS_NOTES = {
                  'pairs. Per kernel (cubic, Gaussian) and precision, 20 launches each of the neighbour update, '
                  'the continuity pass, the momentum pass and the fused pass, all in the uniform form '
                  '`k_pair_uniform<kernel, mode>` / `k_pair_uniform64<kernel, mode>` (kernel 0 cubic, 1 Gaussian; '
-                 'mode 0 fused, 1 continuity, 2 momentum).',
+                 'mode 0 fused, 1 continuity, 2 momentum, + 8 with whole wall exponents).',
     'kt_ens': 'Workload: 256 dam breaks (column width U(0.5, 1.5) m, height U(0.5, 2.5) m, dx from '
               '{0.005, 0.01, 0.02} m, alpha U(0.005, 0.05), 4.0 x 3.0 m tank), 961 to 136,948 fluid particles '
               'each, FP32C pairs, FP64 integrator, PEC, per-instance dt; every stage one launch over all '

@@ -13,8 +13,9 @@
 //   * reductions (bounds, dt) leave partials per chunk or tile, and the
 //     kernel that needs the result folds its instance's in every workgroup,
 //     as the single engine's k_bounds and k_keys do (24 dam breaks, 0.72M
-//     particles: the update's six kernels take 55 us, against 72 with
-//     kernels of their own for the folds, the bins' bases and the bin sort);
+//     particles: the update's five kernels take 42 us; 72 with kernels of
+//     their own for the folds, the bins' bases and the bin sort, LDS permutes
+//     in the folds and a scan that read every count again);
 //   * every instance has its own control block (BInst): clock, dt, grid,
 //     halt flags and constants (alpha, c0, B, r0, D ...).
 // A step needs no host round trip, like the single simulation's. The

@@ -330,9 +330,11 @@ struct DtFold {
 // particles, into the bounds slots (folded by k_keys). In a step every
 // workgroup first folds the dt partials (64 slots, or up to 2,048 partials
 // after k_correct) and decides dt for itself, since the predicted positions
-// need it; the first leaves the decision in ctrl->nx. That fold costs the
-// kernel 1.6 us (5k particles) to 2 us (1M) and saves a single-workgroup
-// kernel of 4.6 to 6.6 us and its launch. Grid-stride over at
+// need it; the first leaves the decision in ctrl->nx. That saves a
+// single-workgroup kernel of 4.6 to 6.6 us and its launch, and the first
+// particles are loaded under it. What is left is a chain of trips to memory:
+// 5.9 us (6.5k particles) to 7.1 us (1.3M; 9.0 and 10.4 with the loads after the
+// fold and LDS permutes in both folds). Grid-stride over at
 // most kBoundsBlocks workgroups, four particles per thread per round with
 // their loads issued together (one workgroup per 256 particles measured 40 %
 // slower, the per-workgroup fold paid in more rounds; 2048 workgroups with
@@ -343,8 +345,8 @@ struct DtFold {
 // predictor the full scan also finds the largest |vx|, |vy| (k_keys keeps it
 // as ctrl->vbound; +inf if one is not finite).
 constexpr int kBoundsBlocks = 1024;
-// workgroups that walk the border cells (one per CU: 8.4 us on the 1M dam
-// break, against 9.6 with all 1,024 and 10.1 with 64)
+// workgroups that walk the border cells (one per CU: on the 1M dam break 1.2
+// us less than with all 1,024 and 1.7 less than with 64)
 constexpr int kBorderBlocks = 256;
 __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const int *cellStart, DtFold D,
                          unsigned long long *bslots, int *clear, int nclear) {
@@ -735,8 +737,8 @@ __global__ void k_reorder(Ctrl *ctrl, ReorderArgs A, const int *perm0) {
 // SLOTS slots for itself and sums the counts before them, with 1,024 threads of
 // which SLOTS carry a slot. Launches, drains and dependent trips to memory are
 // what a small state's update costs: every load is issued in one of two
-// rounds, the bins and states, then the counts and members. Steps in us, by
-// k_scan_one (two kernels above 65,536), k_place and k_reorder and by this:
+// rounds, the bins and states, then the counts and members. Steps in us, with
+// kernels of their own for the scan, the places and the reorder and with this:
 //     FP64, 6.5k particles 38.9, 33.5; 39k 51.6, 45.7; 112k 66.6, 60.8
 //     FP32C, 53k 46.7, 40.5; 112k 55.1, 50.6
 // and the same on grids of up to 18 cells per particle (6.5k: 40.5, 37.0).

@@ -66,9 +66,9 @@ struct Ctrl {
     double nm_beta, nm_gamma;
     int dt_parts;        // workgroups whose dt partials the partials buffer holds (set by their kernel;
                          // kDtSlots: the dt slots hold them)
-    int pec_parts;       // 1 when those partials come from the fused PEC pass (cleared by k_dt_final)
+    int pec_parts;       // 1 when those partials come from the fused PEC pass (cleared when a dt decision takes effect)
     double disp;         // bound on how far any particle's predicted position lies from where it was
-                         // last binned, per axis (k_dt_final; +inf when unknown)
+                         // last binned, per axis (dt_decide; +inf when unknown)
     double vbound;       // bound on every particle's |vx|, |vy| at the start of the step (+inf: unknown)
     double abound;       // bound on every fluid particle's |a| in the rates the step's predictor uses
     long long border_updates;  // neighbour updates whose bounds came from the border cells
