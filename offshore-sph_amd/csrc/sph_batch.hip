@@ -9,7 +9,7 @@
 //     cells from a fixed bin on, so each instance's offsets are scanned from
 //     off_k without the others;
 //   * every workgroup works on one instance (tiles of 256 slots, chunks of
-//     1,024 for the bounds), whose control block it reads once;
+//     1,024 or 4,096 for the bounds), whose control block it reads once;
 //   * reductions (bounds, dt) leave partials per chunk or tile, and the
 //     kernel that needs the result folds its instance's in every workgroup,
 //     as the single engine's k_bounds and k_keys do (24 dam breaks, 0.72M
@@ -36,9 +36,14 @@ using namespace hipsph;
 namespace {
 
 // Two segmentations of the slots, each segment inside one instance: chunks
-// of kChunk for the bounds reduction (one workgroup of kChunkThreads), tiles
+// of chunk_slots for the bounds reduction (one workgroup of kChunkThreads), tiles
 // of kTile for everything else (one 256-thread workgroup per tile).
-constexpr int kChunk = 1024, kChunkThreads = 512;
+constexpr int kChunkThreads = 512;
+// 1,024 slots, or 4,096 in a batch of more than 2,048 such chunks: each
+// workgroup folds its instance's dt partials again, and when the border cells
+// are enough few of its threads have a particle (256 dam breaks, 7.7M
+// particles: 7,500 workgroups took 76 us).
+inline int chunk_slots(long long n) { return n > 2048 * 1024 ? 4096 : 1024; }
 constexpr int kTile = 256;
 static_assert(kTile == 256, "the fused batch pair pass runs one 256-thread workgroup per tile");
 
@@ -110,7 +115,7 @@ __device__ inline void bupd_pos(const BPos &p, bool pred, double dt, double &x, 
     y = f ? pec_half_pos(p.y, p.vy, dt) : p.y;
 }
 
-// Per chunk of 1,024 slots (one instance's): the fold of the instance's dt
+// Per chunk (of one instance's slots): the fold of the instance's dt
 // partials and its decision (every workgroup needs dt; the first chunk's
 // leaves it in I.nx for kb_keys), then the bounds' partials of the chunk,
 // part[c * kBoundsVQ + q]. With PEC's predictor the full scan also finds the
@@ -135,11 +140,10 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
     const bool may = cellStart && pred && I.uh_on && g.ncx >= 3 && g.ncy >= 3;
     const int tid = (c - chunk0[k]) * (int)blockDim.x + (int)threadIdx.x;
     const int nthreads = (chunk0[k + 1] - chunk0[k]) * (int)blockDim.x;
-    constexpr int U = kChunk / kChunkThreads;
+    constexpr int U = 2;
     int slot[U];
     BPos p[U];
     if (may) {
-        static_assert(U == 2, "the border's rows and runs");
         const BorderWalk W(cellStart, I.cellBase, g, tid, nthreads);
         slot[0] = W.first_row();
         slot[1] = W.first_run();
@@ -190,17 +194,33 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
             if (slot[u] >= 0) take(slot[u], p[u]);
         BorderWalk(cellStart, I.cellBase, g, tid, nthreads).rest([&](int i) { take(i, bpos_load(a, i, pred)); });
     } else {
+        auto speed = [&](const BPos &q) {
+            if (!pred) return;
+            const double ux = fabs(q.vx), uy = fabs(q.vy);
+            const double w = (isfinite(ux) && isfinite(uy)) ? (ux > uy ? ux : uy) : INFINITY;
+            vmx = w > vmx ? w : vmx;
+        };
+        const int end = cs[c + 1];
+        int i0 = cs[c] + (int)threadIdx.x;
+        if (!may) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = cs[c] + (int)threadIdx.x + u * kChunkThreads;
-            if (i >= cs[c + 1]) continue;
-            if (may) p[u] = bpos_load(a, i, pred);
-            take(i, p[u]);
-            if (pred) {
-                const double ux = fabs(p[u].vx), uy = fabs(p[u].vy);
-                const double w = (isfinite(ux) && isfinite(uy)) ? (ux > uy ? ux : uy) : INFINITY;
-                vmx = w > vmx ? w : vmx;
-            }
+            for (int u = 0; u < U; ++u)
+                if (slot[u] >= 0) {
+                    take(slot[u], p[u]);
+                    speed(p[u]);
+                }
+            i0 += U * kChunkThreads;
+        }
+        for (; i0 < end; i0 += U * kChunkThreads) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * kChunkThreads < end) p[u] = bpos_load(a, i0 + u * kChunkThreads, pred);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * kChunkThreads < end) {
+                    take(i0 + u * kChunkThreads, p[u]);
+                    speed(p[u]);
+                }
         }
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
@@ -725,12 +745,13 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     // chunk and tile tables
     std::vector<int> cs, chunkInst, chunk0, ts, tileInst, tile0;
     std::vector<BInst> hI(ninst);
+    const int chunk = chunk_slots(ntot);
     long long off = 0, base = 0;
     int tbase = 0;
     for (int k = 0; k < ninst; ++k) {
         const sph_params_t &P = params[k];
         chunk0.push_back((int)cs.size());
-        for (long long c = 0; c < P.n; c += kChunk) {
+        for (long long c = 0; c < P.n; c += chunk) {
             cs.push_back((int)(off + c));
             chunkInst.push_back(k);
         }
