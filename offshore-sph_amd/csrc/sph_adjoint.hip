@@ -294,50 +294,54 @@ __global__ void k_tape_pair(const Ctrl *ctrl, State s, State o, const int *perm,
         const long long lim = m < cap ? m : cap;
         for (long long k = t; k < lim; k += (long long)gridDim.x * blockDim.x) T.cellStart[k] = cellStart[k];
         if (t < n) {
+            // every load before the first store (which it may alias for the
+            // compiler): two trips to memory instead of four
             const int i = s.id[t];
             const int q = perm[t];
-            const double ax = o.ax[q], ay = o.ay[q];
-            T.vx0[i] = o.vx[q];
-            T.vy0[i] = o.vy[q];
-            T.axp[i] = ax;
-            T.ayp[i] = ay;
-            T.drhop[i] = o.drho[q];
             const int8_t lab = s.label[t];
-            const double m = s.m[t], h = s.h[t];
-            double x, y, vx, vy, rho;
-            if (lean && lab == 0) {
-                const double dt = ctrl->dt, damping = ctrl->damping;
-                x = pec_half_pos(o.x[q], o.vx[q], dt);
-                y = pec_half_pos(o.y[q], o.vy[q], dt);
-                vx = pec_half_vel(o.vx[q], ax, dt, damping);
-                vy = pec_half_vel(o.vy[q], ay, dt, damping);
-                rho = pec_half_rho(o.rho[q], o.drho[q], dt, strict);
-            } else {
+            const double m = s.m[t], h = s.h[t], sax = s.ax[t], say = s.ay[t], sdr = s.drho[t];
+            const int2 c = cxy[t];
+            const bool half = lean && lab == 0;
+            double x = 0.0, y = 0.0, vx = 0.0, vy = 0.0, rho = 0.0;
+            if (!half) {
                 x = s.x[t];
                 y = s.y[t];
                 vx = s.vx[t];
                 vy = s.vy[t];
                 rho = s.rho[t];
             }
+            const double ax = o.ax[q], ay = o.ay[q], vx0 = o.vx[q], vy0 = o.vy[q], dr0 = o.drho[q], r0 = o.rho[q];
+            const double dt = ctrl->dt, damping = ctrl->damping;
+            if (half) {
+                x = pec_half_pos(o.x[q], vx0, dt);
+                y = pec_half_pos(o.y[q], vy0, dt);
+                vx = pec_half_vel(vx0, ax, dt, damping);
+                vy = pec_half_vel(vy0, ay, dt, damping);
+                rho = pec_half_rho(r0, dr0, dt, strict);
+            }
+            T.vx0[i] = vx0;
+            T.vy0[i] = vy0;
+            T.axp[i] = ax;
+            T.ayp[i] = ay;
+            T.drhop[i] = dr0;
             // PEC's strict clamp (src/Integrators/PEC.py:57-58, 87-88): whether it
             // took the predicted or the corrected density (the adjoint of a
             // clamped density is zero)
             int8_t cl = 0;
             if (strict && lab == 0) {
-                const double dt = ctrl->dt, r0 = o.rho[q];
-                const double rp = r0 + 0.5 * dt * o.drho[q];
-                const double rc = 2 * (r0 + 0.5 * dt * s.drho[t]) - r0;
+                const double rp = r0 + 0.5 * dt * dr0;
+                const double rc = 2 * (r0 + 0.5 * dt * sdr) - r0;
                 cl = (int8_t)((rp < 0.0 ? 1 : 0) | (rc < 0.0 ? 2 : 0));
             }
             T.clamp[i] = cl;
             T.vxh[i] = vx;
             T.vyh[i] = vy;
-            T.ax[i] = s.ax[t];
-            T.ay[i] = s.ay[t];
-            T.drho[i] = s.drho[t];
+            T.ax[i] = sax;
+            T.ay[i] = say;
+            T.drho[i] = sdr;
             T.slot[i] = t;
             T.id[t] = i;
-            T.cxy[t] = cxy[t];
+            T.cxy[t] = c;
             T.pa[t] = make_double4(x, y, h, lab == 0 ? m : -(double)lab);
             T.pb[t] = make_double4(vx, vy, rho, m);
             if (lab == 0) {
@@ -380,33 +384,38 @@ __global__ void k_adj_correct(const TapeHdr *hdr, TapeSlot T, const int8_t *labe
     const double dt = hdr->dt, e = 1.0 + 0.5 * damping;
     double v[kAdjQ] = {0.0, 0.0, 0.0, 0.0};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (label[i] != 0) {
-            lk[T.slot[i]] = make_double4(0.0, 0.0, 0.0, 0.0);
+        // every load before the first store, as k_tape_pair
+        const int8_t lab = label[i];
+        const int slot = T.slot[i];
+        const double xb = A.x[i], yb = A.y[i], vxb = A.vx[i], vyb = A.vy[i], rb = A.rho[i];
+        const double axb = A.ax[i], ayb = A.ay[i], drb = A.drho[i];
+        const double tax = T.ax[i], tay = T.ay[i], tdr = T.drho[i];
+        const double tvx = euler ? T.vx0[i] : T.vxh[i], tvy = euler ? T.vy0[i] : T.vyh[i];
+        const bool cc = (T.clamp[i] & 2) != 0;
+        if (lab != 0) {
+            lk[slot] = make_double4(0.0, 0.0, 0.0, 0.0);
             vbx[i] = vby[i] = 0.0;
             A.x[i] = A.y[i] = A.vx[i] = A.vy[i] = A.rho[i] = A.ax[i] = A.ay[i] = A.drho[i] = 0.0;
             continue;
         }
-        const double xb = A.x[i], yb = A.y[i], vxb = A.vx[i], vyb = A.vy[i], rb = A.rho[i];
         if (euler) {
             // x' = x + dt v + dt^2/2 a, v' = v + dt a, rho' = rho + dt drho (pair at the start state)
-            lk[T.slot[i]] = make_double4(A.ax[i] + dt * vxb + 0.5 * dt * dt * xb, A.ay[i] + dt * vyb + 0.5 * dt * dt * yb,
-                                         A.drho[i] + dt * rb, 0.0);
+            lk[slot] = make_double4(axb + dt * vxb + 0.5 * dt * dt * xb, ayb + dt * vyb + 0.5 * dt * dt * yb,
+                                    drb + dt * rb, 0.0);
             vbx[i] = 0.0;
             vby[i] = 0.0;
             A.vx[i] = vxb + dt * xb;
             A.vy[i] = vyb + dt * yb;
-            const double vx = T.vx0[i], vy = T.vy0[i], ax = T.ax[i], ay = T.ay[i];
-            v[0] += xb * (vx + dt * ax) + yb * (vy + dt * ay) + vxb * ax + vyb * ay + rb * T.drho[i];
+            v[0] += xb * (tvx + dt * tax) + yb * (tvy + dt * tay) + vxb * tax + vyb * tay + rb * tdr;
         } else {
             // a density the strict clamp set to 0 passes no adjoint back
-            const bool cc = (T.clamp[i] & 2) != 0;
             const double rbe = cc ? 0.0 : rb;
-            lk[T.slot[i]] = make_double4(A.ax[i] + dt / e * vxb, A.ay[i] + dt / e * vyb, A.drho[i] + dt * rbe, 0.0);
+            lk[slot] = make_double4(axb + dt / e * vxb, ayb + dt / e * vyb, drb + dt * rbe, 0.0);
             vbx[i] = dt * xb;
             vby[i] = dt * yb;
             A.vx[i] = (2.0 / e - 1.0) * vxb;
             A.vy[i] = (2.0 / e - 1.0) * vyb;
-            v[0] += xb * T.vxh[i] + yb * T.vyh[i] + (vxb * T.ax[i] + vyb * T.ay[i]) / e + rbe * T.drho[i];
+            v[0] += xb * tvx + yb * tvy + (vxb * tax + vyb * tay) / e + rbe * tdr;
             if (cc) A.rho[i] = 0.0;
         }
         // x and rho pass through with coefficient 1 (A.x, A.y, A.rho unchanged,
