@@ -321,15 +321,19 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     }
 }
 
-// Each instance's offsets, scanned from its first slot, up to scan_tiles(K)
-// tiles at a time.
+// Each instance's offsets, scanned from its first slot, up to T =
+// scan_tiles(K) tiles at a time: workgroups k T ... k T + T - 1 are instance
+// k's (on the grid's x axis: the others hold 65,535 workgroups, a batch up to
+// 2^20 instances).
 inline int scan_tiles(int K) { return K >= 256 ? 8 : (K >= 64 ? 16 : 64); }
-__global__ __launch_bounds__(kBlock) void kb_scan(const BInst *inst, int *counts, const int *tileSums, int *cellStart) {
+__global__ __launch_bounds__(kBlock) void kb_scan(const BInst *inst, int *counts, const int *tileSums, int *cellStart,
+                                                  int T) {
     __shared__ int lds[16];
-    const BInst &I = inst[blockIdx.y];
+    const int k = (int)blockIdx.x / T;
+    const BInst &I = inst[k];
     if (!I.active) return;
     const long long nbins = I.grid.ncells + 1;
-    for (long long tile = blockIdx.x; tile * kScanTile < nbins; tile += gridDim.x)
+    for (long long tile = (int)blockIdx.x - k * T; tile * kScanTile < nbins; tile += T)
         scan_tile(counts + I.cellBase, tileSums + (size_t)I.tileBase * kTileStride, cellStart + I.cellBase, nbins,
                   tile, I.off, lds);
 }
@@ -621,7 +625,8 @@ int b_nn(sph_batch *b, hipStream_t s) {
                                               b->view);
     kb_keys<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->chunk0, b->inst, a, pec, b->part_b, b->counts,
                                     b->bin, b->rank, b->binflag, b->tileSums, b->view);
-    kb_scan<<<dim3(scan_tiles(b->K), b->K), kBlock, 0, s>>>(b->inst, b->counts, b->tileSums, b->cellStart);
+    const int T = scan_tiles(b->K);
+    kb_scan<<<b->K * T, kBlock, 0, s>>>(b->inst, b->counts, b->tileSums, b->cellStart, T);
     kb_place<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->inst, b->cellStart, b->bin, b->rank, b->perm0,
                                      b->tileSums);
     const int fmt = b->precision == SPH_PREC_FP32C ? (b->uni ? kRecUniform : kRecFp32)
