@@ -175,8 +175,11 @@ __global__ void k_ke_final(double *part, int R) {
 // ---------------------------------------------------------------------------
 // integrators (fluid only: src/Solver.py:380,396 pass pA[f_indexes])
 // ---------------------------------------------------------------------------
-__global__ void k_pec_predict(const Ctrl *ctrl, State s, int n, int strict, int xs) {
-    if (!ctrl->active) return;
+// same: x0 ... rho0 are the state and not in memory, where they go also if
+// the predictor does not run (the host cannot know).
+__global__ void k_pec_predict(const Ctrl *ctrl, State s, int n, int strict, int xs, int same) {
+    const int act = ctrl->active;
+    if (!act && !same) return;
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n || s.label[j] != kFluid) return;
     const double dt = ctrl->dt, damping = ctrl->damping;
@@ -185,11 +188,12 @@ __global__ void k_pec_predict(const Ctrl *ctrl, State s, int n, int strict, int 
     s.y0[j] = y;
     s.vx0[j] = vx;
     s.vy0[j] = vy;
+    s.rho0[j] = rho;
+    if (!act) return;
     s.x[j] = pec_half_pos(x, xs ? s.xsphx[j] : vx, dt);  // PEC.py:43-48
     s.y[j] = pec_half_pos(y, xs ? s.xsphy[j] : vy, dt);
     s.vx[j] = pec_half_vel(vx, s.ax[j], dt, damping);
     s.vy[j] = pec_half_vel(vy, s.ay[j], dt, damping);
-    s.rho0[j] = rho;
     s.rho[j] = pec_half_rho(rho, s.drho[j], dt, strict);
 }
 
@@ -586,7 +590,9 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
 // from the position the keys were computed from.
 // carry: keep x0 ... rho0 with the state (between a predictor and its
 // corrector; skipped where they are still the state itself, which saves 80 of
-// 263 bytes per particle).
+// 263 bytes per particle). A step that does not run moves nobody: its x0 ...
+// rho0 stay with the state, or are written from it (same: they were the state
+// and not in memory).
 // pred as for upd_pos; xs: carry the XSPH velocity with the state; dyn:
 // dynamic h for the fluid, formed here, after the keys were binned with the
 // previous h (Solver._compute: nn.update :238, then computeH :242-246) and
@@ -610,7 +616,7 @@ struct ReorderArgs {
     void *recA, *recB;
     int pred, strict, lean, xs, dyn;
     HmConst hc;
-    int carry;
+    int carry, same;
 };
 __device__ inline Moved reorder_load(const Ctrl *ctrl, const ReorderArgs &A, int act, int s) {
     const State &a = A.a;
@@ -674,7 +680,13 @@ __device__ inline void reorder_store(Ctrl *ctrl, const ReorderArgs &A, int act, 
             b.vy0[t] = p.vy0;
             b.rho0[t] = p.rho0;
         }
-    } else if (A.carry) {
+    } else if (A.same && A.pred && !act) {
+        b.x0[t] = p.x0;
+        b.y0[t] = p.y0;
+        b.vx0[t] = p.vx0;
+        b.vy0[t] = p.vy0;
+        b.rho0[t] = p.rho0;
+    } else if (A.carry || (A.pred && !act)) {
         b.x0[t] = a.x0[s];
         b.y0[t] = a.y0[s];
         b.vx0[t] = a.vx0[s];
@@ -1855,7 +1867,7 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
     c->rec_fmt = rec_format(c);
     const ReorderArgs ra{a, b, c->perm, c->cellStart, c->binflag, c->cxy_s, make_phys(c->P), n, c->rec_fmt, c->recA,
                          c->recB, pred, c->P.strict, lean, c->P.use_xsph, c->P.dynamic_h, hc,
-                         pred == 0 && !c->x0_same};
+                         pred == 0 && !c->x0_same, c->x0_same};
     if (!w.members)
         k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, ra, c->perm0);
     else if (n <= kReorderScanMax / 2)
@@ -1958,9 +1970,10 @@ static int dt_step(sph_ctx *c, hipStream_t s) {
 
 static int predict(sph_ctx *c, hipStream_t s) {
     if (c->P.integrator != SPH_INTEGRATOR_PEC) return 0;  // Euler.predict is a no-op
-    c->x0_same = false;
-    k_pec_predict<<<nblk(c->n), kBlock, 0, s>>>(c->ctrl, c->buf[c->cur], c->n, c->P.strict, c->P.use_xsph);
+    k_pec_predict<<<nblk(c->n), kBlock, 0, s>>>(c->ctrl, c->buf[c->cur], c->n, c->P.strict, c->P.use_xsph,
+                                               c->x0_same);
     HIPCHK(hipGetLastError());
+    c->x0_same = false;
     return 0;
 }
 
