@@ -1529,8 +1529,11 @@ bool hipsph::uniform_eligible(const sph_params_t &P, double h) {
     if (P.n > kUniformMaxN) return false;  // records addressed with 32-bit byte offsets
     if (P.use_xsph || P.use_summation_density || P.dynamic_h) return false;
     if (!(h > 0.0)) return false;
-    // the double pass's pair_root and pair_quotient scale nothing
-    if (P.precision == SPH_PREC_FP64 && !(h > 1e-100 && h < 1e100)) return false;
+    // the double pass's pair_root and pair_quotient scale nothing: grad W /
+    // (h r), of (2 - q)^2 / h^4 and Wendland's of (2 - q)^5 / h^4 with 2 - q
+    // down to 2^-52, must stay a normal number
+    const double top = P.kernel == SPH_KERNEL_WENDLAND ? 1e57 : 1e68;
+    if (P.precision == SPH_PREC_FP64 && !(h > 1e-100 && h < top)) return false;
     const double cut = 0.99 * P.qmax * h;
     if (P.kernel == SPH_KERNEL_GAUSSIAN)  // support 3h, cut by the cut-off unless q_max >= 3
         return P.qmax >= 3.0 && P.r0 < 0.99 * 3.0 * h;

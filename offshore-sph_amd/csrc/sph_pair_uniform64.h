@@ -74,12 +74,20 @@ __device__ inline bool not_fluid64(double prs) { return prs != prs; }
 
 // Square roots and quotients of the pair terms with the bits of sqrt() and /,
 // without what those spend on the ends of the exponent range (scaling before
-// and after, 6 of a root's 16 instructions and 3 of a quotient's 11): the
-// launcher takes this pass for 1e-100 < h < 1e100 only and the walk lists no
-// pair with r^2 <= 1e-280, which adds nothing anywhere (r < 1e-12). Newton steps
-// on the hardware's estimates, then one correction by the exact remainder,
+// and after, 6 of a root's 16 instructions and 3 of a quotient's 11). A root is
+// Goldschmidt's coupled iteration for a^1/2 and a^-1/2 / 2 (R. E. Goldschmidt,
+// MIT, 1964) from the hardware's estimate, a quotient a Newton step on the
+// hardware's reciprocal; each ends with a correction by the exact remainder,
 // which rounds a quotient as / does when the reciprocal is itself the rounded
-// one (P. Markstein, IBM J. Res. Dev. 34, 1990).
+// one (P. Markstein, IBM J. Res. Dev. 34, 1990; no bit differed in 2.1e9
+// random operands of each form). That needs an exact remainder and a normal
+// result: the walk lists no pair with r^2 <= 1e-280, which adds nothing anywhere
+// (r < 1e-12), and uniform_eligible keeps h between 1e-100 and 1e68 (1e57 for
+// Wendland), which keeps the roots and the quotients by h and h r of pairs that
+// count (r >= 1e-10) inside. The viscosity's operands depend on velocities and
+// densities and may lie anywhere, so they are divided by / (without scaling the
+// last bits of rates below 1e-300 differed; 30 steps of 500k particles take 3.62
+// ms instead of 3.58).
 //
 // root(a) also leaves half = 0.5 / root(a) to about 2^-50, from which the
 // quotient by h root(a) needs no estimate of its own.
@@ -101,11 +109,6 @@ __device__ inline double pair_quotient(double a, double b, double y) {
 // 1 / b from an estimate y
 __device__ inline double pair_recip(double b, double y) {
     return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
-}
-// a / b, any a (a zero or non-finite a or b as /)
-__device__ inline double pair_divide(double a, double b) {
-    const double y = pair_recip(b, pair_recip(b, __builtin_amdgcn_rcp(b)));
-    return __builtin_amdgcn_div_fixup(pair_quotient(a, b, y), b, a);
 }
 
 // Whether the target at (X, Y) in cell c has a neighbour: one whose own cell
@@ -187,9 +190,9 @@ __device__ inline bool uniform64_rates_listed(const Uniform64Args &P, const Unif
                 double PI_ij = 0.0;
                 if (dv < 0) {
                     const double rhoij = 0.5 * (bt.z + b.z);
-                    const double muij = pair_divide(K.h * dv, r * r + K.c01);
+                    const double muij = K.h * dv / (r * r + K.c01);
                     const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                    PI_ij = pair_divide(ppij, rhoij);
+                    PI_ij = ppij / rhoij;
                 }
                 const double factor = bt.w + b.w + PI_ij;
                 a0 += -K.m * factor * dwx;
@@ -300,9 +303,9 @@ __device__ inline bool uniform64_rates_direct(const Uniform64Args &P, const Unif
                     double PI_ij = 0.0;
                     if (dv < 0) {
                         const double rhoij = 0.5 * (bt.z + b.z);
-                        const double muij = pair_divide(K.h * dv, xij2 + K.c01);
+                        const double muij = K.h * dv / (xij2 + K.c01);
                         const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                        PI_ij = pair_divide(ppij, rhoij);
+                        PI_ij = ppij / rhoij;
                     }
                     const double factor = bt.w + b.w + PI_ij;
                     a0 += -K.m * factor * dwx;
@@ -392,9 +395,9 @@ __device__ inline bool uniform64_rates_staged(const Uniform64Args &P, const Unif
                 double PI_ij = 0.0;
                 if (dv < 0) {
                     const double rhoij = 0.5 * (bt.z + b.z);
-                    const double muij = pair_divide(K.h * dv, r * r + K.c01);
+                    const double muij = K.h * dv / (r * r + K.c01);
                     const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                    PI_ij = pair_divide(ppij, rhoij);
+                    PI_ij = ppij / rhoij;
                 }
                 const double factor = bt.w + b.w + PI_ij;
                 a0 += -K.m * factor * dwx;
@@ -764,9 +767,9 @@ struct Uniform64Group {
             if (dv < 0) {
                 const double rhoij = 0.5 * (rho0 + b.z);
                 const double rr = KERNEL == SPH_KERNEL_GAUSSIAN ? xij2 : r * r;
-                const double muij = pair_divide(K.h * dv, rr + K.c01);
+                const double muij = K.h * dv / (rr + K.c01);
                 const double ppij = muij * (K.beta * muij - K.alpha * K.cij);
-                PI_ij = pair_divide(ppij, rhoij);
+                PI_ij = ppij / rhoij;
             }
             const double factor = prs + b.w + PI_ij;
             a0 = -K.m * factor * dwx;
