@@ -155,14 +155,15 @@ __device__ inline bool exact_q_test(double xi, double yi, double hi, double xj, 
 // h is -2 alpha / h^2 exp(-r^2 / h^2), which needs no square root and no
 // division per pair (ih2 = 1 / h^2, g2 = -2 alpha / h^2). The reference's
 // conditions, q <= 3 and r h > 1e-12, take its expressions where r^2 is
-// within rounding of the limit, so they decide as it does.
+// within rounding of the limit, so they decide as it does. (h |h|: a pair whose
+// h is negative, r h <= 0, adds nothing.)
 __device__ inline bool gauss_factor(double r2, double h, double ih2, double g2, double &f) {
     const double q2 = r2 * ih2;
     if (!(q2 <= 9.0 * (1.0 - 1e-12))) {
         if (!(q2 <= 9.0 * (1.0 + 1e-12))) return false;
         if (!(sqrt(r2) / h <= 3)) return false;
     }
-    if (r2 * (h * h) < 4e-24 && !(sqrt(r2) * h > 1e-12)) return false;
+    if (r2 * (h * fabs(h)) < 4e-24 && !(sqrt(r2) * h > 1e-12)) return false;
     f = g2 * exp(-q2);
     return true;
 }
