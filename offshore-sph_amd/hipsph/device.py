@@ -147,7 +147,7 @@ class Engine:
         """Whether the library can read field k from v itself."""
         import torch
         return (isinstance(v, torch.Tensor) and v.device == self.io[k].device and v.dtype == self.io[k].dtype and
-                v.numel() == self.n and v.is_contiguous())
+                v.numel() == self.n and v.is_contiguous() and not v.is_neg())
 
     def close(self):
         if self._ctx:
