@@ -470,8 +470,16 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
     }
 }
 
-// The least number of a bin's indices that k_keys lists for k_reorder_scan.
-constexpr int kBinMembers = 16;
+// The indices of a bin that k_keys lists for k_reorder_scan: as many as the
+// table's `room` entries hold for every bin of this update's grid, from
+// kBinMembers (the table has those for every cell of the capacity) to
+// kBinMost. A bin of a water column holds 7, of walls without h (cells of 1 m,
+// whatever the spacing) or a wider scale more, in fewer bins.
+constexpr int kBinMembers = 16, kBinMost = 256;
+__device__ inline int bin_most(int room, long long ncells) {
+    const int m = (int)((unsigned)room / ((unsigned)ncells + 1u)) & ~3;  // whole rows of four
+    return m < kBinMost ? m : kBinMost;
+}
 // _bin :129-141: cid = floor((x - xmin) / cs) per axis (:146-176), flat key
 // cx + ncx * cy (:200-208). Counts per bin; the rank inside a bin comes from
 // one atomic per run of equal bins within a wavefront (the state is already
@@ -486,10 +494,11 @@ constexpr int kBinMembers = 16;
 // slots that k_bounds has folded.
 __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double scale, long long cap,
                        const unsigned long long *bslots, unsigned long long *dslots, double *hist, int *counts, int *bin,
-                       int *rank, int *binflag, int *tiles, int *members, int most) {
+                       int *rank, int *binflag, int *tiles, int *members, int room) {
     __shared__ double s_v[kBoundsVQ];
     __shared__ Grid s_g;
     __shared__ unsigned s_halt;
+    __shared__ int s_most;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     // loaded together with the control block
@@ -521,7 +530,9 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         const unsigned halt = derive_grid(s_v, scale, cap, g);
         s_halt = halt;
         s_g = g;
+        s_most = members && !halt ? bin_most(room, g.ncells) : 0;
         if (blockIdx.x == 0) {
+            ctrl->most = s_most;
             if (fold) dt_commit(ctrl, ctrl->nx, hist);
             if (s_v[7] >= 0.0) ctrl->vbound = s_v[7];  // a full scan's velocity bound
             if (halt) {
@@ -570,7 +581,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         const int r = base + (lane - leader);
         bin[t] = b;
         rank[t] = r;
-        if (members && r < most) members[(size_t)b * most + r] = id;  // for k_reorder_scan
+        if (members && r < s_most) members[(size_t)b * s_most + r] = id;  // for k_reorder_scan
     }
 }
 
@@ -760,14 +771,6 @@ constexpr int kReorderShares = 32;
 constexpr int kScanBins = 1 << 13;  // bins in LDS at a time
 constexpr int kReorderScanMax = (256 - kReorderShares) * 512;
 constexpr long long kReorderScanCap = 1 << 20;  // most cells
-constexpr size_t kMembersBytes = 128u << 20;
-// Indices per bin that k_keys lists: a bin of a water column holds 7, of
-// walls without h (cells of 1 m, whatever the spacing) or a wider scale more.
-inline int bin_members(long long cap) {
-    int m = 256;
-    while (m > kBinMembers && sizeof(int) * m * (size_t)(cap + 1) > kMembersBytes) m /= 2;
-    return m;
-}
 
 // For every slot of the workgroup whose bin holds more than are listed (key
 // >= 0), the number of smaller indices in the bin, from all particles' bins:
@@ -810,12 +813,12 @@ __device__ inline int crowded_ranks(int key, int id, int n, const int *bin, cons
 template <int SLOTS>
 __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, ReorderArgs A, const int *counts,
                                                                int *cellStart, const int *bin, const int *rank,
-                                                               const int *members, int most,
+                                                               const int *members,
                                                                unsigned long long *bslots) {
     __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
     __shared__ int lds[16], s_lo[SLOTS / 64], s_hi[SLOTS / 64];
     constexpr bool kPacked = SLOTS <= kBlock;  // n < 65,536
-    const int act = ctrl->active, n = A.n, tid = threadIdx.x;
+    const int act = ctrl->active, most = ctrl->most, n = A.n, tid = threadIdx.x;
     if (blockIdx.x < kReorderShares) {
         if (blockIdx.x == 0 && tid < kBoundsSlots * kBoundsStride) bslots[tid] = 0;  // as k_place
         if (!act) return;
@@ -1438,6 +1441,11 @@ static int read_ctrl(sph_ctx *c, hipStream_t s, Ctrl &h) {
     return 0;
 }
 
+// Entries of the members' table of at most cap cells: 64 bytes a cell, so that
+// a small state's engine stays small (6,500 particles at the default capacity:
+// 7.5 MB; 256 entries for every cell would be 120).
+static int member_room(long long cap) { return (int)(kBinMembers * (cap + 1)); }
+
 static int alloc_cells(sph_ctx *c, long long cap) {
     if (c->counts) hipFree(c->counts);
     if (c->cellStart) hipFree(c->cellStart);
@@ -1460,7 +1468,7 @@ static int alloc_cells(sph_ctx *c, long long cap) {
     HIPCHK(hipMalloc(&c->binflag, sizeof(int) * (cap + 1)));
     HIPCHK(hipMemset(c->binflag, 0, sizeof(int) * (cap + 1)));
     if (c->n <= kReorderScanMax && cap <= kReorderScanCap &&
-        hipMalloc(&c->members, sizeof(int) * bin_members(cap) * (cap + 1)) != hipSuccess) {
+        hipMalloc(&c->members, sizeof(int) * member_room(cap)) != hipSuccess) {
         c->members = nullptr;  // the update of a larger state needs none
         (void)hipGetLastError();
     }
@@ -1822,7 +1830,7 @@ struct NnWork {
     Slots slots;
     int *counts, *cellStart, *tileSums, *binflag, *bin, *rank, *perm0;
     int *members;  // not null: k_reorder_scan follows (then no places, and the counts stay until the next k_bounds)
-    int most;      // members per bin
+    int room;      // its entries
     long long cap;
 };
 static void nn_launch(const NnWork &w, const State &a, int n, int pred, const HmConst &hc, const int *border,
@@ -1831,7 +1839,7 @@ static void nn_launch(const NnWork &w, const State &a, int n, int pred, const Hm
     k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b, w.members ? w.counts : nullptr,
                                  (int)w.cap + 1);
     k_keys<<<nblk(n), kBlock, 0, s>>>(w.ctrl, a, n, pred, D.on, scale, w.cap, w.slots.b, w.slots.d, D.hist, w.counts,
-                                      w.bin, w.rank, w.binflag, w.members ? nullptr : w.tileSums, w.members, w.most);
+                                      w.bin, w.rank, w.binflag, w.members ? nullptr : w.tileSums, w.members, w.room);
     if (w.members) return;  // k_reorder_scan does the rest
     const long long tiles = (w.cap + 1 + kScanTile - 1) / kScanTile;
     k_scan<<<(int)(tiles < 2048 ? tiles : 2048), kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums, w.cellStart);
@@ -1864,7 +1872,7 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
     const HmConst hc = hm_const(c);
     const Slots sl = slots_of(c->slots);
     const NnWork w{c->ctrl, sl, c->counts, c->cellStart, c->tileSums, c->binflag, c->bin, c->rank, c->perm0,
-                   c->members, bin_members(c->cap_cells), c->cap_cells};
+                   c->members, c->members ? member_room(c->cap_cells) : 0, c->cap_cells};
     nn_launch(w, a, n, pred, hc, border, c->P.scale,
               DtFold{fold, c->P.gamma_c, c->P.gamma_f, c->uni_h, c->dt_hist, c->part_d, sl.d}, s);
     c->rec_fmt = rec_format(c);
@@ -1875,10 +1883,10 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
         k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, ra, c->perm0);
     else if (n <= kReorderScanMax / 2)
         k_reorder_scan<256><<<kReorderShares + nblk(n, 256), kScanThreads, 0, s>>>(
-            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, w.most, sl.b);
+            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, sl.b);
     else
         k_reorder_scan<512><<<kReorderShares + nblk(n, 512), kScanThreads, 0, s>>>(
-            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, w.most, sl.b);
+            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, sl.b);
     HIPCHK(hipGetLastError());
     if (pred) c->x0_same = false;
     if (!c->P.use_xsph) c->xs_fluid_zero = true;

@@ -74,6 +74,7 @@ struct Ctrl {
     long long border_updates;  // neighbour updates whose bounds came from the border cells
     DtNext nx;
     int epoch;           // neighbour updates so far: a bin flag holds the update that set it
+    int most;            // indices that the last update's keys listed of each bin
     int counted;         // bins whose counts the last update left for the next one's k_bounds to clear
 };
 
