@@ -552,32 +552,38 @@ __global__ __launch_bounds__(kBlock) void k_scan(const Ctrl *ctrl, int *counts, 
 }
 
 // Share i of S of the exclusive scan of counts[0 .. nbins) (16-byte aligned)
-// into cellStart, from `first` on: the workgroup sums every count before its
-// share itself, then scans its share, four bins per thread. Returns whether
-// the share holds the last bin; sum is then the scan's total. lds holds 16
-// ints.
-__device__ inline bool scan_share(const int *counts, int *cellStart, long long nbins, int i, int S, int first, int *lds,
-                                  int &sum) {
-    const long long share = ((nbins + S - 1) / S + 3) / 4 * 4;
-    const long long b0 = i * share;
-    if (b0 >= nbins) return false;
-    const long long b1 = b0 + share < nbins ? b0 + share : nbins;
+// into cellStart: the workgroup sums what lies before its share itself, the
+// counts or, in a grid of more than kPlainBins (whose keys left them), the
+// tiles' sums, and scans its share, four bins per thread. lds holds 16 ints.
+constexpr int kPlainBins = 1 << 17;
+__device__ inline void scan_share(const int *counts, const int *tileSums, int *cellStart, int nbins, int i, int S,
+                                  int *lds) {
+    const bool tiles = nbins > kPlainBins;
+    const int unit = tiles ? kScanTile : 4;
+    const int share = ((nbins + S - 1) / S + unit - 1) / unit * unit;
+    const long long at = (long long)i * share;
+    if (at >= nbins) return;
+    const int b0 = (int)at, b1 = nbins - b0 > share ? b0 + share : nbins;
     int pre = 0;
-    constexpr int U = 8;  // loads in flight per thread
-    const long long step = 4 * (long long)blockDim.x;
-    for (long long j = 4 * (long long)threadIdx.x; j < b0; j += U * step) {  // b0 is a multiple of 4
-        int4 c[U];
+    const int step = 4 * (int)blockDim.x;
+    if (tiles) {
+        for (int j = threadIdx.x; j < b0 / kScanTile; j += blockDim.x) pre += tileSums[(size_t)j * kTileStride];
+    } else {
+        constexpr int U = 8;  // loads in flight per thread
+        for (int j = 4 * (int)threadIdx.x; j < b0; j += U * step) {  // b0 is a multiple of 4
+            int4 c[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            c[u] = j + u * step < b0 ? *reinterpret_cast<const int4 *>(counts + j + u * step) : make_int4(0, 0, 0, 0);
+            for (int u = 0; u < U; ++u)
+                c[u] = j + u * step < b0 ? *reinterpret_cast<const int4 *>(counts + j + u * step)
+                                         : make_int4(0, 0, 0, 0);
 #pragma unroll
-        for (int u = 0; u < U; ++u) pre += c[u].x + c[u].y + c[u].z + c[u].w;
+            for (int u = 0; u < U; ++u) pre += c[u].x + c[u].y + c[u].z + c[u].w;
+        }
     }
     int run, tot;
     block_scan_excl(pre, lds, &run);  // run: the sum before the share
-    run += first;
-    for (long long b = b0; b < b1; b += step) {
-        const long long k = b + 4 * (long long)threadIdx.x;
+    for (int b = b0; b < b1; b += step) {
+        const int k = b + 4 * (int)threadIdx.x;
         int v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) v[u] = k + u < b1 ? counts[k + u] : 0;
@@ -589,8 +595,6 @@ __device__ inline bool scan_share(const int *counts, int *cellStart, long long n
         }
         run += tot;
     }
-    sum = run;
-    return b1 == nbins;
 }
 
 constexpr int kScanThreads = 1024;  // of the kernels that use scan_share

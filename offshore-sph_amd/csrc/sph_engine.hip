@@ -353,11 +353,14 @@ constexpr int kBoundsBlocks = 1024;
 // us less than with all 1,024 and 1.7 less than with 64)
 constexpr int kBorderBlocks = 256;
 __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const int *cellStart, DtFold D,
-                         unsigned long long *bslots, int *clear, int nclear) {
+                         unsigned long long *bslots, int *clear, int *tiles, int nclear) {
     __shared__ double lds[kBoundsVQ * 16];
-    if (clear) {  // the last update's counts, all of whose readers (k_reorder_scan) are done
+    if (clear) {  // the last update's counts and tile sums, all of whose readers (k_reorder_scan) are done
         const int m = ctrl->counted < nclear ? ctrl->counted : nclear;
         for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < m; b += gridDim.x * blockDim.x) clear[b] = 0;
+        if (m > kPlainBins)
+            for (int j = blockIdx.x * blockDim.x + threadIdx.x; j <= (m - 1) / kScanTile; j += gridDim.x * blockDim.x)
+                tiles[(size_t)j * kTileStride] = 0;
     }
     __shared__ double s_dt, s_disp;
     __shared__ int s_active;
@@ -575,7 +578,8 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         // flagged; the store is idempotent, so no atomic is needed.
         if (base != 0) binflag[b] = epoch;
     }
-    if (tiles) tile_add(tiles, b < 0 ? -1 : b / kScanTile);
+    // k_reorder_scan reads the tiles' sums of a large grid only
+    if (!members || g.ncells >= kPlainBins) tile_add(tiles, b < 0 ? -1 : b / kScanTile);
     base = __shfl(base, leader, 64);
     if (t < n) {
         const int r = base + (lane - leader);
@@ -845,7 +849,8 @@ __device__ inline int crowded_ranks(int key, int id, int n, const int *bin, cons
 
 template <int SLOTS>
 __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, ReorderArgs A, const int *counts,
-                                                               int *cellStart, const int *bin, const int *rank,
+                                                               const int *tileSums, int *cellStart,
+                                                               const int *bin, const int *rank,
                                                                const int *members,
                                                                unsigned long long *bslots) {
     __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
@@ -856,8 +861,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
         if (blockIdx.x == 0 && tid < kBoundsSlots * kBoundsStride) bslots[tid] = 0;  // as k_place
         if (!act) return;
         const int nbins = (int)ctrl->grid.ncells + 1;
-        int sum;
-        scan_share(counts, cellStart, nbins, blockIdx.x, kReorderShares, 0, lds, sum);
+        scan_share(counts, tileSums, cellStart, nbins, blockIdx.x, kReorderShares, lds);
         if (blockIdx.x == 0 && tid == 0) {
             ctrl->nn_valid = 1;
             ctrl->counted = nbins;
@@ -901,8 +905,14 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
         const int from0 = lo & ~3, to = (hi | 3) + 1;
         unsigned pre = 0;
         {
+            int whole = 0;  // bins whose sums the tiles hold
+            if (ctrl->grid.ncells >= kPlainBins) {
+                whole = from0 / kScanTile * kScanTile;
+                for (int j = tid; j < whole / kScanTile; j += kScanThreads)
+                    pre += (unsigned)tileSums[(size_t)j * kTileStride];
+            }
             constexpr int U = 4;  // loads in flight per thread
-            for (int j = 4 * tid; j < from0; j += 4 * U * kScanThreads) {
+            for (int j = whole + 4 * tid; j < from0; j += 4 * U * kScanThreads) {
                 int4 c[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -1870,9 +1880,9 @@ static void nn_launch(const NnWork &w, const State &a, int n, int pred, const Hm
                       double scale, const DtFold &D, hipStream_t s) {
     const int R = redblk(n) < kBoundsBlocks ? redblk(n) : kBoundsBlocks;
     k_bounds<<<R, kBlock, 0, s>>>(w.ctrl, a, n, pred, hc, border, D, w.slots.b, w.members ? w.counts : nullptr,
-                                 (int)w.cap + 1);
+                                 w.tileSums, (int)w.cap + 1);
     k_keys<<<nblk(n), kBlock, 0, s>>>(w.ctrl, a, n, pred, D.on, scale, w.cap, w.slots.b, w.slots.d, D.hist, w.counts,
-                                      w.bin, w.rank, w.binflag, w.members ? nullptr : w.tileSums, w.members, w.room);
+                                      w.bin, w.rank, w.binflag, w.tileSums, w.members, w.room);
     if (w.members) return;  // k_reorder_scan does the rest
     const long long tiles = (w.cap + 1 + kScanTile - 1) / kScanTile;
     k_scan<<<(int)(tiles < 2048 ? tiles : 2048), kBlock, 0, s>>>(w.ctrl, w.counts, w.tileSums, w.cellStart);
@@ -1916,10 +1926,10 @@ static int nn_update(sph_ctx *c, hipStream_t s, int pred = 0, int lean = 0, int 
         k_reorder<<<nblk(n), kBlock, 0, s>>>(c->ctrl, ra, c->perm0);
     else if (n <= kReorderScanMax / 2)
         k_reorder_scan<256><<<kReorderShares + nblk(n, 256), kScanThreads, 0, s>>>(
-            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, sl.b);
+            c->ctrl, ra, c->counts, c->tileSums, c->cellStart, c->bin, c->rank, c->members, sl.b);
     else
         k_reorder_scan<512><<<kReorderShares + nblk(n, 512), kScanThreads, 0, s>>>(
-            c->ctrl, ra, c->counts, c->cellStart, c->bin, c->rank, c->members, sl.b);
+            c->ctrl, ra, c->counts, c->tileSums, c->cellStart, c->bin, c->rank, c->members, sl.b);
     HIPCHK(hipGetLastError());
     if (pred) c->x0_same = false;
     if (!c->P.use_xsph) c->xs_fluid_zero = true;
