@@ -501,7 +501,6 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
     __shared__ double s_v[kBoundsVQ];
     __shared__ Grid s_g;
     __shared__ unsigned s_halt;
-    __shared__ int s_most;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     // loaded together with the control block
@@ -533,9 +532,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         const unsigned halt = derive_grid(s_v, scale, cap, g);
         s_halt = halt;
         s_g = g;
-        s_most = members && !halt ? bin_most(room, g.ncells) : 0;
         if (blockIdx.x == 0) {
-            ctrl->most = s_most;
             if (fold) dt_commit(ctrl, ctrl->nx, hist);
             if (s_v[7] >= 0.0) ctrl->vbound = s_v[7];  // a full scan's velocity bound
             if (halt) {
@@ -570,14 +567,15 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
     int leader, next;
     bin_run(b, id, leader, next);
     int base = 0;
-    if (lane == leader && b >= 0) {
-        base = atomicAdd(&counts[b], next - leader);
-        // A bin filled by more than one run may be out of reference-index
-        // order: flag it with this update's epoch. Every
-        // run but the first to arrive sees base != 0, so such a bin is always
-        // flagged; the store is idempotent, so no atomic is needed.
-        if (base != 0) binflag[b] = epoch;
-    }
+    const bool counts_run = lane == leader && b >= 0;
+    if (counts_run) base = atomicAdd(&counts[b], next - leader);
+    const int most = members ? bin_most(room, g.ncells) : 0;  // formed while the atomics return
+    if (t == 0) ctrl->most = most;
+    // A bin filled by more than one run may be out of reference-index
+    // order: flag it with this update's epoch. Every
+    // run but the first to arrive sees base != 0, so such a bin is always
+    // flagged; the store is idempotent, so no atomic is needed.
+    if (counts_run && base != 0) binflag[b] = epoch;
     // k_reorder_scan reads the tiles' sums of a large grid only
     if (!members || g.ncells >= kPlainBins) tile_add(tiles, b < 0 ? -1 : b / kScanTile);
     base = __shfl(base, leader, 64);
@@ -585,7 +583,7 @@ __global__ void k_keys(Ctrl *ctrl, State a, int n, int pred, int fold, double sc
         const int r = base + (lane - leader);
         bin[t] = b;
         rank[t] = r;
-        if (members && r < s_most) members[(size_t)b * s_most + r] = id;  // for k_reorder_scan
+        if (r < most) members[(size_t)b * most + r] = id;  // for k_reorder_scan
     }
 }
 
@@ -856,11 +854,10 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
     __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
     __shared__ int lds[16], s_lo[SLOTS / 64], s_hi[SLOTS / 64];
     constexpr bool kPacked = SLOTS <= kBlock;  // n < 65,536
-    const int act = ctrl->active, most = ctrl->most, n = A.n, tid = threadIdx.x;
+    const int act = ctrl->active, most = ctrl->most, nbins = (int)ctrl->grid.ncells + 1, n = A.n, tid = threadIdx.x;
     if (blockIdx.x < kReorderShares) {
         if (blockIdx.x == 0 && tid < kBoundsSlots * kBoundsStride) bslots[tid] = 0;  // as k_place
         if (!act) return;
-        const int nbins = (int)ctrl->grid.ncells + 1;
         scan_share(counts, tileSums, cellStart, nbins, blockIdx.x, kReorderShares, lds);
         if (blockIdx.x == 0 && tid == 0) {
             ctrl->nn_valid = 1;
@@ -906,7 +903,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
         unsigned pre = 0;
         {
             int whole = 0;  // bins whose sums the tiles hold
-            if (ctrl->grid.ncells >= kPlainBins) {
+            if (nbins > kPlainBins) {
                 whole = from0 / kScanTile * kScanTile;
                 for (int j = tid; j < whole / kScanTile; j += kScanThreads)
                     pre += (unsigned)tileSums[(size_t)j * kTileStride];
