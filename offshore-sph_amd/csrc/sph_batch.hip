@@ -23,6 +23,7 @@
 // instance evolves exactly as it would alone.
 //
 // Built with -ffp-contract=off (as sph_engine.hip).
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -45,6 +46,13 @@ constexpr int kChunkThreads = 512;
 // particles: 7,500 workgroups took 76 us).
 inline int chunk_slots(long long n) { return n > 2048 * 1024 ? 4096 : 1024; }
 constexpr int kTile = 256;
+// Entries of dt partials (tiles) and bounds partials (chunks) an instance has
+// at most: every workgroup of the next kernel reads all of its instance's, so
+// without a limit that grows with the square of its size. An instance of more
+// shares them by atomic maxima, cleared after their readers. Steps in us without
+// and with a limit (and the scan's workgroups by size): one FP32C instance of 4M
+// particles 764, 558; of 1M 190, 151; 2 of 2M 639, 554; 24 of 30k 127, 127.
+constexpr int kDtEntries = 512, kBoundsEntries = 128;
 static_assert(kTile == 256, "the fused batch pair pass runs one 256-thread workgroup per tile");
 
 struct BState {  // the concatenated cell-ordered state (as State)
@@ -55,31 +63,32 @@ struct BState {  // the concatenated cell-ordered state (as State)
 // per-instance dt (src/Solver.py:210-230, src/Equations/TimeStep.py:40-90)
 // ---------------------------------------------------------------------------
 // segment c (a tile) covers [cs[c], cs[c + 1]) inside one instance
-__global__ void kb_dt_partial(const int *cs, const int *segInst, const BInst *inst, State s, double *part,
-                              Ctrl *view) {
+__global__ void kb_dt_partial(const int *cs, const int *segInst, const int *entry, const BInst *inst, State s,
+                              unsigned long long *part, Ctrl *view) {
     __shared__ double lds[kDtQ * 16];
-    const int c = blockIdx.x, NC = gridDim.x;
+    const int c = blockIdx.x, e = entry[c];
     if (c == 0 && threadIdx.x == 0) view->pec_parts = 0;
     const BInst &I = inst[segInst[c]];
     DtVars v;
     for (int t = cs[c] + threadIdx.x; t < cs[c + 1]; t += blockDim.x)
         if (s.label[t] == kFluid) v.add(I.uh_on ? I.uh : s.h[t], s.ax[t], s.ay[t]);
-    v.store(part, NC, c, lds);
+    v.publish(part, e, lds);
 }
 
-// One workgroup's fold of its instance's dt partials (tiles [t0, t1) of NT);
-// the result is valid in thread 0. lds holds kDtQ * 16 doubles.
-__device__ inline void bdt_fold(const double *part, int NT, int t0, int t1, double (&v)[kDtQ], double *lds) {
+// One workgroup's fold of its instance's dt partials; the result is valid in
+// thread 0. lds holds kDtQ * 16 doubles.
+__device__ inline void bdt_fold(const unsigned long long *part, const BInst &I, double (&v)[kDtQ], double *lds) {
     const int kind[kDtQ] = {0, 1, 2, 2};
     v[0] = INFINITY;
     v[1] = -INFINITY;
     v[2] = v[3] = 0.0;
-    for (int c = t0 + threadIdx.x; c < t1; c += blockDim.x) {
-        const double a = part[0 * NT + c], b = part[1 * NT + c];
-        v[0] = a < v[0] ? a : v[0];
-        v[1] = b > v[1] ? b : v[1];
-        v[2] += part[2 * NT + c];
-        v[3] += part[3 * NT + c];
+    for (int j = threadIdx.x; j < I.dtn; j += blockDim.x) {
+        const ulonglong2 *p = reinterpret_cast<const ulonglong2 *>(part + (size_t)kDtQ * (I.dt0 + j));
+        const ulonglong2 a = p[0], b = p[1];
+        v[0] = -max_of(-v[0], order_value(a.x));
+        v[1] = max_of(v[1], order_value(a.y));
+        v[2] = max_of(v[2], order_value(b.x));
+        v[3] = max_of(v[3], order_value(b.y));
     }
     block_fold<kDtQ>(v, kind, lds);
 }
@@ -117,22 +126,23 @@ __device__ inline void bupd_pos(const BPos &p, bool pred, double dt, double &x, 
 
 // Per chunk (of one instance's slots): the fold of the instance's dt
 // partials and its decision (every workgroup needs dt; the first chunk's
-// leaves it in I.nx for kb_keys), then the bounds' partials of the chunk,
-// part[c * kBoundsVQ + q]. With PEC's predictor the full scan also finds the
+// leaves it in I.nx for kb_keys), then the chunk's bounds into an entry of its
+// instance's partials (kBoundsVQ order keys, as maxima), or one that it shares
+// (~entry). With PEC's predictor the full scan also finds the
 // largest |vx|, |vy| (kb_keys keeps it as the instance's vbound). With
 // cellStart (the fused PEC step) and an instance whose carried bound allows
 // it (as the single engine's k_bounds), the instance's chunks share the walk
 // of its border cells instead.
-__global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const int *chunkInst, const int *chunk0,
-                                                           const int *tile0, BInst *inst, State a, int pec,
-                                                           const double *part_d, int NT, double *part,
+__global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const int *chunkInst, const int *entry,
+                                                           const int *chunk0, BInst *inst, State a, int pec,
+                                                           const unsigned long long *part_d, unsigned long long *part,
                                                            const int *cellStart, Ctrl *view) {
     __shared__ double lds[kBoundsVQ * 16];
     __shared__ double s_dt, s_disp;
     __shared__ int s_active;
     const int c = blockIdx.x;
+    const int k = chunkInst[c], e = entry[c];
     if (c == 0 && threadIdx.x == 0) view->epoch += 1;
-    const int k = chunkInst[c];
     BInst &I = inst[k];
     const bool pred = pec != 0;
     // the first particles of either scan, in flight under the dt fold
@@ -160,7 +170,7 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
     {
         const DtIn in(I, view->pec_parts);
         double v[kDtQ];
-        bdt_fold(part_d, NT, tile0[k], tile0[k + 1], v, lds);
+        bdt_fold(part_d, I, v, lds);
         if (threadIdx.x == 0) {
             const DtNext x = dt_decide(in, v, I.gamma_c, I.gamma_f);
             s_dt = x.dt;
@@ -227,25 +237,34 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
     double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
     __syncthreads();  // lds held the dt fold
     block_fold<kBoundsVQ>(v, kind, lds);
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
+        unsigned long long *p = part + (size_t)kBoundsVQ * (e < 0 ? ~e : e);
+        v[0] = -v[0];  // minima as maxima
+        v[2] = -v[2];
+        v[4] = -v[4];
 #pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q) part[c * kBoundsVQ + q] = v[q];
+        for (int q = 0; q < kBoundsVQ; ++q)
+            if (e >= 0)
+                p[q] = order_key(v[q]);
+            else
+                atomicMax(p + q, order_key(v[q]));
+    }
 }
 
 // _bin :129-141 with the instance's grid; rank by runs as k_keys does. One
-// tile per workgroup, which derives its instance's grid from the chunks'
-// partials itself (32 lanes per quantity); the instance's first tile moves the grid and the dt decision into
+// tile per workgroup, which derives its instance's grid from the bounds'
+// partials itself (32 lanes per quantity) and clears a dt entry that is shared; the instance's first tile moves the grid and the dt decision into
 // its control block, whose fields no workgroup reads here (they take I.nx and
 // their own grid). An instance that is not active is left where it is.
-__global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileInst, const int *tile0,
-                                                 const int *chunk0, BInst *inst, State a, int pec, const double *part,
-                                                 int *counts, int *bin, int *rank, int *binflag, int *tileSums, Ctrl *view) {
+__global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileInst, const int *entry,
+                                                 const int *tile0, BInst *inst, State a, int pec, const unsigned long long *part,
+                                                 unsigned long long *part_d, int *counts, int *bin, int *rank, int *binflag, int *tileSums, Ctrl *view) {
     __shared__ double s_v[kBoundsVQ];
     __shared__ Grid s_g;
     __shared__ unsigned s_halt;
     const int c = blockIdx.x;
     if (c == 0 && threadIdx.x == 0) view->pec_parts = 0;  // kb_bounds has read it
-    const int k = tileInst[c];
+    const int k = tileInst[c], e = entry[c];
     BInst &I = inst[k];
     const bool first = c == tile0[k];
     // loaded together with the instance's control block
@@ -255,6 +274,8 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     const int t0 = in ? t : ts[c];
     const BPos p = bpos_load(a, t0, pec != 0);
     const int id = in ? a.id[t0] : 0x7fffffff;
+    if (e < 0 && ~e == I.dt0 + c - tile0[k] && threadIdx.x < kDtQ)  // its entry's first tile
+        part_d[(size_t)kDtQ * ~e + threadIdx.x] = 0;                // kb_bounds has folded it
     if (!I.nx.active) {
         if (first && threadIdx.x == 0) bdt_commit(I, I.nx);
         return;
@@ -262,18 +283,14 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     const int epoch = view->epoch;
     double x, y;
     bupd_pos(p, pec != 0, I.nx.dt, x, y);
-    {  // 32 lanes per quantity fold the instance's chunks, all as maxima (the count: zero or not)
+    {  // 32 lanes per quantity fold the instance's bounds, all as maxima
         const int q = threadIdx.x >> 5;
-        const bool mn = q == 0 || q == 2 || q == 4;
-        double u = q == 6 ? 0.0 : -INFINITY;
-        for (int j = chunk0[k] + (threadIdx.x & 31); j < chunk0[k + 1]; j += 32) {
-            const double w = part[j * kBoundsVQ + q];
-            u = max_of(u, mn ? -w : w);
-        }
-        double u2 = u;
+        unsigned long long u = 0;
+        for (int j = threadIdx.x & 31; j < I.bn; j += 32) u = max_of(u, part[(size_t)kBoundsVQ * (I.b0 + j) + q]);
+        unsigned long long u2 = u;
         row_swap<16>(u, u2);
         u = group_max<4>(max_of(u, u2));
-        if ((threadIdx.x & 31) == 0) s_v[q] = mn ? -u : u;
+        if ((threadIdx.x & 31) == 0) s_v[q] = q == 0 || q == 2 || q == 4 ? -order_value(u) : order_value(u);
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -321,37 +338,54 @@ __global__ __launch_bounds__(kTile) void kb_keys(const int *ts, const int *tileI
     }
 }
 
-// Each instance's offsets, scanned from its first slot, up to T =
-// scan_tiles(K) tiles at a time: workgroups k T ... k T + T - 1 are instance
-// k's (on the grid's x axis: the others hold 65,535 workgroups, a batch up to
-// 2^20 instances).
-inline int scan_tiles(int K) { return K >= 256 ? 8 : (K >= 64 ? 16 : 64); }
+// Each instance's offsets, scanned from its first slot by scan_groups
+// workgroups, a tile of bins each at a time: those of row blockIdx.y, or, with
+// the tables, wg0[k] ... wg0[k + 1] - 1 of the x axis (the others hold 65,535
+// workgroups, a batch up to 2^20 instances), whose instances wgInst gives.
+// As many as keep the chip busy with few instances, or one for every 2,048
+// slots (about 800 bins of a dam break) of a large one: with 64 whatever
+// its size the scan of one instance of 4M particles took 111 us, now 17.
+constexpr int kScanAlike = 4096;  // most workgroups in rows of as many for each instance
+inline int scan_groups(int K, long long n, long long tiles) {
+    const long long few = K < 2048 ? (K > 32 ? 2048 / K : 64) : 1;
+    return (int)std::min(tiles, std::max(few, n / 2048));
+}
 __global__ __launch_bounds__(kBlock) void kb_scan(const BInst *inst, int *counts, const int *tileSums, int *cellStart,
-                                                  int T) {
+                                                  const int *wgInst, const int *wg0) {
     __shared__ int lds[16];
-    const int k = (int)blockIdx.x / T;
+    int k = (int)blockIdx.y, first = (int)blockIdx.x, w = (int)gridDim.x;
+    if (wgInst) {
+        k = wgInst[first];
+        w = wg0[k + 1] - wg0[k];
+        first -= wg0[k];
+    }
     const BInst &I = inst[k];
     if (!I.active) return;
     const long long nbins = I.grid.ncells + 1;
-    for (long long tile = (int)blockIdx.x - k * T; tile * kScanTile < nbins; tile += T)
+    for (long long tile = first; tile * kScanTile < nbins; tile += w)
         scan_tile(counts + I.cellBase, tileSums + (size_t)I.tileBase * kTileStride, cellStart + I.cellBase, nbins,
                   tile, I.off, lds);
 }
 
 // Each particle's place (k_place); an instance that is not active keeps its
-// order. Also zeroes the instance's tile sums for the next update.
+// order. Also zeroes the instance's tile sums for the next update, and its
+// bounds entries if it shares them, active or not.
 __global__ __launch_bounds__(kTile) void kb_place(const int *ts, const int *tileInst, const int *tile0,
                                                   const BInst *inst, const int *cellStart, const int *bin,
-                                                  const int *rank, int *perm0, int *tileSums) {
+                                                  const int *rank, int *perm0, int *tileSums,
+                                                  unsigned long long *part_b) {
     const int c = blockIdx.x, k = tileInst[c];
     const BInst &I = inst[k];
     const int t = ts[c] + (int)threadIdx.x;
     const bool in = t < ts[c + 1];
-    if (!I.active) {
+    const int active = I.active, shares = I.shares, first = tile0[k];  // one trip to memory
+    if (shares && c == first)
+        for (int j = threadIdx.x; j < kBoundsVQ * I.bn; j += kTile) part_b[(size_t)kBoundsVQ * I.b0 + j] = 0;
+    if (!active) {
         if (in) perm0[t] = t;
         return;
     }
-    const int j = c - tile0[k], nt = tile0[k + 1] - tile0[k];
+    const int j = c - first, nt = tile0[k + 1] - first;
     for (long long q = j * kTile + (int)threadIdx.x; q * kScanTile <= I.grid.ncells; q += (long long)nt * kTile)
         tileSums[(I.tileBase + q) * kTileStride] = 0;
     if (in) perm0[cellStart[bin[t]] + rank[t]] = t;
@@ -447,10 +481,10 @@ __global__ void kb_hm_range(const BInst *inst, State st, double *out) {
 // PEC.correct / Euler (fluid of active instances) + the next dt partials.
 // PEC's start-of-step values come from the buffer before the reorder, at the
 // particle's previous slot perm[j] (the lean reorder did not copy them).
-__global__ void kb_correct(const int *cs, const int *chunkInst, const BInst *inst, State s, State o,
-                           const int *perm, int euler, double *part, Ctrl *view) {
+__global__ void kb_correct(const int *cs, const int *chunkInst, const int *entry, const BInst *inst, State s, State o,
+                           const int *perm, int euler, unsigned long long *part, Ctrl *view) {
     __shared__ double lds[kDtQ * 16];
-    const int c = blockIdx.x, NC = gridDim.x;
+    const int c = blockIdx.x, e = entry[c];
     if (c == 0 && threadIdx.x == 0) view->pec_parts = 0;
     const BInst &I = inst[chunkInst[c]];
     const double dt = I.dt, damping = I.damping;
@@ -486,7 +520,7 @@ __global__ void kb_correct(const int *cs, const int *chunkInst, const BInst *ins
             s.rho[j] = s.rho[j] + dt * s.drho[j];
         }
     }
-    v.store(part, NC, c, lds);
+    v.publish(part, e, lds);
 }
 
 __global__ void kb_upload(State d, sph_state_t in, int n) {
@@ -555,10 +589,14 @@ struct sph_batch {
     int *instOf = nullptr, *cs = nullptr, *chunkInst = nullptr, *chunk0 = nullptr;
     int NT = 0;  // tiles: starts ts (NT + 1), instance of each, first tile of each instance (K + 1)
     int *ts = nullptr, *tileInst = nullptr, *tile0 = nullptr;
+    dim3 scan;  // the scan's workgroups: a row for each instance, or by the tables
+    int *wgInst = nullptr, *wg0 = nullptr;
     int *bin = nullptr, *rank = nullptr, *perm0 = nullptr, *perm = nullptr;
     int2 *cxy_s = nullptr;
     int *counts = nullptr, *cellStart = nullptr, *binflag = nullptr, *tileSums = nullptr;
-    double *part_b = nullptr, *part_d = nullptr;
+    unsigned long long *part_b = nullptr, *part_d = nullptr;  // bounds and dt partials
+    int *bEntry = nullptr, *dtEntry = nullptr;  // of each chunk and tile (~: shared)
+    size_t part_d_bytes = 0;
     void *recA = nullptr, *recB = nullptr;
     long long capBins = 0;
     bool dt_fresh = false;
@@ -591,7 +629,7 @@ void free_batch(sph_batch *b) {
         if (b->arena[k]) hipFree(b->arena[k]);
     }
     void *ptrs[] = {b->inst, b->view, b->instOf, b->cs, b->chunkInst, b->chunk0, b->ts, b->tileInst, b->tile0,
-                    b->bin, b->rank, b->perm,
+                    b->wgInst, b->wg0, b->bEntry, b->dtEntry, b->bin, b->rank, b->perm,
                     b->perm0, b->cxy_s, b->counts, b->cellStart, b->binflag, b->tileSums,
                     b->part_b, b->part_d, b->recA, b->recB, b->queue, b->uniK, b->hm};
     for (void *p : ptrs)
@@ -617,18 +655,16 @@ int b_nn(sph_batch *b, hipStream_t s) {
     const int pec = b->integrator == SPH_INTEGRATOR_PEC;
     State a = b->buf[b->cur], c = b->buf[1 - b->cur];
     if (!b->dt_fresh)
-        kb_dt_partial<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->inst, a, b->part_d, b->view);
+        kb_dt_partial<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->dtEntry, b->inst, a, b->part_d, b->view);
     // the border-cell bounds only in the fused PEC step's update
     const bool fused = b->uni && !b->persistent && pec;
-    kb_bounds<<<b->NC, kChunkThreads, 0, s>>>(b->cs, b->chunkInst, b->chunk0, b->tile0, b->inst, a, pec, b->part_d,
-                                              b->NT, b->part_b, fused && b->border_bounds ? b->cellStart : nullptr,
-                                              b->view);
-    kb_keys<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->chunk0, b->inst, a, pec, b->part_b, b->counts,
-                                    b->bin, b->rank, b->binflag, b->tileSums, b->view);
-    const int T = scan_tiles(b->K);
-    kb_scan<<<b->K * T, kBlock, 0, s>>>(b->inst, b->counts, b->tileSums, b->cellStart, T);
+    kb_bounds<<<b->NC, kChunkThreads, 0, s>>>(b->cs, b->chunkInst, b->bEntry, b->chunk0, b->inst, a, pec, b->part_d,
+                                              b->part_b, fused && b->border_bounds ? b->cellStart : nullptr, b->view);
+    kb_keys<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->dtEntry, b->tile0, b->inst, a, pec, b->part_b, b->part_d,
+                                    b->counts, b->bin, b->rank, b->binflag, b->tileSums, b->view);
+    kb_scan<<<b->scan, kBlock, 0, s>>>(b->inst, b->counts, b->tileSums, b->cellStart, b->wgInst, b->wg0);
     kb_place<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->tile0, b->inst, b->cellStart, b->bin, b->rank, b->perm0,
-                                     b->tileSums);
+                                     b->tileSums, b->part_b);
     const int fmt = b->precision == SPH_PREC_FP32C ? (b->uni ? kRecUniform : kRecFp32)
                                                    : (b->uni ? kRecUniform64 : kRecFp64);
     kb_reorder<<<b->NT, kTile, 0, s>>>(b->ts, b->tileInst, b->inst, a, c, b->perm0, b->perm, b->cellStart, b->binflag,
@@ -675,7 +711,8 @@ int b_pair_pec(sph_batch *b, hipStream_t s) {
     State st = b->buf[b->cur];
     PairIn in{b->recA, b->recB, st.h, b->cxy_s, b->cellStart};
     PairOut out{st.ax, st.ay, st.drho, nullptr, 0};
-    const PecArgs pec{st, b->buf[1 - b->cur], b->perm, b->part_d, nullptr, HmConst{}, 0, &b->view->pec_parts};
+    const PecArgs pec{st, b->buf[1 - b->cur], b->perm, b->part_d, nullptr, HmConst{}, 0, b->dtEntry,
+                      &b->view->pec_parts};
     hipError_t e = b->precision == SPH_PREC_FP32C
                        ? launch_pair_batch_fp32u_pec(b->inst, b->ts, b->tileInst, b->NT, in, out, b->uniK, b->kernel,
                                                      b->n, b->whole, pec, s)
@@ -694,7 +731,7 @@ int b_step(sph_batch *b, hipStream_t s) {
         if ((rc = b_pair_pec(b, s))) return rc;
     } else {
         if ((rc = b_pair(b, s))) return rc;
-        kb_correct<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->inst, b->buf[b->cur], b->buf[1 - b->cur],
+        kb_correct<<<b->NT, kBlock, 0, s>>>(b->ts, b->tileInst, b->dtEntry, b->inst, b->buf[b->cur], b->buf[1 - b->cur],
                                             b->perm, b->integrator == SPH_INTEGRATOR_EULER, b->part_d, b->view);
         HIPCHK(hipGetLastError());
     }
@@ -748,14 +785,16 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     b->capBins = capTot;
     const size_t n = (size_t)ntot;
     // chunk and tile tables
-    std::vector<int> cs, chunkInst, chunk0, ts, tileInst, tile0;
+    std::vector<int> cs, chunkInst, chunk0, ts, tileInst, tile0, dtEntry, bEntry;
+    size_t ND = 0, NB = 0;  // entries of dt and of bounds partials
     std::vector<BInst> hI(ninst);
     const int chunk = chunk_slots(ntot);
     long long off = 0, base = 0;
     int tbase = 0;
     for (int k = 0; k < ninst; ++k) {
         const sph_params_t &P = params[k];
-        chunk0.push_back((int)cs.size());
+        const int c0 = (int)cs.size();
+        chunk0.push_back(c0);
         for (long long c = 0; c < P.n; c += chunk) {
             cs.push_back((int)(off + c));
             chunkInst.push_back(k);
@@ -767,6 +806,16 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
         }
         BInst &I = hI[k];
         std::memset(&I, 0, sizeof I);
+        const int nt = (int)ts.size() - tile0.back(), nc = (int)cs.size() - c0;
+        I.dt0 = (int)ND;
+        I.dtn = std::min(nt, kDtEntries);
+        for (int j = 0; j < nt; ++j) dtEntry.push_back(nt <= kDtEntries ? I.dt0 + j : ~(I.dt0 + j % kDtEntries));
+        ND += I.dtn;
+        I.b0 = (int)NB;
+        I.bn = std::min(nc, kBoundsEntries);
+        I.shares = nc > kBoundsEntries;
+        for (int j = 0; j < nc; ++j) bEntry.push_back(nc <= kBoundsEntries ? I.b0 + j : ~(I.b0 + j % kBoundsEntries));
+        NB += I.bn;
         I.disp = I.vbound = I.abound = INFINITY;
         I.off = (int)off;
         I.n = (int)P.n;
@@ -809,6 +858,21 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
     ts.push_back((int)off);
     tile0.push_back((int)tileInst.size());
     b->NT = (int)tileInst.size();
+    // the scan's workgroups: as many for each instance where that is few enough
+    std::vector<int> wg0{0}, wgInst;
+    int most = 1;
+    for (int k = 0; k < ninst; ++k) {
+        const int w = scan_groups(ninst, hI[k].n, tile_room(hI[k].cap));
+        most = std::max(most, w);
+        wg0.push_back(wg0.back() + w);
+    }
+    if ((long long)most * ninst <= kScanAlike) {
+        b->scan = dim3(most, ninst);
+    } else {
+        b->scan = dim3(wg0.back());
+        wgInst.resize(wg0.back());
+        for (int k = 0; k < ninst; ++k) std::fill(wgInst.begin() + wg0[k], wgInst.begin() + wg0[k + 1], k);
+    }
     std::vector<int> instOf(n);
     for (int k = 0; k < ninst; ++k)
         for (int i = b->offs[k]; i < b->offs[k + 1]; ++i) instOf[i] = k;
@@ -837,6 +901,8 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
                       sizeof(Rec<double>::B) >= sizeof(double4) && sizeof(float4) >= sizeof(Rec<float>::B),
                   "record buffers hold every format");
     const size_t uk = b->precision == SPH_PREC_FP32C ? uniform_const_size_fp32() : uniform_const_size_fp64();
+    const size_t part_b_bytes = sizeof(unsigned long long) * kBoundsVQ * NB;
+    b->part_d_bytes = sizeof(unsigned long long) * kDtQ * ND;
     ok = ok && hipMalloc(&b->inst, sizeof(BInst) * ninst) == hipSuccess &&
          hipMalloc(&b->view, sizeof(Ctrl)) == hipSuccess && hipMalloc(&b->instOf, sizeof(int) * n) == hipSuccess &&
          hipMalloc(&b->cs, sizeof(int) * cs.size()) == hipSuccess &&
@@ -845,6 +911,8 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMalloc(&b->ts, sizeof(int) * ts.size()) == hipSuccess &&
          hipMalloc(&b->tileInst, sizeof(int) * tileInst.size()) == hipSuccess &&
          hipMalloc(&b->tile0, sizeof(int) * tile0.size()) == hipSuccess &&
+         hipMalloc(&b->wg0, sizeof(int) * wg0.size()) == hipSuccess &&
+         (wgInst.empty() || hipMalloc(&b->wgInst, sizeof(int) * wgInst.size()) == hipSuccess) &&
          hipMalloc(&b->bin, sizeof(int) * n) == hipSuccess && hipMalloc(&b->rank, sizeof(int) * n) == hipSuccess &&
          hipMalloc(&b->perm, sizeof(int) * n) == hipSuccess && hipMalloc(&b->perm0, sizeof(int) * n) == hipSuccess &&
          hipMalloc(&b->cxy_s, sizeof(int2) * n) == hipSuccess &&
@@ -853,8 +921,11 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMalloc(&b->binflag, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMalloc(&b->tileSums, sizeof(int) * kTileStride * tiles) == hipSuccess &&
          hipMemset(b->tileSums, 0, sizeof(int) * kTileStride * tiles) == hipSuccess &&
-         hipMalloc(&b->part_b, sizeof(double) * kBoundsVQ * b->NC) == hipSuccess &&
-         hipMalloc(&b->part_d, sizeof(double) * kDtQ * b->NT) == hipSuccess &&
+         hipMalloc(&b->part_b, part_b_bytes) == hipSuccess &&
+         hipMalloc(&b->part_d, b->part_d_bytes) == hipSuccess &&
+         hipMalloc(&b->bEntry, sizeof(int) * bEntry.size()) == hipSuccess &&
+         hipMalloc(&b->dtEntry, sizeof(int) * dtEntry.size()) == hipSuccess &&
+         hipMemset(b->part_b, 0, part_b_bytes) == hipSuccess &&
          hipMalloc(&b->recA, ra * n) == hipSuccess && hipMalloc(&b->recB, rb * n) == hipSuccess &&
          hipMalloc(&b->queue, sizeof(int) * kQueueInts) == hipSuccess &&
          hipMalloc(&b->uniK, uk * ninst) == hipSuccess && hipMalloc(&b->hm, sizeof(double) * 4 * ninst) == hipSuccess;
@@ -876,6 +947,11 @@ int sph_batch_create(const sph_params_t *params, int32_t ninst, sph_batch_t **ou
          hipMemcpy(b->tileInst, tileInst.data(), sizeof(int) * tileInst.size(), hipMemcpyHostToDevice) ==
              hipSuccess &&
          hipMemcpy(b->tile0, tile0.data(), sizeof(int) * tile0.size(), hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(b->bEntry, bEntry.data(), sizeof(int) * bEntry.size(), hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(b->dtEntry, dtEntry.data(), sizeof(int) * dtEntry.size(), hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(b->wg0, wg0.data(), sizeof(int) * wg0.size(), hipMemcpyHostToDevice) == hipSuccess &&
+         (wgInst.empty() ||
+          hipMemcpy(b->wgInst, wgInst.data(), sizeof(int) * wgInst.size(), hipMemcpyHostToDevice) == hipSuccess) &&
          hipMemset(b->counts, 0, sizeof(int) * (capTot + 1)) == hipSuccess &&
          hipMemset(b->cellStart, 0, sizeof(int) * (capTot + 2)) == hipSuccess &&
          hipMemset(b->binflag, 0, sizeof(int) * (capTot + 1)) == hipSuccess &&
@@ -905,6 +981,8 @@ int sph_batch_upload(sph_batch_t *b, const sph_state_t *st, void *stream) {
     hipStream_t s = (hipStream_t)stream;
     b->cur = 0;
     b->dt_fresh = false;
+    // the last state's partials, which shared entries would keep
+    HIPCHK(hipMemsetAsync(b->part_d, 0, b->part_d_bytes, s));
     kb_upload<<<nblk_b(b->n), kBlock, 0, s>>>(b->buf[0], *st, b->n);
     HIPCHK(hipGetLastError());
     b->loaded = true;

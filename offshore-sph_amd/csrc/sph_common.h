@@ -315,6 +315,22 @@ struct DtVars {
         block_partials<kDtQ>(v, kind, lds, part, R, k);
     }
     __device__ void publish(double *part, double *lds) { store(part, gridDim.x, blockIdx.x, lds); }
+    // a batch tile's, into entry e of its instance's (kDtQ order keys, the
+    // minimum as a maximum), or into ~e, which other tiles share
+    __device__ void publish(unsigned long long *part, int e, double *lds) {
+        const int kind[kDtQ] = {0, 1, 2, 2};
+        double v[kDtQ] = {mn, mx, cnt, bad};
+        block_fold<kDtQ>(v, kind, lds);
+        if (threadIdx.x != 0) return;
+        v[0] = -v[0];
+        unsigned long long *p = part + (size_t)kDtQ * (e < 0 ? ~e : e);
+#pragma unroll
+        for (int q = 0; q < kDtQ; ++q)
+            if (e >= 0)
+                p[q] = order_key(v[q]);
+            else
+                atomicMax(p + q, order_key(v[q]));
+    }
     // into the dt slots (one h for every particle: min h is not folded).
     // |a|^2 >= 0 orders as its bits. lds holds 4 * 16 doubles.
     __device__ void publish_slots(unsigned long long *d, double *lds) {

@@ -143,15 +143,15 @@ struct HmConst {
 // PEC's corrector fused into the uniform pair passes (a step whose reorder
 // ran lean): slot j of s (this step's cell order) came from slot perm[j] of
 // o (the start-of-step buffer), which holds the start-of-step state and the
-// previous rates; the next dt's partials go to part (kDtQ per workgroup) or
-// the dt slots.
+// previous rates; the next dt's partials go to part or the dt slots.
 struct PecArgs {
     State s, o;
     const int *perm;
-    double *part;                      // the batch: one partial per tile
+    unsigned long long *part;              // the batch: its instances' dt partials (DtVars::publish)
     unsigned long long *dslots = nullptr;  // the single engine: the dt slots
     HmConst hc;
     int strict;
+    const int *entry = nullptr;  // the batch: each tile's entry in part
     int *mark = nullptr;  // when set, the pass stores 1 there (its partials come from a corrector that moved the fluid)
 };
 
@@ -307,7 +307,7 @@ hipError_t launch_pair_batch_fp64u(const BInst *inst, const int *instOf, PairIn 
 // The batch's uniform passes with PEC's corrector and the dt partials
 // fused in: one 256-thread workgroup per chunk of one instance (slots
 // cs[c] .. cs[c + 1], c < NC, at most 256 each; chunkInst: the chunk's
-// instance); the partials go to pec.part[q * NC + c] (pec.strict is unused:
+// instance); the partials go to the instance's in pec.part (pec.strict is unused:
 // each instance's own). whole: every instance's wall force exponents are
 // whole numbers (whole_exponent).
 hipError_t launch_pair_batch_fp32u_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC, PairIn in,
@@ -336,6 +336,8 @@ struct BInst {
     long long cellBase;
     int tileBase;  // the first of its bins' scan tiles
     int off, n;
+    int dt0, dtn, b0, bn;  // the first and the number of its entries of dt and of bounds partials
+    int shares;            // whether its chunks share bounds entries
     int advance_t;
     int nfluid;
     long long cap;  // most cells this instance's grid may have

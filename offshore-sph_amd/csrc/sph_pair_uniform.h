@@ -562,8 +562,8 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_queue(const BInst *i
 // The batched ensemble with PEC's corrector and the dt partials fused in:
 // one workgroup per chunk (slots cs[c] .. cs[c + 1], at most 256 of one
 // instance), so the instance's grid, constants and integrator fields are the
-// same for the whole workgroup. The chunk's dt partials go to
-// C.part[q * NC + c], where the batch's corrector stores them. An instance
+// same for the whole workgroup. The chunk's dt partials go to its instance's
+// in C.part, where the batch's corrector puts them. An instance
 // that is not active keeps its state; its fluid still enters the partials.
 // The tile's walk is staged in LDS as the single-simulation pass's (one
 // instance per tile: its grid and bins).
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_pec(const BInst *ins
     __shared__ int s_red[6 * 4];
     const int c = xcd_remap(blockIdx.x, gridDim.x);
     if (c >= NC) return;  // the whole workgroup
-    const int k = chunkInst[c];
+    const int k = chunkInst[c], entry = C.entry[c];
     const BInst &I = inst[k];
     const Grid &g = I.grid;
     const int ncx = (int)g.ncx, ncy = (int)g.ncy;
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform_pec(const BInst *ins
             v.add(I.uh_on ? I.uh : C.s.h[t], ax, ay);
         }
     }
-    v.store(C.part, NC, c, lds);
+    v.publish(C.part, entry, lds);
     if (c == 0 && threadIdx.x == 0 && C.mark) *C.mark = 1;
 }
 

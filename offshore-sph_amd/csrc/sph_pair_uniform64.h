@@ -639,8 +639,8 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_queue(const BInst 
 // The batched ensemble with PEC's corrector and the dt partials fused in:
 // one workgroup per chunk (slots cs[c] .. cs[c + 1], at most 256 of one
 // instance), so the instance's grid, constants and integrator fields are the
-// same for the whole workgroup. The chunk's dt partials go to
-// C.part[q * NC + c], where the batch's corrector stores them. An instance
+// same for the whole workgroup. The chunk's dt partials go to its instance's
+// in C.part, where the batch's corrector puts them. An instance
 // that is not active keeps its state; its fluid still enters the partials.
 template <int KERNEL, int MODE>
 __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *inst, const int *cs, const int *chunkInst, int NC,
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *i
     __shared__ double lds[kDtQ * 16];
     const int c = xcd_remap(blockIdx.x, gridDim.x);
     if (c >= NC) return;  // the whole workgroup
-    const int k = chunkInst[c];
+    const int k = chunkInst[c], entry = C.entry[c];
     const BInst &I = inst[k];
     DtVars v;
     const int t = cs[c] + (int)threadIdx.x;
@@ -685,7 +685,7 @@ __global__ __launch_bounds__(256) void k_pair_batch_uniform64_pec(const BInst *i
             v.add(I.uh_on ? I.uh : C.s.h[t], ax, ay);
         }
     }
-    v.store(C.part, NC, c, lds);
+    v.publish(C.part, entry, lds);
     if (c == 0 && threadIdx.x == 0 && C.mark) *C.mark = 1;
 }
 
