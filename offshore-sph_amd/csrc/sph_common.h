@@ -46,14 +46,6 @@ __device__ inline T block_reduce(T v, Op op, T *lds) {
     return v;  // valid in wave 0
 }
 
-struct MinOp {
-    __device__ static double identity() { return INFINITY; }
-    __device__ double operator()(double a, double b) const { return b < a ? b : a; }
-};
-struct MaxOp {
-    __device__ static double identity() { return -INFINITY; }
-    __device__ double operator()(double a, double b) const { return b > a ? b : a; }
-};
 struct AddOp {
     __device__ static double identity() { return 0.0; }
     __device__ double operator()(double a, double b) const { return a + b; }
@@ -119,15 +111,19 @@ __device__ inline T lane_value(T x, int lane) {  // of a lane that is the same f
 }
 // Of the lane before (lane 0: its own).
 __device__ inline int lane_before(int x) { return __builtin_amdgcn_update_dpp(x, x, 0x138, 0xf, 0xf, false); }
-// The sum over the lanes up to this one.
-__device__ inline int wave_scan(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // within the rows
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // a row's last lane into the next row
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // the lower half's into the upper
-    return x;
+// The sum over the lanes up to this one; unsigned, since two sums packed into
+// one word use its top bit.
+template <int CTRL, int ROWS>
+__device__ inline unsigned scan_step(unsigned x) {
+    return x + (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ inline unsigned wave_scan(unsigned x) {
+    x = scan_step<0x111, 0xf>(x);  // within the rows
+    x = scan_step<0x112, 0xf>(x);
+    x = scan_step<0x114, 0xf>(x);
+    x = scan_step<0x118, 0xf>(x);
+    x = scan_step<0x142, 0xa>(x);  // a row's last lane into the next row
+    return scan_step<0x143, 0xc>(x);  // the lower half's into the upper
 }
 
 // f over the values of all lanes, in all of them: the pairs of an xor tree of
@@ -509,21 +505,27 @@ __device__ inline void tile_add(int *tileSums, int tile) {
     __syncthreads();
     if (threadIdx.x == 0) atomicAdd(&tileSums[(size_t)s_tile * kTileStride], s_sum);
 }
-__device__ inline int block_scan_excl(int v, int *lds, int *total) {
+__device__ inline unsigned block_scan_excl(unsigned v, unsigned *lds, unsigned *total) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int s = wave_scan(v);
+    const unsigned s = wave_scan(v);
     if (lane == 63) lds[w] = s;
     __syncthreads();
     int nw = blockDim.x >> 6;
-    int off = 0, tot = 0;
+    unsigned off = 0, tot = 0;
     for (int k = 0; k < nw; ++k) {
-        int ws = lds[k];
+        const unsigned ws = lds[k];
         if (k < w) off += ws;
         tot += ws;
     }
     __syncthreads();
     *total = tot;
     return off + s - v;
+}
+__device__ inline int block_scan_excl(int v, int *lds, int *total) {
+    unsigned tot;
+    const unsigned ex = block_scan_excl((unsigned)v, reinterpret_cast<unsigned *>(lds), &tot);
+    *total = (int)tot;
+    return (int)ex;
 }
 
 // Tile `tile` of the scan of nbins counts, from `first` on (workgroups of
@@ -573,17 +575,17 @@ __global__ __launch_bounds__(kBlock) void k_scan(const Ctrl *ctrl, int *counts, 
 // tiles' sums, and scans its share, four bins per thread. lds holds 16 ints.
 constexpr int kPlainBins = 1 << 17;
 __device__ inline void scan_share(const int *counts, const int *tileSums, int *cellStart, int nbins, int i, int S,
-                                  int *lds) {
+                                  unsigned *lds) {
     const bool tiles = nbins > kPlainBins;
     const int unit = tiles ? kScanTile : 4;
     const int share = ((nbins + S - 1) / S + unit - 1) / unit * unit;
     const long long at = (long long)i * share;
     if (at >= nbins) return;
     const int b0 = (int)at, b1 = nbins - b0 > share ? b0 + share : nbins;
-    int pre = 0;
+    unsigned pre = 0;
     const int step = 4 * (int)blockDim.x;
     if (tiles) {
-        for (int j = threadIdx.x; j < b0 / kScanTile; j += blockDim.x) pre += tileSums[(size_t)j * kTileStride];
+        for (int j = threadIdx.x; j < b0 / kScanTile; j += blockDim.x) pre += (unsigned)tileSums[(size_t)j * kTileStride];
     } else {
         constexpr int U = 8;  // loads in flight per thread
         for (int j = 4 * (int)threadIdx.x; j < b0; j += U * step) {  // b0 is a multiple of 4
@@ -593,17 +595,17 @@ __device__ inline void scan_share(const int *counts, const int *tileSums, int *c
                 c[u] = j + u * step < b0 ? *reinterpret_cast<const int4 *>(counts + j + u * step)
                                          : make_int4(0, 0, 0, 0);
 #pragma unroll
-            for (int u = 0; u < U; ++u) pre += c[u].x + c[u].y + c[u].z + c[u].w;
+            for (int u = 0; u < U; ++u) pre += (unsigned)(c[u].x + c[u].y + c[u].z + c[u].w);
         }
     }
-    int run, tot;
+    unsigned run, tot;
     block_scan_excl(pre, lds, &run);  // run: the sum before the share
     for (int b = b0; b < b1; b += step) {
         const int k = b + 4 * (int)threadIdx.x;
         int v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) v[u] = k + u < b1 ? counts[k + u] : 0;
-        int ex = block_scan_excl(v[0] + v[1] + v[2] + v[3], lds, &tot) + run;
+        int ex = (int)(block_scan_excl((unsigned)(v[0] + v[1] + v[2] + v[3]), lds, &tot) + run);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if (k + u < b1) cellStart[k + u] = ex;

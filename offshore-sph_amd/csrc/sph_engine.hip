@@ -852,7 +852,8 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
                                                                const int *members,
                                                                unsigned long long *bslots) {
     __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
-    __shared__ int lds[16], s_lo[SLOTS / 64], s_hi[SLOTS / 64];
+    __shared__ unsigned lds[16];
+    __shared__ int s_lo[SLOTS / 64], s_hi[SLOTS / 64];
     constexpr bool kPacked = SLOTS <= kBlock;  // n < 65,536
     const int act = ctrl->active, most = ctrl->most, nbins = (int)ctrl->grid.ncells + 1, n = A.n, tid = threadIdx.x;
     if (blockIdx.x < kReorderShares) {
@@ -933,19 +934,20 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
                 c[u] = u < rows && j < m ? *reinterpret_cast<const int4 *>(counts + from + j) : make_int4(0, 0, 0, 0);
                 sum += (unsigned)(c[u].x + c[u].y + c[u].z + c[u].w);
             }
-            int tot, ex;
+            unsigned tot;
+            int ex;
             if (kPacked) {  // the stretch's sum below, that of the counts before it above
-                const unsigned both = (unsigned)block_scan_excl((int)(sum | pre << 16), lds, &tot);
-                run += (int)((unsigned)tot >> 16);
+                const unsigned both = block_scan_excl(sum | pre << 16, lds, &tot);
+                run += (int)(tot >> 16);
                 ex = run + (int)(both & 0xffff);
-                run += (int)((unsigned)tot & 0xffff);
+                run += (int)(tot & 0xffff);
             } else {
                 if (from == from0) {
-                    block_scan_excl((int)pre, lds, &tot);
-                    run += tot;
+                    block_scan_excl(pre, lds, &tot);
+                    run += (int)tot;
                 }
-                ex = run + block_scan_excl((int)sum, lds, &tot);
-                run += tot;
+                ex = run + (int)block_scan_excl(sum, lds, &tot);
+                run += (int)tot;
             }
             pre = 0;
 #pragma unroll
