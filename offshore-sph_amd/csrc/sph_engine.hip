@@ -1711,9 +1711,11 @@ int sph_ctx_create(const sph_params_t *params, sph_ctx_t **out) {
     h.advance_t = 1;
     h.active = 1;
     h.disp = h.vbound = h.abound = INFINITY;
-    if (hipMemcpy(c->ctrl, &h, sizeof h, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(c->dt_hist, 0, sizeof(double) * 3 * SPH_DT_HISTORY) != hipSuccess ||
-        hipMemset(c->slots, 0, sizeof(unsigned long long) * kSlotWords) != hipSuccess) {
+    // the fills, then a copy that waits for them: a caller's stream may not
+    // wait for the null stream
+    if (hipMemset(c->dt_hist, 0, sizeof(double) * 3 * SPH_DT_HISTORY) != hipSuccess ||
+        hipMemset(c->slots, 0, sizeof(unsigned long long) * kSlotWords) != hipSuccess ||
+        hipMemcpy(c->ctrl, &h, sizeof h, hipMemcpyHostToDevice) != hipSuccess) {
         free_ctx(c);
         return fail(SPH_EHIP, "control block init failed");
     }
