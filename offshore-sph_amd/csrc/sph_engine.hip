@@ -759,7 +759,8 @@ __global__ void k_reorder(Ctrl *ctrl, ReorderArgs A, const int *perm0) {
 // of smaller indices in the bin (k_keys has listed the bin's first `most`;
 // crowded_ranks counts in a bin of more). The first kReorderShares workgroups
 // write cellStart (scan_share); each of the others scans the bins of its
-// SLOTS slots for itself and sums the counts before them, with 1,024 threads of
+// SLOTS slots for itself and sums the counts before them (above kPlainBins bins the
+// tiles' sums: 107k particles on 0.88M cells, an update 66 -> 44 us), with 1,024 threads of
 // which SLOTS carry a slot. Launches, drains and dependent trips to memory are
 // what a small state's update costs: every load is issued in one of two
 // rounds, the bins and states, then the counts and members. Steps in us, with
@@ -1738,8 +1739,7 @@ int sph_ctx_set_params(sph_ctx_t *ctx, const sph_params_t *params) {
     int rc = check_params(params);
     if (rc) return rc;
     // The control block is rewritten whole: steps still in flight on any
-    // stream (the caller's, or the context's own graph stream, which the
-    // null stream does not wait for) must finish first.
+    // stream (which the null stream may not wait for) must finish first.
     HIPCHK(hipDeviceSynchronize());
     ctx->P = *params;
     ctx->dt_fresh = false;

@@ -28,8 +28,8 @@ constexpr int kFluid = 0;
 constexpr int kCoupled = 3;
 constexpr int kBlock = 256;        // threads per block of streaming kernels
 // bins per thread in the cell scan (tiles of 1,024 bins: 438 tiles on the
-// 1M dam break's 447k cells; against 2,048-bin tiles the apply kernel takes
-// 5.13 us instead of 5.85 and the step 1.5 us less; 512 no better)
+// 1M dam break's 447k cells; with tiles of 2,048 the step took 1.5 us more; 512
+// no better)
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kBlock * kScanItems;
 constexpr int kRedBlocks = 2048;   // max workgroups of a grid-wide reduction
@@ -383,8 +383,7 @@ hipError_t launch_pair_batch_fp64(const BInst *inst, const int *instOf, PairIn i
                                   int threads, int list, int *queue, int grid, hipStream_t s);
 hipError_t launch_pair_batch_fp32c(const BInst *inst, const int *instOf, PairIn in, PairOut out, int kernel, int n,
                                    int threads, int list, int *queue, int grid, hipStream_t s);
-// Resident workgroups per CU of the persistent form (not to be called under
-// stream capture).
+// Resident workgroups per CU of the persistent form.
 int pair_batch_queue_occupancy_fp64(int kernel, int list, int threads);
 int pair_batch_queue_occupancy_fp32c(int kernel, int list, int threads);
 

@@ -770,8 +770,8 @@ __global__ __launch_bounds__(kPairThreads) void k_pair_batch(const BInst *inst, 
 // dispatcher hands to an XCD (blockIdx % 8) take from that XCD's counter, so
 // neighbouring tiles still share an L2. Every workgroup ends once its
 // counter has passed the end of its range; none waits for another. The last
-// workgroup out (a separate counter) clears all counters, so the next launch,
-// graph replays included, starts from zero without a memset. Each target's
+// workgroup out (a separate counter) clears all counters, so the next launch
+// starts from zero without a memset. Each target's
 // sums do not depend on which workgroup runs it: results are those of
 // k_pair_batch bit for bit.
 template <typename R, int KERNEL, bool EXACT, int LIST>
@@ -831,7 +831,7 @@ void launch_batch_list(const BInst *inst, const int *instOf, const PairArgs<R> &
 }
 
 // Resident workgroups per CU of the persistent batch pass (hipOccupancy), for
-// sizing its grid outside any stream capture.
+// sizing its grid.
 template <typename R, int KERNEL, bool EXACT>
 int queue_occupancy_list(int list, int threads) {
     if (list == 0) list = list_len<R, KERNEL>();

@@ -31,7 +31,7 @@ namespace hipsph {
 namespace {
 
 #ifndef HIPSPH_PEC64_EARLY
-#define HIPSPH_PEC64_EARLY 0  // 1: the corrector's gathers before the walk (97 VGPRs instead of 83, 4 waves: no faster)
+#define HIPSPH_PEC64_EARLY 0  // 1: the corrector's gathers before the walk (99 VGPRs instead of 85, 4 waves: no faster)
 #endif
 
 #ifndef HIPSPH_UNIFORM64_UNROLL
