@@ -854,7 +854,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
                                                                unsigned long long *bslots) {
     __shared__ __attribute__((aligned(16))) int s_start[kScanBins];
     __shared__ unsigned lds[16];
-    __shared__ int s_lo[SLOTS / 64], s_hi[SLOTS / 64];
+    __shared__ int s_lo[SLOTS / 64], s_hi[SLOTS / 64], s_crowded;
     constexpr bool kPacked = SLOTS <= kBlock;  // n < 65,536
     const int act = ctrl->active, most = ctrl->most, nbins = (int)ctrl->grid.ncells + 1, n = A.n, tid = threadIdx.x;
     if (blockIdx.x < kReorderShares) {
@@ -878,6 +878,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
         p = reorder_load(ctrl, A, act, s);
     }
     if (act) {
+        if (tid == 0) s_crowded = 0;
         if (tid < SLOTS) {
             const int lo = -wave_max(live ? -key : -0x7fffffff), hi = wave_max(live ? key : -1);
             if ((tid & 63) == 0) {
@@ -964,6 +965,7 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
             if (live && k >= 0 && k < m) {
                 begin = s_start[k];
                 end = k + 1 < m ? s_start[k + 1] : run;
+                if (flagged && end - begin > most) s_crowded = 1;
             }
             __syncthreads();
         }
@@ -986,8 +988,8 @@ __global__ __launch_bounds__(kScanThreads) void k_reorder_scan(Ctrl *ctrl, Reord
                     r += j + 3 < cnt && c.w < p.id;
                 }
         }
-        const bool crowded = flagged && cnt > most;
-        if (__syncthreads_or(crowded)) {
+        if (s_crowded) {  // set before the last barrier, so no vote of its own
+            const bool crowded = flagged && cnt > most;
             const int rc = crowded_ranks<SLOTS>(crowded ? key : -1, p.id, n, bin, A.a.id, s_start);
             if (crowded) r = rc;
         }
