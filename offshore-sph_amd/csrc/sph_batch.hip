@@ -51,7 +51,7 @@ constexpr int kTile = 256;
 // without a limit that grows with the square of its size. An instance of more
 // shares them by atomic maxima, cleared after their readers. Steps in us without
 // and with a limit (and the scan's workgroups by size): one FP32C instance of 4M
-// particles 764, 558; of 1M 190, 151; 2 of 2M 639, 554; 24 of 30k 127, 127.
+// particles 764, 556; of 1M 190, 148; 2 of 2M 639, 554; 24 of 30k 127, 127.
 constexpr int kDtEntries = 512, kBoundsEntries = 128;
 static_assert(kTile == 256, "the fused batch pair pass runs one 256-thread workgroup per tile");
 
@@ -234,21 +234,9 @@ __global__ __launch_bounds__(kChunkThreads) void kb_bounds(const int *cs, const 
         }
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
-    double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
+    const double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
     __syncthreads();  // lds held the dt fold
-    block_fold<kBoundsVQ>(v, kind, lds);
-    if (threadIdx.x == 0) {
-        unsigned long long *p = part + (size_t)kBoundsVQ * (e < 0 ? ~e : e);
-        v[0] = -v[0];  // minima as maxima
-        v[2] = -v[2];
-        v[4] = -v[4];
-#pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q)
-            if (e >= 0)
-                p[q] = order_key(v[q]);
-            else
-                atomicMax(p + q, order_key(v[q]));
-    }
+    publish_maxima<kBoundsVQ>(v, kind, lds, part + (size_t)kBoundsVQ * (e < 0 ? ~e : e), e < 0);
 }
 
 // _bin :129-141 with the instance's grid; rank by runs as k_keys does. One

@@ -185,14 +185,20 @@ __device__ inline T wave_maxima(T (&m)[P]) {
 
 // Fold NQ (at most 8) quantities over a whole workgroup (up to 16
 // wavefronts). kind: 0 min, 1 max, 2 a count of which only zero or not is
-// kept: all are taken as maxima, inside a wavefront by wave_maxima (as 96 LDS
-// permutes per wavefront they kept a CU's LDS pipe busy for 3 us in the bounds
-// kernels); one LDS round, then wavefront 0
-// folds the wavefronts' values, a group of lanes per quantity. The result is valid
-// in wavefront 0. lds holds P * 16 doubles, P the next of 4 and 8.
+// kept: all are taken as maxima (the minima negated), inside a wavefront by
+// wave_maxima (as 96 LDS permutes per wavefront they kept a CU's LDS pipe busy for 3
+// us in the bounds kernels); one LDS round, then wavefront 0
+// folds the wavefronts' values, a group of lanes per quantity. block_maxima: the
+// maximum of quantity q in the q-th group of fold_lanes lanes of wavefront 0.
+// block_fold: the results in all lanes of wavefront 0. lds holds P * 16 doubles, P
+// the next of 4 and 8.
 template <int NQ>
-__device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double *lds) {
-    constexpr int P = NQ <= 4 ? 4 : 8, L = 64 / P;
+constexpr int fold_lanes() {
+    return NQ <= 4 ? 16 : 8;
+}
+template <int NQ>
+__device__ inline double block_maxima(const double (&v)[NQ], const int (&kind)[NQ], double *lds) {
+    constexpr int P = NQ <= 4 ? 4 : 8, L = fold_lanes<NQ>();
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     double m[P];
 #pragma unroll
@@ -200,15 +206,20 @@ __device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double
     const double top = wave_maxima<P>(m);
     if (lane % L == 0) lds[(lane / L) * 16 + w] = top;
     __syncthreads();
-    if (w != 0) return;
+    if (w != 0) return 0.0;
     double x = -INFINITY;
 #pragma unroll
     for (int u = 0; u < 16; u += L)
         if (u + lane % L < nw) x = max_of(x, lds[(lane / L) * 16 + u + lane % L]);
-    x = group_max<P>(x);
+    return group_max<P>(x);
+}
+template <int NQ>
+__device__ inline void block_fold(double (&v)[NQ], const int (&kind)[NQ], double *lds) {
+    const double x = block_maxima<NQ>(v, kind, lds);
+    if (threadIdx.x >= 64) return;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const double r = lane_value(x, q * L);
+        const double r = lane_value(x, q * fold_lanes<NQ>());
         v[q] = kind[q] == 0 ? -r : r;
     }
 }
@@ -232,6 +243,20 @@ __device__ inline unsigned long long order_key(double x) {
 }
 __device__ inline double order_value(unsigned long long k) {
     return __longlong_as_double((long long)(k ^ ((k >> 63) ? 0x8000000000000000ull : ~0ull)));
+}
+
+// A workgroup's maxima of NQ quantities (block_maxima) as order keys into
+// p[0 .. NQ), or raised there (shared).
+template <int NQ>
+__device__ inline void publish_maxima(const double (&v)[NQ], const int (&kind)[NQ], double *lds, unsigned long long *p,
+                                      bool shared) {
+    const double x = block_maxima<NQ>(v, kind, lds);
+    const int t = threadIdx.x, q = t / fold_lanes<NQ>();
+    if (t >= 64 || t % fold_lanes<NQ>() || q >= NQ) return;
+    if (shared)
+        atomicMax(p + q, order_key(x));
+    else
+        p[q] = order_key(x);
 }
 
 // src/Integrators/PEC.py:32-59 (useXSPH = False branch), one particle. The
@@ -315,17 +340,8 @@ struct DtVars {
     // minimum as a maximum), or into ~e, which other tiles share
     __device__ void publish(unsigned long long *part, int e, double *lds) {
         const int kind[kDtQ] = {0, 1, 2, 2};
-        double v[kDtQ] = {mn, mx, cnt, bad};
-        block_fold<kDtQ>(v, kind, lds);
-        if (threadIdx.x != 0) return;
-        v[0] = -v[0];
-        unsigned long long *p = part + (size_t)kDtQ * (e < 0 ? ~e : e);
-#pragma unroll
-        for (int q = 0; q < kDtQ; ++q)
-            if (e >= 0)
-                p[q] = order_key(v[q]);
-            else
-                atomicMax(p + q, order_key(v[q]));
+        const double v[kDtQ] = {mn, mx, cnt, bad};
+        publish_maxima<kDtQ>(v, kind, lds, part + (size_t)kDtQ * (e < 0 ? ~e : e), e < 0);
     }
     // into the dt slots (one h for every particle: min h is not folded).
     // |a|^2 >= 0 orders as its bits. lds holds 4 * 16 doubles.

@@ -460,17 +460,9 @@ __global__ void k_bounds(Ctrl *ctrl, State a, int n, int pred, HmConst hc, const
         }
     }
     const int kind[kBoundsVQ] = {0, 1, 0, 1, 0, 1, 2, 1};
-    double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
+    const double v[kBoundsVQ] = {xmn, xmx, ymn, ymx, hmn, hmx, bad, vmx};
     __syncthreads();  // lds held the dt fold
-    block_fold<kBoundsVQ>(v, kind, lds);
-    if (threadIdx.x == 0) {
-        unsigned long long *p = bslots + (size_t)(blockIdx.x % kBoundsSlots) * kBoundsStride;
-        v[0] = -v[0];  // minima as maxima
-        v[2] = -v[2];
-        v[4] = -v[4];
-#pragma unroll
-        for (int q = 0; q < kBoundsVQ; ++q) atomicMax(p + q, order_key(v[q]));
-    }
+    publish_maxima<kBoundsVQ>(v, kind, lds, bslots + (size_t)(blockIdx.x % kBoundsSlots) * kBoundsStride, true);
 }
 
 // The indices of a bin that k_keys lists for k_reorder_scan: as many as the
@@ -760,7 +752,7 @@ __global__ void k_reorder(Ctrl *ctrl, ReorderArgs A, const int *perm0) {
 // crowded_ranks counts in a bin of more). The first kReorderShares workgroups
 // write cellStart (scan_share); each of the others scans the bins of its
 // SLOTS slots for itself and sums the counts before them (above kPlainBins bins the
-// tiles' sums: 107k particles on 0.88M cells, an update 66 -> 44 us), with 1,024 threads of
+// tiles' sums: 107k particles on 0.88M cells, an update 66 -> 43 us), with 1,024 threads of
 // which SLOTS carry a slot. Launches, drains and dependent trips to memory are
 // what a small state's update costs: every load is issued in one of two
 // rounds, the bins and states, then the counts and members. Steps in us, with
@@ -780,7 +772,7 @@ constexpr long long kReorderScanCap = 1 << 20;  // most cells
 // particles' bins, kCrowdTile at a time, keeps those in its own crowded bins
 // (a hash table in LDS) and counts among these, its threads sharing each slot.
 // Most of a tile lies in other bins: counting among all of them took a state of
-// 107k particles 1.2 ms, this 60 us.
+// 107k particles 1.2 ms, this 52 us.
 constexpr int kCrowdTile = kScanBins / 2;
 template <int SLOTS>
 __device__ inline int crowded_ranks(int key, int id, int n, const int *bin, const int *ids, int *s_tile) {
