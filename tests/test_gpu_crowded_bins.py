@@ -43,13 +43,18 @@ def test_cells_of_one_metre(dx, far, capacity):
     _check(pA, sc.method(), capacity, 62)
 
 
+@pytest.mark.parametrize('far', [False, True])
 @pytest.mark.parametrize('n', [57344, 57345, 114688, 114689])
-def test_one_crowded_cell(n):
-    """One cell of 400 particles in a dam break."""
+def test_one_crowded_cell(n, far):
+    """One cell of 400 particles in a dam break; far: a wall particle so far
+    away that the grid has about 4 cells per particle."""
     sc = scenarios.dam_break(1.0, 2.0, float(np.sqrt(2.0 / n)), name='wide')
     pA = perturbed(sc.pA, 63)
     pA = pA[np.sort(np.random.default_rng(64).permutation(len(pA))[:n])]
     f = np.nonzero(pA['label'] == 0)[0][:400]
     pA['x'][f] = 0.31 + 1e-5 * np.arange(400)  # 400 particles in one cell
     pA['y'][f] = 0.47 + 1e-5 * (np.arange(400) % 20)
+    if far:
+        cs = 2.0 * pA['h'].min()
+        pA['x'][np.nonzero(pA['label'] != 0)[0][-1]] += 4 * n / np.ceil(np.ptp(pA['y']) / cs) * cs
     _check(pA, sc.method(), 0, 65)
